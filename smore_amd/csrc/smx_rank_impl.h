@@ -300,6 +300,12 @@ __device__ __forceinline__ void add_step(float& total, float& err, float step) {
   err += step - (t - total);
   total = t;
 }
+// The sum with its error.  Past fp32 the error is a difference of infinities: the total alone then is what a plain sum
+// would be (a diverged row scores -inf and ranks last, it does not turn into a NaN above every logit).
+__device__ __forceinline__ float with_error(float total, float err) {
+#pragma clang fp contract(off)
+  return __builtin_isfinite(total) ? total + err : total;
+}
 __device__ __forceinline__ float beta_eighths(const float (&x)[8]) {
 #pragma clang fp contract(off)
   return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
@@ -411,9 +417,9 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
     if (M == mBox && k.fast_box) sums(std::integral_constant<bool, M == mBox>{});   // uniform
     else sums(std::false_type{});
 #pragma unroll
-    for (int i = 0; i < O::kSums; ++i) tot[i] += err[i];
+    for (int i = 0; i < O::kSums; ++i) tot[i] = with_error(tot[i], err[i]);
 #pragma unroll
-    for (int i = 0; i < NS; ++i) rtot[i] += rerr[i];
+    for (int i = 0; i < NS; ++i) rtot[i] = with_error(rtot[i], rerr[i]);
     const float su = O::score(tot, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), k, A.p);
     if (u == 0 || union_takes(su, best)) best = su;
   }
@@ -644,7 +650,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       const unsigned long long id = (unsigned long long)g * kScanRows + lane + 64 * r;
       float rsum[NS];
 #pragma unroll
-      for (int i = 0; i < NS; ++i) rsum[i] = rtot[r][i] + rerr[r][i];
+      for (int i = 0; i < NS; ++i) rsum[i] = with_error(rtot[r][i], rerr[r][i]);
 #pragma unroll
       for (int l = 0; l < NL; ++l) {
         float s = 0.f;
@@ -652,7 +658,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
         for (int u = 0; u < UP; ++u) {
           float sum[O::kSums];
 #pragma unroll
-          for (int i = 0; i < O::kSums; ++i) sum[i] = tot[l * UP + u][r][i] + err[l * UP + u][r][i];
+          for (int i = 0; i < O::kSums; ++i) sum[i] = with_error(tot[l * UP + u][r][i], err[l * UP + u][r][i]);
           const float su = O::score(sum, rsum, row_const[r], qc[l * UP + u], k, A.p);
           if (u == 0 || union_takes(su, s)) s = su;
         }

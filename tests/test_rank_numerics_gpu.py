@@ -1,0 +1,86 @@
+"""All-entity ranking: values that are not finite, keys from elsewhere, rows that occur twice, and the rounding error of the
+scores against that of the scoring kernels (a row per wavefront, summed as a tree)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+GAMMA = {"l1": 24.0, "l2": 12.0, "box": 24.0, "rotate": 9.0, "beta_kl": 60.0, "complex": 0.0, "distmult": 0.0}
+TWO_HALVES = ("rotate", "beta_kl", "complex")
+ONE_QUERY = ("l1", "l2", "distmult")
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
+
+
+def _row(model, dim):
+    return dim * (2 if model in TWO_HALVES else 1)
+
+
+def _keys(model, table, q1, q2, params, ids, branches=1):
+    """smx_rank_answer_keys_union on the device ids [B, A]: scores and keys (as signed 64-bit)."""
+    from smore_amd import _lib
+    from smore_amd.fused import MODELS
+    b, a = ids.shape
+    counts = torch.full((b,), a, dtype=torch.int32, device="cuda")
+    keys, scores = torch.empty((b, a), dtype=torch.int64, device="cuda"), torch.empty((b, a), device="cuda")
+    _lib.call("smx_rank_answer_keys_union", MODELS[model], None, _ptr(table), table.shape[0], _ptr(q1), _ptr(q2), b, branches,
+              q1.shape[-1], ctypes.byref(params), _ptr(ids), _ptr(counts), a, _ptr(scores), _ptr(keys))
+    return scores, keys
+
+
+def _scan(model, table, q1, q2, params, ids, keys, branches=1):
+    """smx_rank_scan_union with the keys given, in the slots of `ids`."""
+    from smore_amd import _lib
+    from smore_amd.fused import MODELS
+    b, a = ids.shape
+    counts = torch.full((b,), a, dtype=torch.int32, device="cuda")
+    order = torch.argsort(keys ^ -(1 << 63), dim=1, descending=True, stable=True)
+    ids_s, keys_s = torch.gather(ids, 1, order).contiguous(), torch.gather(keys, 1, order).contiguous()
+    ranks = torch.empty((b, a), dtype=torch.int64, device="cuda")
+    ws = torch.empty(_lib.load().smx_rank_workspace_bytes(b, a), dtype=torch.uint8, device="cuda")
+    _lib.call("smx_rank_scan_union", MODELS[model], None, _ptr(table), table.shape[0], _ptr(q1), _ptr(q2), b, branches,
+              q1.shape[-1], ctypes.byref(params), _ptr(ids_s), _ptr(keys_s), _ptr(counts), a, _ptr(ranks), _ptr(ws), ws.numel())
+    return torch.empty_like(ranks).scatter_(1, order, ranks)
+
+
+def _all_ids(b, n):
+    return torch.arange(n, device="cuda").expand(b, n).contiguous()
+
+
+@pytest.mark.parametrize("model", ["l1", "l2", "box", "rotate", "complex", "distmult"])
+@pytest.mark.parametrize("b,dim", [(1, 100), (5, 36), (5, 33)])
+def test_rows_that_are_not_finite_rank_where_the_scoring_kernels_put_them(model, b, dim):
+    """A diverged row (an infinite feature, sums or squares beyond fp32) scores -inf or +inf, not NaN: it must not move the
+    ranks of the others.  Integer coordinates elsewhere: every finite sum is exact."""
+    from smore_amd import fused
+    from smore_amd.evaluation import filtered_ranks
+    rng = np.random.default_rng(dim)
+    n = 300
+    table = rng.integers(-3, 4, (n, _row(model, dim))).astype(np.float32)
+    q1 = rng.integers(1, 4, (b, dim)).astype(np.float32)
+    q2 = None if model in ONE_QUERY else rng.integers(1, 4, (b, dim)).astype(np.float32)
+    table[3, 5], table[130, dim - 1], table[131, 0] = np.inf, -np.inf, 1e38
+    if model in ("l1", "l2", "box", "rotate"):
+        table[7], table[299] = 3e38, -1e30
+    t, a, c = (None if x is None else torch.tensor(x, device="cuda") for x in (table, q1, q2))
+    params = fused.score_params(GAMMA[model], 0.5 if model == "box" else 0.0)
+    want = fused.score_forward(model, t, _all_ids(b, n), a, c, params)
+    got, _ = _keys(model, t, a, c, params, _all_ids(b, n))
+    assert not want.isnan().any() and int(want.isinf().sum()) >= b
+    assert torch.equal(got.isinf(), want.isinf()) and not got.isnan().any()
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    answers = [rng.choice(n, size=9, replace=False).tolist() + [3] for _ in range(b)]
+    answers = [list(dict.fromkeys(x)) for x in answers]
+    ranks = filtered_ranks(model, t, a, c, params, [x[:4] for x in answers], [x[4:] for x in answers])
+    # (rotate: irrational sums, the order of two rows within rounding is either kernel's own)
+    scores = (got if model == "rotate" else want).cpu().numpy().astype(np.float64)
+    for i in range(b):
+        want_h, want_e = orc.filtered_ranks(scores[i], answers[i][:4], answers[i][4:])
+        assert ranks[i][0].tolist() == want_h.tolist() and ranks[i][1].tolist() == want_e.tolist()
