@@ -490,7 +490,7 @@ int smx_rank_candidates_union(int model, void* stream, const float* table, size_
 /* Filtered ranks in one call: smx_rank_answer_keys, the answers' order, smx_rank_scan, and the ranks back in the slots
  * the answers were given in (filtered_rank [B, A], 0 in unused slots).  U branch rows per query (1: plain queries).
  * ans_id need not be sorted; ans_score [B, A] may be NULL.  The same ranks as the two calls with a sort between them,
- * without that sort's launches, and the box model's offsets are scaled once per call.
+ * without that sort's launches.
  * workspace: smx_filtered_ranks_workspace_bytes(model, B, U, A, dim), 256-byte aligned. */
 size_t smx_filtered_ranks_workspace_bytes(int model, size_t B, size_t U, size_t A, size_t dim);
 int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_rows, const float* q1, const float* q2,

@@ -16,18 +16,17 @@ constexpr size_t kRankMaxAnswers = 2048;  // per query; bins and keys of a pass 
 
 static size_t rank_ws_bytes(size_t B, size_t A) { return (B * (A + 1) * sizeof(unsigned) + 255) & ~(size_t)255; }
 
-// smx_filtered_ranks: bins | keys | keys in order | their slots | scaled offsets (box)
+// smx_filtered_ranks: bins | keys | keys in order | their slots
 struct RanksWs {
-  size_t key, sorted, slot, offsets, bytes;
+  size_t key, sorted, slot, bytes;
 };
-static RanksWs ranks_ws(int model, size_t B, size_t U, size_t A, size_t dim) {
+static RanksWs ranks_ws(size_t B, size_t A) {
   auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
   RanksWs w;
   w.key = rank_ws_bytes(B, A);
   w.sorted = w.key + up(B * A * sizeof(unsigned long long));
   w.slot = w.sorted + up(B * A * sizeof(unsigned long long));
-  w.offsets = w.slot + up(B * A * sizeof(int));
-  w.bytes = w.offsets + (model == mBox ? up(B * U * dim * sizeof(float)) : 0);
+  w.bytes = w.slot + up(B * A * sizeof(int));
   return w;
 }
 
@@ -131,8 +130,8 @@ int smx_rank_scan_union(int model, void* stream, const float* table, size_t n_ro
   return rank_run(model, as_stream(stream), R, vec, nit, kRankScan);
 }
 
-size_t smx_filtered_ranks_workspace_bytes(int model, size_t B, size_t U, size_t A, size_t dim) {
-  return smx::ranks_ws(model, B, U, A, dim).bytes;
+size_t smx_filtered_ranks_workspace_bytes(int, size_t B, size_t, size_t A, size_t) {
+  return smx::ranks_ws(B, A).bytes;
 }
 
 int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_rows, const float* q1, const float* q2,
@@ -145,7 +144,7 @@ int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_row
   if (int rc = rank_common(&R, &vec, &nit, model, table, n_rows, q1, q2, B, U, dim, params, ans_id, ans_count, A)) return rc;
   if (!filtered_rank || !workspace) return fail(SMX_ERR_ARG, "null pointer");
   if (int rc = scan_branches(model, nit, U)) return rc;
-  const RanksWs ws = ranks_ws(model, B, U, A, dim);
+  const RanksWs ws = ranks_ws(B, A);
   if (workspace_bytes < ws.bytes) return fail(SMX_ERR_WORKSPACE, "rank workspace too small: %zu < %zu", workspace_bytes, ws.bytes);
   hipStream_t st = as_stream(stream);
   char* base = static_cast<char*>(workspace);
@@ -156,11 +155,8 @@ int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_row
   R.key_out = key;
   if (int rc = rank_run(model, st, R, vec, nit, kRankKeys)) return rc;
   R.bins = reinterpret_cast<unsigned*>(base);
-  float* offsets = rank_scales_offsets(model, R.p.cen) ? reinterpret_cast<float*>(base + ws.offsets) : nullptr;
-  hipLaunchKernelGGL(rank_prepare_kernel, dim3((unsigned)B), dim3(256), A * sizeof(unsigned long long), st, R, sorted, slot,
-                     offsets);
+  hipLaunchKernelGGL(rank_prepare_kernel, dim3((unsigned)B), dim3(256), A * sizeof(unsigned long long), st, R, sorted, slot);
   if (int rc = check_launch("rank preparation")) return rc;
-  R.offsets = offsets;
   R.ans_key = sorted;
   R.slot = slot;
   R.rank_out = reinterpret_cast<long long*>(filtered_rank);

@@ -45,7 +45,6 @@ struct RankArgs {
   int first_list;                    // query of the launch's first list of answers
   long long* rank_out;               // [B, A]
   const int* slot;                   // [B, A] slot of the j-th key in the order the answers were given in, or null
-  const float* offsets;              // [B * U, dim] the box model's offsets as the scan's inner loop takes them, or null
   // ranking among sampled candidates (rank_candidates_kernel)
   const long long* cand;             // [B, C], -1 = padding
   int C, H;
@@ -57,9 +56,6 @@ struct RankArgs {
 };
 
 enum RankMode : int { kRankScan = 0, kRankKeys = 1, kRankCandidates = 2 };
-
-// the box model's offsets are scaled once per call instead of once per (row, query): see ScanOps
-__host__ __device__ inline bool rank_scales_offsets(int model, float cen) { return model == mBox && cen > 0.f && cen <= 1.f; }
 
 __device__ __forceinline__ unsigned sortable_bits(float s) {
   const unsigned u = __float_as_uint(s);
@@ -168,10 +164,10 @@ __device__ __forceinline__ void load_rank_query(const float* __restrict__ q1, co
 // owns two of the rows and sums their scores feature by feature, a wavefront does so for NB query rows of its own whose
 // values are scalars.  Every lane then works on every feature (a row spread over the lanes leaves 22 % of them without
 // a column at 400 floats), nothing is summed across lanes, and the table crosses the fabric once per sixteen queries.
-// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, multiply-add, maximum, add (and half an
-// instruction that scales the offset where the call has not done so beforehand).  1 M x 400 rows, 16 queries: 0.64 ms,
-// the 25.6 G operations at the issue rate of 39 T lanes/s (a row per wavefront, a pass per four queries, five operations
-// and two cross-lane reductions per row and query: 1.64 ms).
+// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, minimum, subtract, add, multiply-add.
+// (Four operations would do: out + cen * in over cen is max(|d|, |d| / cen - o (1 - cen) / cen) for 0 < cen <= 1, 0.64 ms.
+// But that rounds values up to 1 / cen times larger than the result: 84 times the error where distances are near the
+// offsets, D = 400, cen = 0.02, twice the error elsewhere.)
 // The sums of a step (32 features, 16 of two-halves models, 8 of BetaE) are added to the row's total with the rounding
 // error carried along, so the long serial sum is no less accurate than the tree over lanes that it replaces.
 constexpr int kScanRows = 128;
@@ -188,41 +184,13 @@ __device__ __forceinline__ ScalarRow scalar_row(const float* p) {
 //   kGroup  groups of values a feature has in LDS: 1 (e), 2 (first, second half), 4 (BetaE: ea, eb, psi(ea) - psi(se),
 //           psi(eb) - psi(se), evaluated once per row for all queries)
 //   kSums   sums per (row, query);  kRowSums  sums per row
-struct ScanConst {
-  int fast_box;      // 0 < cen <= 1
-  float inv_cen, out_pos, out_neg;
-};
-__device__ __forceinline__ ScanConst scan_const(const ScoreParams& p) {
-#pragma clang fp contract(off)
-  ScanConst c;
-  c.fast_box = rank_scales_offsets(mBox, p.cen);
-  c.inv_cen = 1.f / p.cen;
-  c.out_pos = -(1.f - p.cen) / p.cen;   // factor of a non-negative offset, and of a negative one
-  c.out_neg = -(1.f + p.cen) / p.cen;
-  return c;
-}
-
 template <int M, bool NORM> struct ScanOps {
   static constexpr int kGroup = M == mBetaKL ? 4 : model_mul(M);
   static constexpr int kFeat = 32 / kGroup;   // features per step
   static constexpr int kSums = NORM ? model_mul(M) : 1;
   static constexpr int kRowSums = NORM ? model_mul(M) : 0;
 
-  // FAST (box with 0 < cen <= 1):  out + cen * in  over  cen  is
-  //   max(|d|, |d| / cen + o')   with  o' = -o (1 - cen) / cen   (o < 0: -o (1 + cen) / cen),
-  // since out = max(|d| - o, 0) and in = min(|d|, o) for o >= 0 (o < 0: out = |d| - o, in = |o|).  scaled_offset is
-  // the first form of o', which is the larger of the two for o >= 0; negative_offset takes the larger.
-  static __device__ __forceinline__ float scaled_offset(float b, const ScanConst& k) {
-#pragma clang fp contract(off)
-    return b * k.out_pos;
-  }
-  static __device__ __forceinline__ float negative_offset(float scaled, float b, const ScanConst& k) {
-#pragma clang fp contract(off)
-    return fmaxf(scaled, b * k.out_neg);
-  }
-  template <bool FAST>
-  static __device__ __forceinline__ void add(const float (&e)[kGroup], float a, float b, const ScanConst& k, float cen,
-                                             float (&s)[kSums]) {
+  static __device__ __forceinline__ void add(const float (&e)[kGroup], float a, float b, float cen, float (&s)[kSums]) {
 #pragma clang fp contract(off)
     if constexpr (M == mL1) {
       s[0] += fabsf(e[0] - a);
@@ -231,13 +199,9 @@ template <int M, bool NORM> struct ScanOps {
       s[0] = __builtin_fmaf(d, d, s[0]);
     } else if constexpr (M == mBox) {
       const float d = e[0] - a;
-      if constexpr (FAST) {
-        s[0] += fmaxf(fabsf(d), __builtin_fmaf(fabsf(d), k.inv_cen, b));
-      } else {
-        const float mn = ModelOps<mBox>::min_abs(d, b);
-        s[0] += fabsf(d) - mn;
-        s[0] = __builtin_fmaf(fabsf(mn), cen, s[0]);
-      }
+      const float mn = ModelOps<mBox>::min_abs(d, b);
+      s[0] += fabsf(d) - mn;
+      s[0] = __builtin_fmaf(fabsf(mn), cen, s[0]);
     } else if constexpr (M == mRotate) {
       const float x = e[0] - a, y = e[1] - b;
       s[0] += __builtin_amdgcn_sqrtf(__builtin_fmaf(y, y, __builtin_fmaf(x, x, 1e-20f)));
@@ -260,11 +224,9 @@ template <int M, bool NORM> struct ScanOps {
   // logit from the sums; row_const: BetaE's sum over the row of lgamma(se) - lgamma(ea) - lgamma(eb), query_const: the
   // same of the query with the other sign
   static __device__ __forceinline__ float score(const float (&s)[kSums], const float (&r)[kRowSums > 0 ? kRowSums : 1],
-                                                float row_const, float query_const, const ScanConst& k,
-                                                const ScoreParams& p) {
+                                                float row_const, float query_const, const ScoreParams& p) {
 #pragma clang fp contract(off)
     if constexpr (M == mL2) return p.gamma - __builtin_amdgcn_sqrtf(s[0]);
-    else if constexpr (M == mBox) return k.fast_box ? __builtin_fmaf(-p.cen, s[0], p.gamma) : p.gamma - s[0];
     else if constexpr (M == mBetaKL) return p.gamma - (s[0] + (row_const + query_const));
     else if constexpr (M == mComplex || M == mDistmult) {
       float dot = NORM ? s[0] * inv_norm(r[0]) : s[0];
@@ -337,7 +299,6 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
   unsigned long long id = valid ? (unsigned long long)A.ans_id[(size_t)b * A.A + j] : 0ull;
   if (id >= A.n_rows) id = 0;  // the host wrapper has already refused such ids
   const float* row = A.table + id * (size_t)dim * model_mul(M);
-  const ScanConst k = scan_const(A.p);
   float best = 0.f;
   for (int u = 0; u < A.U; ++u) {  // uniform
     const int bq = b * A.U + u;
@@ -372,8 +333,7 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
         }
       }
     };
-    auto sums = [&](auto fast_tag) {
-      constexpr bool FAST = decltype(fast_tag)::value;
+    {
       request(0);
       for (int d0 = 0; d0 < dim; d0 += F) {
 #pragma unroll
@@ -390,8 +350,7 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
           float e[O::kGroup];
           const float l = O::expand(now[0][f], now[MUL - 1][f], A.p, e);
           if constexpr (M == mBetaKL) lb[f & 7] += l;
-          if constexpr (FAST) qb = O::negative_offset(O::scaled_offset(qb, k), qb, k);
-          O::template add<FAST>(e, qa, qb, k, A.p.cen, s);
+          O::add(e, qa, qb, A.p.cen, s);
           O::add_row(e, r);
         };
         if (d0 + F <= dim) {   // (uniform) the query's values of the step in a few wide scalar loads
@@ -413,14 +372,12 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
 #pragma unroll
         for (int i = 0; i < NS; ++i) add_step(rtot[i], rerr[i], r[i]);
       }
-    };
-    if (M == mBox && k.fast_box) sums(std::integral_constant<bool, M == mBox>{});   // uniform
-    else sums(std::false_type{});
+    }
 #pragma unroll
     for (int i = 0; i < O::kSums; ++i) tot[i] = with_error(tot[i], err[i]);
 #pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = with_error(rtot[i], rerr[i]);
-    const float su = O::score(tot, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), k, A.p);
+    const float su = O::score(tot, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), A.p);
     if (u == 0 || union_takes(su, best)) best = su;
   }
   if (j < A.A) {
@@ -448,7 +405,6 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
   const int block_list = A.first_list + (int)blockIdx.y * 4 * NL;
   const int first_list = block_list + wave * NL;   // this wavefront's lists of answers
   const bool active = first_list < A.B;
-  const ScanConst k = scan_const(A.p);
   if (A.lds_bins) {
     for (int i = t; i < 4 * NL * A1; i += kScanThreads) lds_bins[i] = 0u;
     __syncthreads();
@@ -460,7 +416,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
     const int b = min(first_list + x / UP, A.B - 1);   // a list past the last query repeats it and is not counted
     const int bq = b * A.U + min(x % UP, A.U - 1);
     q1[x] = scalar_row(A.q1 + (size_t)bq * dim);
-    q2[x] = scalar_row(model_nq(M) == 2 ? (M == mBox && A.offsets ? A.offsets : A.q2) + (size_t)bq * dim : A.q1);
+    q2[x] = scalar_row(model_nq(M) == 2 ? A.q2 + (size_t)bq * dim : A.q1);
     qc[x] = active ? query_const<M>(A, bq, dim, lane) : 0.f;
   }
 
@@ -512,20 +468,15 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
 
   float tot[NB][R][O::kSums], err[NB][R][O::kSums], rtot[R][NS], rerr[R][NS];
   // N features (4 or 1) of the staged step, from feature f on
-  // (form: 0 plain, 1 the box's fast form, 2 the same with the offsets scaled beforehand)
-  auto features = [&](auto form_tag, auto n_tag, const float* from, int d0, int f, float (&s)[NB][R][O::kSums], float (&rs)[R][NS]) {
-    constexpr int FORM = decltype(form_tag)::value;
-    constexpr bool FAST = FORM != 0;
+  auto features = [&](auto n_tag, const float* from, int d0, int f, float (&s)[NB][R][O::kSums], float (&rs)[R][NS]) {
     constexpr int N = decltype(n_tag)::value;
     float a[NB][N], b[NB][N], e[R][N][G];
-    bool negative = false;
 #pragma unroll
     for (int x = 0; x < NB; ++x)
 #pragma unroll
       for (int v = 0; v < N; ++v) {
         a[x][v] = q1[x][d0 + f + v];
         b[x][v] = model_nq(M) == 2 ? (float)q2[x][d0 + f + v] : 0.f;
-        if constexpr (FORM == 1) negative |= (int)__float_as_uint(b[x][v]) < 0;
       }
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -539,28 +490,12 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
           e[r][0][x] = at[0];
         }
       }
-    if constexpr (FORM == 1) {
-      float raw[NB][N];
-#pragma unroll
-      for (int x = 0; x < NB; ++x)
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          raw[x][v] = b[x][v];
-          b[x][v] = O::scaled_offset(raw[x][v], k);
-        }
-      if (negative) {   // uniform, and not in a trained box
-#pragma unroll
-        for (int x = 0; x < NB; ++x)
-#pragma unroll
-          for (int v = 0; v < N; ++v) b[x][v] = O::negative_offset(b[x][v], raw[x][v], k);
-      }
-    }
 #pragma unroll
     for (int v = 0; v < N; ++v)
 #pragma unroll
       for (int r = 0; r < R; ++r) {
 #pragma unroll
-        for (int x = 0; x < NB; ++x) O::template add<FAST>(e[r][v], a[x][v], b[x][v], k, A.p.cen, s[x][r]);
+        for (int x = 0; x < NB; ++x) O::add(e[r][v], a[x][v], b[x][v], A.p.cen, s[x][r]);
         O::add_row(e[r][v], rs[r]);
       }
   };
@@ -576,18 +511,9 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       for (int i = 0; i < NS; ++i) rs[r][i] = 0.f;
     }
     const int n = min(F, dim - d0);
-    auto walk = [&](auto form_tag) {
-      int f = 0;
-      for (; f + 4 <= n; f += 4) features(form_tag, std::integral_constant<int, 4>{}, from, d0, f, s, rs);
-      for (; f < n; ++f) features(form_tag, std::integral_constant<int, 1>{}, from, d0, f, s, rs);
-    };
-    if constexpr (M == mBox) {   // (uniform)
-      if (A.offsets) walk(std::integral_constant<int, 2>{});
-      else if (k.fast_box) walk(std::integral_constant<int, 1>{});
-      else walk(std::integral_constant<int, 0>{});
-    } else {
-      walk(std::integral_constant<int, 0>{});
-    }
+    int f = 0;
+    for (; f + 4 <= n; f += 4) features(std::integral_constant<int, 4>{}, from, d0, f, s, rs);
+    for (; f < n; ++f) features(std::integral_constant<int, 1>{}, from, d0, f, s, rs);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
@@ -659,7 +585,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
           float sum[O::kSums];
 #pragma unroll
           for (int i = 0; i < O::kSums; ++i) sum[i] = with_error(tot[l * UP + u][r][i], err[l * UP + u][r][i]);
-          const float su = O::score(sum, rsum, row_const[r], qc[l * UP + u], k, A.p);
+          const float su = O::score(sum, rsum, row_const[r], qc[l * UP + u], A.p);
           if (u == 0 || union_takes(su, s)) s = su;
         }
         const int b = first_list + l;
@@ -851,22 +777,13 @@ static __global__ __launch_bounds__(64) void rank_finish_kernel(RankArgs A) {
 }
 
 // One workgroup per query, everything the scan needs beside the keys: the keys in descending order with the slot each
-// came from (unused slots have key 0 and go last), the query's bins cleared, its offsets scaled (box).
-static __global__ __launch_bounds__(256) void rank_prepare_kernel(RankArgs A, unsigned long long* sorted, int* slot,
-                                                                  float* offsets) {
+// came from (unused slots have key 0 and go last), the query's bins cleared.
+static __global__ __launch_bounds__(256) void rank_prepare_kernel(RankArgs A, unsigned long long* sorted, int* slot) {
   extern __shared__ unsigned long long sort_keys[];
   const int n = A.A, b = blockIdx.x;
   const size_t base = (size_t)b * n;
   for (int i = threadIdx.x; i < n; i += 256) sort_keys[i] = A.key_out[base + i];
   for (int i = threadIdx.x; i <= n; i += 256) A.bins[(size_t)b * (n + 1) + i] = 0u;
-  if (offsets) {
-    const ScanConst k = scan_const(A.p);
-    const size_t first = (size_t)b * A.U * A.dim;
-    for (int i = threadIdx.x; i < A.U * A.dim; i += 256) {
-      const float o = A.q2[first + i];
-      offsets[first + i] = ScanOps<mBox, false>::negative_offset(ScanOps<mBox, false>::scaled_offset(o, k), o, k);
-    }
-  }
   __syncthreads();
   for (int j = threadIdx.x; j < n; j += 256) {
     const unsigned long long mine = sort_keys[j];

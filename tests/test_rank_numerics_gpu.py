@@ -84,3 +84,36 @@ def test_rows_that_are_not_finite_rank_where_the_scoring_kernels_put_them(model,
     for i in range(b):
         want_h, want_e = orc.filtered_ranks(scores[i], answers[i][:4], answers[i][4:])
         assert ranks[i][0].tolist() == want_h.tolist() and ranks[i][1].tolist() == want_e.tolist()
+
+
+def _rms(x):
+    return float(np.sqrt(np.mean(np.square(x))))
+
+
+@pytest.mark.parametrize("dim", [100, 400])
+def test_box_scores_keep_their_digits_where_distances_are_near_the_offsets(dim):
+    """Outside distances near zero: |d| - offset is exact there, and what a form that scales it by 1 / cen rounds away is
+    1 / cen times larger.  Bound: up to 64 additions one after another round by sqrt(64 / 3) x 2^-24 / sqrt(3) of the sum,
+    2.7 x 2^-24."""
+    from smore_amd import fused
+    rng = np.random.default_rng(dim)
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    n, b, cen = 1500, 3, float(np.float32(0.02))
+    table = f32(rng.choice([-1.0, 1.0], (n, dim)) * 0.05 * (1 + 0.01 * rng.random((n, dim))))
+    q1, q2 = np.zeros((b, dim)), f32(0.05 * (1 + 0.001 * rng.random((b, dim))))
+    want = orc.score_forward("box", np.broadcast_to(table[None], (b, n, dim)), q1[:, None], q2[:, None], 0.0, cen)
+    t, a, c = (torch.tensor(x, dtype=torch.float32, device="cuda") for x in (table, q1, q2))
+    got, _ = _keys("box", t, a, c, fused.score_params(0.0, cen), _all_ids(b, n))
+    assert _rms(got.cpu().numpy() - want) <= 4 * 2.0 ** -24 * _rms(want)
+
+
+def test_box_scores_with_a_weight_too_small_to_invert():
+    from smore_amd import fused
+    rng = np.random.default_rng(0)
+    n, b, dim = 200, 2, 40
+    table, q1 = rng.integers(-3, 4, (n, dim)).astype(np.float32), rng.integers(-3, 4, (b, dim)).astype(np.float32)
+    q2 = rng.integers(0, 3, (b, dim)).astype(np.float32)
+    want = -np.maximum(np.abs(table[None] - q1[:, None]) - q2[:, None], 0).sum(axis=-1)
+    t, a, c = (torch.tensor(x, device="cuda") for x in (table, q1, q2))
+    got, _ = _keys("box", t, a, c, fused.score_params(0.0, 1e-40), _all_ids(b, n))
+    assert np.array_equal(got.cpu().numpy(), want)
