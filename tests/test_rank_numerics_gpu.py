@@ -117,3 +117,25 @@ def test_box_scores_with_a_weight_too_small_to_invert():
     t, a, c = (torch.tensor(x, device="cuda") for x in (table, q1, q2))
     got, _ = _keys("box", t, a, c, fused.score_params(0.0, 1e-40), _all_ids(b, n))
     assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("model", ["l1", "l2", "box", "rotate", "complex", "distmult", "complex_norm", "distmult_norm"])
+@pytest.mark.parametrize("dim", [12, 33, 100, 255, 400])
+def test_scores_round_no_worse_than_those_of_the_scoring_kernels(model, dim):
+    """The scan sums a row feature by feature in one lane, the scoring kernels as a tree over a wavefront: error against
+    float64, a tenth for the spread of two samples of a few thousand logits."""
+    from smore_amd import fused
+    rng = np.random.default_rng(dim)
+    model, norm = model.removesuffix("_norm"), model.endswith("_norm")
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    n, b, cen = 1500, 4, float(np.float32(0.02))
+    r = 26.0 / dim
+    table, q1 = f32(rng.uniform(-r, r, (n, _row(model, dim)))), f32(rng.uniform(-r, r, (b, dim)))
+    q2 = None if model in ONE_QUERY else f32(rng.uniform(0 if model == "box" else -r, r, (b, dim)))
+    want = orc.score_forward(model, np.broadcast_to(table[None], (b,) + table.shape), q1[:, None],
+                             None if q2 is None else q2[:, None], 0.0, cen, norm=norm)
+    t, a, c = (None if x is None else torch.tensor(x, dtype=torch.float32, device="cuda") for x in (table, q1, q2))
+    params = fused.score_params(0.0, cen if model == "box" else 0.0, norm=norm)
+    scan, _ = _keys(model, t, a, c, params, _all_ids(b, n))
+    tree = fused.score_forward(model, t, _all_ids(b, n), a, c, params)
+    assert _rms(scan.cpu().numpy() - want) <= 1.1 * _rms(tree.cpu().numpy() - want)
