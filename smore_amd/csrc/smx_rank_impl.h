@@ -186,6 +186,25 @@ __device__ __forceinline__ ScalarRow scalar_row(const float* p) {
 //   kGroup  groups of values a feature has in LDS: 1 (e), 2 (first, second half), 4 (BetaE: ea, eb, psi(ea) - psi(se),
 //           psi(eb) - psi(se), evaluated once per row for all queries)
 //   kSums   sums per (row, query);  kRowSums  sums per row
+// BetaE's log-Beta terms depend on the row or on the query alone; a divergence is what is left when they and the sum over
+// psi cancel, digits that its fp32 sums would round away.  They are summed, and the three parts added, in 64 bits: once
+// per row, once per query, three additions per pair.  log_beta: with what the rounding of ea + eb changes in lgamma(ea + eb)
+// (the pair's sum is over ea and eb themselves, not over that rounded value).
+__device__ __forceinline__ double log_beta(float a, float b, float& pa, float& pb, float& ps) {
+#pragma clang fp contract(off)
+  float lb;
+  beta_terms(a, b, lb, pa, pb, ps);
+  const float sum = a + b, from_b = sum - a;
+  const float rest = (a - (sum - from_b)) + (b - from_b);   // a + b = sum + rest
+  return (double)lb + (double)(rest * ps);
+}
+// The sum with its error.  Past fp32 the error is a difference of infinities: the total alone then is what a plain sum
+// would be (a diverged row scores -inf and ranks last, it does not turn into a NaN above every logit).
+__device__ __forceinline__ float with_error(float total, float err) {
+#pragma clang fp contract(off)
+  return __builtin_isfinite(total) ? total + err : total;
+}
+
 template <int M, bool NORM> struct ScanOps {
   static constexpr int kGroup = M == mBetaKL ? 4 : model_mul(M);
   static constexpr int kFeat = 32 / kGroup;   // features per step
@@ -242,13 +261,20 @@ template <int M, bool NORM> struct ScanOps {
       s[0] = 0.f;
     }
   }
-  // logit from the sums; row_const: BetaE's sum over the row of lgamma(se) - lgamma(ea) - lgamma(eb), query_const: the
-  // same of the query with the other sign
-  static __device__ __forceinline__ float score(const float (&s)[kSums], const float (&r)[kRowSums > 0 ? kRowSums : 1],
-                                                float row_const, float query_const, const ScoreParams& p) {
+  // logit from the sums and their errors; row_const: BetaE's sum over the row of lgamma(se) - lgamma(ea) - lgamma(eb),
+  // query_const: the same of the query with the other sign
+  static __device__ __forceinline__ float score(const float (&total)[kSums], const float (&err)[kSums],
+                                                const float (&r)[kRowSums > 0 ? kRowSums : 1], double row_const,
+                                                double query_const, const ScoreParams& p) {
 #pragma clang fp contract(off)
+    if constexpr (M == mBetaKL) {
+      const double sum = __builtin_isfinite(total[0]) ? (double)total[0] + (double)err[0] : (double)total[0];
+      return p.gamma - (float)(sum + (row_const + query_const));
+    }
+    float s[kSums];
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) s[i] = with_error(total[i], err[i]);
     if constexpr (M == mL2) return p.gamma - __builtin_amdgcn_sqrtf(s[0]);
-    else if constexpr (M == mBetaKL) return p.gamma - (s[0] + (row_const + query_const));
     else if constexpr (M == mComplex || M == mDistmult) {
       float dot = NORM ? s[0] * inv_norm(r[0]) : s[0];
       if constexpr (NORM && kSums == 2) dot += s[1] * inv_norm(r[1]);
@@ -258,20 +284,20 @@ template <int M, bool NORM> struct ScanOps {
     }
   }
   // a feature's values in LDS from the row's (regularized) values; returns BetaE's log-Beta term
-  static __device__ __forceinline__ float expand(float x1, float x2, const ScoreParams& p, float (&e)[kGroup]) {
+  static __device__ __forceinline__ double expand(float x1, float x2, const ScoreParams& p, float (&e)[kGroup]) {
 #pragma clang fp contract(off)
     if constexpr (M == mBetaKL) {
-      float lb, pa, pb, ps;
+      float pa, pb, ps;
       e[0] = reg_apply(x1, p);
       e[1] = reg_apply(x2, p);
-      beta_terms(e[0], e[1], lb, pa, pb, ps);
+      const double lb = log_beta(e[0], e[1], pa, pb, ps);
       e[2] = pa - ps;
       e[3] = pb - ps;
       return lb;
     } else {
       e[0] = x1;
       if constexpr (kGroup == 2) e[1] = x2;
-      return 0.f;
+      return 0.0;
     }
   }
 };
@@ -283,28 +309,21 @@ __device__ __forceinline__ void add_step(float& total, float& err, float step) {
   err += step - (t - total);
   total = t;
 }
-// The sum with its error.  Past fp32 the error is a difference of infinities: the total alone then is what a plain sum
-// would be (a diverged row scores -inf and ranks last, it does not turn into a NaN above every logit).
-__device__ __forceinline__ float with_error(float total, float err) {
-#pragma clang fp contract(off)
-  return __builtin_isfinite(total) ? total + err : total;
-}
-__device__ __forceinline__ float beta_eighths(const float (&x)[8]) {
-#pragma clang fp contract(off)
+__device__ __forceinline__ double beta_eighths(const double (&x)[8]) {
   return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
 }
 // BetaE: minus the log-Beta terms of query row bq, summed by a whole wavefront
 template <int M>
-__device__ __forceinline__ float query_const(const RankArgs& A, int bq, int dim, int lane) {
-#pragma clang fp contract(off)
-  if constexpr (M != mBetaKL) return 0.f;
-  float mine = 0.f;
+__device__ __forceinline__ double query_const(const RankArgs& A, int bq, int dim, int lane) {
+  if constexpr (M != mBetaKL) return 0.0;
+  double mine = 0.0;
   for (int d = lane; d < dim; d += 64) {
-    float lb, pa, pb, ps;
-    beta_terms(A.q1[(size_t)bq * dim + d], A.q2[(size_t)bq * dim + d], lb, pa, pb, ps);
-    mine -= lb;
+    float pa, pb, ps;
+    mine -= log_beta(A.q1[(size_t)bq * dim + d], A.q2[(size_t)bq * dim + d], pa, pb, ps);
   }
-  return wave_sum_f32(mine);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) mine += __shfl_xor(mine, d);   // (either order of a pair: the same sum in every lane)
+  return __longlong_as_double(uniform64(__double_as_longlong(mine)));
 }
 
 // Keys (and scores) of the answers: a wavefront takes up to 64 answer slots of one query, one per lane.
@@ -325,13 +344,14 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
     const int bq = b * A.U + u;
     const ScalarRow q1 = scalar_row(A.q1 + (size_t)bq * dim);
     const ScalarRow q2 = scalar_row(model_nq(M) == 2 ? A.q2 + (size_t)bq * dim : A.q1);
-    float tot[O::kSums], err[O::kSums], rtot[NS], rerr[NS], lb[8];
+    float tot[O::kSums], err[O::kSums], rtot[NS], rerr[NS];
+    double lb[8];
 #pragma unroll
     for (int i = 0; i < O::kSums; ++i) tot[i] = err[i] = 0.f;
 #pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = rerr[i] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) lb[i] = 0.f;
+    for (int i = 0; i < 8; ++i) lb[i] = 0.0;
     // the values of the next step are on their way while this one's are summed
     constexpr int F = O::kFeat, MUL = model_mul(M);
     float now[MUL][F], next[MUL][F];
@@ -373,7 +393,7 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
           float e[N][O::kGroup], qa[N], qb[N];
 #pragma unroll
           for (int v = 0; v < N; ++v) {
-            const float l = O::expand(now[0][f + v], now[MUL - 1][f + v], A.p, e[v]);
+            const double l = O::expand(now[0][f + v], now[MUL - 1][f + v], A.p, e[v]);
             if constexpr (M == mBetaKL) lb[(f + v) & 7] += l;
             qa[v] = q1[d0 + f + v];
             qb[v] = model_nq(M) == 2 ? (float)q2[d0 + f + v] : 0.f;
@@ -422,10 +442,8 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int sl
       }
     }
 #pragma unroll
-    for (int i = 0; i < O::kSums; ++i) tot[i] = with_error(tot[i], err[i]);
-#pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = with_error(rtot[i], rerr[i]);
-    const float su = O::score(tot, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), A.p);
+    const float su = O::score(tot, err, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), A.p);
     if (u == 0 || union_takes(su, best)) best = su;
   }
   if (j < A.A) {
@@ -458,14 +476,14 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
     __syncthreads();
   }
   ScalarRow q1[NB], q2[NB];
-  float qc[NB];
+  double qc[NB];
 #pragma unroll
   for (int x = 0; x < NB; ++x) {
     const int b = min(first_list + x / UP, A.B - 1);   // a list past the last query repeats it and is not counted
     const int bq = b * A.U + min(x % UP, A.U - 1);
     q1[x] = scalar_row(A.q1 + (size_t)bq * dim);
     q2[x] = scalar_row(model_nq(M) == 2 ? A.q2 + (size_t)bq * dim : A.q1);
-    qc[x] = active ? query_const<M>(A, bq, dim, lane) : 0.f;
+    qc[x] = active ? query_const<M>(A, bq, dim, lane) : 0.0;
   }
 
   // Staging.  Rows of 16-byte columns: thread t brings column t % 8 of rows t / 8 + 32 i (two halves: columns 0-3 from
@@ -495,15 +513,15 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       }
     }
   };
-  float lb[kBeta ? kItems : 1];
+  double lb[kBeta ? kItems : 1];
   auto put = [&](float* to, int d0) {
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
       float* at = to + ((t >> kRowShift) + kRowStep * i) * kScanStride;
       if constexpr (kBeta) {
         float e[G];
-        const float l = O::expand(in1[i], in2[i], A.p, e);
-        lb[i] += d0 + feat < dim ? l : 0.f;
+        const double l = O::expand(in1[i], in2[i], A.p, e);
+        lb[i] += d0 + feat < dim ? l : 0.0;
 #pragma unroll
         for (int x = 0; x < G; ++x) at[x * F + sub] = e[x];
       } else if constexpr (VEC == 4) {
@@ -616,7 +634,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
     }
     if constexpr (kBeta) {
 #pragma unroll
-      for (int i = 0; i < kItems; ++i) lb[i] = 0.f;
+      for (int i = 0; i < kItems; ++i) lb[i] = 0.0;
     }
     for (int c = 0; c < steps; ++c) {
       // the other buffer's readers are behind the barrier of the step before
@@ -627,23 +645,23 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       if (active) consume(stage[parity], c * F);
       parity ^= 1;
     }
-    float row_const[R];
+    double row_const[R];
     if constexpr (kBeta) {   // eight partial sums per row, added in a fixed order
-      float* part = stage[parity];
+      double* part = reinterpret_cast<double*>(stage[parity]);
 #pragma unroll
-      for (int i = 0; i < kItems; ++i) part[((t >> kRowShift) + kRowStep * i) * kScanStride + sub] = lb[i];
+      for (int i = 0; i < kItems; ++i) part[((t >> kRowShift) + kRowStep * i) * (kScanStride / 2) + sub] = lb[i];
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        float x[8];
+        double x[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = part[(lane + 64 * r) * kScanStride + i];
+        for (int i = 0; i < 8; ++i) x[i] = part[(lane + 64 * r) * (kScanStride / 2) + i];
         row_const[r] = beta_eighths(x);
       }
       parity ^= 1;
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r) row_const[r] = 0.f;
+      for (int r = 0; r < R; ++r) row_const[r] = 0.0;
     }
     if (!active) continue;
 #pragma unroll
@@ -657,10 +675,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
         float s = 0.f;
 #pragma unroll
         for (int u = 0; u < UP; ++u) {
-          float sum[O::kSums];
-#pragma unroll
-          for (int i = 0; i < O::kSums; ++i) sum[i] = with_error(tot[l * UP + u][r][i], err[l * UP + u][r][i]);
-          const float su = O::score(sum, rsum, row_const[r], qc[l * UP + u], A.p);
+          const float su = O::score(tot[l * UP + u][r], err[l * UP + u][r], rsum, row_const[r], qc[l * UP + u], A.p);
           if (u == 0 || union_takes(su, s)) s = su;
         }
         const int b = first_list + l;

@@ -139,3 +139,22 @@ def test_scores_round_no_worse_than_those_of_the_scoring_kernels(model, dim):
     scan, _ = _keys(model, t, a, c, params, _all_ids(b, n))
     tree = fused.score_forward(model, t, _all_ids(b, n), a, c, params)
     assert _rms(scan.cpu().numpy() - want) <= 1.1 * _rms(tree.cpu().numpy() - want)
+
+
+@pytest.mark.parametrize("low,high", [(0.05, 3.0), (1.0, 20.0), (20.0, 100.0)])
+@pytest.mark.parametrize("dim", [30, 100, 404])
+def test_divergences_round_no_worse_than_those_of_the_scoring_kernels(low, high, dim):
+    """BetaE: the log-Beta terms of row and query, thousands of times the divergence's last digits, cancel.  Whole error, and
+    the part that can reorder entities (without each query's mean); a tenth for the spread of two samples."""
+    from smore_amd import fused
+    rng = np.random.default_rng(dim)
+    f32 = lambda x: x.astype(np.float32).astype(np.float64)
+    n, b = 600, 3
+    table, q1, q2 = (f32(rng.uniform(low, high, s)) for s in ((n, 2 * dim), (b, dim), (b, dim)))
+    want = orc.score_forward("beta_kl", np.broadcast_to(table[None], (b,) + table.shape), q1[:, None], q2[:, None], 0.0, 0.0)
+    t, a, c = (torch.tensor(x, dtype=torch.float32, device="cuda") for x in (table, q1, q2))
+    params = fused.score_params(0.0)
+    scan = _keys("beta_kl", t, a, c, params, _all_ids(b, n))[0].cpu().numpy() - want
+    tree = fused.score_forward("beta_kl", t, _all_ids(b, n), a, c, params).cpu().numpy() - want
+    assert _rms(scan) <= 1.1 * _rms(tree)
+    assert _rms(scan - scan.mean(axis=1, keepdims=True)) <= 1.1 * _rms(tree - tree.mean(axis=1, keepdims=True))
