@@ -210,9 +210,10 @@ template <int M, bool NORM> struct ScanOps {
   static constexpr int kFeat = 32 / kGroup;   // features per step
   static constexpr int kSums = NORM ? model_mul(M) : 1;
   static constexpr int kRowSums = NORM ? model_mul(M) : 0;
+  static constexpr int kKeyStride = kFeat == 8 ? 8 : kFeat + 4;   // floats between two steps of a row in the answers' kernel
 
-  // Sum over N (4 or 1) features; terms that are not products are added as a tree.
-  template <int N>
+  // Sum over N (4 or 1) features; terms that are not products are added as a tree.  SCALAR: a and b are wavefront-uniform.
+  template <int N, bool SCALAR>
   static __device__ __forceinline__ void block(const float (&e)[N][kGroup], const float (&a)[N], const float (&b)[N], float cen,
                                                float (&s)[kSums]) {
 #pragma clang fp contract(off)
@@ -224,7 +225,9 @@ template <int M, bool NORM> struct ScanOps {
         if constexpr (M == mL1) {
           t[v] = fabsf(d);
         } else if constexpr (M == mBox) {
-          const float mn = ModelOps<mBox>::min_abs(d, b[v]);
+          float mn;
+          if constexpr (SCALAR) asm("v_min_f32_e64 %0, |%1|, %2" : "=v"(mn) : "v"(d), "s"(b[v]));   // (no move of the offset)
+          else mn = ModelOps<mBox>::min_abs(d, b[v]);
           t[v] = __builtin_fmaf(fabsf(mn), cen, fabsf(d) - mn);
         } else {
           const float y = e[v][1] - b[v];
@@ -326,127 +329,167 @@ __device__ __forceinline__ double query_const(const RankArgs& A, int bq, int dim
   return __longlong_as_double(uniform64(__double_as_longlong(mine)));
 }
 
-// Keys (and scores) of the answers: a wavefront takes up to 64 answer slots of one query, one per lane.
+// Keys (and scores) of the answers.  What bounds it: latency, most calls have a few dozen answers.  2^group_bits lanes share
+// an answer and take a step of its features each, out of rows staged in LDS; the steps' sums meet there and are added in
+// the scan's order.  (A lane per answer, step after step: 13 us instead of 9 for box at D = 400, 110 for BetaE with its chain
+// of special functions.  Lanes that fetch their steps themselves, 64 bytes apart: 59 us instead of 30 for 32,000 answers of
+// 2 x 250 floats.)
 template <int M, bool NORM, int VEC>
-__global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int slices) {
+__global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int group_bits, int tiles) {
 #pragma clang fp contract(off)
   using O = ScanOps<M, NORM>;
-  constexpr int NS = O::kRowSums > 0 ? O::kRowSums : 1;
-  const int lane = threadIdx.x;
-  const int b = blockIdx.x / slices, j = (blockIdx.x - b * slices) * 64 + lane;
-  const int dim = A.dim;
+  constexpr int NS = O::kRowSums > 0 ? O::kRowSums : 1, F = O::kFeat, MUL = model_mul(M), kVals = O::kSums + O::kRowSums;
+  constexpr bool kBeta = M == mBetaKL;
+  // per answer: BetaE's log-Beta terms [steps][8] | (all answers') sums [steps][kVals] | rows [MUL][steps][kKeyStride]
+  // | the query's row
+  extern __shared__ __attribute__((aligned(16))) double keys_lds[];
+  const int lane = threadIdx.x, group = 1 << group_bits, slots = 64 >> group_bits;
+  const int mine = lane >> group_bits, s0 = lane & (group - 1);
+  const int b = blockIdx.x / tiles, j = (blockIdx.x - b * tiles) * slots + mine;
+  const int dim = A.dim, steps = (dim + F - 1) / F;
   const bool valid = j < min(A.ans_count[b], A.A);
   unsigned long long id = valid ? (unsigned long long)A.ans_id[(size_t)b * A.A + j] : 0ull;
   if (id >= A.n_rows) id = 0;  // the host wrapper has already refused such ids
-  const float* row = A.table + id * (size_t)dim * model_mul(M);
+  double* lb = keys_lds + mine * steps * 8;
+  float* const parts = reinterpret_cast<float*>(keys_lds + (kBeta ? slots * steps * 8 : 0));
+  float* part = parts + mine * steps * kVals;
+  float* const rows = parts + ((slots * steps * kVals + 3) & ~3);
+  float* const query = rows + slots * MUL * steps * O::kKeyStride;
+  {
+    typedef std::conditional_t<VEC == 4, float4, float> Piece;
+    const int halves = slots * MUL;
+    for (int d0 = 0; d0 < dim; d0 += 64 * VEC) {
+      const int d = d0 + lane * VEC;
+      for (int q0 = 0; q0 < halves; q0 += 8) {   // eight half rows at a time are on their way
+        Piece w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int q = min(q0 + i, halves - 1), from = q / MUL * group;   // (uniform)
+          const unsigned long long at = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(id >> 32), from) << 32) |
+                                        (unsigned)__builtin_amdgcn_readlane((int)id, from);
+          w[i] = *reinterpret_cast<const Piece*>(A.table + (at * MUL + q % MUL) * (size_t)dim + min(d, dim - VEC));
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (q0 + i < halves && d < dim) *reinterpret_cast<Piece*>(rows + ((q0 + i) * steps + d / F) * O::kKeyStride + d % F) = w[i];
+      }
+    }
+  }
+  auto fetch = [&](float (&to)[F], const float* from) {   // (what lies past the row's end is not used)
+#pragma unroll
+    for (int f = 0; f < F; f += 4) {
+      const float4 w = reinterpret_cast<const float4*>(from)[f / 4];
+      to[f] = w.x;
+      to[f + 1] = w.y;
+      to[f + 2] = w.z;
+      to[f + 3] = w.w;
+    }
+  };
   float best = 0.f;
   for (int u = 0; u < A.U; ++u) {  // uniform
     const int bq = b * A.U + u;
-    const ScalarRow q1 = scalar_row(A.q1 + (size_t)bq * dim);
-    const ScalarRow q2 = scalar_row(model_nq(M) == 2 ? A.q2 + (size_t)bq * dim : A.q1);
+#pragma unroll
+    for (int h = 0; h < model_nq(M); ++h) {
+      const float* from = (h == 0 ? A.q1 : A.q2) + (size_t)bq * dim;
+      for (int d = lane * VEC; d < dim; d += 64 * VEC) {
+        float* to = query + (h * steps + d / F) * O::kKeyStride + d % F;
+        if constexpr (VEC == 4) *reinterpret_cast<float4*>(to) = *reinterpret_cast<const float4*>(from + d);
+        else *to = from[d];
+      }
+    }
+    __syncthreads();
+    for (int c = s0; c < steps; c += group) {
+      const int d0 = c * F, n = min(F, dim - d0);
+      float x[MUL][F], q1[F], q2[F], s[O::kSums], r[NS];
+#pragma unroll
+      for (int h = 0; h < MUL; ++h) fetch(x[h], rows + ((mine * MUL + h) * steps + c) * O::kKeyStride);
+      fetch(q1, query + c * O::kKeyStride);
+      if constexpr (model_nq(M) == 2) fetch(q2, query + (steps + c) * O::kKeyStride);
+#pragma unroll
+      for (int i = 0; i < O::kSums; ++i) s[i] = 0.f;
+#pragma unroll
+      for (int i = 0; i < NS; ++i) r[i] = 0.f;
+      // N features from f on; the order is the scan's (its `consume`)
+      auto block = [&](auto n_tag, int f, float (&ps)[O::kSums], float (&pr)[NS]) {
+        constexpr int N = decltype(n_tag)::value;
+        float e[N][O::kGroup], qa[N], qb[N];
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+          const double l = O::expand(x[0][f + v], x[MUL - 1][f + v], A.p, e[v]);
+          if constexpr (kBeta) lb[c * 8 + f + v] = l;
+          qa[v] = q1[f + v];
+          qb[v] = model_nq(M) == 2 ? q2[f + v] : 0.f;
+        }
+        O::template block<N, false>(e, qa, qb, A.p.cen, ps);
+        O::template block_row<N>(e, pr);
+      };
+      auto take = [&](const float (&ps)[O::kSums], const float (&pr)[NS]) {
+#pragma unroll
+        for (int i = 0; i < O::kSums; ++i) s[i] += ps[i];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) r[i] += pr[i];
+      };
+      float ps[O::kSums], pr[NS], ps2[O::kSums], pr2[NS];
+#pragma unroll
+      for (int f = 0; f < F; f += 8) {
+        if (f + 8 <= n) {
+          block(std::integral_constant<int, 4>{}, f, ps, pr);
+          block(std::integral_constant<int, 4>{}, f + 4, ps2, pr2);
+#pragma unroll
+          for (int i = 0; i < O::kSums; ++i) ps[i] += ps2[i];
+#pragma unroll
+          for (int i = 0; i < NS; ++i) pr[i] += pr2[i];
+          take(ps, pr);
+        } else if (f < n) {
+          const bool four = f + 4 <= n;
+          if (four) {
+            block(std::integral_constant<int, 4>{}, f, ps, pr);
+            take(ps, pr);
+          }
+#pragma unroll
+          for (int v = 0; v < 8; ++v) {
+            if (v >= (four ? 4 : 0) && f + v < n) {
+              block(std::integral_constant<int, 1>{}, f + v, ps, pr);
+              take(ps, pr);
+            } else if (kBeta && f + v >= n) {
+              lb[c * 8 + f + v] = 0.0;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < O::kSums; ++i) part[c * kVals + i] = s[i];
+#pragma unroll
+      for (int i = 0; i < O::kRowSums; ++i) part[c * kVals + O::kSums + i] = r[i];
+    }
+    __syncthreads();
     float tot[O::kSums], err[O::kSums], rtot[NS], rerr[NS];
-    double lb[8];
 #pragma unroll
     for (int i = 0; i < O::kSums; ++i) tot[i] = err[i] = 0.f;
 #pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = rerr[i] = 0.f;
+#pragma unroll 4
+    for (int c = 0; c < steps; ++c) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) lb[i] = 0.0;
-    // the values of the next step are on their way while this one's are summed
-    constexpr int F = O::kFeat, MUL = model_mul(M);
-    float now[MUL][F], next[MUL][F];
-    auto request = [&](int d0) {
+      for (int i = 0; i < O::kSums; ++i) add_step(tot[i], err[i], part[c * kVals + i]);
 #pragma unroll
-      for (int h = 0; h < MUL; ++h) {
-        const float* half = row + h * dim;
-        if constexpr (VEC == 4) {   // (rows of whole 16-byte columns; past the end the last one again, not used)
-#pragma unroll
-          for (int f = 0; f < F; f += 4) {
-            const float4 w = *reinterpret_cast<const float4*>(half + min(d0 + f, dim - 4));
-            next[h][f] = w.x;
-            next[h][f + 1] = w.y;
-            next[h][f + 2] = w.z;
-            next[h][f + 3] = w.w;
-          }
-        } else {
-#pragma unroll
-          for (int f = 0; f < F; ++f) next[h][f] = half[min(d0 + f, dim - 1)];
-        }
-      }
-    };
-    {
-      request(0);
-      for (int d0 = 0; d0 < dim; d0 += F) {
-#pragma unroll
-        for (int h = 0; h < MUL; ++h)
-#pragma unroll
-          for (int f = 0; f < F; ++f) now[h][f] = next[h][f];
-        if (d0 + F < dim) request(d0 + F);
-        float s[O::kSums], r[NS];
-#pragma unroll
-        for (int i = 0; i < O::kSums; ++i) s[i] = 0.f;
-#pragma unroll
-        for (int i = 0; i < NS; ++i) r[i] = 0.f;
-        // N features from f on
-        auto block = [&](auto n_tag, int f, float (&ps)[O::kSums], float (&pr)[NS]) {
-          constexpr int N = decltype(n_tag)::value;
-          float e[N][O::kGroup], qa[N], qb[N];
-#pragma unroll
-          for (int v = 0; v < N; ++v) {
-            const double l = O::expand(now[0][f + v], now[MUL - 1][f + v], A.p, e[v]);
-            if constexpr (M == mBetaKL) lb[(f + v) & 7] += l;
-            qa[v] = q1[d0 + f + v];
-            qb[v] = model_nq(M) == 2 ? (float)q2[d0 + f + v] : 0.f;
-          }
-          O::template block<N>(e, qa, qb, A.p.cen, ps);
-          O::template block_row<N>(e, pr);
-        };
-        auto take = [&](const float (&ps)[O::kSums], const float (&pr)[NS]) {
-#pragma unroll
-          for (int i = 0; i < O::kSums; ++i) s[i] += ps[i];
-#pragma unroll
-          for (int i = 0; i < NS; ++i) r[i] += pr[i];
-        };
-        const int n = min(F, dim - d0);   // uniform
-        float ps[O::kSums], pr[NS], ps2[O::kSums], pr2[NS];
-#pragma unroll
-        for (int f = 0; f < F; f += 8) {
-          if (f + 8 <= n) {
-            block(std::integral_constant<int, 4>{}, f, ps, pr);
-            block(std::integral_constant<int, 4>{}, f + 4, ps2, pr2);
-#pragma unroll
-            for (int i = 0; i < O::kSums; ++i) ps[i] += ps2[i];
-#pragma unroll
-            for (int i = 0; i < NS; ++i) pr[i] += pr2[i];
-            take(ps, pr);
-          } else if (f < n) {
-            int done = f;
-            if (f + 4 <= n) {
-              block(std::integral_constant<int, 4>{}, f, ps, pr);
-              take(ps, pr);
-              done = f + 4;
-            }
-#pragma unroll
-            for (int v = 0; v < 7; ++v) {
-              if (f + v >= done && f + v < n) {
-                block(std::integral_constant<int, 1>{}, f + v, ps, pr);
-                take(ps, pr);
-              }
-            }
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < O::kSums; ++i) add_step(tot[i], err[i], s[i]);
-#pragma unroll
-        for (int i = 0; i < NS; ++i) add_step(rtot[i], rerr[i], r[i]);
-      }
+      for (int i = 0; i < O::kRowSums; ++i) add_step(rtot[i], rerr[i], part[c * kVals + O::kSums + i]);
     }
+    double row_const = 0.0;
+    if constexpr (kBeta) {   // (the group has at least eight lanes)
+      double sum = 0.0, eighths[8];
+      for (int c = 0; c < steps; ++c) sum += lb[c * 8 + (s0 & 7)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) eighths[i] = __shfl(sum, mine * group + i);
+      row_const = beta_eighths(eighths);
+    }
+    __syncthreads();  // the next branch writes there
 #pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = with_error(rtot[i], rerr[i]);
-    const float su = O::score(tot, err, rtot, beta_eighths(lb), query_const<M>(A, bq, dim, lane), A.p);
+    const float su = O::score(tot, err, rtot, row_const, query_const<M>(A, bq, dim, lane), A.p);
     if (u == 0 || union_takes(su, best)) best = su;
   }
-  if (j < A.A) {
+  if (s0 == 0 && j < A.A) {
     if (A.score_out) A.score_out[(size_t)b * A.A + j] = valid ? best : 0.f;
     A.key_out[(size_t)b * A.A + j] = valid ? rank_key(best, id) : 0ull;  // key 0 sorts last and is never counted
   }
@@ -561,7 +604,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int x = 0; x < NB; ++x) O::template block<N>(e[r], a[x], b[x], A.p.cen, s[x][r]);
+      for (int x = 0; x < NB; ++x) O::template block<N, true>(e[r], a[x], b[x], A.p.cen, s[x][r]);
       O::template block_row<N>(e[r], rs[r]);
     }
   };
@@ -941,9 +984,17 @@ int launch_scan_vec(hipStream_t st, const RankArgs& A) {
 template <int M, bool NORM>
 int launch_rank_all(hipStream_t st, RankArgs A, int vec, int mode) {
   if (mode == kRankKeys) {
-    const int slices = (A.A + 63) / 64;
-    if (vec == 4) hipLaunchKernelGGL((rank_answer_keys_kernel<M, NORM, 4>), dim3((unsigned)A.B * slices), dim3(64), 0, st, A, slices);
-    else hipLaunchKernelGGL((rank_answer_keys_kernel<M, NORM, 1>), dim3((unsigned)A.B * slices), dim3(64), 0, st, A, slices);
+    using O = ScanOps<M, NORM>;
+    const int steps = (A.dim + O::kFeat - 1) / O::kFeat;   // at most 256 (BetaE, 2,048 floats per half)
+    int bits = M == mBetaKL ? 3 : 0;
+    while (bits < 6 && (1 << bits) < steps) ++bits;
+    const int slots = 64 >> bits, tiles = (A.A + slots - 1) / slots;
+    // (at most 50 KiB: BetaE's 256 steps of one answer, 16 KiB each of them log-Beta terms, row and query)
+    const size_t sums = ((size_t)slots * steps * (O::kSums + O::kRowSums) + 3) & ~(size_t)3;
+    const size_t lds = (M == mBetaKL ? (size_t)slots * steps * 8 * sizeof(double) : 0) +
+                       (sums + ((size_t)slots * model_mul(M) + model_nq(M)) * steps * O::kKeyStride) * sizeof(float);
+    if (vec == 4) hipLaunchKernelGGL((rank_answer_keys_kernel<M, NORM, 4>), dim3((unsigned)A.B * tiles), dim3(64), lds, st, A, bits, tiles);
+    else hipLaunchKernelGGL((rank_answer_keys_kernel<M, NORM, 1>), dim3((unsigned)A.B * tiles), dim3(64), lds, st, A, bits, tiles);
     return check_launch("rank answer keys");
   }
   if (!A.slot) {   // (smx_filtered_ranks has cleared them: rank_prepare_kernel)
