@@ -9,8 +9,8 @@
 // row that reaches the lowest of a query's answers finds its place among them by a binary search and is counted in
 // that place's bin (integer atomics: exact, order-free).  A prefix sum over the bins gives every answer its count.
 // Order of equal scores: the lower entity id ranks first (one of the orders an unstable argsort may produce).
-// "Beats" is one unsigned compare of (sortable(score) << 32 | ~id) keys; the answers' keys come from the same
-// arithmetic, operation by operation, so that an answer is recognised in the stream by its key.
+// "Beats" is one unsigned compare of (sortable(score) << 32 | ~id) keys; an answer is recognised in the stream by its id.
+// The answers' keys come from the same arithmetic, operation by operation, so that equal rows tie.
 #pragma once
 #include "smx_common.h"
 #include "smx_models.h"
@@ -737,7 +737,13 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
             else lo = mid + 1;
           }
         }
-        const bool is_answer = lo > 0 && keys[lo - 1] == key;
+        // rows that are answers themselves, by the ids in the keys: their own scores may come from elsewhere
+        bool is_answer = false;
+        for (int j0 = 0; j0 < count; j0 += 64) {
+          const unsigned in_group = j0 + lane < count ? ~(unsigned)keys[j0 + lane] - (g * kScanRows + 64 * r) : 64u;
+          for (unsigned long long hits = __ballot(in_group < 64u); hits != 0ull; hits &= hits - 1)
+            is_answer |= (unsigned)lane == (unsigned)__builtin_amdgcn_readlane((int)in_group, __builtin_ctzll(hits));
+        }
         if (reaches && lo < count && !is_answer)
           atomicAdd(A.lds_bins ? &lds_bins[(wave * NL + l) * A1 + lo] : &A.bins[(size_t)b * A1 + lo], 1u);
       }

@@ -158,3 +158,28 @@ def test_divergences_round_no_worse_than_those_of_the_scoring_kernels(low, high,
     tree = fused.score_forward("beta_kl", t, _all_ids(b, n), a, c, params).cpu().numpy() - want
     assert _rms(scan) <= 1.1 * _rms(tree)
     assert _rms(scan - scan.mean(axis=1, keepdims=True)) <= 1.1 * _rms(tree - tree.mean(axis=1, keepdims=True))
+
+
+@pytest.mark.parametrize("model", ["l1", "box", "rotate", "beta_kl", "complex_norm", "l2"])
+@pytest.mark.parametrize("b,branches,dim", [(1, 1, 100), (6, 1, 37), (3, 2, 36)])
+def test_answers_are_known_by_their_ids_not_by_their_scores(model, b, branches, dim):
+    """Every entity is an answer, one of them listed twice: nothing ranks before any of them, whatever the keys' scores --
+    those of smx_rank_answer_keys, the same an ulp off, or scores of the scoring kernels."""
+    from smore_amd import fused
+    from smore_amd.evaluation import filtered_ranks
+    rng = np.random.default_rng(dim)
+    model, norm = model.removesuffix("_norm"), model.endswith("_norm")
+    n = 333
+    low, high = (0.1, 4.0) if model == "beta_kl" else (-0.2, 0.2)
+    t = torch.tensor(rng.uniform(low, high, (n, _row(model, dim))), dtype=torch.float32, device="cuda")
+    q = [torch.tensor(np.abs(rng.uniform(low, high, (b, branches, dim))), dtype=torch.float32, device="cuda") for _ in range(2)]
+    q1, q2 = q[0], None if model in ONE_QUERY else q[1]
+    params = fused.score_params(GAMMA[model], 0.02 if model == "box" else 0.0, norm=norm)
+    ids = torch.cat([_all_ids(b, n), torch.full((b, 1), 7, device="cuda")], dim=1).contiguous()
+    _, keys = _keys(model, t, q1, q2, params, ids, branches)
+    ulp = torch.tensor(rng.integers(-1, 2, tuple(keys.shape)), device="cuda") << 32
+    elsewhere = (torch.tensor(rng.integers(0, 2 ** 31, tuple(keys.shape)), device="cuda") << 32) | (keys & 0xFFFFFFFF)
+    for k in (keys, keys + ulp, elsewhere):
+        assert (_scan(model, t, q1, q2, params, ids, k, branches) == 1).all()
+    ranks = filtered_ranks(model, t, q1, q2, params, [list(range(0, n, 2))] * b, [list(range(1, n, 2))] * b, branches)
+    assert all((x == 1).all() for pair in ranks for x in pair)
