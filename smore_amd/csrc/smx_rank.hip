@@ -155,7 +155,9 @@ int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_row
   R.key_out = key;
   if (int rc = rank_run(model, st, R, vec, nit, kRankKeys)) return rc;
   R.bins = reinterpret_cast<unsigned*>(base);
-  hipLaunchKernelGGL(rank_prepare_kernel, dim3((unsigned)B), dim3(256), A * sizeof(unsigned long long), st, R, sorted, slot);
+  const int tiles = (int)((A + 63) / 64);
+  hipLaunchKernelGGL(rank_prepare_kernel, dim3((unsigned)B * tiles), dim3(256), A * sizeof(unsigned long long), st, R, tiles,
+                     sorted, slot);
   if (int rc = check_launch("rank preparation")) return rc;
   R.ans_key = sorted;
   R.slot = slot;

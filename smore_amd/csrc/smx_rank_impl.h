@@ -915,20 +915,27 @@ static __global__ __launch_bounds__(64) void rank_finish_kernel(RankArgs A) {
   }
 }
 
-// One workgroup per query, everything the scan needs beside the keys: the keys in descending order with the slot each
-// came from (unused slots have key 0 and go last), the query's bins cleared.
-static __global__ __launch_bounds__(256) void rank_prepare_kernel(RankArgs A, unsigned long long* sorted, int* slot) {
+// Everything the scan needs beside the keys: the keys in descending order with the slot each came from (unused slots have
+// key 0 and go last), the query's bins cleared.  A workgroup places 64 keys, each of its wavefronts by a quarter of the
+// query's (one workgroup for all of them: 0.48 ms for a list of 2,000, 6 us now).
+static __global__ __launch_bounds__(256) void rank_prepare_kernel(RankArgs A, int tiles, unsigned long long* sorted, int* slot) {
   extern __shared__ unsigned long long sort_keys[];
-  const int n = A.A, b = blockIdx.x;
+  __shared__ int before[4][64];
+  const int n = A.A, b = blockIdx.x / tiles, tile = blockIdx.x - b * tiles;
   const size_t base = (size_t)b * n;
   for (int i = threadIdx.x; i < n; i += 256) sort_keys[i] = A.key_out[base + i];
-  for (int i = threadIdx.x; i <= n; i += 256) A.bins[(size_t)b * (n + 1) + i] = 0u;
+  for (int i = tile * 256 + threadIdx.x; i <= n; i += 256 * tiles) A.bins[(size_t)b * (n + 1) + i] = 0u;
   __syncthreads();
-  for (int j = threadIdx.x; j < n; j += 256) {
-    const unsigned long long mine = sort_keys[j];
-    int at = 0;
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+  const int j = tile * 64 + lane, per = (n + 3) / 4;
+  const unsigned long long mine = sort_keys[min(j, n - 1)];
+  int at = 0;
 #pragma unroll 8
-    for (int i = 0; i < n; ++i) at += sort_keys[i] > mine || (sort_keys[i] == mine && i < j);
+  for (int i = wave * per; i < min(n, (wave + 1) * per); ++i) at += sort_keys[i] > mine || (sort_keys[i] == mine && i < j);
+  before[wave][lane] = at;
+  __syncthreads();
+  if (wave == 0 && j < n) {
+    at = (before[0][lane] + before[1][lane]) + (before[2][lane] + before[3][lane]);
     sorted[base + at] = mine;
     slot[base + at] = j;
   }
