@@ -439,7 +439,9 @@ int smx_sample_loss_static(void* stream, const float* pos, const float* neg, con
  * smx_rank_answer_keys: ans_score [B, A] = the answers' logits, ans_key [B, A] = their order keys
  *   (larger key = ranked earlier; 0 in unused slots).
  * smx_rank_scan: ans_id / ans_key must be sorted by key, descending, within each query (unused slots
- *   last); filtered_rank [B, A] int64, 1-based, in that order (0 in unused slots).
+ *   last); filtered_rank [B, A] int64, 1-based, in that order (0 in unused slots).  An answer is known by the id in its
+ *   key.  Equal rows tie with an answer exactly if its key comes from a smx_rank_answer_keys call of the same B, U and A
+ *   (the order of a score's sum depends on them; other keys may be an ulp off).
  * workspace: smx_rank_workspace_bytes(B, A).  At most 2048 answers per query, n_rows <= 2^32. */
 size_t smx_rank_workspace_bytes(size_t B, size_t A);
 int smx_rank_answer_keys(int model, void* stream, const float* table, size_t n_rows, const float* q1,

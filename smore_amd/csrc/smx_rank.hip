@@ -1,5 +1,6 @@
 // Host side of the all-entity ranking (see smx_rank_impl.h).
 #include "smx_rank_impl.h"
+#include "smx_rank_stream_impl.h"
 
 namespace smx {
 
@@ -10,6 +11,12 @@ extern template int rank_dispatch<mRotate>(hipStream_t, const RankArgs&, int, in
 extern template int rank_dispatch<mBetaKL>(hipStream_t, const RankArgs&, int, int, int);
 extern template int rank_dispatch<mComplex>(hipStream_t, const RankArgs&, int, int, int);
 extern template int rank_dispatch<mDistmult>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mL1>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mL2>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mBox>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mRotate>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mComplex>(hipStream_t, const RankArgs&, int, int, int);
+extern template int rank_stream_dispatch<mDistmult>(hipStream_t, const RankArgs&, int, int, int);
 
 constexpr size_t kRankMaxCandidates = 4096;  // per query: their keys live in LDS
 constexpr size_t kRankMaxAnswers = 2048;  // per query; bins and keys of a pass live in LDS (per query of the pass 2049 x 4 + 2048 x 8 bytes)
@@ -72,15 +79,25 @@ static int rank_common(RankArgs* R, int* vec, int* nit, int model, const float* 
   return SMX_OK;
 }
 
-static int rank_run(int model, hipStream_t st, const RankArgs& R, int vec, int nit, int keys_only) {
+static int rank_run(int model, hipStream_t st, const RankArgs& R, int vec, int nit, int mode) {
+  if (mode != kRankCandidates && rank_streams(model, R.n_rows, (size_t)R.dim, (size_t)R.B, (size_t)R.U, (size_t)R.A)) {
+    switch (model) {
+      case mL1: return rank_stream_dispatch<mL1>(st, R, vec, nit, mode);
+      case mL2: return rank_stream_dispatch<mL2>(st, R, vec, nit, mode);
+      case mBox: return rank_stream_dispatch<mBox>(st, R, vec, nit, mode);
+      case mRotate: return rank_stream_dispatch<mRotate>(st, R, vec, nit, mode);
+      case mComplex: return rank_stream_dispatch<mComplex>(st, R, vec, nit, mode);
+      case mDistmult: return rank_stream_dispatch<mDistmult>(st, R, vec, nit, mode);
+    }
+  }
   switch (model) {
-    case mL1: return rank_dispatch<mL1>(st, R, vec, nit, keys_only);
-    case mL2: return rank_dispatch<mL2>(st, R, vec, nit, keys_only);
-    case mBox: return rank_dispatch<mBox>(st, R, vec, nit, keys_only);
-    case mRotate: return rank_dispatch<mRotate>(st, R, vec, nit, keys_only);
-    case mBetaKL: return rank_dispatch<mBetaKL>(st, R, vec, nit, keys_only);
-    case mComplex: return rank_dispatch<mComplex>(st, R, vec, nit, keys_only);
-    case mDistmult: return rank_dispatch<mDistmult>(st, R, vec, nit, keys_only);
+    case mL1: return rank_dispatch<mL1>(st, R, vec, nit, mode);
+    case mL2: return rank_dispatch<mL2>(st, R, vec, nit, mode);
+    case mBox: return rank_dispatch<mBox>(st, R, vec, nit, mode);
+    case mRotate: return rank_dispatch<mRotate>(st, R, vec, nit, mode);
+    case mBetaKL: return rank_dispatch<mBetaKL>(st, R, vec, nit, mode);
+    case mComplex: return rank_dispatch<mComplex>(st, R, vec, nit, mode);
+    case mDistmult: return rank_dispatch<mDistmult>(st, R, vec, nit, mode);
   }
   return fail(SMX_ERR_KIND, "unknown score model %d", model);
 }

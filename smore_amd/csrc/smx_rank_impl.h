@@ -41,6 +41,7 @@ struct RankArgs {
   int A;
   unsigned* bins;                    // [B, A + 1]
   int lds_bins;                      // the scan counts in LDS first (the bins of its queries fit)
+  int lds_keys;                      // and keeps their keys there
   unsigned groups;                   // the scan's groups of kScanRows rows
   int first_list;                    // query of the launch's first list of answers
   long long* rank_out;               // [B, A]
@@ -120,7 +121,8 @@ __device__ __forceinline__ void unit_row(float (&e1)[NIT][VEC], float (&e2)[NIT]
   }
 }
 
-template <int VEC, int NIT, int MUL>
+// STREAM: the row is read once (non-temporal)
+template <int VEC, int NIT, int MUL, bool STREAM = false>
 __device__ __forceinline__ void load_entity(const float* __restrict__ row, int dim, int ncol, int lane,
                                             float (&e1)[NIT][VEC], float (&e2)[NIT][VEC]) {
   typedef float vec4f __attribute__((ext_vector_type(4)));
@@ -129,16 +131,16 @@ __device__ __forceinline__ void load_entity(const float* __restrict__ row, int d
     const int c = min(lane + 64 * it, ncol - 1);
     if constexpr (VEC == 4) {
       const vec4f* pa = reinterpret_cast<const vec4f*>(row) + c;
-      const vec4f a = *pa;
+      const vec4f a = STREAM ? __builtin_nontemporal_load(pa) : *pa;
       e1[it][0] = a.x; e1[it][1] = a.y; e1[it][2] = a.z; e1[it][3] = a.w;
       if (MUL == 2) {
         const vec4f* pb = reinterpret_cast<const vec4f*>(row + dim) + c;
-        const vec4f b = *pb;
+        const vec4f b = STREAM ? __builtin_nontemporal_load(pb) : *pb;
         e2[it][0] = b.x; e2[it][1] = b.y; e2[it][2] = b.z; e2[it][3] = b.w;
       }
     } else {
-      e1[it][0] = row[c];
-      if (MUL == 2) e2[it][0] = row[dim + c];
+      e1[it][0] = STREAM ? __builtin_nontemporal_load(row + c) : row[c];
+      if (MUL == 2) e2[it][0] = STREAM ? __builtin_nontemporal_load(row + dim + c) : row[dim + c];
     }
   }
 }
@@ -506,7 +508,8 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
   constexpr int R = kScanRows / 64, G = O::kGroup, F = O::kFeat, NL = NB / UP;
   constexpr bool kBeta = M == mBetaKL;
   __shared__ __attribute__((aligned(16))) float stage[2][kScanRows * kScanStride];
-  extern __shared__ unsigned lds_bins[];  // [4 * NL][A + 1], when A.lds_bins
+  // keys [lists][A], when A.lds_keys | bins [lists][A + 1], when A.lds_bins; the lists of this workgroup
+  extern __shared__ unsigned long long lds_keys[];
   const int t = threadIdx.x, lane = t & 63, wave = uniform(t >> 6);
   const int dim = A.dim;
   const size_t row_len = (size_t)dim * model_mul(M);
@@ -514,9 +517,20 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
   const int block_list = A.first_list + (int)blockIdx.y * 4 * NL;
   const int first_list = block_list + wave * NL;   // this wavefront's lists of answers
   const bool active = first_list < A.B;
-  if (A.lds_bins) {
-    for (int i = t; i < 4 * NL * A1; i += kScanThreads) lds_bins[i] = 0u;
-    __syncthreads();
+  const int lists = min(4 * NL, A.B - block_list);
+  unsigned* const lds_bins = reinterpret_cast<unsigned*>(lds_keys + (A.lds_keys ? min(4 * NL, A.B) * A.A : 0));
+  if (A.lds_bins)
+    for (int i = t; i < lists * A1; i += kScanThreads) lds_bins[i] = 0u;
+  if (A.lds_keys)
+    for (int i = t; i < lists * A.A; i += kScanThreads) lds_keys[i] = A.ans_key[(size_t)block_list * A.A + i];
+  __syncthreads();
+  int count[NL];                    // answers of the wavefront's lists, and the lowest key of each (uniform)
+  unsigned long long lowest[NL];
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    const int b = first_list + l;
+    count[l] = b < A.B ? uniform(min(max(A.ans_count[b], 0), A.A)) : 0;
+    lowest[l] = count[l] > 0 ? (unsigned long long)uniform64((long long)A.ans_key[(size_t)b * A.A + count[l] - 1]) : ~0ull;
   }
   ScalarRow q1[NB], q2[NB];
   double qc[NB];
@@ -535,12 +549,18 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
   constexpr int kItems = kBeta ? 4 : (VEC == 4 ? 4 : 16);
   constexpr int kRowShift = kBeta || VEC == 4 ? 3 : 5, kRowStep = kBeta || VEC == 4 ? 32 : 8;
   typedef float vec4f __attribute__((ext_vector_type(4)));
-  vec4f in4[kBeta || VEC != 4 ? 1 : kItems];
-  float in1[kBeta || VEC != 4 ? kItems : 1], in2[kBeta ? kItems : 1];
+  // Two halves and few queries, where memory is what bounds: two steps at a time, so that whole 128-byte lines of either half
+  // are asked for at once (thread: the same column of both halves; half of the threads then have the first step's).  Four
+  // queries, 300 k rows, RotatE 2 x 250 floats 177 -> 167 us, ComplEx 2 x 200 119 -> 117.
+  constexpr bool kPairs = G == 2 && NB <= 2;
+  typedef std::conditional_t<VEC == 4, vec4f, float> Piece;
+  Piece in[kBeta ? 1 : kItems], in_b[kPairs ? kItems : 1];
+  float in1[kBeta ? kItems : 1], in2[kBeta ? kItems : 1];
   const int sub = t & ((1 << kRowShift) - 1);
-  const int half = G == 2 ? (VEC == 4 ? sub >> 2 : sub >> 4) : 0;
-  const int feat = kBeta ? sub : (VEC == 4 ? 4 * (sub - half * 4) : sub - half * 16);   // first feature within the step
+  const int half = G == 2 && !kPairs ? (VEC == 4 ? sub >> 2 : sub >> 4) : 0;
+  const int feat = kBeta ? sub : VEC * sub - half * 16;   // first feature within the step (or pair of steps)
   auto request = [&](unsigned g, int d0) {
+    if (kPairs && (d0 / F & 1)) return;   // (uniform: on its way since the step before)
     const int d = min(d0 + feat, dim - (kBeta ? 1 : VEC)) + half * dim;
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
@@ -549,10 +569,9 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       if constexpr (kBeta) {
         in1[i] = p[0];
         in2[i] = p[dim];
-      } else if constexpr (VEC == 4) {
-        in4[i] = *reinterpret_cast<const vec4f*>(p);
       } else {
-        in1[i] = p[0];
+        in[i] = *reinterpret_cast<const Piece*>(p);
+        if constexpr (kPairs) in_b[i] = *reinterpret_cast<const Piece*>(p + dim);
       }
     }
   };
@@ -567,10 +586,14 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
         lb[i] += d0 + feat < dim ? l : 0.0;
 #pragma unroll
         for (int x = 0; x < G; ++x) at[x * F + sub] = e[x];
-      } else if constexpr (VEC == 4) {
-        *reinterpret_cast<vec4f*>(at + 4 * sub) = in4[i];
+      } else if constexpr (kPairs) {
+        const int f = feat - 16 * (d0 / F & 1);
+        if (f >= 0 && f < 16) {
+          *reinterpret_cast<Piece*>(at + f) = in[i];
+          *reinterpret_cast<Piece*>(at + 16 + f) = in_b[i];
+        }
       } else {
-        at[sub] = in1[i];
+        *reinterpret_cast<Piece*>(at + VEC * sub) = in[i];
       }
     }
   };
@@ -721,41 +744,41 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
           const float su = O::score(tot[l * UP + u][r], err[l * UP + u][r], rsum, row_const[r], qc[l * UP + u], A.p);
           if (u == 0 || union_takes(su, s)) s = su;
         }
-        const int b = first_list + l;
-        const int count = b < A.B ? min(max(A.ans_count[b], 0), A.A) : 0;   // uniform
-        if (count == 0) continue;
-        const unsigned long long* keys = A.ans_key + (size_t)b * A.A;
         const unsigned long long key = rank_key(s, id);
-        const bool reaches = id < A.n_rows && key >= keys[count - 1];
+        const bool reaches = count[l] > 0 && id < A.n_rows && key >= lowest[l];
         if (__ballot(reaches) == 0ull) continue;   // uniform: no row of these beats any answer of the query
-        // answers that the row does not beat: the keys are sorted descending
-        int lo = 0, hi = count;
-        while (__ballot(lo < hi) != 0ull) {
-          const int mid = (lo + hi) >> 1;
-          if (lo < hi) {
-            if (key > keys[mid]) hi = mid;
-            else lo = mid + 1;
+        auto place = [&](const unsigned long long* keys) {
+          // answers that the row does not beat: the keys are sorted descending
+          int lo = 0, hi = count[l];
+          while (__ballot(lo < hi) != 0ull) {
+            const int mid = (lo + hi) >> 1;
+            if (lo < hi) {
+              if (key > keys[mid]) hi = mid;
+              else lo = mid + 1;
+            }
           }
-        }
-        // rows that are answers themselves, by the ids in the keys: their own scores may come from elsewhere
-        bool is_answer = false;
-        for (int j0 = 0; j0 < count; j0 += 64) {
-          const unsigned in_group = j0 + lane < count ? ~(unsigned)keys[j0 + lane] - (g * kScanRows + 64 * r) : 64u;
-          for (unsigned long long hits = __ballot(in_group < 64u); hits != 0ull; hits &= hits - 1)
-            is_answer |= (unsigned)lane == (unsigned)__builtin_amdgcn_readlane((int)in_group, __builtin_ctzll(hits));
-        }
-        if (reaches && lo < count && !is_answer)
-          atomicAdd(A.lds_bins ? &lds_bins[(wave * NL + l) * A1 + lo] : &A.bins[(size_t)b * A1 + lo], 1u);
+          // rows that are answers themselves, by the ids in the keys: their own scores may come from elsewhere
+          bool is_answer = false;
+          for (int j0 = 0; j0 < count[l]; j0 += 64) {
+            const unsigned in_group = j0 + lane < count[l] ? ~(unsigned)keys[j0 + lane] - (g * kScanRows + 64 * r) : 64u;
+            for (unsigned long long hits = __ballot(in_group < 64u); hits != 0ull; hits &= hits - 1)
+              is_answer |= (unsigned)lane == (unsigned)__builtin_amdgcn_readlane((int)in_group, __builtin_ctzll(hits));
+          }
+          if (reaches && lo < count[l] && !is_answer) {
+            if (A.lds_bins) atomicAdd(&lds_bins[(wave * NL + l) * A1 + lo], 1u);
+            else atomicAdd(&A.bins[(size_t)(first_list + l) * A1 + lo], 1u);
+          }
+        };
+        if (A.lds_keys) place(lds_keys + (wave * NL + l) * A.A);
+        else place(A.ans_key + (size_t)(first_list + l) * A.A);
       }
     }
   }
   if (A.lds_bins) {
     __syncthreads();
-    for (int i = t; i < 4 * NL * A1; i += kScanThreads) {
+    for (int i = t; i < lists * A1; i += kScanThreads) {
       const unsigned v = lds_bins[i];
-      const int l = i / A1;
-      const int b = block_list + l;
-      if (v && b < A.B) atomicAdd(&A.bins[(size_t)b * A1 + (i - l * A1)], v);
+      if (v) atomicAdd(&A.bins[(size_t)block_list * A1 + i], v);
     }
   }
 }
@@ -957,19 +980,38 @@ int launch_candidates(hipStream_t st, const RankArgs& A) {
   return check_launch("candidate ranks");
 }
 
+template <class K>
+unsigned long long resident_workgroups(K kernel, int threads, size_t lds) {
+  int dev = 0, cus = 256, per_cu = 2;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds) != hipSuccess || per_cu < 1) per_cu = 2;
+  return (unsigned long long)cus * per_cu;
+}
+
+inline int clear_bins(hipStream_t st, const RankArgs& A) {
+  if (A.slot) return SMX_OK;   // (smx_filtered_ranks has cleared them: rank_prepare_kernel)
+  const size_t n_bins = (size_t)A.B * (A.A + 1);
+  hipLaunchKernelGGL(rank_clear_kernel, dim3((unsigned)((n_bins + 255) / 256)), dim3(256), 0, st, A.bins, n_bins);
+  return check_launch("rank scan (bins)");
+}
+inline int finish_ranks(hipStream_t st, const RankArgs& A) {
+  hipLaunchKernelGGL(rank_finish_kernel, dim3((unsigned)A.B), dim3(64), 0, st, A);
+  return check_launch("rank scan");
+}
+
 template <int M, bool NORM, int VEC, int NB, int UP>
 int launch_scan(hipStream_t st, RankArgs A) {
   constexpr int kLists = 4 * (NB / UP);   // lists of answers a workgroup serves
-  const size_t bins = (size_t)kLists * (A.A + 1) * sizeof(unsigned);
-  A.lds_bins = bins <= (size_t)24 << 10;  // (beside 36 KB of staged rows; longer lists count in memory directly)
-  const size_t lds = A.lds_bins ? bins : 0;
-  int dev = 0, cus = 256, per_cu = 2;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, rank_scan_kernel<M, NORM, VEC, NB, UP>, kScanThreads, lds) != hipSuccess ||
-      per_cu < 1)
-    per_cu = 2;
+  // Keys and bins in LDS beside 36 KB of staged rows while four workgroups still fit a compute unit; then bins alone up to
+  // 24 KB; longer lists count in memory directly.
+  const size_t lists = A.B < kLists ? A.B : kLists, bins = lists * (A.A + 1) * sizeof(unsigned);
+  const size_t keys = lists * A.A * sizeof(unsigned long long);
+  A.lds_bins = bins <= (size_t)24 << 10;
+  A.lds_keys = keys + bins <= (size_t)4 << 10;
+  const size_t lds = (A.lds_bins ? bins : 0) + (A.lds_keys ? keys : 0);
   // several workgroups per slot: the last ones then spread evenly (BetaE's evaluate their queries first: one per slot)
-  const unsigned long long most = (unsigned long long)cus * per_cu * (M == mBetaKL ? 1 : 4);
+  const unsigned long long most =
+      resident_workgroups(rank_scan_kernel<M, NORM, VEC, NB, UP>, kScanThreads, lds) * (M == mBetaKL ? 1 : 4);
   const unsigned blocks = (unsigned)(A.groups < most ? A.groups : most);
   const unsigned passes = (unsigned)((A.B + kLists - 1) / kLists);
   for (unsigned done = 0; done < passes; done += 65535u) {   // (the second grid extent's limit)
@@ -1010,48 +1052,48 @@ int launch_rank_all(hipStream_t st, RankArgs A, int vec, int mode) {
     else hipLaunchKernelGGL((rank_answer_keys_kernel<M, NORM, 1>), dim3((unsigned)A.B * tiles), dim3(64), lds, st, A, bits, tiles);
     return check_launch("rank answer keys");
   }
-  if (!A.slot) {   // (smx_filtered_ranks has cleared them: rank_prepare_kernel)
-    const size_t n_bins = (size_t)A.B * (A.A + 1);
-    hipLaunchKernelGGL(rank_clear_kernel, dim3((unsigned)((n_bins + 255) / 256)), dim3(256), 0, st, A.bins, n_bins);
-  }
+  if (int rc = clear_bins(st, A)) return rc;
   A.groups = (unsigned)((A.n_rows + kScanRows - 1) / kScanRows);
   if (int rc = vec == 4 ? launch_scan_vec<M, NORM, 4>(st, A) : launch_scan_vec<M, NORM, 1>(st, A)) return rc;
-  hipLaunchKernelGGL(rank_finish_kernel, dim3((unsigned)A.B), dim3(64), 0, st, A);
-  return check_launch("rank scan");
+  return finish_ranks(st, A);
+}
+
+// f(VEC, NIT, REG as integral constants) for a call's row shape
+template <int M, class F>
+int with_row_shape(const RankArgs& A, int vec, int nit, F f) {
+  using std::integral_constant;
+  auto with_reg = [&](auto vec_tag, auto nit_tag) {
+    if constexpr (M == mBetaKL || M == mComplex || M == mDistmult) {
+      if (M == mBetaKL ? A.p.reg_on : A.p.norm_on) return f(vec_tag, nit_tag, std::true_type{});
+    }
+    return f(vec_tag, nit_tag, std::false_type{});
+  };
+  if (vec == 4) {
+    switch (nit) {
+      case 1: return with_reg(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+      case 2: return with_reg(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+      case 4: return with_reg(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+      default: return with_reg(integral_constant<int, 4>{}, integral_constant<int, 8>{});
+    }
+  }
+  switch (nit) {
+    case 1: return with_reg(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    case 2: return with_reg(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+    default: return with_reg(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  }
 }
 
 // Instantiated once per model in its own translation unit (smx_rank_inst_*.hip).
 template <int M>
 int rank_dispatch(hipStream_t st, const RankArgs& A, int vec, int nit, int mode) {
-  constexpr bool kHasReg = M == mBetaKL || M == mComplex || M == mDistmult;
-  const bool reg = kHasReg && (M == mBetaKL ? A.p.reg_on : A.p.norm_on);
-  if (mode != kRankCandidates) {
-    if constexpr (M == mComplex || M == mDistmult) {
-      if (reg) return launch_rank_all<M, true>(st, A, vec, mode);
-    }
-    return launch_rank_all<M, false>(st, A, vec, mode);   // (BetaE's clamp is a run-time switch of the scan)
+  if (mode == kRankCandidates)
+    return with_row_shape<M>(A, vec, nit, [&](auto vec_tag, auto nit_tag, auto reg_tag) {
+      return launch_candidates<M, decltype(vec_tag)::value, decltype(nit_tag)::value, decltype(reg_tag)::value>(st, A);
+    });
+  if constexpr (M == mComplex || M == mDistmult) {
+    if (A.p.norm_on) return launch_rank_all<M, true>(st, A, vec, mode);
   }
-  auto candidates = [&](auto vec_tag, auto nit_tag) {
-    constexpr int VEC = decltype(vec_tag)::value, NIT = decltype(nit_tag)::value;
-    if constexpr (kHasReg) {
-      if (reg) return launch_candidates<M, VEC, NIT, true>(st, A);
-    }
-    return launch_candidates<M, VEC, NIT, false>(st, A);
-  };
-  using std::integral_constant;
-  if (vec == 4) {
-    switch (nit) {
-      case 1: return candidates(integral_constant<int, 4>{}, integral_constant<int, 1>{});
-      case 2: return candidates(integral_constant<int, 4>{}, integral_constant<int, 2>{});
-      case 4: return candidates(integral_constant<int, 4>{}, integral_constant<int, 4>{});
-      default: return candidates(integral_constant<int, 4>{}, integral_constant<int, 8>{});
-    }
-  }
-  switch (nit) {
-    case 1: return candidates(integral_constant<int, 1>{}, integral_constant<int, 1>{});
-    case 2: return candidates(integral_constant<int, 1>{}, integral_constant<int, 2>{});
-    default: return candidates(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-  }
+  return launch_rank_all<M, false>(st, A, vec, mode);   // (BetaE's clamp is a run-time switch of the scan)
 }
 
 }  // namespace smx

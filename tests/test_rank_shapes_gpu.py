@@ -75,6 +75,31 @@ def test_ranks_over_the_edges_of_the_scan(model, n, b, dim, most, cen):
         assert parts[i, : len(easy[i]) + len(hard[i])].tolist() == want_e.tolist() + want_h.tolist()
 
 
+@pytest.mark.parametrize("model,b,u,dim,most", [
+    ("l1", 1, 1, 96, 64), ("l1", 1, 1, 33, 40), ("l1", 1, 1, 96, 65), ("box", 2, 1, 100, 64), ("box", 1, 2, 100, 30),
+    ("complex", 1, 1, 50, 9), ("complex", 1, 2, 21, 64), ("complex", 2, 1, 129, 20), ("distmult", 1, 1, 260, 3),
+])
+def test_ranks_of_one_and_two_queries_over_a_long_table(model, b, u, dim, most):
+    """The streaming form: from 20 MB of table, up to two query rows and 64 answers (one case just past each limit)."""
+    from smore_amd import fused
+    from smore_amd.evaluation import filtered_ranks
+    rng = np.random.default_rng(dim)
+    width = dim * (2 if model == "complex" else 1)
+    n = (20 << 20) // (4 * width) + (1 if dim != 50 else -1)
+    table, q1, q2 = _integers(model, n, b * u, dim, rng, offsets=(-2, 5) if model == "box" else (-3, 4))
+    lists = [rng.choice(n, size=most, replace=False).tolist() for _ in range(b)]
+    scores = np.concatenate([orc.score_forward(model, table[None, i:i + 16384].repeat(b * u, 0), q1[:, None],
+                                               None if q2 is None else q2[:, None], 0.0, 0.5) for i in range(0, n, 16384)], axis=1)
+    scores = scores.reshape(b, u, n).max(axis=1)
+    shape = (b, u, dim) if u > 1 else (b, dim)
+    q1, q2 = q1.reshape(shape), None if q2 is None else q2.reshape(shape)
+    got = filtered_ranks(model, dev(table), dev(q1), dev(q2), fused.score_params(0.0, 0.5), [x[::2] for x in lists],
+                         [x[1::2] for x in lists], branches=u)
+    for i in range(b):
+        want_h, want_e = orc.filtered_ranks(scores[i], lists[i][::2], lists[i][1::2])
+        assert got[i][0].tolist() == want_h.tolist() and got[i][1].tolist() == want_e.tolist()
+
+
 @pytest.mark.parametrize("b,u", [(3, 2), (9, 2), (5, 3), (5, 4)])
 def test_union_ranks_with_several_queries_per_pass(b, u):
     from smore_amd import fused
