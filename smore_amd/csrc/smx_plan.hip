@@ -604,7 +604,7 @@ constexpr int kSmallLanes = kSmallThreads / kSmallElems;     // lanes that share
 constexpr int kSmallPer = kSmallPlanMax / kSmallThreads;     // list entries per thread, at most
 constexpr unsigned kSmallEmpty = 0xffffffffu;
 
-// LDS: keys [n], then the hash table [slots] (positions; a power of two, four times n or more), whose place is then taken by
+// LDS: keys [n], then the hash table [slots] (positions; a power of two, two times n or more), whose place is then taken by
 // the keys once more, of first occurrences only
 __global__ __launch_bounds__(kSmallThreads) void plan_small_kernel(const long long* __restrict__ idx, int n, int slot_bits,
                                                                  unsigned long long n_rows,
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kSmallThreads) void plan_small_kernel(const long lo
   }
   if (bad && err && blockIdx.x == 0) *err = 1;
   __syncthreads();
-  // the slot of an id ends up with the first position that holds it (at most a quarter of the slots are taken: a free one
+  // the slot of an id ends up with the first position that holds it (at most half of the slots are taken: a free one
   // or the id's own is always met).  A thread tries its entries' slots together, so that their latencies overlap; an
   // entry that has its slot finds it taken by its own id again, one past the end (compare value 0xfffffffe) takes none.
   const int rounds = (n + kSmallThreads - 1) / kSmallThreads;
@@ -835,25 +835,27 @@ static PlanLayout plan_layout(size_t n, size_t n_rows) {
   return L;
 }
 
+// More than 64 KiB of dynamic LDS: said once per kernel and device (not again under a later stream
+// capture); a runtime that does not know the attribute leaves it to the launch to accept or refuse the size.
+struct LdsAnnouncement {
+  std::mutex mu;
+  bool told[64] = {};
+  void make(const void* kernel, size_t lds) {
+    int dev = 0;
+    if (lds <= 64 * 1024 || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return;
+    std::lock_guard<std::mutex> lock(mu);
+    if (told[dev]) return;
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit());
+    (void)hipGetLastError();
+    told[dev] = true;
+  }
+};
+
 template <int NW, int MAXR, bool IN_IDX, bool OUT_SPLIT>
 static void launch_pass(hipStream_t st, const PlanLayout& L, const SortPassArgs& A) {
   auto kernel = sort_pass_kernel<NW, MAXR, IN_IDX, OUT_SPLIT>;
-  // More than 64 KiB of dynamic LDS: said once per kernel and device (not again under a later stream
-  // capture); a runtime that does not know the attribute leaves it to the launch to accept or refuse the size.
-  if (L.pass_lds > 64 * 1024) {
-    static std::mutex mu;
-    static bool told[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
-      std::lock_guard<std::mutex> lock(mu);
-      if (!told[dev]) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds_limit());
-        (void)hipGetLastError();
-        told[dev] = true;
-      }
-    }
-  }
+  static LdsAnnouncement announcement;
+  announcement.make(reinterpret_cast<const void*>(kernel), L.pass_lds);
   hipLaunchKernelGGL(kernel, dim3((unsigned)L.tiles), dim3(NW * 64), L.pass_lds, st, A);
 }
 
@@ -901,8 +903,11 @@ static int plan_build(void* stream, const int64_t* idx, size_t n_pairs, size_t n
     int slot_bits = 1;
     // 1,024 ids in 2,048 slots 17 us, in 4,096 10 us, in 8,192 8.6 us: the longest probe of the workgroup is what takes the time
     while (slot_bits < 14 && ((size_t)1 << slot_bits) < 5 * n_pairs) ++slot_bits;
-    const size_t lds = (n_pairs + ((size_t)1 << slot_bits)) * sizeof(unsigned);  // at most 80 KiB
-    if (lds > lds_limit()) return fail(SMX_ERR_HIP, "a plan of %zu ids needs %zu bytes of LDS", n_pairs, lds);
+    // at most 80 KiB; where less is to be had, fewer slots do (two per id are 48 KiB for 4,096 ids)
+    while ((n_pairs + ((size_t)1 << slot_bits)) * sizeof(unsigned) > lds_limit() && ((size_t)1 << slot_bits) >= 4 * n_pairs) --slot_bits;
+    const size_t lds = (n_pairs + ((size_t)1 << slot_bits)) * sizeof(unsigned);
+    static LdsAnnouncement announcement;
+    announcement.make(reinterpret_cast<const void*>(plan_small_kernel), lds);
     hipLaunchKernelGGL(plan_small_kernel, dim3((unsigned)((n_pairs + kSmallElems - 1) / kSmallElems)), dim3(kSmallThreads),
                        lds, as_stream(stream), reinterpret_cast<const long long*>(idx), (int)n_pairs, slot_bits,
                        (unsigned long long)n_rows, order, reinterpret_cast<unsigned*>(sorted_ids), seg_of_pos,

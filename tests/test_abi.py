@@ -137,6 +137,20 @@ def test_entity_side_options_are_refused_where_a_model_has_none():
     assert c.sizeof(_lib.ScoreParams) == 28      # seven four-byte fields, as the header declares them
 
 
+@pytest.mark.parametrize("n_ids", [1, 1638, 1639, 4096])
+def test_small_plans_are_not_refused_where_the_lds_limit_cannot_be_asked_for(n_ids):
+    """Without a device the limit reads 64 KiB: a plan comes as far as its launch, which then finds no device."""
+    from smore_amd import _lib
+    import ctypes as c
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the pointers below are not for a device")
+    lib = _lib.load()
+    fake = c.c_void_p(256)
+    rc = lib.smx_plan_build(None, fake, n_ids, 1000, fake, 1 << 30, fake, fake, fake, fake, fake, None, None, fake, None)
+    assert rc != 0 and b"LDS" not in lib.smx_last_error(), lib.smx_last_error()
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from smore_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)
