@@ -793,9 +793,12 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
 // Two launches, so that both halves fill the chip whatever the number of queries: one workgroup per query left 156 of
 // 256 compute units idle at 100 queries of 1,001 candidates (RotatE, 2 x 250 floats: one launch 123 us; scores 34 us, the
 // fabric's rate for random rows, and ranks 12 us).
+// (FUSED, one launch of a workgroup of sixteen wavefronts per query: the second launch costs 3 us, more than it saves up to
+// 64 candidates, 5 us instead of 8.)
 // Scores: a wavefront takes `per_wave` consecutive candidates of one query, the next row on its way while one is summed.
-template <int M, int VEC, int NIT, bool REG, bool UNION>
-__global__ __launch_bounds__(256) void cand_score_kernel(RankArgs A, int tiles, int per_wave) {
+constexpr int kCandFused = 64;
+template <int M, int VEC, int NIT, bool REG, bool UNION, bool FUSED>
+__global__ __launch_bounds__(FUSED ? 1024 : 256) void cand_score_kernel(RankArgs A, int tiles, int per_wave) {
   constexpr int MUL = model_mul(M);
   const int b = blockIdx.x / tiles;
   const int lane = threadIdx.x & 63;
@@ -803,63 +806,89 @@ __global__ __launch_bounds__(256) void cand_score_kernel(RankArgs A, int tiles, 
   const int dim = A.ncol * VEC;
   const int j0 = ((blockIdx.x - b * tiles) * 4 + wave) * per_wave;
   const int n = min(per_wave, A.C - j0);   // (per_wave <= 64: candidate j0 + i lives in lane i)
-  if (n <= 0) return;
-  const long long raw = A.cand[(size_t)b * A.C + j0 + min(lane, n - 1)];
-  const bool pad = raw == -1;
-  unsigned long long id = pad ? 0ull : (unsigned long long)raw;
-  const bool bad = id >= A.n_rows;
-  if (bad) id = 0;
-  if (__ballot(bad) != 0ull && A.err && lane == 0) *A.err = 1;
-  const unsigned long long off = id * (size_t)dim * MUL;
-  typename ModelOps<M>::Q q[NIT][VEC];
-  if constexpr (!UNION) load_rank_query<M, VEC, NIT>(A.q1, A.q2, b, dim, A.ncol, lane, q);
-  float e1[NIT][VEC], e2[NIT][VEC], next1[NIT][VEC], next2[NIT][VEC];
-  auto request = [&](int i) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)off, i);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(off >> 32), i);
-    load_entity<VEC, NIT, MUL>(A.table + (((unsigned long long)hi << 32) | lo), dim, A.ncol, lane, next1, next2);
-  };
-  request(0);
-  for (int i = 0; i < n; ++i) {
+  __shared__ unsigned fused_keys[FUSED ? kCandFused : 1];
+  if (!FUSED && n <= 0) return;
+  if (n > 0) {
+    const long long raw = A.cand[(size_t)b * A.C + j0 + min(lane, n - 1)];
+    const bool pad = raw == -1;
+    unsigned long long id = pad ? 0ull : (unsigned long long)raw;
+    const bool bad = id >= A.n_rows;
+    if (bad) id = 0;
+    if (__ballot(bad) != 0ull && A.err && lane == 0) *A.err = 1;
+    const unsigned long long off = id * (size_t)dim * MUL;
+    typename ModelOps<M>::Q q[NIT][VEC];
+    // The first branch of a union query, or the only row, stays in registers; the others are fetched again per candidate.
+    // (BetaE: all of them, in one set of registers.  100 x 500 candidates, two branches: 228 us, 339 with the first kept.)
+    constexpr bool kKeep = !UNION || M != mBetaKL;
+    if constexpr (kKeep) load_rank_query<M, VEC, NIT>(A.q1, A.q2, b * A.U, dim, A.ncol, lane, q);
+    float e1[NIT][VEC], e2[NIT][VEC], next1[NIT][VEC], next2[NIT][VEC];
+    auto request = [&](int i) {
+      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)off, i);
+      const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(off >> 32), i);
+      load_entity<VEC, NIT, MUL>(A.table + (((unsigned long long)hi << 32) | lo), dim, A.ncol, lane, next1, next2);
+    };
+    request(0);
+    for (int i = 0; i < n; ++i) {
 #pragma unroll
-    for (int it = 0; it < NIT; ++it)
+      for (int it = 0; it < NIT; ++it)
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) {
-        e1[it][v] = next1[it][v];
-        e2[it][v] = MUL == 2 ? next2[it][v] : 0.f;
+        for (int v = 0; v < VEC; ++v) {
+          e1[it][v] = next1[it][v];
+          e2[it][v] = MUL == 2 ? next2[it][v] : 0.f;
+        }
+      request(min(i + 1, n - 1));
+      unit_row<M, VEC, NIT, REG>(e1, e2, A.ncol, lane);
+      float s = 0.f;
+      if constexpr (kKeep) s = row_score<M, VEC, NIT, REG>(e1, e2, q, A.ncol, lane, A.p);
+      if constexpr (UNION) {
+        for (int u = kKeep ? 1 : 0; u < A.U; ++u) {  // uniform
+          typename ModelOps<M>::Q qu[NIT][VEC];
+          load_rank_query<M, VEC, NIT>(A.q1, A.q2, b * A.U + u, dim, A.ncol, lane, qu);
+          const float su = row_score<M, VEC, NIT, REG>(e1, e2, qu, A.ncol, lane, A.p);
+          if (u == 0 || union_takes(su, s)) s = su;
+        }
       }
-    request(min(i + 1, n - 1));
-    unit_row<M, VEC, NIT, REG>(e1, e2, A.ncol, lane);
-    float s = 0.f;
-    if constexpr (UNION) {
-      for (int u = 0; u < A.U; ++u) {  // uniform: the branches of a union query, fetched again per candidate
-        load_rank_query<M, VEC, NIT>(A.q1, A.q2, b * A.U + u, dim, A.ncol, lane, q);
-        const float su = row_score<M, VEC, NIT, REG>(e1, e2, q, A.ncol, lane, A.p);
-        if (u == 0 || union_takes(su, s)) s = su;
+      s += __builtin_amdgcn_readlane((int)pad, i) ? -1e6f : 0.f;
+      if (lane == 63) {
+        const size_t at = (size_t)b * A.C + j0 + i;
+        if (A.cand_logit) A.cand_logit[at] = s;
+        else if (!FUSED) A.cand_rank[at] = (long long)(unsigned long long)__float_as_uint(s);   // the ranking's own slot until it is ranked
+        if constexpr (FUSED) fused_keys[j0 + i] = sortable_bits(s);
       }
-    } else {
-      s = row_score<M, VEC, NIT, REG>(e1, e2, q, A.ncol, lane, A.p);
     }
-    s += __builtin_amdgcn_readlane((int)pad, i) ? -1e6f : 0.f;
-    if (lane == 63) {
-      const size_t at = (size_t)b * A.C + j0 + i;
-      if (A.cand_logit) A.cand_logit[at] = s;
-      else A.cand_rank[at] = (long long)(unsigned long long)__float_as_uint(s);   // the ranking's own slot until it is ranked
+  }
+  if constexpr (FUSED) {   // the ranks, a candidate per lane of the first wavefront
+    __syncthreads();
+    if (wave != 0 || lane >= A.C) return;
+    const unsigned mine = fused_keys[lane];
+    const int n_hard = min(A.n_hard[b], min(A.H, A.C));
+    int before = 0, ahead = 0;
+#pragma unroll 8
+    for (int i = 0; i < A.C; ++i) {
+      const unsigned k = fused_keys[i];
+      const int counts = k > mine || (k == mine && i < lane);
+      before += counts;
+      ahead += i < n_hard ? counts : 0;
     }
+    A.cand_rank[(size_t)b * A.C + lane] = before;
+    if (lane < A.H) A.hard_rank[(size_t)b * A.H + lane] = lane < n_hard ? (long long)(before - ahead + 1) : 0ll;
   }
 }
 
-// Ranks by counting, 64 candidates per workgroup: each of its four wavefronts compares them with a quarter of the
+// Ranks by counting, 64 candidates per workgroup: each of its wavefronts compares them with its share of the
 // query's candidates (four LDS keys per broadcast read) and the counts are added through LDS.  Before position j an
 // equal logit counts, behind it only a larger one does, so one 32-bit compare decides and only the stretch that holds
 // the workgroup's own positions looks at both.  tiles == 1: the workgroup walks all positions of its query (it then may
-// overwrite the scores that stand in the ranking's slots).
-static __global__ __launch_bounds__(256) void cand_rank_kernel(RankArgs A, int tiles) {
-  extern __shared__ __attribute__((aligned(16))) unsigned cand_keys[];  // [C rounded up to a multiple of 16] | int [4][64][2]
+// overwrite the scores that stand in the ranking's slots); it has sixteen wavefronts for that if they
+// have something to do, four otherwise.
+constexpr int cand_padded(int C, int waves) { return (C + 4 * waves - 1) & ~(4 * waves - 1); }
+template <int WAVES>
+static __global__ __launch_bounds__(64 * WAVES) void cand_rank_kernel(RankArgs A, int tiles) {
+  extern __shared__ __attribute__((aligned(16))) unsigned cand_keys[];  // [cand_padded(C, WAVES)] | int [WAVES][64][2]
   const int b = blockIdx.x / tiles, tile = blockIdx.x - b * tiles;
-  const int C16 = (A.C + 15) & ~15;
-  int* part = reinterpret_cast<int*>(cand_keys + C16);
-  for (int i = threadIdx.x; i < C16; i += 256) {
+  const int padded = cand_padded(A.C, WAVES);
+  int* part = reinterpret_cast<int*>(cand_keys + padded);
+  for (int i = threadIdx.x; i < padded; i += 64 * WAVES) {
     unsigned key = 0u;   // (the lowest key, and behind every candidate: never counted)
     if (i < A.C) {
       const size_t at = (size_t)b * A.C + i;
@@ -870,7 +899,7 @@ static __global__ __launch_bounds__(256) void cand_rank_kernel(RankArgs A, int t
   const uint4* keys4 = reinterpret_cast<const uint4*>(cand_keys);
   const int n_hard = min(A.n_hard[b], min(A.H, A.C));
   const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-  const int from = wave * (C16 / 4), to = from + C16 / 4;   // (multiples of 4)
+  const int from = wave * (padded / WAVES), to = from + padded / WAVES;   // (multiples of 4)
   for (int own = tile * 64; own < A.C; own += 64 * tiles) {
     __syncthreads();
     const int j = own + lane;
@@ -904,7 +933,7 @@ static __global__ __launch_bounds__(256) void cand_rank_kernel(RankArgs A, int t
     if (wave == 0 && j < A.C) {
       before = ahead = 0;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
+      for (int w = 0; w < WAVES; ++w) {
         before += part[(w * 64 + lane) * 2];
         ahead += part[(w * 64 + lane) * 2 + 1];
       }
@@ -969,14 +998,22 @@ int launch_candidates(hipStream_t st, const RankArgs& A) {
   int per_wave = 16;   // candidates of a wavefront: fewer when the grid would not fill the chip
   while (per_wave > 1 && (size_t)A.B * ((A.C + 4 * per_wave - 1) / (4 * per_wave)) < 2048) per_wave /= 2;
   const int tiles = (A.C + 4 * per_wave - 1) / (4 * per_wave);
+  if (A.U == 1 && A.C <= kCandFused) {
+    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, false, true>), dim3((unsigned)A.B), dim3(1024), 0, st, A, 1, (A.C + 15) / 16);
+    return check_launch("candidate scores and ranks");
+  }
   if (A.U > 1)
-    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, true>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
+    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, true, false>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
   else
-    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, false>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
+    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, false, false>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
   if (int rc = check_launch("candidate scores")) return rc;
-  const int rank_tiles = A.cand_logit ? (A.C + 63) / 64 : 1;
-  hipLaunchKernelGGL(cand_rank_kernel, dim3((unsigned)A.B * rank_tiles), dim3(256),
-                     (size_t)((A.C + 15) & ~15) * sizeof(unsigned) + 4 * 64 * 2 * sizeof(int), st, A, rank_tiles);
+  auto lds = [&](int waves) { return (size_t)cand_padded(A.C, waves) * sizeof(unsigned) + waves * 64 * 2 * sizeof(int); };
+  if (!A.cand_logit && A.C > 256) {   // (2,048 x 128 candidates: 34 us with sixteen wavefronts, 28 with four)
+    hipLaunchKernelGGL(cand_rank_kernel<16>, dim3((unsigned)A.B), dim3(1024), lds(16), st, A, 1);
+  } else {
+    const int rank_tiles = A.cand_logit ? (A.C + 63) / 64 : 1;
+    hipLaunchKernelGGL(cand_rank_kernel<4>, dim3((unsigned)A.B * rank_tiles), dim3(256), lds(4), st, A, rank_tiles);
+  }
   return check_launch("candidate ranks");
 }
 
