@@ -260,7 +260,7 @@ def test_shared_negatives_next_to_positives_and_anchors_in_one_step():
 
 @pytest.mark.parametrize("n_ids", [1, 2, 63, 64, 65, 1000, 2049, 4096, 4097])
 def test_small_plans_are_the_bits_of_numpy(n_ids):
-    """Up to 4096 ids are sorted by one workgroup in one launch; 4097 take the radix passes.  Same contract."""
+    """Up to 4096 ids are placed by counting in one launch; 4097 take the radix passes.  Same contract."""
     from smore_amd import fused
     rng = np.random.default_rng(n_ids)
     n_rows = 50 if n_ids > 10 else 3
@@ -290,6 +290,55 @@ def test_small_plans_are_the_bits_of_numpy(n_ids):
     ps = plan.pair_seg.cpu().numpy()
     assert np.array_equal(ps < 0, alone) and np.array_equal(ps[alone] & 0x7fffffff, inverse[alone])
     assert np.all(ps[~alone] == 0)
+
+
+def _ids_of_slots(slots, bits, each, rng):
+    """`each` distinct 32-bit ids per slot of the small plans' hash table of 2^bits slots."""
+    ids = rng.integers(0, 2 ** 32 - 1, each << (bits + 1), dtype=np.uint64)
+    slot = ((ids * 2654435761) & 0xffffffff) >> np.uint64(32 - bits)
+    return np.concatenate([np.unique(ids[slot == s])[:each] for s in slots]).astype(np.int64)
+
+
+@pytest.mark.parametrize("n_rows", [50, 0, 20_000_000, 2 ** 32 - 1, "one slot", "last slots"])
+@pytest.mark.parametrize("n_ids", [15, 17, 511, 513, 1638, 1639, 4095])
+def test_small_plans_of_mostly_distinct_ids(n_ids, n_rows):
+    """Around the rounds of 512, the workgroups of 16 and 64 KiB of LDS; tables from 50 rows over 4 n_ids (0) to the largest;
+    ids that share one slot of the hash table, or fill its last ones so that probes wrap, repeated far apart."""
+    from smore_amd import fused
+    rng = np.random.default_rng(n_ids)
+    bits = 1
+    while bits < 14 and 2 ** bits < 5 * n_ids:
+        bits += 1
+    if isinstance(n_rows, str):
+        slots = [2 ** bits // 3] if n_rows == "one slot" else [2 ** bits - 2, 2 ** bits - 1]
+        some = _ids_of_slots(slots, bits, min(60, max(1, n_ids // 4)), rng)
+        n_rows = 2 ** 32 - 1
+        idx = rng.integers(0, n_rows, n_ids)
+        at = rng.choice(n_ids, size=min(n_ids, 2 * some.size), replace=False)
+        idx[at] = np.tile(some, 2)[:at.size]
+    else:
+        n_rows = n_rows or 4 * n_ids
+        idx = rng.integers(0, n_rows, n_ids)
+    idx[[0, n_ids - 1]] = idx[n_ids // 2]
+    bad = np.zeros(n_ids, bool)
+    if n_ids > 500:
+        idx[[5, 300]], bad[[5, 300]] = [n_rows, -1], True
+    err = fused.new_error_flag("cuda")
+    plan = fused.build_plan(torch.tensor(idx, device="cuda"), n_rows, want_inverse=True, err_flag=err)
+    key = np.where(bad, n_rows, idx)
+    order = np.argsort(key, kind="stable")
+    uniq, inverse, counts = np.unique(key, return_inverse=True, return_counts=True)
+    n_seg = uniq.size
+    assert err.item() == int(bad.any()) and plan.n_uniq == n_seg - int(bad.any())
+    assert np.array_equal(plan.uniq.cpu().numpy(), uniq[:plan.n_uniq])
+    assert np.array_equal(plan.order.cpu().numpy(), order)
+    assert np.array_equal(plan.sorted_ids.cpu().numpy().astype(np.int64) & 0xffffffff, key[order])
+    assert np.array_equal(plan.seg_of_pos.cpu().numpy(), inverse[order])
+    assert np.array_equal(plan.seg_start[: n_seg + 1].cpu().numpy(), np.r_[0, np.cumsum(counts)])
+    assert np.array_equal(plan.inverse.cpu().numpy(), inverse)
+    alone = (counts[inverse] == 1) & ~bad
+    ps = plan.pair_seg.cpu().numpy()
+    assert np.array_equal(ps < 0, alone) and np.array_equal(ps[alone] & 0x7fffffff, inverse[alone]) and np.all(ps[~alone] == 0)
 
 
 def test_a_plan_that_gives_up_is_marked_on_the_device_and_nothing_reads_it():
