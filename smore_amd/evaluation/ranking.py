@@ -10,12 +10,27 @@ from .. import _lib
 from ..fused import MODELS, _dims, _on, _ptr, _stream, _workspace
 
 
-def _int64(ids):
-    """Entity ids of one answer list (any sequence of integers, tensors included) as an int64 array."""
+def _plain(values):
+    """Integers of a list, tuple, range, array or host tensor as a one-dimensional int64 array, None for anything else."""
     try:
-        return np.asarray(ids, dtype=np.int64)
-    except (TypeError, ValueError, RuntimeError):       # device tensors, sequences of them
-        return np.asarray([int(x) for x in ids], dtype=np.int64)
+        a = np.asarray(values)
+    except (TypeError, ValueError, RuntimeError):       # device tensors, sequences of them, ragged lists
+        return None
+    return a.astype(np.int64) if a.ndim == 1 and (a.dtype.kind == "i" or not a.size) else None
+
+
+def _int64(ids):
+    """Entity ids of one answer list as an int64 array: what torch takes for integers and nothing else (no strings, no dates)."""
+    a = _plain(ids)
+    return torch.as_tensor(list(ids), dtype=torch.int64).cpu().numpy() if a is None else a
+
+
+def _counts(n_hard):
+    """Hard-answer counts as an int32 tensor, likewise."""
+    a = _plain(n_hard) if isinstance(n_hard, (list, tuple)) else None
+    if a is None or (a.size and (a.min() < 0 or a.max() > 0x7fffffff)):
+        return torch.as_tensor(n_hard, dtype=torch.int32).reshape(-1)
+    return torch.from_numpy(a.astype(np.int32))
 
 
 def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, branches=1):
@@ -77,9 +92,7 @@ def candidate_ranks(model, table, q1, q2, params, negative_sample, n_hard, err_f
         raise _lib.SmxError("negative_sample must be int64 [B, C]")
     dev = table.device
     cand = negative_sample.to(dev).contiguous()
-    if not torch.is_tensor(n_hard):
-        n_hard = torch.from_numpy(np.asarray(n_hard, dtype=np.int32))
-    counts = n_hard.reshape(-1).to(torch.int32)
+    counts = _counts(n_hard)
     low, high = (int(x) for x in counts.aminmax()) if counts.numel() == b else (-1, 0)
     if low < 0 or high > cand.shape[1]:
         raise _lib.SmxError("one hard-answer count per query, between 0 and C")

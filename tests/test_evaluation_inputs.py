@@ -1,0 +1,39 @@
+"""What the evaluation calls take for entity ids and counts: the integers torch.as_tensor takes, no more and no less."""
+import numpy as np
+import pytest
+import torch
+
+VALUES = {
+    "ints": [3, 4], "tuple": (3, 4), "range": range(3), "set": {3, 4}, "keys": {3: 1}.keys(), "empty": [], "array": np.array([3, 4]),
+    "int32": np.array([3, 4], dtype=np.int32), "uint8": np.array([3, 4], dtype=np.uint8), "tensor": torch.tensor([3, 4]),
+    "scalars": [torch.tensor(3), torch.tensor(4)], "one-element tensors": [torch.tensor([3]), torch.tensor([4])],
+    "floats": [1.5, 2.0], "bools": [True, False], "objects": np.array([3, 4], dtype=object), "numpy scalars": [np.int64(3), np.int32(4)],
+    "strings": ["3", "4"], "string": "34", "bytes": b"34", "string array": np.array(["3"]), "dates": np.array(["2020-01-01"], "M8[D]"),
+    "float tensor": torch.tensor([1.5]), "too large": [2 ** 63], "uint64": np.array([2 ** 63 + 1], dtype=np.uint64), "nan": [float("nan")],
+    "none": [None], "ragged": [[1], [2, 3]], "negative": [-1, 2],
+}
+
+
+def _either(f):
+    try:
+        return f().tolist()
+    except Exception as e:
+        return "refused" if isinstance(e, (TypeError, ValueError, RuntimeError, OverflowError)) else e
+
+
+@pytest.mark.parametrize("kind", VALUES)
+def test_answer_ids(kind):
+    from smore_amd.evaluation.ranking import _int64
+    x = VALUES[kind]
+    want = _either(lambda: torch.as_tensor(list(x), dtype=torch.int64))
+    assert _either(lambda: _int64(x)) == want
+    assert want == "refused" or _int64(x).dtype == np.int64
+
+
+@pytest.mark.parametrize("kind", [*VALUES, "scalar", "too large for 32 bits"])
+def test_hard_answer_counts(kind):
+    from smore_amd.evaluation.ranking import _counts
+    x = {"scalar": 3, "too large for 32 bits": [2 ** 31]}.get(kind, VALUES.get(kind))
+    want = _either(lambda: torch.as_tensor(x, dtype=torch.int32).reshape(-1))
+    assert _either(lambda: _counts(x)) == want
+    assert want == "refused" or _counts(x).dtype == torch.int32
