@@ -163,6 +163,7 @@ int smx_filtered_ranks(int model, void* stream, const float* table, size_t n_row
   if (int rc = scan_branches(model, nit, U)) return rc;
   const RanksWs ws = ranks_ws(B, A);
   if (workspace_bytes < ws.bytes) return fail(SMX_ERR_WORKSPACE, "rank workspace too small: %zu < %zu", workspace_bytes, ws.bytes);
+  if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(SMX_ERR_ARG, "workspace must be 256-byte aligned");
   hipStream_t st = as_stream(stream);
   char* base = static_cast<char*>(workspace);
   unsigned long long* key = reinterpret_cast<unsigned long long*>(base + ws.key);

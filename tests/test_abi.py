@@ -137,6 +137,17 @@ def test_entity_side_options_are_refused_where_a_model_has_none():
     assert c.sizeof(_lib.ScoreParams) == 28      # seven four-byte fields, as the header declares them
 
 
+def test_filtered_ranks_refuses_a_workspace_that_is_not_aligned_as_documented():
+    """Keys of eight bytes and counters of four live in it; decided on the host, before any launch."""
+    from smore_amd import _lib
+    import ctypes as c
+    lib = _lib.load()
+    params, fake = _lib.ScoreParams(24.0, 0.02, 0, 0.0, 0.0, 0.0, 0), c.c_void_p(256)      # never dereferenced
+    rc = lib.smx_filtered_ranks(2, None, fake, 100, fake, fake, 2, 1, 8, c.byref(params), fake, fake, 4, None, fake,
+                                c.c_void_p(256 + 8), 1 << 20)
+    assert rc != 0 and b"256-byte aligned" in lib.smx_last_error()
+
+
 @pytest.mark.parametrize("n_ids", [1, 1638, 1639, 4096])
 def test_small_plans_are_not_refused_where_the_lds_limit_cannot_be_asked_for(n_ids):
     """Without a device the limit reads 64 KiB: a plan comes as far as its launch, which then finds no device."""
