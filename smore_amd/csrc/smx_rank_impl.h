@@ -266,11 +266,19 @@ template <int M, bool NORM> struct ScanOps {
       s[0] = 0.f;
     }
   }
+  // Product of a query with a half row of squared length r scaled to unit length.  Where r leaves fp32, scaling first (as
+  // for candidates) gives zeros, and a NaN for an infinite feature; the product here may be infinite for either.
+  static __device__ __forceinline__ float unit_product(float s, float r, const float* half, int dim) {
+    if (r != __builtin_inff()) return s * inv_norm(r);
+    float zero = 0.f;
+    for (int d = 0; d < dim; ++d) zero += half[d] * 0.f;
+    return zero;
+  }
   // logit from the sums and their errors; row_const: BetaE's sum over the row of lgamma(se) - lgamma(ea) - lgamma(eb),
   // query_const: the same of the query with the other sign
   static __device__ __forceinline__ float score(const float (&total)[kSums], const float (&err)[kSums],
                                                 const float (&r)[kRowSums > 0 ? kRowSums : 1], double row_const,
-                                                double query_const, const ScoreParams& p) {
+                                                double query_const, const ScoreParams& p, const float* row, int dim) {
 #pragma clang fp contract(off)
     if constexpr (M == mBetaKL) {
       const double sum = __builtin_isfinite(total[0]) ? (double)total[0] + (double)err[0] : (double)total[0];
@@ -281,8 +289,8 @@ template <int M, bool NORM> struct ScanOps {
     for (int i = 0; i < kSums; ++i) s[i] = with_error(total[i], err[i]);
     if constexpr (M == mL2) return p.gamma - __builtin_amdgcn_sqrtf(s[0]);
     else if constexpr (M == mComplex || M == mDistmult) {
-      float dot = NORM ? s[0] * inv_norm(r[0]) : s[0];
-      if constexpr (NORM && kSums == 2) dot += s[1] * inv_norm(r[1]);
+      float dot = NORM ? unit_product(s[0], r[0], row, dim) : s[0];
+      if constexpr (NORM && kSums == 2) dot += unit_product(s[1], r[1], row + dim, dim);
       return p.gamma + dot;
     } else {
       return p.gamma - s[0];
@@ -488,7 +496,8 @@ __global__ __launch_bounds__(64) void rank_answer_keys_kernel(RankArgs A, int gr
     __syncthreads();  // the next branch writes there
 #pragma unroll
     for (int i = 0; i < NS; ++i) rtot[i] = with_error(rtot[i], rerr[i]);
-    const float su = O::score(tot, err, rtot, row_const, query_const<M>(A, bq, dim, lane), A.p);
+    const float su = O::score(tot, err, rtot, row_const, query_const<M>(A, bq, dim, lane), A.p,
+                              A.table + id * (size_t)dim * MUL, dim);
     if (u == 0 || union_takes(su, best)) best = su;
   }
   if (s0 == 0 && j < A.A) {
@@ -741,7 +750,8 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
         float s = 0.f;
 #pragma unroll
         for (int u = 0; u < UP; ++u) {
-          const float su = O::score(tot[l * UP + u][r], err[l * UP + u][r], rsum, row_const[r], qc[l * UP + u], A.p);
+          const float su = O::score(tot[l * UP + u][r], err[l * UP + u][r], rsum, row_const[r], qc[l * UP + u], A.p,
+                                    A.table + min(id, A.n_rows - 1) * row_len, dim);
           if (u == 0 || union_takes(su, s)) s = su;
         }
         const unsigned long long key = rank_key(s, id);

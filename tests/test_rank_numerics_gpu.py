@@ -183,3 +183,30 @@ def test_answers_are_known_by_their_ids_not_by_their_scores(model, b, branches, 
         assert (_scan(model, t, q1, q2, params, ids, k, branches) == 1).all()
     ranks = filtered_ranks(model, t, q1, q2, params, [list(range(0, n, 2))] * b, [list(range(1, n, 2))] * b, branches)
     assert all((x == 1).all() for pair in ranks for x in pair)
+
+
+@pytest.mark.parametrize("model", ["complex", "distmult"])
+@pytest.mark.parametrize("b,dim", [(1, 100), (5, 33)])
+def test_unit_length_rows_beyond_fp32_score_as_among_candidates(model, b, dim):
+    """A row whose squared length leaves fp32 is scaled to zeros (its logit is gamma), to a NaN where a feature is infinite,
+    also where its product with the query is infinite: the candidate call scales first."""
+    from smore_amd import fused
+    from smore_amd.evaluation import candidate_ranks
+    rng = np.random.default_rng(dim)
+    n = 200
+    table = rng.uniform(-1, 1, (n, _row(model, dim))).astype(np.float32)
+    table[3], table[77, :5], table[130, dim - 1], table[199, 0] = 3e38, -2e38, np.inf, 1e30
+    q = [torch.tensor(rng.uniform(1, 3, (b, dim)), dtype=torch.float32, device="cuda") for _ in range(2)]
+    t, q2 = torch.tensor(table, device="cuda"), None if model in ONE_QUERY else q[1]
+    params = fused.score_params(0.0, norm=True)
+    want, _, _ = candidate_ranks(model, t, q[0], q2, params, _all_ids(b, n), [1] * b)
+    got, keys = _keys(model, t, q[0], q2, params, _all_ids(b, n))
+    assert torch.equal(got.isnan(), want.isnan()) and want.isnan().sum() == b and (got[:, [3, 77, 199]] - want[:, [3, 77, 199]]).abs().max() < 1e-5
+    ids = torch.tensor([[3, 77, 8, 199]], device="cuda").expand(b, 4).contiguous()
+    _, some = _keys(model, t, q[0], q2, params, ids)
+    ranks = _scan(model, t, q[0], q2, params, ids, some)
+    others = np.setdiff1d(np.arange(n), [3, 77, 8, 199])
+    order = keys ^ -(1 << 63)
+    for i in range(b):
+        beats = (order[i, others][:, None] > order[i, ids[i]][None]).sum(dim=0)
+        assert (ranks[i] == beats + 1).all()
