@@ -433,7 +433,7 @@ int smx_sample_loss_static(void* stream, const float* pos, const float* neg, con
  * Filtered ranks of a query's answers among all n_rows entities (the test_all branch of
  * smore/training/train_process.py:112-160: logits of every entity, argsort, ranks of easy + hard
  * answers, minus the answers ranked before) without materialising or sorting the logit row: the
- * table is streamed once per sixteen query rows and every non-answer entity is counted against the answers
+ * table is streamed once per sixteen query rows (once per call for one or two) and every non-answer entity is counted against the answers
  * it ranks before.  Equal scores: the lower entity id ranks first.
  *   ans_id [B, A] int64, ans_count [B] int32: ans_count[b] <= A valid answers (easy and hard alike) per query.
  * smx_rank_answer_keys: ans_score [B, A] = the answers' logits, ans_key [B, A] = their order keys
@@ -473,8 +473,8 @@ int smx_rank_candidates(int model, void* stream, const float* table, size_t n_ro
  * for smx_score_forward_union), and an entity's logit is the maximum over the branches -- the last line of every
  * custom_cal_logit (smore/models/box.py:163, vec.py:89, rotate.py:141, beta.py:307), which the evaluation loop
  * reaches through the same model call as training (train_process.py:112-123).  Everything else as above; the
- * ranks are those of the maximum logits, not the best of the branches' ranks.  U <= 4 (the scan keeps a query's
- * branch rows in registers: rows of more than 512 floats -- 256 for the two-halves models -- allow U <= 2).
+ * ranks are those of the maximum logits, not the best of the branches' ranks.  U <= 4; smx_rank_scan_union and smx_filtered_ranks
+ * allow U <= 2 for rows of more than 512 floats (256 per half of the two-halves models).
  * U == 1 is the plain call. */
 int smx_rank_answer_keys_union(int model, void* stream, const float* table, size_t n_rows, const float* q1,
                                const float* q2, size_t B, size_t U, size_t dim, const smx_score_params* params,

@@ -1,4 +1,4 @@
-// Host side of the all-entity ranking (see smx_rank_impl.h).
+// Host side of the all-entity ranking (see smx_rank_impl.h, smx_rank_stream_impl.h).
 #include "smx_rank_impl.h"
 #include "smx_rank_stream_impl.h"
 
@@ -19,7 +19,7 @@ extern template int rank_stream_dispatch<mComplex>(hipStream_t, const RankArgs&,
 extern template int rank_stream_dispatch<mDistmult>(hipStream_t, const RankArgs&, int, int, int);
 
 constexpr size_t kRankMaxCandidates = 4096;  // per query: their keys live in LDS
-constexpr size_t kRankMaxAnswers = 2048;  // per query; bins and keys of a pass live in LDS (per query of the pass 2049 x 4 + 2048 x 8 bytes)
+constexpr size_t kRankMaxAnswers = 2048;  // per query: rank_prepare_kernel holds a query's keys in LDS
 
 static size_t rank_ws_bytes(size_t B, size_t A) { return (B * (A + 1) * sizeof(unsigned) + 255) & ~(size_t)255; }
 
@@ -37,6 +37,7 @@ static RanksWs ranks_ws(size_t B, size_t A) {
   return w;
 }
 
+// A documented limit of the calls from a scan that kept the branch rows in registers; the present one would not need it.
 static int scan_branches(int model, int nit, size_t U) {
   if (U > 2 && nit * model_mul(model) > 2)
     return fail(SMX_ERR_SHAPE, "union queries of %zu branches over rows this long are not supported by the scan (2 at most)", U);

@@ -46,7 +46,7 @@ struct RankArgs {
   int first_list;                    // query of the launch's first list of answers
   long long* rank_out;               // [B, A]
   const int* slot;                   // [B, A] slot of the j-th key in the order the answers were given in, or null
-  // ranking among sampled candidates (rank_candidates_kernel)
+  // ranking among sampled candidates (cand_score_kernel, cand_rank_kernel)
   const long long* cand;             // [B, C], -1 = padding
   int C, H;
   const int* n_hard;                 // [B]: the first n_hard[b] candidates of query b are its hard answers
@@ -166,8 +166,9 @@ __device__ __forceinline__ void load_rank_query(const float* __restrict__ q1, co
 // owns two of the rows and sums their scores feature by feature, a wavefront does so for NB query rows of its own whose
 // values are scalars.  Every lane then works on every feature (a row spread over the lanes leaves 22 % of them without
 // a column at 400 floats), nothing is summed across lanes, and the table crosses the fabric once per sixteen queries.
-// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, minimum, subtract, add, multiply-add.
-// (Four operations would do: out + cen * in over cen is max(|d|, |d| / cen - o (1 - cen) / cen) for 0 < cen <= 1, 0.64 ms.
+// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, minimum, subtract, multiply-add, add.
+// 1 M x 400 rows, 16 queries: 0.69 ms for 32 G operations (a row per wavefront, a pass per four queries: 1.57 ms).
+// (Four operations would do: out + cen * in over cen is max(|d|, |d| / cen - o (1 - cen) / cen) for 0 < cen <= 1, 0.65 ms.
 // But that rounds values up to 1 / cen times larger than the result: 84 times the error where distances are near the
 // offsets, D = 400, cen = 0.02, twice the error elsewhere.)
 // The sums of a step (32 features, 16 of two-halves models, 8 of BetaE) are added to the row's total with the rounding
@@ -1101,8 +1102,10 @@ int launch_rank_all(hipStream_t st, RankArgs A, int vec, int mode) {
   }
   if (int rc = clear_bins(st, A)) return rc;
   A.groups = (unsigned)((A.n_rows + kScanRows - 1) / kScanRows);
-  if (int rc = vec == 4 ? launch_scan_vec<M, NORM, 4>(st, A) : launch_scan_vec<M, NORM, 1>(st, A)) return rc;
-  return finish_ranks(st, A);
+  int rc;
+  if constexpr (M == mBetaKL) rc = launch_scan_vec<M, NORM, 1>(st, A);   // (fetches single floats at any alignment)
+  else rc = vec == 4 ? launch_scan_vec<M, NORM, 4>(st, A) : launch_scan_vec<M, NORM, 1>(st, A);
+  return rc ? rc : finish_ranks(st, A);
 }
 
 // f(VEC, NIT, REG as integral constants) for a call's row shape

@@ -72,14 +72,10 @@ __global__ __launch_bounds__(kSbThreads) void shared_backward_kernel(SharedBwdAr
     }
   }
   float acc[R][2][4];
-  [[maybe_unused]] float thr[R][4];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      acc[r][0][x] = acc[r][1][x] = 0.f;
-      if constexpr (M == mBox && !ENTITY) thr[r][x] = ModelOps<M>::neg_threshold(ModelOps<M>::prep(kept[r][0][x], kept[r][1][x]));
-    }
+    for (int x = 0; x < 4; ++x) acc[r][0][x] = acc[r][1][x] = 0.f;
 
   const int per = (n_str + kSbStretches - 1) / kSbStretches;
   const int lo = stretch * per, hi = min(n_str, lo + per);
@@ -95,7 +91,6 @@ __global__ __launch_bounds__(kSbThreads) void shared_backward_kernel(SharedBwdAr
         const float x1 = e[0][x], x2 = MUL == 2 ? e[MUL - 1][x] : 0.f;
         const typename ModelOps<M>::Q qq = ModelOps<M>::prep(q[0][x], NQ == 2 ? q[NQ - 1][x] : 0.f);
         if constexpr (ENTITY) ModelOps<M>::bwd_e(c0, c1, x1, x2, qq, acc[r][0][x], acc[r][1][x]);
-        else if constexpr (M == mBox) ModelOps<M>::bwd_q_thr(c0, c1, x1, qq, thr[r][x], acc[r][0][x], acc[r][1][x]);
         else ModelOps<M>::bwd_q(c0, c1, x1, x2, qq, acc[r][0][x], acc[r][1][x]);
       }
     }
