@@ -143,3 +143,69 @@ def test_candidate_ranks_over_the_edges_of_the_tiles(b, c, h):
             assert np.array_equal(ranking[i].cpu().numpy(), rk)
             assert hard[i].tolist() == filt.tolist() + [0] * (h - len(filt))
             assert logit is None or np.array_equal(logit[i].cpu().numpy(), biased)
+
+
+@pytest.mark.parametrize("model,b,u,dim", [("l2", 1, 1, 200), ("rotate", 2, 1, 130), ("rotate", 1, 2, 75), ("complex_norm", 2, 1, 100),
+                                           ("complex_norm", 1, 1, 61), ("distmult_norm", 1, 1, 260), ("box", 2, 1, 500)])
+def test_streamed_ranks_lie_where_fp32_allows_and_equal_rows_tie(model, b, u, dim):
+    """Random floats; a copy of each answer's row ranks before it from a lower id and does not from a higher one."""
+    from smore_amd import fused
+    from smore_amd.evaluation import filtered_ranks
+    rng = np.random.default_rng(dim)
+    model, norm = model.removesuffix("_norm"), model.endswith("_norm")
+    width = dim * (2 if model in ("rotate", "complex") else 1)
+    n = (20 << 20) // (4 * width) + 5
+    t = dev(rng.uniform(-0.2, 0.2, (n, width)))
+    q1 = dev(rng.uniform(-0.2, 0.2, (b, u, dim)))
+    q2 = None if model in ("l2", "distmult") else dev(rng.uniform(0, 0.2, (b, u, dim)))
+    answers = rng.choice(np.arange(1, n - 1), size=(b, 12), replace=False)
+    t[0], t[n - 1] = t[answers[0, 0]], t[answers[0, 1]]
+    params = fused.score_params(0.0, 0.02 if model == "box" else 0.0, norm=norm)
+    got = filtered_ranks(model, t, q1, q2, params, [[]] * b, answers.tolist(), branches=u)
+    table, a, c = t.cpu().numpy().astype(np.float64), q1.cpu().numpy().reshape(b * u, 1, dim).astype(np.float64), None
+    if q2 is not None:
+        c = q2.cpu().numpy().reshape(b * u, 1, dim).astype(np.float64)
+    scores = np.concatenate([orc.score_forward(model, np.broadcast_to(table[None, i:i + 8192], (b * u,) + table[i:i + 8192].shape), a, c,
+                                               0.0, 0.02, norm=norm) for i in range(0, n, 8192)], axis=1).reshape(b, u, n).max(axis=1)
+    for i in range(b):
+        others = np.sort(np.delete(scores[i], answers[i]))
+        tol = 2e-5 * max(1.0, np.abs(scores[i]).max())
+        ranks = got[i][0].cpu().numpy()
+        for x, r in zip(answers[i], ranks):
+            assert 1 + np.sum(others > scores[i, x] + tol) <= r <= 1 + np.sum(others > scores[i, x] - tol)
+    # without the copies (rows behind every other): one rank less after the lower id, the same before the higher one
+    far = q1[0, 0] if q2 is None or model == "box" else torch.cat([q1[0, 0], q2[0, 0]])
+    t[0] = t[n - 1] = -far if model in ("complex", "distmult") else far + 100.0
+    again = filtered_ranks(model, t, q1, q2, params, [[]] * b, answers.tolist(), branches=u)
+    s0, s1 = scores[0, answers[0, 0]], scores[0, answers[0, 1]]
+    assert abs(s0 - s1) > 1e-5
+    assert got[0][0][0].item() == again[0][0][0].item() + 1 + int(s1 > s0)
+    assert got[0][0][1].item() == again[0][0][1].item() + int(s0 > s1)
+
+
+@pytest.mark.parametrize("model", ["l1", "l2", "box", "rotate", "beta_kl", "complex", "complex_norm", "distmult_norm"])
+@pytest.mark.parametrize("b,c,dim", [(1, 1, 40), (3, 33, 37), (5, 64, 520)])
+def test_short_candidate_lists_are_those_of_long_ones(model, b, c, dim):
+    """Up to 64 candidates one launch scores and ranks them: the same bits as a list padded beyond that."""
+    from smore_amd import fused
+    from smore_amd.evaluation import candidate_ranks
+    if dim == 520 and model != "l1":
+        dim = 264
+    rng = np.random.default_rng(c)
+    model, norm = model.removesuffix("_norm"), model.endswith("_norm")
+    n = 300
+    t = dev(rng.uniform(0.1, 2.0, (n, dim * (2 if model in ("rotate", "complex", "beta_kl") else 1))))
+    q1 = dev(rng.uniform(0.1, 2.0, (b, dim)))
+    q2 = None if model in ("l1", "l2", "distmult") else dev(rng.uniform(0.1, 2.0, (b, dim)))
+    params = fused.score_params(24.0, 0.02 if model == "box" else 0.0, norm=norm)
+    neg = rng.integers(0, n, (b, c))
+    neg[:, c // 2: c // 2 + 3] = -1
+    n_hard = [min(3, c)] * b
+    short = candidate_ranks(model, t, q1, q2, params, dev(neg, torch.int64), n_hard)
+    long = candidate_ranks(model, t, q1, q2, params, dev(np.concatenate([neg, np.full((b, 70), -1)], axis=1), torch.int64), n_hard)
+    assert torch.equal(short[0], long[0][:, :c])
+    for i in range(b):
+        _, rank, filtered = orc.candidate_ranks(short[0][i].cpu().numpy() - np.where(neg[i] == -1, np.float32(-1e6), 0), neg[i], n_hard[i])
+        real = neg[i] != -1
+        assert np.array_equal(short[1][i].cpu().numpy()[real], rank[real]) and short[2][i].tolist() == filtered.tolist()
+        assert torch.equal(short[1][i][dev(real, torch.bool)], long[1][i, :c][dev(real, torch.bool)])
