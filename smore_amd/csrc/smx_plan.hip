@@ -266,7 +266,7 @@ struct SortPassArgs {
 // Digits are owned by threads: thread t owns digit t (and t + threads when there are more digits
 // than threads).
 template <int NW, int MAXR, bool IN_IDX, bool OUT_SPLIT>
-__global__ __launch_bounds__(NW * 64, (MAXR <= 8 ? 8 : 4)) void sort_pass_kernel(SortPassArgs A) {
+__global__ __launch_bounds__(NW * 64, 4) void sort_pass_kernel(SortPassArgs A) {
   constexpr int NT = NW * 64;
   constexpr int PER = (1 << kSortMaxDigitBits) / NT > 1 ? (1 << kSortMaxDigitBits) / NT : 1;  // digits per thread, at most
   extern __shared__ __align__(16) unsigned char smem[];
@@ -868,10 +868,19 @@ static void launch_pass_r(hipStream_t st, const PlanLayout& L, const SortPassArg
 }
 template <int NW>
 static void launch_pass_nw(hipStream_t st, const PlanLayout& L, const SortPassArgs& A, bool first, bool last) {
+  // One form per length of a thread's stretch, each with the registers it needs for one workgroup per CU (there are at
+  // most 256 tiles up to 16 elements per thread).  One form for up to 8 elements, held to the 64 registers of two
+  // workgroups per CU, spilled 164 bytes per lane around the look-back's fifteen loads.  Whole plans: 65,536 pairs of
+  // 300 k ids 42.6 -> 35.1 us, 262,144 of 1 M 57.4 -> 49.9, 524,288 of 1 M 64.3 -> 56.9, 1,048,576 of 2.5 M 89.3 -> 77.3.
+  // Fewer, longer tiles in the passes that look back were measured and not kept: twice the length 48.2 / 56.0 / 80.2 us
+  // at the last three sizes, four times 48.7 / 58.7 / 92.1.
   // (a step of B x (1 + K) pairs -- positives beside the negatives -- lies just beyond 256 tiles of 16 elements
-  // per thread and still fits one tile per CU with 17: the third form saves such steps a second round of
+  // per thread and still fits one tile per CU with 17: the last form saves such steps a second round of
   // workgroups, 51 -> 37 us per pass at 4.2 M pairs, at the price of a few spilled registers)
-  if (L.rounds <= 8) launch_pass_r<NW, 8>(st, L, A, first, last);
+  if (L.rounds <= 1) launch_pass_r<NW, 1>(st, L, A, first, last);
+  else if (L.rounds <= 2) launch_pass_r<NW, 2>(st, L, A, first, last);
+  else if (L.rounds <= 4) launch_pass_r<NW, 4>(st, L, A, first, last);
+  else if (L.rounds <= 8) launch_pass_r<NW, 8>(st, L, A, first, last);
   else if (L.rounds <= 16) launch_pass_r<NW, 16>(st, L, A, first, last);
   else launch_pass_r<NW, kSortMaxRounds>(st, L, A, first, last);
 }

@@ -255,7 +255,7 @@ class SegmentPlan:
         self.uniq_buf = torch.empty(n_pairs, dtype=torch.int64, device=device)
         self.inverse = torch.empty(n_pairs, dtype=torch.int64, device=device) if want_inverse else None
         self.pair_seg = torch.empty(n_pairs, **i32)
-        self.n_uniq_dev = torch.zeros(1, **i32)
+        self.n_uniq_dev = torch.empty(1, **i32)   # (every build writes it)
         self._n_uniq = None
 
     @property

@@ -238,6 +238,27 @@ def test_plan_around_the_tile_geometry_boundaries():
         assert torch.equal(plan.seg_start[: plan.n_uniq].long(), torch.nonzero(heads).reshape(-1))
 
 
+@pytest.mark.parametrize("rounds", [2, 8])
+@pytest.mark.parametrize("n", [40_000, 900_000])
+def test_plan_between_the_forms_of_the_radix_pass(rounds, n):
+    """Pair counts around the lengths of a thread's stretch at which another form of the pass takes over, two-pass
+    plans (16- and 20-bit ids): sorted order, stability and segment table against torch's stable sort."""
+    from smore_amd import fused
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rounds)
+    per = 1024 * 256
+    for n_pairs in (rounds * per - 1, rounds * per, rounds * per + 1):
+        ids = torch.randint(0, n, (n_pairs,), device="cuda", generator=gen)
+        ids[: n_pairs // 50] = ids[0]
+        plan = fused.build_plan(ids, n)
+        want_ids, want_order = torch.sort(ids, stable=True)
+        assert torch.equal(plan.sorted_ids.long(), want_ids) and torch.equal(plan.order.long(), want_order), n_pairs
+        heads = torch.ones(n_pairs, dtype=torch.bool, device="cuda")
+        heads[1:] = want_ids[1:] != want_ids[:-1]
+        assert plan.n_uniq == int(heads.sum().item())
+        assert torch.equal(plan.seg_start[: plan.n_uniq].long(), torch.nonzero(heads).reshape(-1))
+
+
 def test_plan_beyond_4096_tiles():
     """More than 4096 tiles of 18 elements per thread: the look-back's three levels end and the chain of prefixes
     over stretches of 4096 tiles takes over.  Sorted order, stability and segment table against torch's stable sort."""
