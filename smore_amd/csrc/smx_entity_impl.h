@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void entity_segment_coded_kernel(EntityArgs A)
         at[s] = todo != 0ull ? __builtin_ctzll(todo) : -1;
         if (at[s] >= 0) {  // wave-uniform
           todo &= todo - 1;
-          request_state<SRC, VEC, NIT>(A, lane, (unsigned)__builtin_amdgcn_readlane((int)my_id, at[s]), st[s]);
+          request_state<SRC, VEC, NIT, false>(A, lane, (unsigned)__builtin_amdgcn_readlane((int)my_id, at[s]), st[s]);
         }
       }
 #pragma unroll
@@ -953,7 +953,7 @@ __global__ __launch_bounds__(256, 4) void entity_tile_coded_kernel(EntityArgs A)
       const unsigned row_id = (unsigned)at(id, rel);
       const bool whole = s0 >= p0 && s1 <= p1;
       RowState<1, VEC, NIT> st;
-      if (whole) request_state<SRC, VEC, NIT>(A, lane, row_id, st);
+      if (whole) request_state<SRC, VEC, NIT, false>(A, lane, row_id, st);
       float g1[NIT][VEC], g2[NIT][VEC];
       zero_acc<VEC, NIT>(g1, g2);
       for (int gbase = pos; gbase < end; gbase += 64 * W) {  // uniform
