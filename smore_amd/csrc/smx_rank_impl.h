@@ -166,8 +166,11 @@ __device__ __forceinline__ void load_rank_query(const float* __restrict__ q1, co
 // owns two of the rows and sums their scores feature by feature, a wavefront does so for NB query rows of its own whose
 // values are scalars.  Every lane then works on every feature (a row spread over the lanes leaves 22 % of them without
 // a column at 400 floats), nothing is summed across lanes, and the table crosses the fabric once per sixteen queries.
-// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, minimum, subtract, multiply-add, add.
-// 1 M x 400 rows, 16 queries: 0.69 ms for 32 G operations (a row per wavefront, a pass per four queries: 1.57 ms).
+// What bounds it: instruction issue.  Box, per (row, query, feature): subtract, minimum, subtract, multiply-add, add.  An
+// addition or multiply-add issues at up to twice the rate of a minimum, and of any instruction with a scalar operand, so
+// cen sits in a VGPR: 1 M x 400 rows, 16 queries 0.69 -> 0.65 ms for 32 G operations (a row per wavefront, a pass per four
+// queries: 1.57 ms).  (The subtracted query values out of LDS as well, a broadcast read per four features and query row:
+// no faster, and RotatE 2 to 5 % slower, LDS then being what bounds it.)
 // (Four operations would do: out + cen * in over cen is max(|d|, |d| / cen - o (1 - cen) / cen) for 0 < cen <= 1, 0.65 ms.
 // But that rounds values up to 1 / cen times larger than the result: 84 times the error where distances are near the
 // offsets, D = 400, cen = 0.02, twice the error elsewhere.)
@@ -585,6 +588,8 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
       }
     }
   };
+  float cen;   // in a VGPR, see above
+  asm("v_mov_b32 %0, %1" : "=v"(cen) : "s"(A.p.cen));
   double lb[kBeta ? kItems : 1];
   auto put = [&](float* to, int d0) {
 #pragma unroll
@@ -637,7 +642,7 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int x = 0; x < NB; ++x) O::template block<N, true>(e[r], a[x], b[x], A.p.cen, s[x][r]);
+      for (int x = 0; x < NB; ++x) O::template block<N, true>(e[r], a[x], b[x], cen, s[x][r]);
       O::template block_row<N>(e[r], rs[r]);
     }
   };
