@@ -416,6 +416,11 @@ int smx_sample_loss(void* stream, const float* pos, const float* neg, const floa
                     const float* weight, size_t B, size_t K, double temperature, double scale,
                     float* out_loss, float* gpos, float* gneg, void* workspace, size_t workspace_bytes);
 
+/* The same pass, and *total (device) = (pos_loss + neg_loss) * scale, the value the training step logs and differentiates. */
+int smx_sample_loss_total(void* stream, const float* pos, const float* neg, const float* mask,
+                          const float* weight, size_t B, size_t K, double temperature, double scale,
+                          float* out_loss, float* total, float* gpos, float* gneg, void* workspace, size_t workspace_bytes);
+
 /* The same pass for callers that cannot allocate or pass a workspace: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.  The
  * 2 B + 1 floats of scratch live in a static device array of the library (one copy per device, 512 KiB,

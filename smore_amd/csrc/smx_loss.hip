@@ -23,9 +23,10 @@ struct LossArgs {
   int B, K;
   float temperature;    // > 0: self-adversarial weights, 0: plain mean over K
   float scale;
-  float* wsum;          // device scalar: sum of weights (or B)
+  float* wsum;          // device scalar: sum of the weights, or null: each workgroup adds them up
   float* per_query;     // [B,2]: W_b logsigmoid(pos_b), W_b s_b
   float* out_loss;      // [2]
+  float* total;         // their sum times scale, or null
   float* gpos;          // [B]
   float* gneg;          // [B,K]
 };
@@ -64,7 +65,18 @@ __global__ __launch_bounds__(256) void loss_rows_kernel(LossArgs A) {
   const float* __restrict__ neg = A.neg + (size_t)b * A.K;
   const float* __restrict__ mask = A.mask ? A.mask + (size_t)b * A.K : nullptr;
   float* __restrict__ gneg = A.gneg + (size_t)b * A.K;
-  const float W = A.weight ? A.weight[b] / *A.wsum : 1.0f / (float)A.B;
+  float W = 1.0f / (float)A.B;
+  if (A.weight) {
+    float wsum;
+    if (A.wsum) {
+      wsum = *A.wsum;
+    } else {   // few queries: every workgroup adds the weights up itself, as loss_weight_sum_kernel does
+      float part = 0.f;
+      for (int i = threadIdx.x; i < A.B; i += 256) part += A.weight[i];
+      wsum = block_sum(part, lds);
+    }
+    W = A.weight[b] / wsum;
+  }
   const float T = A.temperature;
 
   float mx = 0.f, inv_z = 1.0f / (float)A.K;
@@ -105,6 +117,7 @@ __global__ __launch_bounds__(256) void loss_finish_kernel(LossArgs A) {
   if (threadIdx.x == 0) {
     A.out_loss[0] = -p;
     A.out_loss[1] = -s;
+    if (A.total) *A.total = (-p - s) * A.scale;
   }
 }
 
@@ -134,7 +147,7 @@ static float* static_scratch() {
 // Argument checks and launches shared by the two entry points; `buf` holds 2 B + 1 floats.
 static int launch_loss(void* stream, const float* pos, const float* neg, const float* mask, const float* weight,
                        size_t B, size_t K, double temperature, double scale, float* out_loss, float* gpos, float* gneg,
-                       float* buf) {
+                       float* buf, float* total = nullptr) {
   if (!pos || !neg || !out_loss || !gpos || !gneg || !buf) return fail(SMX_ERR_ARG, "null pointer in sample loss");
   if (B == 0 || K == 0 || B > 0x7fffffffull || K > 0x7fffffffull) return fail(SMX_ERR_SHAPE, "empty or oversized batch");
   if (!(temperature >= 0.0)) return fail(SMX_ERR_ARG, "adversarial temperature must be >= 0 (0 = plain mean)");
@@ -148,12 +161,15 @@ static int launch_loss(void* stream, const float* pos, const float* neg, const f
   A.temperature = (float)temperature;
   A.scale = (float)scale;
   A.per_query = buf;
-  A.wsum = buf + 2 * B;
+  // Up to 2,048 queries every workgroup reads all weights (8 KB out of the L2): less than the launch that would do it once,
+  // 4 us.
+  A.wsum = weight && B > 2048 ? buf + 2 * B : nullptr;
   A.out_loss = out_loss;
+  A.total = total;
   A.gpos = gpos;
   A.gneg = gneg;
   hipStream_t st = as_stream(stream);
-  if (weight) hipLaunchKernelGGL(loss_weight_sum_kernel, dim3(1), dim3(256), 0, st, A);
+  if (A.wsum) hipLaunchKernelGGL(loss_weight_sum_kernel, dim3(1), dim3(256), 0, st, A);
   hipLaunchKernelGGL(loss_rows_kernel, dim3((unsigned)B), dim3(256), 0, st, A);
   hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(256), 0, st, A);
   return check_launch("sample loss");
@@ -174,6 +190,17 @@ int smx_sample_loss(void* stream, const float* pos, const float* neg, const floa
     return fail(SMX_ERR_WORKSPACE, "loss workspace too small: %zu < %zu", workspace_bytes, loss_ws_bytes(B));
   return launch_loss(stream, pos, neg, mask, weight, B, K, temperature, scale, out_loss, gpos, gneg,
                      static_cast<float*>(workspace));
+}
+
+int smx_sample_loss_total(void* stream, const float* pos, const float* neg, const float* mask, const float* weight,
+                          size_t B, size_t K, double temperature, double scale, float* out_loss, float* total, float* gpos,
+                          float* gneg, void* workspace, size_t workspace_bytes) {
+  using namespace smx;
+  if (!workspace || !total) return fail(SMX_ERR_ARG, "null pointer in sample loss");
+  if (workspace_bytes < loss_ws_bytes(B))
+    return fail(SMX_ERR_WORKSPACE, "loss workspace too small: %zu < %zu", workspace_bytes, loss_ws_bytes(B));
+  return launch_loss(stream, pos, neg, mask, weight, B, K, temperature, scale, out_loss, gpos, gneg,
+                     static_cast<float*>(workspace), total);
 }
 
 int smx_sample_loss_static(void* stream, const float* pos, const float* neg, const float* mask, const float* weight,

@@ -67,7 +67,7 @@ class _FusedScoreFunc(torch.autograd.Function):
         """q1 / q2 [B * branches, dim].  ids [1, K] against more than one query row: negatives shared by the batch
         (--share_negative), they stay K ids and every row scores them: returns [B * branches, K].  Else ids [B, K];
         with branches > 1 (union queries) the result is the maximum over a query's branch rows, [B, K], and the
-        second output says which branch held it ([B, K] int64; empty for one branch)."""
+        second output says which branch held it ([B, K] uint8; empty for one branch)."""
         table = embed_opt.sparse_embed.embedding.detach()
         ctx.shared = ids.shape[0] == 1 and q1.shape[0] > 1
         ctx.branches = 1 if ctx.shared else branches
@@ -88,12 +88,15 @@ class _FusedScoreFunc(torch.autograd.Function):
         ctx.save_for_backward(q1.detach(), q2.detach() if q2 is not None else None, score)
         ctx.idx_fwd = embed_opt.n_fwd
         embed_opt.n_fwd += 1
-        index = ctx.winner.long() if ctx.winner is not None else torch.empty(0, dtype=torch.int64, device=score.device)
+        index = ctx.winner if ctx.winner is not None else torch.empty(0, dtype=torch.uint8, device=score.device)
         ctx.mark_non_differentiable(index)
+        ctx.set_materialize_grads(False)    # (no zeros for the index)
         return score, index
 
     @staticmethod
     def backward(ctx, gscore, _gindex):
+        if gscore is None:
+            return (None,) * 9
         q1, q2, score = ctx.saved_tensors
         opt = ctx.embed_opt
         table = opt.sparse_embed.embedding.detach()
@@ -147,6 +150,7 @@ class EmbeddingOptimizer(ABC):
         self.check_ids_synchronously = False   # True: every apply_grad waits for the device and raises for its own step
         self._flag_host = torch.zeros(1, dtype=torch.int32, pin_memory=True)   # where the flag of a step lands
         self._flag_event = None                                                # set while such a copy is under way
+        self._flag_copied = None                                               # the event behind it, recorded anew by every step
         self.lazy_lookup = True
         self.stats = self._new_stats()
         self._warned_fallback = False
@@ -418,8 +422,10 @@ class EmbeddingOptimizer(ABC):
         lookup (no table row was updated for the bad id).  check_ids() after the step, or check_ids_synchronously =
         True, fails before anything uses them."""
         self._flag_host.copy_(self.err_flag, non_blocking=True)
-        self._flag_event = torch.cuda.Event()
-        self._flag_event.record()
+        if self._flag_copied is None:
+            self._flag_copied = torch.cuda.Event()
+        self._flag_copied.record()
+        self._flag_event = self._flag_copied
 
     def apply_grad(self, lr):
         """Unique-merge, segment sum and row update of everything recorded since zero_grad().  Pairs whose id

@@ -1050,6 +1050,8 @@ class _LazyIndices(_Delegating):
         self.scores.materialize()
         if self.scores._index is None:      # one branch
             self.scores._index = torch.zeros(self.shape, dtype=torch.int64, device=self.device)
+        elif self.scores._index.dtype is not torch.int64:   # as the scorer leaves it, one byte each
+            self.scores._index = self.scores._index.long()
         return self.scores._index
 
 

@@ -2,6 +2,7 @@
 them (smore/training/train_process.py:112-160), on the streaming HIP scan instead of
 `argsort` over the [1, nentity] logit row."""
 import ctypes
+from itertools import chain
 
 import numpy as np
 import torch
@@ -33,6 +34,23 @@ def _counts(n_hard):
     return torch.from_numpy(a.astype(np.int32))
 
 
+def _pinned(count, dtype):
+    """Host memory a copy to the device need not be waited for from (it is given out again once that copy has passed).
+    Under graph capture pageable memory: such a call is refused, a replay would copy whatever then lies there."""
+    return torch.empty(count, dtype=dtype, pin_memory=not torch.cuda.is_current_stream_capturing())
+
+
+def _to_device(host, dev):
+    return host.to(dev, non_blocking=host.is_pinned())
+
+
+def _one_array(lists):
+    """The ids of all answer lists in a row, where they are plain lists of integers; None otherwise."""
+    if not all(type(ids) in (list, tuple) for ids in lists):
+        return None
+    return _plain(list(chain.from_iterable(lists)))
+
+
 def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, branches=1):
     """model: score model name; table [N,row]; q1/q2 [B,dim] (q2 None for l1/l2); params from
     fused.score_params (gamma, cen, regularizer); easy_answers / hard_answers: per query a sequence of
@@ -48,16 +66,22 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
     n = table.shape[0]
     sizes = [(len(e), len(h)) for e, h in zip(easy_answers, hard_answers)]
     a = max(1, max(ne + nh for ne, nh in sizes))
-    # ids [B, A] and the counts behind them travel to the device as one array
-    packed = np.zeros(b * a + (b + 1) // 2, dtype=np.int64)
+    # ids [B, A] and the counts behind them travel to the device as one array, which nothing waits for
+    host = _pinned(b * a + (b + 1) // 2, torch.int64)
+    packed = host.numpy()
+    packed[:] = 0
     ids, counts = packed[: b * a].reshape(b, a), packed[b * a:].view(np.int32)
-    for i, (e, h) in enumerate(zip(easy_answers, hard_answers)):
-        ne, nh = sizes[i]
-        counts[i] = ne + nh
-        if ne:
-            ids[i, :ne] = _int64(e)
-        if nh:
-            ids[i, ne: ne + nh] = _int64(h)
+    counts[:b] = [ne + nh for ne, nh in sizes]
+    flat = _one_array([x for pair in zip(easy_answers, hard_answers) for x in pair])
+    if flat is not None:
+        ids[np.arange(a) < counts[:b, None]] = flat
+    else:
+        for i, (e, h) in enumerate(zip(easy_answers, hard_answers)):
+            ne, nh = sizes[i]
+            if ne:
+                ids[i, :ne] = _int64(e)
+            if nh:
+                ids[i, ne: ne + nh] = _int64(h)
     used = np.arange(a) < counts[:b, None]
     if ids.min() < 0 or ids.max() >= n:
         raise IndexError("answer id outside the entity table")
@@ -65,7 +89,7 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
     if (ordered[:, 1:] == ordered[:, :-1]).any():
         raise _lib.SmxError("an entity is listed twice among the answers of one query")
     dev = table.device
-    packed = torch.from_numpy(packed).to(dev)
+    packed = _to_device(host, dev)
     ids, counts = packed[: b * a].view(b, a), packed[b * a:]
     q1c = q1.reshape(b * branches, -1).contiguous()
     q2c = None if q2 is None else q2.reshape(b * branches, -1).contiguous()
@@ -75,7 +99,8 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
         ws = _workspace(_lib.load().smx_filtered_ranks_workspace_bytes(MODELS[model], b, branches, a, dim), dev)
         _lib.call("smx_filtered_ranks", MODELS[model], _stream(table), _ptr(table), n, _ptr(q1c), _ptr(q2c), b, branches,
                   dim, ctypes.byref(params), _ptr(ids), _ptr(counts), a, None, _ptr(ranks), _ptr(ws), ws.numel())
-    return [(ranks[i, ne: ne + nh], ranks[i, :ne]) for i, (ne, nh) in enumerate(sizes)]
+    pieces = torch.split(ranks.view(-1), [s for ne, nh in sizes for s in (ne, nh, a - ne - nh)])   # easy, hard, unused
+    return [(pieces[3 * i + 1], pieces[3 * i]) for i in range(b)]
 
 
 def candidate_ranks(model, table, q1, q2, params, negative_sample, n_hard, err_flag=None, branches=1):
@@ -97,7 +122,10 @@ def candidate_ranks(model, table, q1, q2, params, negative_sample, n_hard, err_f
     if low < 0 or high > cand.shape[1]:
         raise _lib.SmxError("one hard-answer count per query, between 0 and C")
     h = max(1, high)
-    counts = counts.to(dev)
+    if counts.device.type == "cpu":
+        host = _pinned(b, torch.int32)
+        host.copy_(counts)
+        counts = _to_device(host, dev)
     q1c = q1.reshape(b * branches, -1).contiguous()
     q2c = None if q2 is None else q2.reshape(b * branches, -1).contiguous()
     _, _, dim = _dims(model, table, cand, q1c[:b], None if q2c is None else q2c[:b])

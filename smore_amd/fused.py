@@ -58,7 +58,7 @@ def _ptr(t):
 def _f32(t, name):
     if t is None:
         return
-    if t.dtype != torch.float32 or not t.is_contiguous() or t.device.type != "cuda":
+    if t.dtype is not torch.float32 or not t.is_contiguous() or not t.is_cuda:
         raise _lib.SmxError(f"{name} must be a contiguous fp32 device tensor")
 
 
@@ -243,20 +243,40 @@ def gather_rows(table, idx, err_flag=None):
 
 
 class SegmentPlan:
-    """Device-resident result of grouping one step's pairs by entity id (see smx_plan_build)."""
+    """Device-resident result of grouping one step's pairs by entity id (see smx_plan_build).  order, sorted_ids,
+    seg_of_pos, pair_seg, seg_start, uniq_buf, n_uniq_dev and inverse (or None) are stretches of one allocation (eight
+    tensors cost a step of a few launches more host time than its kernels); each becomes a tensor when it is asked for."""
 
     def __init__(self, n_pairs, n_rows, device, want_inverse):
-        i32 = dict(dtype=torch.int32, device=device)
         self.n_pairs, self.n_rows = n_pairs, n_rows
-        self.order = torch.empty(n_pairs, **i32)
-        self.sorted_ids = torch.empty(n_pairs, **i32)
-        self.seg_of_pos = torch.empty(n_pairs, **i32)
-        self.seg_start = torch.empty(n_pairs + 1, **i32)
-        self.uniq_buf = torch.empty(n_pairs, dtype=torch.int64, device=device)
-        self.inverse = torch.empty(n_pairs, dtype=torch.int64, device=device) if want_inverse else None
-        self.pair_seg = torch.empty(n_pairs, **i32)
-        self.n_uniq_dev = torch.empty(1, **i32)   # (every build writes it)
+        at, self._arrays = 0, {}
+        for name, count, dtype in (("n_uniq_dev", 1, torch.int32), ("order", n_pairs, torch.int32),
+                                   ("sorted_ids", n_pairs, torch.int32), ("seg_of_pos", n_pairs, torch.int32),
+                                   ("pair_seg", n_pairs, torch.int32), ("seg_start", n_pairs + 1, torch.int32),
+                                   ("uniq_buf", n_pairs, torch.int64), ("inverse", n_pairs, torch.int64)):
+            if name == "inverse" and not want_inverse:
+                self.inverse = None
+                break
+            size = count * (4 if dtype is torch.int32 else 8)
+            self._arrays[name] = (at, size, dtype)
+            at += (size + 255) & ~255
+        self._memory = torch.empty(at, dtype=torch.uint8, device=device)   # (every build writes all of it that it reads)
+        self._base = self._memory.data_ptr()
         self._n_uniq = None
+
+    def __getattr__(self, name):
+        arrays = self.__dict__.get("_arrays")
+        if arrays is None or name not in arrays:
+            raise AttributeError(name)
+        at, size, dtype = arrays[name]
+        tensor = self._memory[at: at + size].view(dtype)
+        self.__dict__[name] = tensor
+        return tensor
+
+    def _at(self, name):
+        """Address of an array; None for an inverse that was not asked for."""
+        entry = self._arrays.get(name)
+        return None if entry is None else self._base + entry[0]
 
     @property
     def n_uniq(self):
@@ -273,8 +293,9 @@ class SegmentPlan:
         return self.uniq_buf[: self.n_uniq]
 
     def view(self):
-        return _lib.PlanView(_ptr(self.order), _ptr(self.sorted_ids), _ptr(self.seg_of_pos), _ptr(self.seg_start),
-                             _ptr(self.uniq_buf), _ptr(self.n_uniq_dev), _ptr(self.pair_seg), self.n_pairs)
+        at = self._at
+        return _lib.PlanView(at("order"), at("sorted_ids"), at("seg_of_pos"), at("seg_start"), at("uniq_buf"),
+                             at("n_uniq_dev"), at("pair_seg"), self.n_pairs)
 
 
 def _workspace(nbytes, device):
@@ -295,9 +316,10 @@ def build_plan(idx, n_rows, want_inverse=False, err_flag=None, measure=None):
             raise _lib.SmxError("smx_plan_workspace_bytes failed")
         ws = _workspace(nbytes, flat.device)
         entry, extra = ("smx_plan_build", ()) if measure is None else ("smx_measure_plan_build", tuple(measure))
-        _lib.call(entry, _stream(flat), _ptr(flat), n, n_rows, _ptr(ws), ws.numel(), _ptr(plan.order),
-                  _ptr(plan.sorted_ids), _ptr(plan.seg_of_pos), _ptr(plan.uniq_buf), _ptr(plan.seg_start),
-                  _ptr(plan.inverse), _ptr(plan.pair_seg), _ptr(plan.n_uniq_dev), _ptr(err_flag), *extra)
+        at = plan._at
+        _lib.call(entry, _stream(flat), _ptr(flat), n, n_rows, _ptr(ws), ws.numel(), at("order"), at("sorted_ids"),
+                  at("seg_of_pos"), at("uniq_buf"), at("seg_start"), at("inverse"), at("pair_seg"), at("n_uniq_dev"),
+                  _ptr(err_flag), *extra)
     return plan
 
 

@@ -9,30 +9,38 @@ import ctypes
 import torch
 
 from .. import _lib
-from ..fused import _ptr, _stream, _workspace
+from ..fused import _on, _ptr, _stream, _workspace
 
 
 class _SampleLossFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pos, neg, mask, weight, temperature, scale):
         b, k = neg.shape
+        total = torch.empty((), dtype=torch.float32, device=neg.device)
         out = torch.empty(2, dtype=torch.float32, device=neg.device)
-        gpos = torch.empty(b, dtype=torch.float32, device=neg.device)
-        gneg = torch.empty((b, k), dtype=torch.float32, device=neg.device)
-        with torch.cuda.device(neg.device):
+        # both gradients in one allocation (one product with the upstream gradient in backward)
+        n_pairs = b * k
+        at = (n_pairs + 63) & ~63
+        grads = torch.empty(at + b, dtype=torch.float32, device=neg.device)
+        with _on(neg.device):
             ws = _workspace(_lib.load().smx_sample_loss_workspace_bytes(b), neg.device)
-            _lib.call("smx_sample_loss", _stream(neg), _ptr(pos), _ptr(neg), _ptr(mask), _ptr(weight), b, k,
-                      ctypes.c_double(temperature), ctypes.c_double(scale), _ptr(out), _ptr(gpos), _ptr(gneg),
-                      _ptr(ws), ws.numel())
-        ctx.save_for_backward(gpos, gneg)
-        ctx.pos_shape = pos.shape
+            _lib.call("smx_sample_loss_total", _stream(neg), _ptr(pos), _ptr(neg), _ptr(mask), _ptr(weight), b, k,
+                      ctypes.c_double(temperature), ctypes.c_double(scale), _ptr(out), _ptr(total),
+                      grads.data_ptr() + 4 * at, _ptr(grads), _ptr(ws), ws.numel())
+        ctx.save_for_backward(grads)
+        ctx.pos_shape, ctx.neg_shape = pos.shape, neg.shape
         ctx.mark_non_differentiable(out)
-        return (out[0] + out[1]) * scale, out
+        ctx.set_materialize_grads(False)    # (none for `out`: a launch that fills zeros nobody reads)
+        return total, out
 
     @staticmethod
     def backward(ctx, g_total, _g_out):
-        gpos, gneg = ctx.saved_tensors
-        return (gpos * g_total).reshape(ctx.pos_shape), gneg * g_total, None, None, None, None
+        if g_total is None:
+            return None, None, None, None, None, None
+        grads, = ctx.saved_tensors
+        b, k = ctx.neg_shape
+        grads = grads * g_total
+        return (grads[grads.numel() - b:].view(ctx.pos_shape), grads[: b * k].view(b, k), None, None, None, None)
 
 
 def sample_loss(positive_logit, negative_logit, is_negative_mat=None, subsampling_weight=None,

@@ -37,3 +37,15 @@ def test_hard_answer_counts(kind):
     want = _either(lambda: torch.as_tensor(x, dtype=torch.int32).reshape(-1))
     assert _either(lambda: _counts(x)) == want
     assert want == "refused" or _counts(x).dtype == torch.int32
+
+
+@pytest.mark.parametrize("kind", VALUES)
+def test_answer_lists_in_one_array(kind):
+    """Lists taken together give what each would alone, or are left to be taken one by one."""
+    from smore_amd.evaluation.ranking import _int64, _one_array
+    lists = [[7, 8], VALUES[kind], (), [9]]
+    flat = _one_array(lists)
+    if flat is not None:
+        assert flat.dtype == np.int64 and flat.tolist() == [int(v) for x in lists for v in _int64(x)]
+    else:
+        assert kind not in ("ints", "tuple", "empty", "numpy scalars", "negative")

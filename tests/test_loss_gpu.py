@@ -39,6 +39,25 @@ def test_sample_loss_matches_oracle(shape, temperature, weighted, masked):
     assert_close(tn.grad.cpu().numpy(), want[3], REL_F32, "gradient of the negative logits")
 
 
+@pytest.mark.parametrize("b", [255, 257, 2048, 2049])
+def test_sample_loss_around_the_batch_from_which_the_weights_are_summed_once(b):
+    """Up to 2,048 queries every workgroup adds the weights up itself, beyond a launch of its own does: the same
+    bits, so scaling all weights by a power of two changes nothing, and both sides meet the oracle."""
+    from smore_amd.training import sample_loss
+    pos, neg, mask, w = _case(b, 5, b)
+    dev = lambda a: torch.tensor(a, dtype=torch.float32, device="cuda")
+    got = []
+    for scale in (1.0, 4.0):
+        tp, tn = dev(pos).requires_grad_(), dev(neg).requires_grad_()
+        loss, pl, nl = sample_loss(tp, tn, dev(mask), dev(w * scale))
+        (3.0 * loss).backward()
+        got.append((loss.detach(), pl, nl, tp.grad, tn.grad))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    want = orc.sample_loss(pos, neg, mask, w, 0.0, 0.5)
+    assert_close(got[0][3].cpu().numpy(), 3.0 * want[2], REL_F32, "gradient of the positive logits")
+    assert_close(got[0][4].cpu().numpy(), 3.0 * want[3], REL_F32, "gradient of the negative logits")
+
+
 def test_saturated_logits_stay_finite():
     from smore_amd.training import sample_loss
     b, k = 4, 8
