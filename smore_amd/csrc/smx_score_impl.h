@@ -290,10 +290,10 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
 
   // LDS: query | per-wavefront pair slabs | code stage (per wavefront; one for the tile with DEDUP) | DEDUP tables
   unsigned* slab = reinterpret_cast<unsigned*>(lds + model_nq(M) * dim) + wave * kSlabDwords;
-  constexpr int kStaged = DEDUP ? 256 : kStagePairs;  // pairs whose code bytes a stage holds
+  constexpr int kStaged = DEDUP ? 256 : kStagePairs;  // pairs whose code bytes a stage holds (DEDUP: tile_k, at most that)
   unsigned char* stage_base = reinterpret_cast<unsigned char*>(lds + model_nq(M) * dim + 4 * kSlabDwords);
   unsigned char* stage = DEDUP ? stage_base : stage_base + wave * (kStaged * NIT * 64);
-  unsigned char* after_stage = stage_base + (CODED ? (size_t)(DEDUP ? 1 : 4) * kStaged * NIT * 64 : 0);
+  unsigned char* after_stage = stage_base + (CODED ? (size_t)(DEDUP ? tile_k : 4 * kStaged) * NIT * 64 : 0);
   unsigned* slot_id = reinterpret_cast<unsigned*>(after_stage);                   // [kDedupSlots]
   int* slot_pos = reinterpret_cast<int*>(slot_id + kDedupSlots);                   // [kDedupSlots]
   uint2* rep_addr = reinterpret_cast<uint2*>(slot_pos + kDedupSlots);              // [256]
@@ -794,12 +794,17 @@ int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
   // ids given (not the dense layout, whose rows are all different): score each distinct entity of a
   // tile once
   // (not for a list of ids shared by the batch: a sampler's K negatives hardly ever repeat)
-  const bool dedup = A.idx != nullptr && !A.ids_shared;
+  // (and not for the short tiles of small batches: few of their ids repeat, and the tables, the barriers and the LDS they
+  // take -- 49 KiB for sign codes of 400 floats, three workgroups per CU -- cost more than the repeats.  Uniform / skewed ids,
+  // us with and without: box 512 x 128 x 400 46 / 43 -> 23 / 22, 400 x 400 x 400 61 / 57 -> 39 / 30, L1 54 / 46 -> 36 / 27 at
+  // 1024 x 128 x 400, L2 512 x 128 x 200 12.8 / 11.5 -> 11.6 / 10.3.  Tiles of 64, 1024 x 512 x 400: box 116 / 87 -> 113 / 68, but
+  // BetaE, whose pairs are arithmetic, 341 / 300 -> 337 / 336 at 200.  Tiles of 128, 2000 x 1000 x 200: L2 162 / 77 -> 164 / 93.)
+  const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= (M == mBetaKL ? 64 : 128);
   if constexpr (model_coded(M) && !REG) {
     if (A.codes) {
       if (dedup)
         hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, true, true>), dim3((unsigned)(B * tiles)),
-                           dim3(256), lds + 256 * NIT * 64 + kDedupLds, st, A, tiles, tile_k);
+                           dim3(256), lds + (size_t)tile_k * NIT * 64 + kDedupLds, st, A, tiles, tile_k);
       else
         hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, true>), dim3((unsigned)(B * tiles)), dim3(256),
                            lds + 4 * kStagePairs * NIT * 64, st, A, tiles, tile_k);
