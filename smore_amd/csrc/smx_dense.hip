@@ -20,6 +20,8 @@
 // reverse layout (entity [B,1,.] against query [B,N,.]) have kernels of the same build.
 #include <type_traits>
 
+#include <type_traits>
+
 #include "smx_common.h"
 #include "smx_functors.h"
 
@@ -160,79 +162,116 @@ __global__ __launch_bounds__(256) void dense_pq_forward_kernel(const float* __re
   }
 }
 
-// One workgroup of eight wavefronts per query.  Lane l owns the 16-byte columns l, l+64, ... of the row
-// (NIT of them); wavefront w takes rows w, w+8, ...  For every row it writes the row's gradient and adds
-// the row's contribution to its query-gradient registers; the eight partial query gradients are summed
+template <int VEC> using column = float __attribute__((ext_vector_type(VEC)));
+
+// Stores the lane's column (VEC floats) of a half row through a buffer descriptor: a lane past the row's end stores nothing,
+// with no branch around the store.  (Loads and stores share one in-order counter, and a wait has to assume the path that issued
+// least: behind a branch, the stores of one row would have to land before the next row, long requested, may be used.)
+template <int VEC>
+__device__ __forceinline__ void store_column(float* half_row, int dim, int c, column<VEC> v) {
+  const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(half_row, 0, dim * (int)sizeof(float), 0x00027000);
+  constexpr int kNonTemporal = 2;
+  if constexpr (VEC == 1) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), row, c * 4, 0, kNonTemporal);
+  } else {
+    typedef unsigned bits __attribute__((ext_vector_type(VEC)));
+    bits t;
+#pragma unroll
+    for (int x = 0; x < VEC; ++x) t[x] = __float_as_uint(v[x]);
+    if constexpr (VEC == 2) __builtin_amdgcn_raw_buffer_store_b64(t, row, c * 8, 0, kNonTemporal);
+    else __builtin_amdgcn_raw_buffer_store_b128(t, row, c * 16, 0, kNonTemporal);
+  }
+}
+
+// One workgroup of NW wavefronts per query.  Lane l owns the columns l, l+64, ... of the row, VEC floats each
+// (NIT of them); wavefront w takes rows w, w+NW, ...  For every row it writes the row's gradient and adds
+// the row's contribution to its query-gradient registers, the next row on its way; the partial query gradients are summed
 // through LDS in wavefront order, so the result does not depend on timing.
 // SHARED: the entity rows are the same [1,N,.] for every query (--share_negative, online_sampler.py:155-157);
 // this kernel then gives the query gradients only, and dense_shared_entity_backward_kernel the rows'.
-template <int K, int NIT, bool SHARED = false>
-__global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_pq_backward_kernel(
+// What bounds it: memory, given enough rows in flight where a few hundred queries leave a CU one or two workgroups.
+// The next row in flight, and stores that no wait depends on: box 64 x 512 x 400 69 -> 25 us, L1 100 x 400 x 400 50 -> 22,
+// box 300 x 333 x 400 58 -> 55 (5.8 TB/s).
+template <int K, int NIT, bool SHARED = false, int NW = kPqBwdWaves, int VEC = 4>
+__global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
     const float* __restrict__ gout, const float* __restrict__ ent, const float* __restrict__ q1,
     const float* __restrict__ q2, float* __restrict__ gent, float* __restrict__ gq1, float* __restrict__ gq2, int num,
     int dim) {
   constexpr int MUL = kind_mul(K), NQ = kind_nq(K);
+  typedef column<VEC> vec;
   extern __shared__ float lds[];  // [waves][NQ][dim]
   const int b = blockIdx.x;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int ncol = dim / 4;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int ncol = dim / VEC;
   const size_t row_len = (size_t)dim * MUL;
-  const dvec4 zero = {0.f, 0.f, 0.f, 0.f};
-  dvec4 qa[NIT], qb[NIT], acc1[NIT], acc2[NIT];
+  const vec zero = (vec)(0.f);
+  vec qa[NIT], qb[NIT], acc1[NIT], acc2[NIT];
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = min(lane + kWave * it, ncol - 1);
-    qa[it] = reinterpret_cast<const dvec4*>(q1 + (size_t)b * dim)[c];
-    qb[it] = NQ == 2 ? reinterpret_cast<const dvec4*>(q2 + (size_t)b * dim)[c] : zero;
+    qa[it] = reinterpret_cast<const vec*>(q1 + (size_t)b * dim)[c];
+    qb[it] = NQ == 2 ? reinterpret_cast<const vec*>(q2 + (size_t)b * dim)[c] : zero;
     acc1[it] = acc2[it] = zero;
   }
-  for (int k = wave; k < num; k += kPqBwdWaves) {
+  struct Row {
+    float g;
+    vec e1[NIT], e2[NIT];
+  };
+  auto request = [&](int k, Row& row) {   // (past the last row: that one once more)
+    k = min(k, num - 1);
     const size_t r = (size_t)b * num + k;
-    const float g = gout[r];
-    const size_t er = SHARED ? (size_t)k : r;
-    const dvec4* pe = reinterpret_cast<const dvec4*>(ent + er * row_len);
-    dvec4* pg = reinterpret_cast<dvec4*>(gent + er * row_len);
-    dvec4 e1[NIT], e2[NIT];
+    row.g = gout[r];
+    const vec* pe = reinterpret_cast<const vec*>(ent + (SHARED ? (size_t)k : r) * row_len);
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int c = min(lane + kWave * it, ncol - 1);
-      e1[it] = pe[c];
-      e2[it] = MUL == 2 ? pe[c + ncol] : zero;
+      row.e1[it] = pe[c];
+      row.e2[it] = MUL == 2 ? pe[c + ncol] : zero;
     }
+  };
+  auto use = [&](int k, const Row& row) {
+    float* pg = gent + ((size_t)b * num + k) * row_len;
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-      const int c = lane + kWave * it;
-      if (c < ncol) {
-        dvec4 ge1 = zero, ge2 = zero;
+      // lanes past the row end hold a copy of the last column: what they compute is not stored
+      vec ge1 = zero, ge2 = zero;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          float a1 = 0.f, a2 = 0.f, b1 = acc1[it][x], b2 = acc2[it][x];
-          Term<K, float>::bwd(g, e1[it][x], e2[it][x], qa[it][x], qb[it][x], a1, a2, b1, b2);
-          ge1[x] = a1;
-          ge2[x] = a2;
-          acc1[it][x] = b1;
-          acc2[it][x] = b2;
-        }
-        if (!SHARED) {
-          __builtin_nontemporal_store(ge1, pg + c);
-          if (MUL == 2) __builtin_nontemporal_store(ge2, pg + c + ncol);
-        }
+      for (int x = 0; x < VEC; ++x) {
+        float a1 = 0.f, a2 = 0.f, b1 = acc1[it][x], b2 = acc2[it][x];
+        Term<K, float>::bwd(row.g, row.e1[it][x], row.e2[it][x], qa[it][x], qb[it][x], a1, a2, b1, b2);
+        ge1[x] = a1;
+        ge2[x] = a2;
+        acc1[it][x] = b1;
+        acc2[it][x] = b2;
+      }
+      if (!SHARED) {
+        store_column<VEC>(pg, dim, lane + kWave * it, ge1);
+        if (MUL == 2) store_column<VEC>(pg + dim, dim, lane + kWave * it, ge2);
       }
     }
+  };
+  Row row_a, row_b;
+  request(wave, row_a);
+  for (int k = wave; k < num; k += 2 * NW) {
+    request(k + NW, row_b);
+    use(k, row_a);
+    if (k + NW >= num) break;
+    request(k + 2 * NW, row_a);
+    use(k + NW, row_b);
   }
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = lane + kWave * it;
     if (c < ncol) {
-      reinterpret_cast<dvec4*>(lds + (size_t)(wave * NQ + 0) * dim)[c] = acc1[it];
-      if (NQ == 2) reinterpret_cast<dvec4*>(lds + (size_t)(wave * NQ + 1) * dim)[c] = acc2[it];
+      reinterpret_cast<vec*>(lds + (size_t)(wave * NQ + 0) * dim)[c] = acc1[it];
+      if (NQ == 2) reinterpret_cast<vec*>(lds + (size_t)(wave * NQ + 1) * dim)[c] = acc2[it];
     }
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < dim; d += kPqBwdWaves * kWave) {
+  for (int d = threadIdx.x; d < dim; d += NW * kWave) {
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int w = 0; w < kPqBwdWaves; ++w) {
+    for (int w = 0; w < NW; ++w) {
       s1 += lds[(size_t)(w * NQ + 0) * dim + d];
       if (NQ == 2) s2 += lds[(size_t)(w * NQ + 1) * dim + d];
     }
@@ -486,6 +525,18 @@ static bool pq_layout(const Layout& L, int kind, const void* a, const void* b, c
   return aligned16(a) && aligned16(b) && aligned16(c) && aligned16(d) && aligned16(e) && aligned16(f) && aligned16(g);
 }
 
+// Floats per column of the per-query backward for a call, 0: not its layout.  Rows that are not made of 16-byte columns take
+// 8- or 4-byte ones up to 512 floats (the general kernels form each row's and each query's gradient by itself: rotate
+// 300 x 333 x 250 571 us against 76 here, box 300 x 333 x 201 487 against 31, L1 100 x 400 x 330 666 against 30).
+static int pq_backward_vec(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
+                           const void* f, const void* g) {
+  if (pq_layout(L, 0, a, b, c, d, e, f, g)) return 4;
+  if (L.be != L.bsize || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.dim > 512) return 0;
+  if (L.bsize * L.num > 0x7fffffffull || L.bsize > 0x7fffffffull) return 0;
+  auto even = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  return L.dim % 2 == 0 && even(a) && even(b) && even(c) && even(d) && even(e) && even(f) && even(g) ? 2 : 1;
+}
+
 template <int K, bool SHARED = false>
 static int forward_pq(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L) {
   // enough workgroups to fill the chip, at least eight rows each when there are that many
@@ -501,17 +552,35 @@ static int forward_pq(hipStream_t st, const float* ent, const float* q1, const f
 
 template <int K>
 static int backward_pq(hipStream_t st, const float* gout, const float* ent, const float* q1, const float* q2, float* gent,
-                       float* gq1, float* gq2, const Layout& L) {
-  const size_t lds = (size_t)kPqBwdWaves * kind_nq(K) * L.dim * sizeof(float);
-  const dim3 grid((unsigned)L.bsize), block(kPqBwdWaves * kWave);
+                       float* gq1, float* gq2, const Layout& L, int vec) {
   const int num = (int)L.num, dim = (int)L.dim;
-  const size_t ncol = L.dim / 4;
-  if (ncol <= 64)
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, 1>), grid, block, lds, st, gout, ent, q1, q2, gent, gq1, gq2, num, dim);
-  else if (ncol <= 128)
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, 2>), grid, block, lds, st, gout, ent, q1, q2, gent, gq1, gq2, num, dim);
-  else
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, 4>), grid, block, lds, st, gout, ent, q1, q2, gent, gq1, gq2, num, dim);
+  auto launch = [&](auto nit, auto waves, auto vec) {
+    constexpr int NIT = decltype(nit)::value, NW = decltype(waves)::value, VEC = decltype(vec)::value;
+    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, false, NW, VEC>), dim3((unsigned)L.bsize), dim3(NW * kWave),
+                       (size_t)NW * kind_nq(K) * L.dim * sizeof(float), st, gout, ent, q1, q2, gent, gq1, gq2, num, dim);
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 1> one;
+  constexpr integral_constant<int, 2> two;
+  constexpr integral_constant<int, 4> four;
+  constexpr integral_constant<int, 8> eight;
+  constexpr integral_constant<int, 16> sixteen;
+  const size_t ncol = L.dim / vec;
+  if (vec == 2) {
+    ncol <= 128 ? launch(two, eight, two) : launch(four, eight, two);
+  } else if (vec == 1) {
+    ncol <= 256 ? launch(four, eight, one) : launch(eight, eight, one);
+  } else if (ncol <= 32 || (kind_mul(K) == 1 && ncol <= 128 && L.bsize <= 256)) {
+    // (few queries: a CU has one workgroup, or none.  Eight / sixteen wavefronts, box 64 x 512 x 400 32 / 25 us, 512 x 512 x 100
+    // 42 / 37; two halves of long rows, BetaE 200 x 200 x 400, are slower with sixteen: 134 / 234, the registers do not suffice)
+    ncol <= 64 ? launch(one, sixteen, four) : launch(two, sixteen, four);
+  } else if (ncol <= 64) {
+    launch(one, eight, four);
+  } else if (ncol <= 128) {
+    launch(two, eight, four);
+  } else {
+    launch(four, eight, four);
+  }
   return check_launch("dist backward (per-query layout)");
 }
 
@@ -607,11 +676,11 @@ int dense_backward(int kind, void* stream, const T* gout, const T* ent, const T*
     return fail(SMX_ERR_ARG, "null tensor pointer");
   hipStream_t st = as_stream(stream);
   if constexpr (std::is_same<T, float>::value) {
-    if (pq_layout(L, kind, gout, ent, q1, q2, gent, gq1, gq2)) {
+    if (const int vec = pq_backward_vec(L, gout, ent, q1, q2, gent, gq1, gq2)) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L);
+    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, vec);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }

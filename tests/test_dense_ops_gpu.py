@@ -58,6 +58,42 @@ def test_dense_forward_backward(kind, layout, dtype):
 
 
 @pytest.mark.parametrize("kind", list(orc.KINDS))
+@pytest.mark.parametrize("b,k,dims", [(3, 1, (1, 2, 3, 63, 65)), (2, 17, (66, 127, 130, 254, 255)), (5, 9, (257, 258, 510, 511, 514)),
+                                      (3, 33, (4, 128, 132, 256)), (260, 3, (4, 256, 260)), (257, 18, (128, 132))])
+def test_backward_of_per_query_rows_of_any_width(kind, b, k, dims):
+    """The per-query backward with columns of four, two and one floats, from tensors that start on any 4-byte
+    boundary, and with sixteen or eight wavefronts per query (batches of up to 256, or rows of up to 32 columns)."""
+    from smore_amd import extlib_hip as ext
+    for dim in dims:
+        rng = np.random.default_rng(seed(kind, b, k, dim))
+        e, q1, q2 = make_inputs(kind, b, k, b, 1, dim, rng)
+        gout = rng.standard_normal((b, k))
+        e, q1, gout = (x.astype(np.float32).astype(np.float64) for x in (e, q1, gout))
+        q2 = None if q2 is None else q2.astype(np.float32).astype(np.float64)
+        oe, o1, o2 = orc.dist_backward(kind, gout, e, q1, q2)
+        for shift in (0, 1):
+            def place(x):       # contiguous, `shift` floats behind an allocation's start
+                if x is None:
+                    return None
+                flat = torch.full((x.size + 2 * shift,), float("nan"), device="cuda")
+                out = flat[shift: shift + x.size].view(x.shape)
+                return out.copy_(torch.tensor(x, dtype=torch.float32))
+            te, t1, t2, tg = (place(x) for x in (e, q1, q2, gout))
+            ge, g1, g2 = (place(None if x is None else np.full(x.shape, np.nan)) for x in (e, q1, q2))
+            ext.dist_backward(kind, tg, te, t1, t2, ge, g1, g2, t2 is not None)
+            assert_close(ge.cpu().numpy(), oe, REL_F32, f"{kind} gent dim={dim}")
+            # a sum over k signed terms: one fp32 ulp of their magnitudes is the floor of any order (see assert_close)
+            mag = [None if o is None else np.abs(o) + np.abs(gout).sum(axis=1)[:, None, None] for o in (o1, o2)]
+            assert_close(g1.cpu().numpy(), o1, REL_F32, f"{kind} gq1 dim={dim}", sum_abs=mag[0])
+            if t2 is not None:
+                assert_close(g2.cpu().numpy(), o2, REL_F32, f"{kind} gq2 dim={dim}", sum_abs=mag[1])
+            for t in (ge, g1, g2):      # nothing behind or before the tensor's own values was written
+                if t is not None and shift:
+                    store = torch.as_strided(t, (t.numel() + 2,), (1,), 0)
+                    assert bool(store[0].isnan()) and bool(store[-1].isnan())
+
+
+@pytest.mark.parametrize("kind", list(orc.KINDS))
 @pytest.mark.parametrize("layout", [(6, 9, 6, 1), (1, 11, 5, 1), (4, 1, 4, 1), (5, 1, 5, 10)])
 def test_long_rows_in_the_per_query_and_shared_layouts(kind, layout):
     """Rows of two and four 256-float column groups (and one just past the vector kernels' 1024-float limit)
