@@ -283,19 +283,20 @@ __global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
 // Shared entity rows: gradient of row j = sum over the queries i of gout[i,j] * d term / d e.  One
 // workgroup per row, the row in registers; wavefront w takes queries w, w+8, ... in ascending order and
 // the eight partial sums are combined through LDS in wavefront order.
-template <int K, int NIT>
+template <int K, int NIT, int VEC>
 __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backward_kernel(
     const float* __restrict__ gout, const float* __restrict__ ent, const float* __restrict__ q1,
     const float* __restrict__ q2, float* __restrict__ gent, int bsize, int num, int dim) {
   constexpr int MUL = kind_mul(K), NQ = kind_nq(K);
+  typedef column<VEC> vec;
   extern __shared__ float lds[];  // [waves][MUL][dim]
   const int j = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int ncol = dim / 4;
+  const int ncol = dim / VEC;
   const size_t row_len = (size_t)dim * MUL;
-  const dvec4 zero = {0.f, 0.f, 0.f, 0.f};
-  dvec4 e1[NIT], e2[NIT], acc1[NIT], acc2[NIT];
-  const dvec4* pe = reinterpret_cast<const dvec4*>(ent + (size_t)j * row_len);
+  const vec zero = (vec)(0.f);
+  vec e1[NIT], e2[NIT], acc1[NIT], acc2[NIT];
+  const vec* pe = reinterpret_cast<const vec*>(ent + (size_t)j * row_len);
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = min(lane + kWave * it, ncol - 1);
@@ -305,9 +306,9 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backw
   }
   for (int i = wave; i < bsize; i += kPqBwdWaves) {
     const float g = gout[(size_t)i * num + j];
-    const dvec4* pa = reinterpret_cast<const dvec4*>(q1 + (size_t)i * dim);
-    const dvec4* pb = reinterpret_cast<const dvec4*>(q2 + (size_t)i * dim);
-    dvec4 qa[NIT], qb[NIT];
+    const vec* pa = reinterpret_cast<const vec*>(q1 + (size_t)i * dim);
+    const vec* pb = reinterpret_cast<const vec*>(q2 + (size_t)i * dim);
+    vec qa[NIT], qb[NIT];
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int c = min(lane + kWave * it, ncol - 1);
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backw
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
+      for (int x = 0; x < VEC; ++x) {
         float a1 = acc1[it][x], a2 = acc2[it][x], s1 = 0.f, s2 = 0.f;
         Term<K, float>::bwd(g, e1[it][x], e2[it][x], qa[it][x], qb[it][x], a1, a2, s1, s2);
         acc1[it][x] = a1;
@@ -329,8 +330,8 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backw
   for (int it = 0; it < NIT; ++it) {
     const int c = lane + kWave * it;
     if (c < ncol) {
-      reinterpret_cast<dvec4*>(lds + (size_t)(wave * MUL + 0) * dim)[c] = acc1[it];
-      if (MUL == 2) reinterpret_cast<dvec4*>(lds + (size_t)(wave * MUL + 1) * dim)[c] = acc2[it];
+      reinterpret_cast<vec*>(lds + (size_t)(wave * MUL + 0) * dim)[c] = acc1[it];
+      if (MUL == 2) reinterpret_cast<vec*>(lds + (size_t)(wave * MUL + 1) * dim)[c] = acc2[it];
     }
   }
   __syncthreads();
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backw
   }
 }
 
-// entity [1,N,.] shared by the queries [B,1,.]
+// entity [1,N,.] shared by the queries [B,1,.], float4-able
 static bool shared_layout(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
                           const void* f, const void* g) {
   if (L.be != 1 || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.bsize < 2) return false;
@@ -351,27 +352,54 @@ static bool shared_layout(const Layout& L, const void* a, const void* b, const v
   return aligned16(a) && aligned16(b) && aligned16(c) && aligned16(d) && aligned16(e) && aligned16(f) && aligned16(g);
 }
 
+// 8- or 4-byte columns for tensors whose rows are not made of 16-byte ones
+static int narrow_vec(size_t dim, const void* a, const void* b, const void* c, const void* d, const void* e, const void* f,
+                      const void* g) {
+  auto even = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  return dim % 2 == 0 && even(a) && even(b) && even(c) && even(d) && even(e) && even(f) && even(g) ? 2 : 1;
+}
+
+// Floats per column of the shared backward for a call, 0: not its layout (see pq_backward_vec; L1 512 x 1024 x 330 135 us, box
+// 300 x 500 x 283 66, 2,378 and 1,132 with the general kernels).
+static int shared_backward_vec(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
+                               const void* f, const void* g) {
+  if (shared_layout(L, a, b, c, d, e, f, g)) return 4;
+  if (L.be != 1 || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.bsize < 2 || L.dim > 512) return 0;
+  if (L.bsize * L.num > 0x7fffffffull) return 0;
+  return narrow_vec(L.dim, a, b, c, d, e, f, g);
+}
+
 template <int K>
 static int backward_shared(hipStream_t st, const float* gout, const float* ent, const float* q1, const float* q2,
-                           float* gent, float* gq1, float* gq2, const Layout& L) {
+                           float* gent, float* gq1, float* gq2, const Layout& L, int vec) {
   const dim3 block(kPqBwdWaves * kWave);
   const int num = (int)L.num, dim = (int)L.dim, bsize = (int)L.bsize;
-  const size_t ncol = L.dim / 4;
   const size_t lds_q = (size_t)kPqBwdWaves * kind_nq(K) * L.dim * sizeof(float);
   const size_t lds_e = (size_t)kPqBwdWaves * kind_mul(K) * L.dim * sizeof(float);
-#define SMX_SHARED_LAUNCH(NIT_)                                                                                        \
-  hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT_, true>), dim3((unsigned)L.bsize), block, lds_q, st, gout, ent, q1, \
-                     q2, gent, gq1, gq2, num, dim);                                                                    \
-  hipLaunchKernelGGL((dense_shared_entity_backward_kernel<K, NIT_>), dim3((unsigned)L.num), block, lds_e, st, gout, ent,  \
-                     q1, q2, gent, bsize, num, dim);
-  if (ncol <= 64) {
-    SMX_SHARED_LAUNCH(1)
+  auto launch = [&](auto nit, auto v) {
+    constexpr int NIT = decltype(nit)::value, VEC = decltype(v)::value;
+    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, true, kPqBwdWaves, VEC>), dim3((unsigned)L.bsize), block, lds_q, st,
+                       gout, ent, q1, q2, gent, gq1, gq2, num, dim);
+    hipLaunchKernelGGL((dense_shared_entity_backward_kernel<K, NIT, VEC>), dim3((unsigned)L.num), block, lds_e, st, gout, ent,
+                       q1, q2, gent, bsize, num, dim);
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 1> one;
+  constexpr integral_constant<int, 2> two;
+  constexpr integral_constant<int, 4> four;
+  constexpr integral_constant<int, 8> eight;
+  const size_t ncol = L.dim / vec;
+  if (vec == 2) {
+    ncol <= 128 ? launch(two, two) : launch(four, two);
+  } else if (vec == 1) {
+    ncol <= 256 ? launch(four, one) : launch(eight, one);
+  } else if (ncol <= 64) {
+    launch(one, four);
   } else if (ncol <= 128) {
-    SMX_SHARED_LAUNCH(2)
+    launch(two, four);
   } else {
-    SMX_SHARED_LAUNCH(4)
+    launch(four, four);
   }
-#undef SMX_SHARED_LAUNCH
   return check_launch("dist backward (shared entity rows)");
 }
 
@@ -533,8 +561,7 @@ static int pq_backward_vec(const Layout& L, const void* a, const void* b, const 
   if (pq_layout(L, 0, a, b, c, d, e, f, g)) return 4;
   if (L.be != L.bsize || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.dim > 512) return 0;
   if (L.bsize * L.num > 0x7fffffffull || L.bsize > 0x7fffffffull) return 0;
-  auto even = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
-  return L.dim % 2 == 0 && even(a) && even(b) && even(c) && even(d) && even(e) && even(f) && even(g) ? 2 : 1;
+  return narrow_vec(L.dim, a, b, c, d, e, f, g);
 }
 
 template <int K, bool SHARED = false>
@@ -687,11 +714,11 @@ int dense_backward(int kind, void* stream, const T* gout, const T* ent, const T*
     }
   }
   if constexpr (std::is_same<T, float>::value) {
-    if (shared_layout(L, gout, ent, q1, q2, gent, gq1, gq2)) {
+    if (const int vec = shared_backward_vec(L, gout, ent, q1, q2, gent, gq1, gq2)) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return backward_shared<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L);
+    return backward_shared<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, vec);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
