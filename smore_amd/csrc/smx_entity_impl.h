@@ -349,19 +349,18 @@ constexpr int kRunsLong = 4;
 // wavefront then finishes one segment after the other, and while it works on one it already has
 // the next one's w, m, v rows on the way (two register sets used in turn).
 template <int SRC, int VEC, int NIT, bool REG>
-__global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
+__device__ __forceinline__ void segment_pass(const EntityArgs& A, int block, int blocks) {
   constexpr int MUL = src_mul(SRC);
   constexpr int R = kRunsShort;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
-  const int n_waves = gridDim.x * 4;
+  const int n_waves = blocks * 4;
   const int n_chunks = (A.n_pairs + A.chunk - 1) / A.chunk;
   const int n_valid = *A.n_uniq;  // a last segment beyond this one holds the pairs whose id is outside the table: skipped
   if (n_valid < 0) return;  // the plan's build gave up: nothing of it may be read
   const bool mixed = SRC != kSrcRows && A.rows_first < A.n_pairs;  // the plan also holds gradient rows of plain lookups
 
-  for (int chunk = blockIdx.x * 4 + wave; chunk < n_chunks; chunk += n_waves) {
+  for (int chunk = block * 4 + wave; chunk < n_chunks; chunk += n_waves) {
     const int base = chunk * A.chunk;  // the window is 64 positions wide whatever the chunk: a segment that starts in
     const int n_here = min(64, A.n_pairs - base);  // the chunk usually ends inside it
     const int pos = base + min(lane, n_here - 1);
@@ -442,12 +441,12 @@ __global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
 // otherwise the sum goes to the tile's tail row (segment continues past the tile end) or head row
 // (segment came in from the left and ends here).
 template <int SRC, int VEC, int NIT, bool REG>
-__global__ __launch_bounds__(256) void entity_tile_kernel(EntityArgs A) {
+__device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   constexpr int MUL = src_mul(SRC);
   constexpr int R = kRunsLong;
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
-  const int t = blockIdx.x * 4 + wave;
+  const int t = block * 4 + wave;
   const int p0 = t * A.tile;
   if (p0 >= A.n_pairs) return;  // whole wavefront leaves; no workgroup barrier is used below
   const int p1 = min(A.n_pairs, p0 + A.tile);
@@ -457,7 +456,7 @@ __global__ __launch_bounds__(256) void entity_tile_kernel(EntityArgs A) {
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int sg = A.seg_of_pos[p0];
     const int b0 = A.seg_start[sg], b1 = A.seg_start[sg + 1];
-    if (lane == 0 && p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid)
+    if (A.fix_list && lane == 0 && p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid)
       A.fix_list[atomicAdd(A.fix_count, 1)] = t;
   }
 
@@ -516,6 +515,23 @@ __global__ __launch_bounds__(256) void entity_tile_kernel(EntityArgs A) {
   }
 }
 
+// One launch each, or (few pairs: the launch itself, 4 to 5 us, is what costs) one for both, the tiles first.  Nothing is
+// appended to the fix-up's list then (A.fix_list == null): that pass asks every tile itself.
+template <int SRC, int VEC, int NIT, bool REG>
+__global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
+  segment_pass<SRC, VEC, NIT, REG>(A, blockIdx.x, gridDim.x);
+}
+template <int SRC, int VEC, int NIT, bool REG>
+__global__ __launch_bounds__(256) void entity_tile_kernel(EntityArgs A) {
+  tile_pass<SRC, VEC, NIT, REG>(A, blockIdx.x);
+}
+template <int SRC, int VEC, int NIT, bool REG>
+__global__ __launch_bounds__(256) void entity_small_kernel(EntityArgs A, int tile_blocks) {
+  if ((int)blockIdx.x < tile_blocks) tile_pass<SRC, VEC, NIT, REG>(A, blockIdx.x);
+  else segment_pass<SRC, VEC, NIT, REG>(A, (int)blockIdx.x - tile_blocks, (int)gridDim.x - tile_blocks);
+}
+
 // The tiles whose first segment is long, came in from the left and ends inside the tile are on the list the
 // tile pass made; a fixed grid of workgroups takes them in turn.  For each, the workgroup adds that segment's
 // partial rows (tails of the tiles it crossed, then this tile's head) in tile order and finishes the row.
@@ -528,13 +544,19 @@ __global__ __launch_bounds__(NW * 64) void entity_fixup_kernel(EntityArgs A) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = A.ncol * VEC;
   const size_t row_len = (size_t)half * MUL;
-  const int n_fix = *A.fix_count;
+  const int n_fix = A.fix_list ? *A.fix_count : (A.n_pairs + A.tile - 1) / A.tile;
+  const int n_valid = A.fix_list ? 0 : *A.n_uniq;
+  if (n_valid < 0) return;  // the plan's build gave up (then no tile is on the list)
   const bool mixed = SRC != kSrcRows && A.rows_first < A.n_pairs;
   for (int item = blockIdx.x; item < n_fix; item += gridDim.x) {  // uniform over the workgroup
-  const int t = A.fix_list[item];
+  const int t = A.fix_list ? A.fix_list[item] : item;
   const int p0 = t * A.tile;
   const int seg = A.seg_of_pos[p0];
   const int s0 = A.seg_start[seg];
+  if (!A.fix_list) {  // what the tile pass asks before it puts a tile on the list
+    const int end = A.seg_start[seg + 1];
+    if (p0 == 0 || s0 >= p0 || end > min(A.n_pairs, p0 + A.tile) || end - s0 <= A.short_max || seg >= n_valid) continue;
+  }
   const int ts = s0 / A.tile;
   const int n_parts = t - ts + 1;
   const int per_wave = (n_parts + NW - 1) / NW;
@@ -799,21 +821,19 @@ __device__ __forceinline__ void add_coded_runs(const EntityArgs& A, const unsign
 // segments that start in its chunk.  The chunk's gathers are made once for all of them (only by the lanes of those
 // segments), and the w, m, v rows of up to S segments are requested before the first is finished.
 template <int SRC, int VEC, int NIT>
-__global__ __launch_bounds__(256) void entity_segment_coded_kernel(EntityArgs A) {
+__device__ __forceinline__ void segment_pass_coded(const EntityArgs& A, unsigned char* code_lds, int block, int blocks) {
   static_assert(src_mul(SRC) == 1, "sign codes exist for one-half rows");
   constexpr int S = NIT == 1 ? 4 : 2;
-  extern __shared__ unsigned char code_lds[];  // [4 wavefronts][64 records]
-  if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   unsigned char* slab = code_lds + wave * (64 * NIT * 64);
-  const int n_waves = gridDim.x * 4;
+  const int n_waves = blocks * 4;
   const int n_chunks = (A.n_pairs + A.chunk - 1) / A.chunk;
   const int n_valid = *A.n_uniq;  // a last segment beyond this one holds the pairs whose id is outside the table: skipped
   if (n_valid < 0) return;  // the plan's build gave up: nothing of it may be read
   const bool mixed = A.rows_first < A.n_pairs;  // the plan also holds gradient rows of plain lookups
 
-  for (int chunk = blockIdx.x * 4 + wave; chunk < n_chunks; chunk += n_waves) {
+  for (int chunk = block * 4 + wave; chunk < n_chunks; chunk += n_waves) {
     const int base = chunk * A.chunk;  // the window is 64 positions wide whatever the chunk: a segment that starts in
     const int n_here = min(64, A.n_pairs - base);  // the chunk usually ends inside it
     const int pos = base + min(lane, n_here - 1);
@@ -894,15 +914,14 @@ __global__ __launch_bounds__(256) void entity_segment_coded_kernel(EntityArgs A)
 // together (W windows at a time), so the chain position -> pair -> upstream gradient / code record costs three
 // memory latencies per stretch.
 template <int SRC, int VEC, int NIT>
-__global__ __launch_bounds__(256, 4) void entity_tile_coded_kernel(EntityArgs A) {
+__device__ __forceinline__ void tile_pass_coded(const EntityArgs& A, unsigned char* code_lds, int block) {
   static_assert(src_mul(SRC) == 1, "sign codes exist for one-half rows");
   constexpr int TW = kTileWindows;
   constexpr int W = NIT == 1 ? 4 : 2;  // windows whose code records are in registers at a time
-  extern __shared__ unsigned char code_lds[];  // [4 wavefronts][64 records]
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   unsigned char* slab = code_lds + wave * (64 * NIT * 64);
-  const int t = blockIdx.x * 4 + wave;
+  const int t = block * 4 + wave;
   const int p0 = t * kTile;
   if (p0 >= A.n_pairs) return;  // whole wavefront leaves; no workgroup barrier is used below
   const int p1 = min(A.n_pairs, p0 + kTile);
@@ -935,7 +954,7 @@ __global__ __launch_bounds__(256, 4) void entity_tile_coded_kernel(EntityArgs A)
   };
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int s = at(sg, 0), s0 = at(b0, 0), s1 = at(b1, 0);
-    if (lane == 0 && p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid)
+    if (A.fix_list && lane == 0 && p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid)
       A.fix_list[atomicAdd(A.fix_count, 1)] = t;
   }
   bool any_long = false;
@@ -1003,6 +1022,24 @@ __global__ __launch_bounds__(256, 4) void entity_tile_coded_kernel(EntityArgs A)
   }
 }
 
+template <int SRC, int VEC, int NIT>
+__global__ __launch_bounds__(256) void entity_segment_coded_kernel(EntityArgs A) {
+  extern __shared__ unsigned char code_lds[];  // [4 wavefronts][64 records]
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
+  segment_pass_coded<SRC, VEC, NIT>(A, code_lds, blockIdx.x, gridDim.x);
+}
+template <int SRC, int VEC, int NIT>
+__global__ __launch_bounds__(256, 4) void entity_tile_coded_kernel(EntityArgs A) {
+  extern __shared__ unsigned char code_lds[];
+  tile_pass_coded<SRC, VEC, NIT>(A, code_lds, blockIdx.x);
+}
+template <int SRC, int VEC, int NIT>
+__global__ __launch_bounds__(256, 4) void entity_small_coded_kernel(EntityArgs A, int tile_blocks) {
+  extern __shared__ unsigned char code_lds[];
+  if ((int)blockIdx.x < tile_blocks) tile_pass_coded<SRC, VEC, NIT>(A, code_lds, blockIdx.x);
+  else segment_pass_coded<SRC, VEC, NIT>(A, code_lds, (int)blockIdx.x - tile_blocks, (int)gridDim.x - tile_blocks);
+}
+
 // Workgroups of 256 threads of `kernel` (with that much dynamic LDS) the current device keeps resident; asked
 // once per kernel and device.
 template <class K>
@@ -1028,27 +1065,42 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   // short segments: a fixed grid of wavefronts strides over the segment list (its length lives on the device)
   // (as many workgroups as the chip holds at once: a second wave of workgroups would run half empty)
   const unsigned want_blocks = (unsigned)(((A.n_pairs + A.chunk - 1) / A.chunk + 3) / 4);
+  // Few tiles: one launch for both passes.  65,536 pairs, L2 x 200: 24.7 + 4.8 us in two, 24.4 in one, the step 79.0 -> 76.4;
+  // the entity pass of a shared list's step, 1,536 rows of ComplEx, 13.2 + 5.0 -> 12.3.  (Beyond, the launch is below 2 % of the passes.)
+  const bool small = tiles <= 512;
+  const unsigned tile_blocks = (tiles + 3) / 4;
+  EntityArgs F = A;
+  if (small) F.fix_list = nullptr;
   bool coded = false;
   // (sign codes exist for rows of up to two column groups)
   if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) coded = A.codes != nullptr;
   if (coded) {
     if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) {
       const size_t slabs = (size_t)4 * 64 * NIT * 64;  // one code record per lane and wavefront
+      if (small) {
+        const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_coded_kernel<SRC, VEC, NIT>, (int)slabs));
+        hipLaunchKernelGGL((entity_small_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks + seg_blocks), dim3(256), slabs, st, F,
+                           (int)tile_blocks);
+      } else {
       const unsigned seg_blocks =
           min(want_blocks, resident_blocks(entity_segment_coded_kernel<SRC, VEC, NIT>, (int)slabs));
       hipLaunchKernelGGL((entity_segment_coded_kernel<SRC, VEC, NIT>), dim3(seg_blocks), dim3(256), slabs, st, A);
-      hipLaunchKernelGGL((entity_tile_coded_kernel<SRC, VEC, NIT>), dim3((tiles + 3) / 4), dim3(256), slabs, st, A);
+      hipLaunchKernelGGL((entity_tile_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks), dim3(256), slabs, st, A);
+      }
     }
+  } else if (small) {
+    const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_kernel<SRC, VEC, NIT, REG>, 0));
+    hipLaunchKernelGGL((entity_small_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks + seg_blocks), dim3(256), 0, st, F,
+                       (int)tile_blocks);
   } else {
     const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_segment_kernel<SRC, VEC, NIT, REG>, 0));
     hipLaunchKernelGGL((entity_segment_kernel<SRC, VEC, NIT, REG>), dim3(seg_blocks), dim3(256), 0, st, A);
-    hipLaunchKernelGGL((entity_tile_kernel<SRC, VEC, NIT, REG>), dim3((tiles + 3) / 4), dim3(256), 0, st, A);
+    hipLaunchKernelGGL((entity_tile_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks), dim3(256), 0, st, A);
   }
   const size_t row_bytes = (size_t)A.ncol * VEC * src_mul(SRC) * sizeof(float);
   const bool mixed = SRC != kSrcRows && A.rows_first < A.n_pairs;
   // the fix-up pass: a fixed grid takes the listed tiles in turn (at most one per tile; usually far fewer)
   const unsigned fix_blocks = min(tiles, 1024u);
-  EntityArgs F = A;
   if (7 * row_bytes <= 60 * 1024) {
     F.share_rows = mixed && 14 * row_bytes <= 60 * 1024;
     hipLaunchKernelGGL((entity_fixup_kernel<SRC, VEC, NIT, 8, REG>), dim3(fix_blocks), dim3(8 * 64),

@@ -1268,3 +1268,42 @@ def test_gradient_rows_at_a_size_that_forks():
     touched = torch.zeros(n, dtype=torch.bool, device="cuda")
     touched[plan.uniq] = True
     assert torch.equal(out["fused"][0][~touched], table[~touched])
+
+
+@pytest.mark.parametrize("n_pairs", [1, 255, 257, 131_072, 131_073])
+def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n_pairs):
+    """Up to 512 tiles of 256 pairs short and long segments go through one launch, and the fix-up finds its tiles by
+    itself: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
+    gradient rows and, from sign codes and without, of box pairs, against float64."""
+    from smore_amd import fused
+    n, dim = 3000, 12
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n_pairs)
+    ids = torch.randint(20, n, (n_pairs,), device="cuda", generator=gen)
+    lengths = (700, 68, 256, 65, 100, 64, 1024, 1) if n_pairs > 4000 else (130, 66)
+    at = 0
+    for i, length in enumerate(lengths):
+        ids[at: at + length] = i
+        at += length
+    ids = ids[torch.randperm(n_pairs, device="cuda", generator=gen)].view(1, -1)
+    plan = fused.build_plan(ids, n, want_inverse=True)
+    rows = torch.randn((n_pairs, dim), device="cuda", generator=gen)
+
+    def sums(x):
+        return torch.zeros((plan.n_uniq, dim), dtype=torch.float64, device="cuda").index_add_(0, plan.inverse, x.double())
+    got = torch.full((plan.n_uniq, dim), float("nan"), device="cuda")
+    fused.rows_backward(plan, rows, merged=got)
+    assert_close(got.cpu().numpy(), sums(rows).cpu().numpy(), 1e-6, "summed rows", sum_abs=8 * sums(rows.abs()).cpu().numpy())
+    table = torch.randn((n, dim), device="cuda", generator=gen)
+    q1, q2 = torch.randn((1, dim), device="cuda", generator=gen), torch.rand((1, dim), device="cuda", generator=gen)
+    gs = torch.randn((1, n_pairs), device="cuda", generator=gen)
+    params = fused.score_params(24.0, 0.5)
+    codes = fused.new_codes("box", table, ids, q1)
+    score = fused.score_forward("box", table, ids, q1, q2, params, codes=codes)
+    d = table.double()[ids[0]] - q1.double()
+    outside = d.abs() >= q2.double()
+    want = -gs[0, :, None].double() * torch.where(outside, 1.0, 0.5) * d.sign()
+    for c in (None, codes):
+        got.fill_(float("nan"))
+        fused.score_backward_entity("box", plan, table, q1, q2, score, gs, params, merged=got, codes=c)
+        assert_close(got.cpu().numpy(), sums(want).cpu().numpy(), 1e-6, "box rows", sum_abs=8 * sums(want.abs()).cpu().numpy())
