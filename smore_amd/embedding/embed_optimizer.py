@@ -424,7 +424,7 @@ class EmbeddingOptimizer(ABC):
         self._flag_host.copy_(self.err_flag, non_blocking=True)
         if self._flag_copied is None:
             self._flag_copied = torch.cuda.Event()
-        self._flag_copied.record()
+        self._flag_copied.record(torch.cuda.current_stream(self.err_flag.device))   # where the copy is, whatever device is current
         self._flag_event = self._flag_copied
 
     def apply_grad(self, lr):

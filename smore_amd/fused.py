@@ -261,7 +261,6 @@ class SegmentPlan:
             self._arrays[name] = (at, size, dtype)
             at += (size + 255) & ~255
         self._memory = torch.empty(at, dtype=torch.uint8, device=device)   # (every build writes all of it that it reads)
-        self._base = self._memory.data_ptr()
         self._n_uniq = None
 
     def __getattr__(self, name):
@@ -274,9 +273,13 @@ class SegmentPlan:
         return tensor
 
     def _at(self, name):
-        """Address of an array; None for an inverse that was not asked for."""
+        """Address of an array; None for an inverse that was not asked for.  Asked of the tensors that are there now: a
+        deep copy of a plan has memory of its own, and an array that the caller put in another's place is the one to read."""
+        tensor = self.__dict__.get(name)
+        if tensor is not None:
+            return tensor.data_ptr()
         entry = self._arrays.get(name)
-        return None if entry is None else self._base + entry[0]
+        return None if entry is None else self._memory.data_ptr() + entry[0]
 
     @property
     def n_uniq(self):
