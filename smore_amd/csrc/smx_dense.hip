@@ -20,6 +20,8 @@
 // reverse layout (entity [B,1,.] against query [B,N,.]) have kernels of the same build.
 #include <type_traits>
 
+#include <type_traits>
+
 #include "smx_common.h"
 #include "smx_functors.h"
 
