@@ -45,6 +45,16 @@ int smx_measure_plan_build(void* stream, const int64_t* idx, size_t n_pairs, siz
                            int64_t* uniq, int32_t* seg_start, int64_t* inverse, int32_t* pair_seg, int32_t* n_uniq,
                            int* err_flag, unsigned spin_limit, int force_abort);
 
+/* No counterpart in the reference.  Which kernels smx_dist_backward_f32 takes for a call of these sizes (entity
+ * [be,ne,.], query [bc,nc,.], output [bsize,num], features per half).
+ *   addresses   the addresses of all tensors or'ed together (their alignment; nothing is read)
+ *   path        out: 0 the general kernels, 1 those of the per-query layout, 2 of entity rows shared by the queries, 3 of the
+ *               reverse layout
+ *   vec, waves  out: floats per column of a row, wavefronts of the workgroup a query gets; 0 with the general kernels
+ * Host only: no device is asked. */
+int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc,
+                                    size_t dim, size_t addresses, int* path, int* vec, int* waves);
+
 #ifdef __cplusplus
 }
 #endif

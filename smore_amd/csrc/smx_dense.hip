@@ -22,7 +22,9 @@
 
 #include <type_traits>
 
+#include "../../include/smx_measure.h"
 #include "smx_common.h"
+#include "smx_dense_rules.h"
 #include "smx_functors.h"
 
 namespace smx {
@@ -33,10 +35,6 @@ __device__ __forceinline__ T wave_sum(T v) {
   for (int m = kWave / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
   return v;
 }
-
-struct Layout {
-  size_t bsize, num, be, ne, bc, nc, dim;
-};
 
 template <int K, typename T>
 __global__ __launch_bounds__(256) void dense_forward_kernel(const T* __restrict__ ent, const T* __restrict__ q1,
@@ -112,7 +110,6 @@ __global__ __launch_bounds__(128) void dense_backward_kernel(const T* __restrict
 
 // ---- per-query layout, fp32 -------------------------------------------------------------------
 typedef float dvec4 __attribute__((ext_vector_type(4)));
-constexpr int kPqBwdWaves = 8;
 
 template <int K>
 __device__ __forceinline__ float pq_row_terms(const dvec4* __restrict__ pe, const float* lds, int ncol, int dim, int lane) {
@@ -344,31 +341,6 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_shared_entity_backw
   }
 }
 
-// entity [1,N,.] shared by the queries [B,1,.], float4-able
-static bool shared_layout(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
-                          const void* f, const void* g) {
-  if (L.be != 1 || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.bsize < 2) return false;
-  if (L.dim % 4 != 0 || L.dim > 1024 || L.bsize * L.num > 0x7fffffffull) return false;
-  return aligned16(a) && aligned16(b) && aligned16(c) && aligned16(d) && aligned16(e) && aligned16(f) && aligned16(g);
-}
-
-// 8- or 4-byte columns for tensors whose rows are not made of 16-byte ones
-static int narrow_vec(size_t dim, const void* a, const void* b, const void* c, const void* d, const void* e, const void* f,
-                      const void* g) {
-  auto even = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
-  return dim % 2 == 0 && even(a) && even(b) && even(c) && even(d) && even(e) && even(f) && even(g) ? 2 : 1;
-}
-
-// Floats per column of the shared backward for a call, 0: not its layout (see pq_backward_vec; L1 512 x 1024 x 330 135 us, box
-// 300 x 500 x 283 66, 2,378 and 1,132 with the general kernels).
-static int shared_backward_vec(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
-                               const void* f, const void* g) {
-  if (shared_layout(L, a, b, c, d, e, f, g)) return 4;
-  if (L.be != 1 || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.bsize < 2 || L.dim > 512) return 0;
-  if (L.bsize * L.num > 0x7fffffffull) return 0;
-  return narrow_vec(L.dim, a, b, c, d, e, f, g);
-}
-
 template <int K>
 static int backward_shared(hipStream_t st, const float* gout, const float* ent, const float* q1, const float* q2,
                            float* gent, float* gq1, float* gq2, const Layout& L, int vec) {
@@ -509,14 +481,6 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_rev_backward_kernel
   }
 }
 
-// entity [B,1,.] against query [B,N,.]
-static bool reverse_layout(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
-                           const void* f, const void* g) {
-  if (L.be != L.bsize || L.bc != L.bsize || L.ne != 1 || L.nc != L.num || L.num < 2) return false;
-  if (L.dim % 4 != 0 || L.dim > 1024 || L.bsize * L.num > 0x7fffffffull) return false;
-  return aligned16(a) && aligned16(b) && aligned16(c) && aligned16(d) && aligned16(e) && aligned16(f) && aligned16(g);
-}
-
 template <int K>
 static int forward_rev(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L) {
   int rows_per_tile = (int)L.num;
@@ -544,26 +508,6 @@ static int backward_rev(hipStream_t st, const float* gout, const float* ent, con
   return check_launch("dist backward (reverse layout)");
 }
 
-// entity [B,N,.] against query [B,1,.], float4-able, and small enough for the kernels above
-static bool pq_layout(const Layout& L, int kind, const void* a, const void* b, const void* c, const void* d,
-                      const void* e, const void* f, const void* g) {
-  if (L.be != L.bsize || L.bc != L.bsize || L.ne != L.num || L.nc != 1) return false;
-  if (L.dim % 4 != 0 || L.dim > 1024 || L.bsize * L.num > 0x7fffffffull || L.num > 0x7fffffffull) return false;
-  (void)kind;
-  return aligned16(a) && aligned16(b) && aligned16(c) && aligned16(d) && aligned16(e) && aligned16(f) && aligned16(g);
-}
-
-// Floats per column of the per-query backward for a call, 0: not its layout.  Rows that are not made of 16-byte columns take
-// 8- or 4-byte ones up to 512 floats (the general kernels form each row's and each query's gradient by itself: rotate
-// 300 x 333 x 250 571 us against 76 here, box 300 x 333 x 201 487 against 31, L1 100 x 400 x 330 666 against 30).
-static int pq_backward_vec(const Layout& L, const void* a, const void* b, const void* c, const void* d, const void* e,
-                           const void* f, const void* g) {
-  if (pq_layout(L, 0, a, b, c, d, e, f, g)) return 4;
-  if (L.be != L.bsize || L.bc != L.bsize || L.ne != L.num || L.nc != 1 || L.dim > 512) return 0;
-  if (L.bsize * L.num > 0x7fffffffull || L.bsize > 0x7fffffffull) return 0;
-  return narrow_vec(L.dim, a, b, c, d, e, f, g);
-}
-
 template <int K, bool SHARED = false>
 static int forward_pq(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L) {
   // enough workgroups to fill the chip, at least eight rows each when there are that many
@@ -579,7 +523,7 @@ static int forward_pq(hipStream_t st, const float* ent, const float* q1, const f
 
 template <int K>
 static int backward_pq(hipStream_t st, const float* gout, const float* ent, const float* q1, const float* q2, float* gent,
-                       float* gq1, float* gq2, const Layout& L, int vec) {
+                       float* gq1, float* gq2, const Layout& L, int vec, int waves) {
   const int num = (int)L.num, dim = (int)L.dim;
   auto launch = [&](auto nit, auto waves, auto vec) {
     constexpr int NIT = decltype(nit)::value, NW = decltype(waves)::value, VEC = decltype(vec)::value;
@@ -597,9 +541,7 @@ static int backward_pq(hipStream_t st, const float* gout, const float* ent, cons
     ncol <= 128 ? launch(two, eight, two) : launch(four, eight, two);
   } else if (vec == 1) {
     ncol <= 256 ? launch(four, eight, one) : launch(eight, eight, one);
-  } else if (ncol <= 32 || (kind_mul(K) == 1 && ncol <= 128 && L.bsize <= 256)) {
-    // (few queries: a CU has one workgroup, or none.  Eight / sixteen wavefronts, box 64 x 512 x 400 32 / 25 us, 512 x 512 x 100
-    // 42 / 37; two halves of long rows, BetaE 200 x 200 x 400, are slower with sixteen: 134 / 234, the registers do not suffice)
+  } else if (waves == 16) {
     ncol <= 64 ? launch(one, sixteen, four) : launch(two, sixteen, four);
   } else if (ncol <= 64) {
     launch(one, eight, four);
@@ -644,6 +586,12 @@ static int backward_k(hipStream_t st, const T* gout, const T* ent, const T* q1, 
 #define SMX_FOR_EACH_KIND(X) \
   X(kL1) X(kL2) X(kBoxOut) X(kBoxIn) X(kRotate) X(kBetaKL) X(kComplex) X(kDistmult) X(kBetaL2) X(kBetaFisher)
 
+// Addresses or'ed together: what their lowest bits say holds for all of them.
+template <typename... P>
+static size_t low_bits(const P*... p) {
+  return (size_t)(reinterpret_cast<uintptr_t>(p) | ...);
+}
+
 template <typename T>
 int dense_forward(int kind, void* stream, const T* ent, const T* q1, const T* q2, T* dst, size_t bsize, size_t num,
                   size_t be, size_t ne, size_t bc, size_t nc, size_t dim) {
@@ -653,7 +601,8 @@ int dense_forward(int kind, void* stream, const T* ent, const T* q1, const T* q2
   if (!ent || !q1 || !dst || (kind_nq(kind) == 2 && !q2)) return fail(SMX_ERR_ARG, "null tensor pointer");
   hipStream_t st = as_stream(stream);
   if constexpr (std::is_same<T, float>::value) {
-    if (pq_layout(L, kind, ent, q1, q2, dst, nullptr, nullptr, nullptr)) {
+    const bool rows = rows_of_16_bytes(L, low_bits(ent, q1, q2, dst));
+    if (rows && per_query_layout(L)) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
@@ -662,9 +611,7 @@ int dense_forward(int kind, void* stream, const T* ent, const T* q1, const T* q2
 #undef X
       }
     }
-  }
-  if constexpr (std::is_same<T, float>::value) {
-    if (shared_layout(L, ent, q1, q2, dst, nullptr, nullptr, nullptr)) {
+    if (rows && shared_layout(L)) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
@@ -673,7 +620,7 @@ int dense_forward(int kind, void* stream, const T* ent, const T* q1, const T* q2
 #undef X
       }
     }
-    if (reverse_layout(L, ent, q1, q2, dst, nullptr, nullptr, nullptr)) {
+    if (rows && reverse_layout(L)) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
@@ -703,27 +650,26 @@ int dense_backward(int kind, void* stream, const T* gout, const T* ent, const T*
     return fail(SMX_ERR_ARG, "null tensor pointer");
   hipStream_t st = as_stream(stream);
   if constexpr (std::is_same<T, float>::value) {
-    if (const int vec = pq_backward_vec(L, gout, ent, q1, q2, gent, gq1, gq2)) {
+    const BackwardForm form = dense_backward_form(L, kind_mul(kind), low_bits(gout, ent, q1, q2, gent, gq1, gq2));
+    if (form.path == kPathPerQuery) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, vec);
+    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, form.vec, form.waves);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
     }
-  }
-  if constexpr (std::is_same<T, float>::value) {
-    if (const int vec = shared_backward_vec(L, gout, ent, q1, q2, gent, gq1, gq2)) {
+    if (form.path == kPathShared) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return backward_shared<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, vec);
+    return backward_shared<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, form.vec);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
     }
-    if (reverse_layout(L, gout, ent, q1, q2, gent, gq1, gq2)) {
+    if (form.path == kPathReverse) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
@@ -764,6 +710,18 @@ int smx_dist_backward_f64(int kind, void* stream, const double* gout, const doub
                           const double* q2, double* gent, double* gq1, double* gq2, size_t bsize, size_t num,
                           size_t be, size_t ne, size_t bc, size_t nc, size_t dim) {
   return smx::dense_backward<double>(kind, stream, gout, ent, q1, q2, gent, gq1, gq2, bsize, num, be, ne, bc, nc, dim);
+}
+int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc, size_t dim,
+                                    size_t addresses, int* path, int* vec, int* waves) {
+  using namespace smx;
+  if (kind < 0 || kind >= kNumKinds) return fail(SMX_ERR_KIND, "unknown dist kind %d", kind);
+  const Layout L{bsize, num, be, ne, bc, nc, dim};
+  if (int rc = check_layout(L)) return rc;
+  const BackwardForm form = dense_backward_form(L, kind_mul(kind), addresses);
+  *path = form.path;
+  *vec = form.vec;
+  *waves = form.waves;
+  return SMX_OK;
 }
 
 }  // extern "C"
