@@ -51,9 +51,10 @@ int smx_measure_plan_build(void* stream, const int64_t* idx, size_t n_pairs, siz
  *   path        out: 0 the general kernels, 1 those of the per-query layout, 2 of entity rows shared by the queries, 3 of the
  *               reverse layout
  *   vec, waves  out: floats per column of a row, wavefronts of the workgroup a query gets; 0 with the general kernels
+ *   ahead       out: 1 where a wavefront has its next row on the way while it works on one
  * Host only: no device is asked. */
 int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc,
-                                    size_t dim, size_t addresses, int* path, int* vec, int* waves);
+                                    size_t dim, size_t addresses, int* path, int* vec, int* waves, int* ahead);
 
 #ifdef __cplusplus
 }

@@ -180,25 +180,26 @@ __device__ __forceinline__ void store_column(float* half_row, int dim, int c, co
   }
 }
 
-// One workgroup of NW wavefronts per query.  Lane l owns the columns l, l+64, ... of the row, VEC floats each
-// (NIT of them); wavefront w takes rows w, w+NW, ...  For every row it writes the row's gradient and adds
-// the row's contribution to its query-gradient registers, the next row on its way; the partial query gradients are summed
-// through LDS in wavefront order, so the result does not depend on timing.
+// One workgroup per query, of NW wavefronts (NW = 0: as many as launched, at most eight).  Lane l owns the columns l, l+64, ... of the row, VEC floats each
+// (NIT of them); wavefront w of nw takes rows w, w+nw, ...  For every row it writes the row's gradient and adds
+// the row's contribution to its query-gradient registers, with AHEAD the next row on its way; the partial query gradients are
+// summed through LDS in wavefront order, so the result does not depend on timing.
 // SHARED: the entity rows are the same [1,N,.] for every query (--share_negative, online_sampler.py:155-157);
 // this kernel then gives the query gradients only, and dense_shared_entity_backward_kernel the rows'.
-// What bounds it: memory, given enough rows in flight where a few hundred queries leave a CU one or two workgroups.
-// The next row in flight, and stores that no wait depends on: box 64 x 512 x 400 69 -> 25 us, L1 100 x 400 x 400 50 -> 22,
-// box 300 x 333 x 400 58 -> 55 (5.8 TB/s).
-template <int K, int NIT, bool SHARED = false, int NW = kPqBwdWaves, int VEC = 4>
-__global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
+// What bounds it: memory, given enough rows in flight, which is what the number of wavefronts and AHEAD are for (rule and figures
+// at per_query_form); arithmetic for BetaE and Fisher.  Box 300 x 333 x 400 54 us, 5.9 TB/s.
+template <int K, int NIT, bool SHARED, int NW, int VEC, bool AHEAD>
+__global__ __launch_bounds__((NW > 0 ? NW : kPqBwdWaves) * kWave) void dense_pq_backward_kernel(
     const float* __restrict__ gout, const float* __restrict__ ent, const float* __restrict__ q1,
     const float* __restrict__ q2, float* __restrict__ gent, float* __restrict__ gq1, float* __restrict__ gq2, int num,
     int dim) {
   constexpr int MUL = kind_mul(K), NQ = kind_nq(K);
+  constexpr bool kHeavy = kind_heavy(K);
   typedef column<VEC> vec;
   extern __shared__ float lds[];  // [waves][NQ][dim]
   const int b = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int nw = NW > 0 ? NW : (int)blockDim.x / kWave;
   const int ncol = dim / VEC;
   const size_t row_len = (size_t)dim * MUL;
   const vec zero = (vec)(0.f);
@@ -214,8 +215,7 @@ __global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
     float g;
     vec e1[NIT], e2[NIT];
   };
-  auto request = [&](int k, Row& row) {   // (past the last row: that one once more)
-    k = min(k, num - 1);
+  auto request = [&](int k, Row& row) {
     const size_t r = (size_t)b * num + k;
     row.g = gout[r];
     const vec* pe = reinterpret_cast<const vec*>(ent + (SHARED ? (size_t)k : r) * row_len);
@@ -230,7 +230,9 @@ __global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
     float* pg = gent + ((size_t)b * num + k) * row_len;
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-      // lanes past the row end hold a copy of the last column: what they compute is not stored
+      const int c = lane + kWave * it;
+      if (kHeavy && kWave * it >= ncol) continue;   // uniform: no column of the row in this group
+      if (!AHEAD && c >= ncol) continue;   // (AHEAD: such lanes hold a copy of the last column, what they compute is not stored)
       vec ge1 = zero, ge2 = zero;
 #pragma unroll
       for (int x = 0; x < VEC; ++x) {
@@ -241,20 +243,36 @@ __global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
         acc1[it][x] = b1;
         acc2[it][x] = b2;
       }
-      if (!SHARED) {
-        store_column<VEC>(pg, dim, lane + kWave * it, ge1);
-        if (MUL == 2) store_column<VEC>(pg + dim, dim, lane + kWave * it, ge2);
+      if (SHARED) continue;
+      if constexpr (AHEAD) {
+        store_column<VEC>(pg, dim, c, ge1);
+        if (MUL == 2) store_column<VEC>(pg + dim, dim, c, ge2);
+      } else {
+        __builtin_nontemporal_store(ge1, reinterpret_cast<vec*>(pg) + c);
+        if (MUL == 2) __builtin_nontemporal_store(ge2, reinterpret_cast<vec*>(pg + dim) + c);
       }
     }
   };
-  Row row_a, row_b;
-  request(wave, row_a);
-  for (int k = wave; k < num; k += 2 * NW) {
-    request(k + NW, row_b);
-    use(k, row_a);
-    if (k + NW >= num) break;
-    request(k + 2 * NW, row_a);
-    use(k + NW, row_b);
+  if constexpr (AHEAD) {
+    if (wave < num) {
+      Row row_a, row_b;
+      auto next = [&](int k) { return min(k + nw, num - 1); };   // (behind a wavefront's last row: one that is read anyway)
+      request(wave, row_a);
+      for (int k = wave; k < num; k += nw) {
+        request(next(k), row_b);
+        use(k, row_a);
+        k += nw;
+        if (k >= num) break;
+        request(next(k), row_a);
+        use(k, row_b);
+      }
+    }
+  } else {
+    for (int k = wave; k < num; k += nw) {
+      Row row;
+      request(k, row);
+      use(k, row);
+    }
   }
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
@@ -265,10 +283,10 @@ __global__ __launch_bounds__(NW * kWave) void dense_pq_backward_kernel(
     }
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < dim; d += NW * kWave) {
+  for (int d = threadIdx.x; d < dim; d += nw * kWave) {
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
+    for (int w = 0; w < nw; ++w) {
       s1 += lds[(size_t)(w * NQ + 0) * dim + d];
       if (NQ == 2) s2 += lds[(size_t)(w * NQ + 1) * dim + d];
     }
@@ -350,7 +368,7 @@ static int backward_shared(hipStream_t st, const float* gout, const float* ent, 
   const size_t lds_e = (size_t)kPqBwdWaves * kind_mul(K) * L.dim * sizeof(float);
   auto launch = [&](auto nit, auto v) {
     constexpr int NIT = decltype(nit)::value, VEC = decltype(v)::value;
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, true, kPqBwdWaves, VEC>), dim3((unsigned)L.bsize), block, lds_q, st,
+    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, true, kPqBwdWaves, VEC, true>), dim3((unsigned)L.bsize), block, lds_q, st,
                        gout, ent, q1, q2, gent, gq1, gq2, num, dim);
     hipLaunchKernelGGL((dense_shared_entity_backward_kernel<K, NIT, VEC>), dim3((unsigned)L.num), block, lds_e, st, gout, ent,
                        q1, q2, gent, bsize, num, dim);
@@ -523,32 +541,45 @@ static int forward_pq(hipStream_t st, const float* ent, const float* q1, const f
 
 template <int K>
 static int backward_pq(hipStream_t st, const float* gout, const float* ent, const float* q1, const float* q2, float* gent,
-                       float* gq1, float* gq2, const Layout& L, int vec, int waves) {
+                       float* gq1, float* gq2, const Layout& L, const BackwardForm& form) {
   const int num = (int)L.num, dim = (int)L.dim;
-  auto launch = [&](auto nit, auto waves, auto vec) {
-    constexpr int NIT = decltype(nit)::value, NW = decltype(waves)::value, VEC = decltype(vec)::value;
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, false, NW, VEC>), dim3((unsigned)L.bsize), dim3(NW * kWave),
-                       (size_t)NW * kind_nq(K) * L.dim * sizeof(float), st, gout, ent, q1, q2, gent, gq1, gq2, num, dim);
-  };
   using std::integral_constant;
+  auto launch = [&](auto nit, auto v) {
+    constexpr int NIT = decltype(nit)::value, VEC = decltype(v)::value;
+    auto go = [&](auto most, auto ahead) {
+      constexpr int NW = decltype(most)::value;
+      constexpr bool AHEAD = decltype(ahead)::value;
+      hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, false, NW, VEC, AHEAD>), dim3((unsigned)L.bsize),
+                         dim3(form.waves * kWave), (size_t)form.waves * kind_nq(K) * L.dim * sizeof(float), st, gout, ent, q1,
+                         q2, gent, gq1, gq2, num, dim);
+    };
+    constexpr integral_constant<int, 0> as_launched;
+    constexpr integral_constant<int, 8> eight;
+    constexpr integral_constant<int, 16> sixteen;
+    if (form.waves < kPqBwdWaves) return go(as_launched, std::false_type());
+    if constexpr (VEC == 4 && (NIT == 1 || (NIT == 2 && kind_mul(K) == 1))) {
+      if (form.waves == 16) return go(sixteen, std::true_type());
+    }
+    if constexpr (VEC == 4 && NIT == (kind_heavy(K) ? 4 : 1)) {
+      if (!form.ahead) return go(eight, std::false_type());
+    }
+    if constexpr (!(VEC == 4 && NIT == 4 && kind_heavy(K))) go(eight, std::true_type());
+  };
   constexpr integral_constant<int, 1> one;
   constexpr integral_constant<int, 2> two;
   constexpr integral_constant<int, 4> four;
   constexpr integral_constant<int, 8> eight;
-  constexpr integral_constant<int, 16> sixteen;
-  const size_t ncol = L.dim / vec;
-  if (vec == 2) {
-    ncol <= 128 ? launch(two, eight, two) : launch(four, eight, two);
-  } else if (vec == 1) {
-    ncol <= 256 ? launch(four, eight, one) : launch(eight, eight, one);
-  } else if (waves == 16) {
-    ncol <= 64 ? launch(one, sixteen, four) : launch(two, sixteen, four);
+  const size_t ncol = L.dim / form.vec;
+  if (form.vec == 2) {
+    ncol <= 128 ? launch(two, two) : launch(four, two);
+  } else if (form.vec == 1) {
+    ncol <= 256 ? launch(four, one) : launch(eight, one);
   } else if (ncol <= 64) {
-    launch(one, eight, four);
+    launch(one, four);
   } else if (ncol <= 128) {
-    launch(two, eight, four);
+    launch(two, four);
   } else {
-    launch(four, eight, four);
+    launch(four, four);
   }
   return check_launch("dist backward (per-query layout)");
 }
@@ -650,12 +681,12 @@ int dense_backward(int kind, void* stream, const T* gout, const T* ent, const T*
     return fail(SMX_ERR_ARG, "null tensor pointer");
   hipStream_t st = as_stream(stream);
   if constexpr (std::is_same<T, float>::value) {
-    const BackwardForm form = dense_backward_form(L, kind_mul(kind), low_bits(gout, ent, q1, q2, gent, gq1, gq2));
+    const BackwardForm form = dense_backward_form(L, kind, low_bits(gout, ent, q1, q2, gent, gq1, gq2));
     if (form.path == kPathPerQuery) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, form.vec, form.waves);
+    return backward_pq<KK>(st, gout, ent, q1, q2, gent, gq1, gq2, L, form);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
@@ -712,15 +743,17 @@ int smx_dist_backward_f64(int kind, void* stream, const double* gout, const doub
   return smx::dense_backward<double>(kind, stream, gout, ent, q1, q2, gent, gq1, gq2, bsize, num, be, ne, bc, nc, dim);
 }
 int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc, size_t dim,
-                                    size_t addresses, int* path, int* vec, int* waves) {
+                                    size_t addresses, int* path, int* vec, int* waves,
+                                    int* ahead) {
   using namespace smx;
   if (kind < 0 || kind >= kNumKinds) return fail(SMX_ERR_KIND, "unknown dist kind %d", kind);
   const Layout L{bsize, num, be, ne, bc, nc, dim};
   if (int rc = check_layout(L)) return rc;
-  const BackwardForm form = dense_backward_form(L, kind_mul(kind), addresses);
+  const BackwardForm form = dense_backward_form(L, kind, addresses);
   *path = form.path;
   *vec = form.vec;
   *waves = form.waves;
+  *ahead = form.ahead;
   return SMX_OK;
 }
 

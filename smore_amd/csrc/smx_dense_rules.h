@@ -3,6 +3,8 @@
 #pragma once
 #include <cstddef>
 
+#include "smx_functors.h"
+
 namespace smx {
 
 struct Layout {
@@ -11,12 +13,16 @@ struct Layout {
 
 enum BackwardPath { kPathGeneral = 0, kPathPerQuery = 1, kPathShared = 2, kPathReverse = 3 };
 
-// vec: floats per column of a row, waves: wavefronts of the workgroup that a query gets (both 0 where the path has no choice)
+// vec: floats per column of a row; waves: wavefronts of the workgroup that a query gets; ahead: a wavefront has its next row
+// on the way while it works on one.  (0 where the path has no choice.)
 struct BackwardForm {
-  int path, vec, waves;
+  int path, vec, waves, ahead;
 };
 
 constexpr int kPqBwdWaves = 8;
+
+// Kinds bound by their arithmetic (logarithms, digamma and trigamma functions), not by their rows' way from memory.
+constexpr bool kind_heavy(int kind) { return kind == kBetaKL || kind == kBetaFisher; }
 
 // HIP counts the threads of a launch in 32 bits.
 constexpr bool launchable(size_t workgroups, size_t waves) { return workgroups < (1ull << 32) / (waves * 64); }
@@ -43,26 +49,47 @@ inline int column_floats(const Layout& L, size_t low) {
   return L.dim % 2 == 0 && (low & 7) == 0 ? 2 : 1;
 }
 
-// halves: of an entity row.  Batches and row counts whose launch HIP would refuse take the general kernels, whose workgroups
-// are of two wavefronts (and one per row on either side).
-inline BackwardForm dense_backward_form(const Layout& L, int halves, size_t low) {
+// Wavefronts per query and whether they read ahead, us a call:
+// Few rows: a wavefront each (two rows for the arithmetic-bound kinds), because one without a row takes registers and LDS from
+// other queries.  (Up to eight rows: of their workgroups of five wavefronts and more a CU holds one.)  Eight wavefronts / this, box 16384 x 1 x 400 37 / 25, 262144 x 1 x 32 254 / 62, rotate 16384 x 1 x 100
+// 23 / 11, BetaE 16384 x 1 x 400 378 / 64, 4096 x 8 x 400 134 / 97.
+// Few queries: a CU has one workgroup of the launch, or none, and sixteen wavefronts.  Eight / sixteen, box 64 x 512 x 400
+// 33 / 25, 256 x 512 x 100 29 / 22, 512 x 512 x 32 36 / 26, BetaE 256 x 512 x 100 156 / 137.  Not rows of two long halves,
+// whose registers do not suffice (BetaE 300 x 333 x 400 408 / 663), nor larger batches (box 1024 x 256 x 100 35 / 41).
+// Reading ahead costs registers and, for the last row, a read.  Short rows of many queries do without, their wavefronts being
+// many (box 600 x 512 x 100 49 / 44, L1 16384 x 16 x 64 31 / 29, complex 1024 x 512 x 200 347 / 337 us with / without), and so
+// do long rows of the arithmetic-bound kinds, which it makes spill (BetaE 512 x 128 x 600 395 / 278).  With / without where it
+// stays: box 1024 x 512 x 200 174 / 181, 64 x 512 x 400 33 / 41, rotate 8192 x 32 x 400 307 / 324, BetaE 300 x 333 x 400 408 / 462.
+inline BackwardForm per_query_form(const Layout& L, int kind, int vec) {
+  const size_t ncol = L.dim / vec;
+  const bool one_half = kind_mul(kind) == 1;
+  if (kind_heavy(kind) && L.num <= 8) return {kPathPerQuery, vec, (int)(L.num + 1) / 2, 0};
+  if (L.num < kPqBwdWaves) return {kPathPerQuery, vec, (int)L.num, 0};
+  if (vec == 4) {
+    const size_t sixteen = ncol <= 32 ? (one_half ? 512 : 256) : one_half && ncol <= 128 ? 256 : 0;
+    if (L.bsize <= sixteen && L.num >= 128) return {kPathPerQuery, vec, 16, 1};
+    if (kind_heavy(kind)) return {kPathPerQuery, vec, kPqBwdWaves, ncol <= 128};
+    if (ncol <= (one_half ? 32 : 64) && L.bsize > 256) return {kPathPerQuery, vec, kPqBwdWaves, 0};
+  }
+  return {kPathPerQuery, vec, kPqBwdWaves, 1};
+}
+
+// Batches and row counts whose launch HIP would refuse take the general kernels, whose workgroups are of two wavefronts (and
+// one per row on either side).
+inline BackwardForm dense_backward_form(const Layout& L, int kind, size_t low) {
   if (per_query_layout(L)) {
     const int vec = column_floats(L, low);
-    if (vec == 0 || !launchable(L.bsize, kPqBwdWaves)) return {kPathGeneral, 0, 0};
-    const size_t ncol = L.dim / vec;
-    // Sixteen wavefronts for short rows, and for few queries: a CU has one workgroup, or none.  Eight / sixteen, box
-    // 64 x 512 x 400 32 / 25 us, 512 x 512 x 100 42 / 37; two halves of long rows, BetaE 200 x 200 x 400, are slower with
-    // sixteen: 134 / 234, the registers do not suffice.
-    const bool many = vec == 4 && (ncol <= 32 || (halves == 1 && ncol <= 128 && L.bsize <= 256));
-    return {kPathPerQuery, vec, many && launchable(L.bsize, 16) ? 16 : kPqBwdWaves};
+    if (vec == 0) return {kPathGeneral, 0, 0, 0};
+    const BackwardForm form = per_query_form(L, kind, vec);
+    return launchable(L.bsize, form.waves) ? form : BackwardForm{kPathGeneral, 0, 0, 0};
   }
   if (shared_layout(L)) {
     const int vec = column_floats(L, low);
-    if (vec == 0 || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0};
-    return {kPathShared, vec, kPqBwdWaves};
+    if (vec == 0 || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0, 0};
+    return {kPathShared, vec, kPqBwdWaves, 1};
   }
-  if (reverse_layout(L) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves};
-  return {kPathGeneral, 0, 0};
+  if (reverse_layout(L) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
+  return {kPathGeneral, 0, 0, 0};
 }
 
 }  // namespace smx

@@ -61,10 +61,12 @@ def test_dense_forward_backward(kind, layout, dtype):
 @pytest.mark.parametrize("be,b,k,dims", [(3, 3, 1, (1, 2, 3, 63, 65)), (2, 2, 17, (66, 127, 130, 254, 255)),
                                          (5, 5, 9, (257, 258, 510, 511, 514)), (3, 3, 33, (4, 128, 132, 256)),
                                          (260, 260, 3, (4, 256, 260)), (257, 257, 18, (128, 132)),
+                                         (2, 2, 127, (4, 132, 516)), (2, 2, 128, (4, 128, 132, 512, 516)), (2, 2, 131, (128, 260)),
+                                         (513, 513, 16, (4, 256, 260)), (3, 3, 7, (33, 132, 516)), (3, 3, 15, (34, 260, 516)),
                                          (1, 2, 3, (1, 2, 63, 65, 130)), (1, 9, 17, (254, 255, 257, 258, 510, 511, 513, 400))])
 def test_backward_of_rows_of_any_width(kind, be, b, k, dims):
     """The per-query backward (be = b) and that of rows shared by the queries (be = 1) with columns of four, two and one floats, from tensors that start on any 4-byte
-    boundary, and with sixteen or eight wavefronts per query (batches of up to 256, or rows of up to 32 columns)."""
+    boundary, and with as many wavefronts per query as it has rows, with eight that read ahead or do not, and with sixteen."""
     from smore_amd import extlib_hip as ext
     for dim in dims:
         rng = np.random.default_rng(seed(kind, b, k, dim))

@@ -9,13 +9,13 @@ GENERAL, PER_QUERY, SHARED, REVERSE = range(4)
 
 
 def form(kind, bsize, num, dim, be=None, ne=None, bc=None, nc=1, low=0):
-    """(path, floats per column, wavefronts); entity [B,N,.] against query [B,1,.] unless told otherwise."""
-    path, vec, waves = (ctypes.c_int() for _ in range(3))
+    """(path, floats per column, wavefronts, reads ahead); entity [B,N,.] against query [B,1,.] unless told otherwise."""
+    path, vec, waves, ahead = (ctypes.c_int() for _ in range(4))
     lib = _lib.load()
     rc = lib.smx_measure_dense_backward_form(lib.smx_kind_from_name(kind.encode()), bsize, num, be or bsize, ne or num,
-                                             bc or bsize, nc, dim, low, *(ctypes.byref(x) for x in (path, vec, waves)))
+                                             bc or bsize, nc, dim, low, *(ctypes.byref(x) for x in (path, vec, waves, ahead)))
     assert rc == 0, lib.smx_last_error()
-    return path.value, vec.value, waves.value
+    return path.value, vec.value, waves.value, ahead.value
 
 
 @pytest.mark.parametrize("kind", ["l1", "box_out", "rotate", "beta_kl"])
@@ -25,23 +25,26 @@ def test_every_launch_is_one_that_hip_takes(kind, dim, low, layout):
     """HIP takes launches of fewer than 2^32 threads, and a batch brings a workgroup per query: at the batches around which
     workgroups of sixteen, eight and two wavefronts reach that limit, the kernels taken are below it, or the general ones."""
     for bsize in (1 << 8, (1 << 22) - 1, 1 << 22, 5_000_000, (1 << 23) - 1, 1 << 23, (1 << 25) - 1):
-        for num in (1, 8, 32):
-            path, vec, waves = form(kind, bsize, num, dim, low=low, **(dict(be=1) if layout == "shared" else {}))
+        for num in (1, 2, 8, 32):
+            path, vec, waves, _ = form(kind, bsize, num, dim, low=low, **(dict(be=1) if layout == "shared" else {}))
             assert path in ((GENERAL, PER_QUERY) if layout == "per query" else (GENERAL, SHARED))
-            assert (path == GENERAL) == (bsize * 512 >= 1 << 32)
+            few = num if kind != "beta_kl" else (num + 1) // 2
+            least = 8 if layout == "shared" else min(few, 8)
+            assert (path == GENERAL) == (bsize * least * 64 >= 1 << 32)
             assert path == GENERAL or bsize * waves * 64 < 1 << 32
+            assert layout == "shared" or waves <= few, "a wavefront without a row"
     if layout == "shared":      # a workgroup per shared row, too
         for num in ((1 << 23) - 1, 1 << 23):
-            path, _, _ = form(kind, 2, num, dim, be=1, low=low)
+            path, _, _, _ = form(kind, 2, num, dim, be=1, low=low)
             assert path == (SHARED if num * 512 < 1 << 32 else GENERAL)
 
 
 def test_columns_by_row_length_and_alignment():
     for dim, low, want in ((400, 0, 4), (1024, 0, 4), (1024, 16, 4), (400, 8, 2), (402, 8, 2), (400, 4, 1), (401, 0, 1),
                            (512, 4, 1), (513, 0, 0), (514, 0, 0), (1020, 4, 0), (1028, 0, 0)):
-        path, vec, _ = form("box_out", 64, 40, dim, low=low)
+        path, vec, _, _ = form("box_out", 64, 40, dim, low=low)
         assert vec == want and path == (PER_QUERY if want else GENERAL)
-        path, vec, _ = form("box_out", 64, 40, dim, be=1, low=low)
+        path, vec, _, _ = form("box_out", 64, 40, dim, be=1, low=low)
         assert vec == want and path == (SHARED if want else GENERAL)
     assert form("box_out", 64, 40, 400, ne=1, nc=40)[0] == REVERSE
     assert form("box_out", 64, 40, 401, ne=1, nc=40)[0] == GENERAL
