@@ -194,7 +194,8 @@ __global__ __launch_bounds__((NW > 0 ? NW : kPqBwdWaves) * kWave) void dense_pq_
     const float* __restrict__ q2, float* __restrict__ gent, float* __restrict__ gq1, float* __restrict__ gq2, int num,
     int dim) {
   constexpr int MUL = kind_mul(K), NQ = kind_nq(K);
-  constexpr bool kHeavy = kind_heavy(K);
+  // (a branch that costs one-half rows more than the group's arithmetic: box 200 x 300 x 800, shared, 47.1 / 48.7 us)
+  constexpr bool kSkip = kind_heavy(K) || (SHARED && MUL == 2 && NIT * VEC == 16);
   typedef column<VEC> vec;
   extern __shared__ float lds[];  // [waves][NQ][dim]
   const int b = blockIdx.x;
@@ -231,7 +232,7 @@ __global__ __launch_bounds__((NW > 0 ? NW : kPqBwdWaves) * kWave) void dense_pq_
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int c = lane + kWave * it;
-      if (kHeavy && kWave * it >= ncol) continue;   // uniform: no column of the row in this group
+      if (kSkip && kWave * it >= ncol) continue;   // uniform: no column of the row in this group
       if (!AHEAD && c >= ncol) continue;   // (AHEAD: such lanes hold a copy of the last column, what they compute is not stored)
       vec ge1 = zero, ge2 = zero;
 #pragma unroll
@@ -368,7 +369,9 @@ static int backward_shared(hipStream_t st, const float* gout, const float* ent, 
   const size_t lds_e = (size_t)kPqBwdWaves * kind_mul(K) * L.dim * sizeof(float);
   auto launch = [&](auto nit, auto v) {
     constexpr int NIT = decltype(nit)::value, VEC = decltype(v)::value;
-    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, true, kPqBwdWaves, VEC, true>), dim3((unsigned)L.bsize), block, lds_q, st,
+    // (long rows of the arithmetic-bound kinds would spill, see per_query_form: BetaE 512 x 128 x 600 474 / 432 us)
+    constexpr bool AHEAD = !(VEC == 4 && NIT == 4 && kind_heavy(K));
+    hipLaunchKernelGGL((dense_pq_backward_kernel<K, NIT, true, kPqBwdWaves, VEC, AHEAD>), dim3((unsigned)L.bsize), block, lds_q, st,
                        gout, ent, q1, q2, gent, gq1, gq2, num, dim);
     hipLaunchKernelGGL((dense_shared_entity_backward_kernel<K, NIT, VEC>), dim3((unsigned)L.num), block, lds_e, st, gout, ent,
                        q1, q2, gent, bsize, num, dim);

@@ -51,8 +51,9 @@ inline int column_floats(const Layout& L, size_t low) {
 
 // Wavefronts per query and whether they read ahead, us a call:
 // Few rows: a wavefront each (two rows for the arithmetic-bound kinds), because one without a row takes registers and LDS from
-// other queries.  (Up to eight rows: of their workgroups of five wavefronts and more a CU holds one.)  Eight wavefronts / this, box 16384 x 1 x 400 37 / 25, 262144 x 1 x 32 254 / 62, rotate 16384 x 1 x 100
-// 23 / 11, BetaE 16384 x 1 x 400 378 / 64, 4096 x 8 x 400 134 / 97.
+// other queries.  (Up to eight rows: of their workgroups of five wavefronts and more a CU holds one.)  Eight wavefronts / this,
+// box 16384 x 1 x 400 37 / 25, 262144 x 1 x 32 254 / 62, rotate 16384 x 1 x 100 23 / 11, BetaE 16384 x 1 x 400 378 / 64,
+// 4096 x 8 x 400 134 / 97.
 // Few queries: a CU has one workgroup of the launch, or none, and sixteen wavefronts.  Eight / sixteen, box 64 x 512 x 400
 // 33 / 25, 256 x 512 x 100 29 / 22, 512 x 512 x 32 36 / 26, BetaE 256 x 512 x 100 156 / 137.  Not rows of two long halves,
 // whose registers do not suffice (BetaE 300 x 333 x 400 408 / 663), nor larger batches (box 1024 x 256 x 100 35 / 41).
@@ -86,7 +87,7 @@ inline BackwardForm dense_backward_form(const Layout& L, int kind, size_t low) {
   if (shared_layout(L)) {
     const int vec = column_floats(L, low);
     if (vec == 0 || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0, 0};
-    return {kPathShared, vec, kPqBwdWaves, 1};
+    return {kPathShared, vec, kPqBwdWaves, !(kind_heavy(kind) && vec == 4 && L.dim > 512)};
   }
   if (reverse_layout(L) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
   return {kPathGeneral, 0, 0, 0};
