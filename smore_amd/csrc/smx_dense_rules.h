@@ -27,6 +27,9 @@ constexpr bool kind_heavy(int kind) { return kind == kBetaKL || kind == kBetaFis
 // HIP counts the threads of a launch in 32 bits.
 constexpr bool launchable(size_t workgroups, size_t waves) { return workgroups < (1ull << 32) / (waves * 64); }
 
+// Row and query counts that the kernels step through by up to 2 x 16 with an int.
+constexpr bool steppable(size_t n) { return n <= 0x7fffffffull - 32; }
+
 // The layouts of the kernels below; low: the addresses of all tensors or'ed together.
 inline bool rows_of_16_bytes(const Layout& L, size_t low) { return L.dim % 4 == 0 && L.dim <= 1024 && (low & 15) == 0; }
 inline bool per_query_layout(const Layout& L) {   // entity [B,N,.] against query [B,1,.]
@@ -80,16 +83,16 @@ inline BackwardForm per_query_form(const Layout& L, int kind, int vec) {
 inline BackwardForm dense_backward_form(const Layout& L, int kind, size_t low) {
   if (per_query_layout(L)) {
     const int vec = column_floats(L, low);
-    if (vec == 0) return {kPathGeneral, 0, 0, 0};
+    if (vec == 0 || !steppable(L.num)) return {kPathGeneral, 0, 0, 0};
     const BackwardForm form = per_query_form(L, kind, vec);
     return launchable(L.bsize, form.waves) ? form : BackwardForm{kPathGeneral, 0, 0, 0};
   }
   if (shared_layout(L)) {
     const int vec = column_floats(L, low);
-    if (vec == 0 || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0, 0};
+    if (vec == 0 || !steppable(L.num) || !steppable(L.bsize) || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0, 0};
     return {kPathShared, vec, kPqBwdWaves, !(kind_heavy(kind) && vec == 4 && L.dim > 512)};
   }
-  if (reverse_layout(L) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
+  if (reverse_layout(L) && steppable(L.num) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
   return {kPathGeneral, 0, 0, 0};
 }
 

@@ -39,6 +39,16 @@ def test_every_launch_is_one_that_hip_takes(kind, dim, low, layout):
             assert path == (SHARED if num * 512 < 1 << 32 else GENERAL)
 
 
+@pytest.mark.parametrize("dim", [4, 3])
+def test_row_counts_that_an_int_cannot_be_stepped_through(dim):
+    """A wavefront's row number goes up to 2 x 16 beyond the last row before it is compared: not beyond 2^31 - 1."""
+    top = (1 << 31) - 1
+    for num, special in ((top, False), (top - 31, False), (top - 32, True)):
+        assert (form("l1", 1, num, dim)[0] == PER_QUERY) == special
+        assert (form("l1", 1, num, dim, ne=1, nc=num)[0] == REVERSE) == (special and dim == 4)
+    assert form("l1", 1, 1 << 31, dim, ne=1, nc=1)[0] == GENERAL
+
+
 def test_columns_by_row_length_and_alignment():
     for dim, low, want in ((400, 0, 4), (1024, 0, 4), (1024, 16, 4), (400, 8, 2), (402, 8, 2), (400, 4, 1), (401, 0, 1),
                            (512, 4, 1), (513, 0, 0), (514, 0, 0), (1020, 4, 0), (1028, 0, 0)):
