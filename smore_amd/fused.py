@@ -273,13 +273,12 @@ class SegmentPlan:
         return tensor
 
     def _at(self, name):
-        """Address of an array; None for an inverse that was not asked for.  Asked of the tensors that are there now: a
-        deep copy of a plan has memory of its own, and an array that the caller put in another's place is the one to read."""
-        tensor = self.__dict__.get(name)
-        if tensor is not None:
-            return tensor.data_ptr()
-        entry = self._arrays.get(name)
-        return None if entry is None else self._memory.data_ptr() + entry[0]
+        """Address of an array; None for an inverse that was not asked for and for an array that the caller took away.
+        Asked of the tensors that are there now: a deep copy of a plan has memory of its own, and an array that the caller
+        put in another's place is the one to read."""
+        if name in self.__dict__:
+            return _ptr(self.__dict__[name])
+        return self._memory.data_ptr() + self._arrays[name][0]
 
     @property
     def n_uniq(self):

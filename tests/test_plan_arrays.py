@@ -49,3 +49,16 @@ def test_an_array_that_the_caller_replaced_is_the_one_handed_out():
     plan = SegmentPlan(100, 1000, torch.device("cpu"), False)
     plan.pair_seg = torch.zeros(100, dtype=torch.int32)
     assert _addresses(plan)[FIELDS["pair_seg"]] == plan.pair_seg.data_ptr()
+
+
+@pytest.mark.parametrize("touched", [False, True])
+@pytest.mark.parametrize("name", ARRAYS)
+def test_an_array_that_the_caller_took_away_is_a_null_pointer(name, touched):
+    """pair_seg may be missing (the one-pair fast path is not used then); without another array the library refuses the plan."""
+    from smore_amd.fused import SegmentPlan
+    plan = SegmentPlan(100, 1000, torch.device("cpu"), True)
+    if touched:
+        getattr(plan, name)
+    setattr(plan, name, None)
+    assert getattr(plan, name) is None and _addresses(plan)[FIELDS[name]] is None
+    assert all(a for n, a in zip(ARRAYS, _addresses(plan)) if n != name)
