@@ -44,6 +44,14 @@ def _to_device(host, dev):
     return host.to(dev, non_blocking=host.is_pinned())
 
 
+def _counts_on(counts, dev):
+    if counts.device.type != "cpu":
+        return counts.to(dev)
+    host = _pinned(counts.numel(), torch.int32)
+    host.copy_(counts)
+    return _to_device(host, dev)
+
+
 def _one_array(lists):
     """The ids of all answer lists in a row, where they are plain lists of integers; None otherwise."""
     if not all(type(ids) in (list, tuple) for ids in lists):
@@ -122,10 +130,7 @@ def candidate_ranks(model, table, q1, q2, params, negative_sample, n_hard, err_f
     if low < 0 or high > cand.shape[1]:
         raise _lib.SmxError("one hard-answer count per query, between 0 and C")
     h = max(1, high)
-    if counts.device.type == "cpu":
-        host = _pinned(b, torch.int32)
-        host.copy_(counts)
-        counts = _to_device(host, dev)
+    counts = _counts_on(counts, dev)
     q1c = q1.reshape(b * branches, -1).contiguous()
     q2c = None if q2 is None else q2.reshape(b * branches, -1).contiguous()
     _, _, dim = _dims(model, table, cand, q1c[:b], None if q2c is None else q2c[:b])

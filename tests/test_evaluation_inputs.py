@@ -49,3 +49,18 @@ def test_answer_lists_in_one_array(kind):
         assert flat.dtype == np.int64 and flat.tolist() == [int(v) for x in lists for v in _int64(x)]
     else:
         assert kind not in ("ints", "tuple", "empty", "numpy scalars", "negative")
+
+
+def test_counts_on_another_device_are_brought_to_the_table():
+    """Counts that are on a device already are those of the table's device, whichever they came from."""
+    from smore_amd.evaluation.ranking import _counts_on
+
+    class Counts:
+        device, dtype = torch.device("cuda", 1), torch.int32
+
+        def to(self, device):
+            return "counts on", device
+
+    for index in (0, 1):
+        dev = torch.device("cuda", index)
+        assert _counts_on(Counts(), dev) == ("counts on", dev)
