@@ -34,20 +34,20 @@ def _counts(n_hard):
     return torch.from_numpy(a.astype(np.int32))
 
 
-def _pinned(count, dtype):
+def _pinned(count, dtype, dev):
     """Host memory a copy to the device need not be waited for from (it is given out again once that copy has passed).
     Under graph capture pageable memory: such a call is refused, a replay would copy whatever then lies there."""
-    return torch.empty(count, dtype=dtype, pin_memory=not torch.cuda.is_current_stream_capturing())
+    return torch.empty(count, dtype=dtype, pin_memory=dev.type == "cuda" and not torch.cuda.is_current_stream_capturing())
 
 
 def _to_device(host, dev):
-    return host.to(dev, non_blocking=host.is_pinned())
+    return host.to(dev, non_blocking=dev.type == "cuda" and host.is_pinned())
 
 
 def _counts_on(counts, dev):
     if counts.device.type != "cpu":
         return counts.to(dev)
-    host = _pinned(counts.numel(), torch.int32)
+    host = _pinned(counts.numel(), torch.int32, dev)
     host.copy_(counts)
     return _to_device(host, dev)
 
@@ -75,7 +75,7 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
     sizes = [(len(e), len(h)) for e, h in zip(easy_answers, hard_answers)]
     a = max(1, max(ne + nh for ne, nh in sizes))
     # ids [B, A] and the counts behind them travel to the device as one array, which nothing waits for
-    host = _pinned(b * a + (b + 1) // 2, torch.int64)
+    host = _pinned(b * a + (b + 1) // 2, torch.int64, table.device)
     packed = host.numpy()
     packed[:] = 0
     ids, counts = packed[: b * a].reshape(b, a), packed[b * a:].view(np.int32)

@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 import torch
 
+from smore_amd import _lib
+
 VALUES = {
     "ints": [3, 4], "tuple": (3, 4), "range": range(3), "set": {3, 4}, "keys": {3: 1}.keys(), "empty": [], "array": np.array([3, 4]),
     "int32": np.array([3, 4], dtype=np.int32), "uint8": np.array([3, 4], dtype=np.uint8), "tensor": torch.tensor([3, 4]),
@@ -64,3 +66,20 @@ def test_counts_on_another_device_are_brought_to_the_table():
     for index in (0, 1):
         dev = torch.device("cuda", index)
         assert _counts_on(Counts(), dev) == ("counts on", dev)
+
+
+@pytest.mark.parametrize("easy,hard,error,message", [([[9]], [[1]], IndexError, "outside the entity table"),
+                                                     ([[1]], [[1]], _lib.SmxError, "listed twice"),
+                                                     ([[2]], [[1]], _lib.SmxError, "fp32 device tensor")])
+def test_a_table_on_the_host_is_refused_for_the_reason_it_always_was(easy, hard, error, message):
+    """Pinned memory is for copies to a device: none is asked for (and none is needed) where the table is on the host."""
+    from smore_amd.evaluation.ranking import filtered_ranks
+    table, q = torch.rand(5, 4), torch.rand(1, 4)
+    with pytest.raises(error, match=message):
+        filtered_ranks("l1", table, q, None, None, easy, hard)
+
+
+def test_candidates_on_the_host_are_refused_for_the_reason_they_always_were():
+    from smore_amd.evaluation.ranking import candidate_ranks
+    with pytest.raises(_lib.SmxError, match="fp32 device tensor"):
+        candidate_ranks("l1", torch.rand(5, 4), torch.rand(1, 4), None, None, torch.tensor([[1, 2]]), [1])
