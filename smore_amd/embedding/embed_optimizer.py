@@ -95,9 +95,9 @@ class _FusedScoreFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gscore, _gindex):
-        if gscore is None:
-            return (None,) * 9
         q1, q2, score = ctx.saved_tensors
+        if gscore is None:      # undefined: zeros, so that the lookup still counts as one of the step
+            gscore = torch.zeros_like(score)
         opt = ctx.embed_opt
         table = opt.sparse_embed.embedding.detach()
         with torch.no_grad():

@@ -35,9 +35,9 @@ class _SampleLossFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_total, _g_out):
-        if g_total is None:
-            return None, None, None, None, None, None
         grads, = ctx.saved_tensors
+        if g_total is None:     # undefined: zeros
+            g_total = grads.new_zeros(())
         b, k = ctx.neg_shape
         grads = grads * g_total
         return (grads[grads.numel() - b:].view(ctx.pos_shape), grads[: b * k].view(b, k), None, None, None, None)

@@ -532,3 +532,35 @@ def test_fused_records_of_two_query_batches_and_a_plain_lookup_in_one_step(gamma
     assert_close(emb.state_sum_fo.cpu().numpy()[uniq], m[uniq], REL_F32, "first moment")
     assert_close(emb.state_sum_sq.cpu().numpy()[uniq], v[uniq], REL_F32, "second moment", rms_floor=False)
     assert_adam_weights(emb.embedding.detach().cpu().numpy(), w, merged, uniq, lr, "weights")
+
+
+class _NoGradient(torch.autograd.Function):
+    """x, with an undefined gradient (what autograd hands on for None)."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def test_an_undefined_gradient_of_the_scores_is_one_of_zeros():
+    """The lookup still counts as one of the step: its rows are updated from their moments (embed_optimizer.py:155-163)."""
+    n, d, b, k, lr = 50, 16, 3, 4, 1e-2
+    emb, opt = _setup(n, d, 5)
+    ids = torch.arange(b * k, device="cuda").view(b, k)
+    q = torch.zeros((b, d), device="cuda", requires_grad=True)
+    w0 = emb.embedding.detach().clone()
+    for step in (1, 2):
+        opt.zero_grad()
+        q.grad = None
+        logit = opt.score_negatives("l1", ids, q, None, gamma=12.0)
+        (logit if step == 1 else _NoGradient.apply(logit)).sum().backward()
+        assert len(opt.fused_list) == 1
+        before = emb.embedding.detach().clone()
+        opt.apply_grad(lr)
+        opt.check_ids()
+        assert not torch.equal(emb.embedding[: b * k], before[: b * k]) and torch.equal(emb.embedding[b * k:], w0[b * k:])
+    assert q.grad is not None and not bool(q.grad.any())

@@ -101,6 +101,24 @@ def test_loss_gradient_feeds_the_scoring_backward():
     assert_close(gq2.cpu().numpy(), o2[:, 0], 2 * REL_F32, "offset gradient through the loss")
 
 
+def test_an_undefined_gradient_of_the_loss_is_one_of_zeros():
+    from smore_amd.training import sample_loss
+
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    pos, neg = torch.randn(3, device="cuda", requires_grad=True), torch.randn((3, 4), device="cuda", requires_grad=True)
+    NoGradient.apply(sample_loss(pos, neg)[0]).backward()
+    for t in (pos, neg):
+        assert t.grad is not None and t.grad.shape == t.shape and not bool(t.grad.any())
+
+
 def test_argument_errors():
     from smore_amd import _lib
     from smore_amd.training import sample_loss
