@@ -515,7 +515,7 @@ __device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   }
 }
 
-// One launch each, or (few pairs: the launch itself, 4 to 5 us, is what costs) one for both, the tiles first.  Nothing is
+// One launch each, or (one_launch_tiles) one for both, the tiles first.  Nothing is
 // appended to the fix-up's list then (A.fix_list == null): that pass asks every tile itself.
 template <int SRC, int VEC, int NIT, bool REG>
 __global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
@@ -1040,6 +1040,24 @@ __global__ __launch_bounds__(256, 4) void entity_small_coded_kernel(EntityArgs A
   else segment_pass_coded<SRC, VEC, NIT>(A, code_lds, (int)blockIdx.x - tile_blocks, (int)gridDim.x - tile_blocks);
 }
 
+// Tiles of a plan up to which short and long segments go through one launch.  That saves a launch of 4 to 5 us, and with skewed
+// ids the two passes share the chip (28 us of 104 at 32,768 box pairs of 400 floats).  But the kernel has the registers
+// of the greater of the two, and the tiles' workgroups, which hardly find a long segment where ids are uniform, stand before the
+// segments': where two or fewer workgroups fit a CU, or fewer than of the segment pass alone, uniform ids lose from some size on.
+// The whole backward, uniform ids, two launches -> one, us:
+//   gradient rows 400 floats, 256 tiles 50 -> 47, 1600 floats 227 -> 248;  L2 200, 256 tiles 43 -> 40, 400 65 -> 63, 800 106 -> 114
+//   box 400, 32 tiles 31 -> 30, 128 61 -> 62, 512 90 -> 94;  from sign codes 200, 32 tiles 21 -> 20, 128 33 -> 36, 400 52 -> 51
+//   rotate 200, 32 tiles 29 -> 28, 256 62 -> 64;  400, 128 tiles 104 -> 102, 512 152 -> 157;  800, 8 tiles 43 -> 50
+template <int SRC, int VEC, int NIT>
+constexpr unsigned one_launch_tiles(bool coded) {
+  if (coded) return VEC == 4 && NIT == 2 ? 512 : 32;
+  if (VEC == 1) return 512;
+  if (SRC == kSrcRows) return NIT <= 4 ? 512 : 0;
+  if (NIT > 2) return 0;
+  if (src_mul(SRC) == 2) return NIT == 1 ? 32 : 128;
+  return SRC == mBox && NIT == 2 ? 64 : 512;
+}
+
 // Workgroups of 256 threads of `kernel` (with that much dynamic LDS) the current device keeps resident; asked
 // once per kernel and device.
 template <class K>
@@ -1065,34 +1083,36 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   // short segments: a fixed grid of wavefronts strides over the segment list (its length lives on the device)
   // (as many workgroups as the chip holds at once: a second wave of workgroups would run half empty)
   const unsigned want_blocks = (unsigned)(((A.n_pairs + A.chunk - 1) / A.chunk + 3) / 4);
-  // Few tiles: one launch for both passes.  65,536 pairs, L2 x 200: 24.7 + 4.8 us in two, 24.4 in one, the step 79.0 -> 76.4;
-  // the entity pass of a shared list's step, 1,536 rows of ComplEx, 13.2 + 5.0 -> 12.3.  (Beyond, the launch is below 2 % of the passes.)
-  const bool small = tiles <= 512;
+  constexpr unsigned kOneLaunch = one_launch_tiles<SRC, VEC, NIT>(false), kOneLaunchCoded = one_launch_tiles<SRC, VEC, NIT>(true);
   const unsigned tile_blocks = (tiles + 3) / 4;
   EntityArgs F = A;
-  if (small) F.fix_list = nullptr;
   bool coded = false;
   // (sign codes exist for rows of up to two column groups)
   if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) coded = A.codes != nullptr;
   if (coded) {
     if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) {
       const size_t slabs = (size_t)4 * 64 * NIT * 64;  // one code record per lane and wavefront
-      if (small) {
+      if (tiles <= kOneLaunchCoded) {
+        F.fix_list = nullptr;
         const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_coded_kernel<SRC, VEC, NIT>, (int)slabs));
         hipLaunchKernelGGL((entity_small_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks + seg_blocks), dim3(256), slabs, st, F,
                            (int)tile_blocks);
       } else {
-      const unsigned seg_blocks =
-          min(want_blocks, resident_blocks(entity_segment_coded_kernel<SRC, VEC, NIT>, (int)slabs));
-      hipLaunchKernelGGL((entity_segment_coded_kernel<SRC, VEC, NIT>), dim3(seg_blocks), dim3(256), slabs, st, A);
-      hipLaunchKernelGGL((entity_tile_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks), dim3(256), slabs, st, A);
+        const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_segment_coded_kernel<SRC, VEC, NIT>, (int)slabs));
+        hipLaunchKernelGGL((entity_segment_coded_kernel<SRC, VEC, NIT>), dim3(seg_blocks), dim3(256), slabs, st, A);
+        hipLaunchKernelGGL((entity_tile_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks), dim3(256), slabs, st, A);
       }
     }
-  } else if (small) {
-    const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_kernel<SRC, VEC, NIT, REG>, 0));
-    hipLaunchKernelGGL((entity_small_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks + seg_blocks), dim3(256), 0, st, F,
-                       (int)tile_blocks);
-  } else {
+  }
+  if constexpr (kOneLaunch > 0) {
+    if (!coded && tiles <= kOneLaunch) {
+      F.fix_list = nullptr;
+      const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_kernel<SRC, VEC, NIT, REG>, 0));
+      hipLaunchKernelGGL((entity_small_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks + seg_blocks), dim3(256), 0, st, F,
+                         (int)tile_blocks);
+    }
+  }
+  if (!coded && tiles > kOneLaunch) {
     const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_segment_kernel<SRC, VEC, NIT, REG>, 0));
     hipLaunchKernelGGL((entity_segment_kernel<SRC, VEC, NIT, REG>), dim3(seg_blocks), dim3(256), 0, st, A);
     hipLaunchKernelGGL((entity_tile_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks), dim3(256), 0, st, A);

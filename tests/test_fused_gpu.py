@@ -1270,13 +1270,9 @@ def test_gradient_rows_at_a_size_that_forks():
     assert torch.equal(out["fused"][0][~touched], table[~touched])
 
 
-@pytest.mark.parametrize("n_pairs", [1, 255, 257, 131_072, 131_073])
-def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n_pairs):
-    """Up to 512 tiles of 256 pairs short and long segments go through one launch, and the fix-up finds its tiles by
-    itself: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
-    gradient rows and, from sign codes and without, of box pairs, against float64."""
+def _entity_pass_in_both_forms(n_pairs, dim):
     from smore_amd import fused
-    n, dim = 3000, 12
+    n = 3000
     gen = torch.Generator(device="cuda")
     gen.manual_seed(n_pairs)
     ids = torch.randint(20, n, (n_pairs,), device="cuda", generator=gen)
@@ -1307,3 +1303,19 @@ def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n
         got.fill_(float("nan"))
         fused.score_backward_entity("box", plan, table, q1, q2, score, gs, params, merged=got, codes=c)
         assert_close(got.cpu().numpy(), sums(want).cpu().numpy(), 1e-6, "box rows", sum_abs=8 * sums(want.abs()).cpu().numpy())
+
+
+@pytest.mark.parametrize("n_pairs", [1, 255, 257, 131_072, 131_073])
+def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n_pairs):
+    """Up to 512 tiles of 256 pairs short and long segments of short rows go through one launch, and the fix-up finds its
+    tiles by itself: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
+    gradient rows and, from sign codes and without, of box pairs, against float64."""
+    _entity_pass_in_both_forms(n_pairs, 12)
+
+
+@pytest.mark.parametrize("n_pairs,dim", [(8192, 12), (8193, 12), (16_384, 260), (16_385, 260), (131_072, 50), (131_073, 50),
+                                         (8193, 30), (256, 516), (257, 1100)])
+def test_entity_pass_around_the_sizes_of_other_row_lengths(n_pairs, dim):
+    """Where sign codes (32 tiles), box rows of two column groups (64) and rows of 4-byte columns (512) get launches of their
+    own for short and long segments, and rows so long that they always do."""
+    _entity_pass_in_both_forms(n_pairs, dim)
