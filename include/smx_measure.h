@@ -56,6 +56,11 @@ int smx_measure_plan_build(void* stream, const int64_t* idx, size_t n_pairs, siz
 int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc,
                                     size_t dim, size_t addresses, int* path, int* vec, int* waves, int* ahead);
 
+/* No counterpart in the reference.  The same question for smx_dist_forward_f32 (its addresses: entity, queries, output);
+ * rows_per_tile: entity rows (reverse layout: query rows) that a workgroup takes, 0 with the general kernel.  Host only. */
+int smx_measure_dense_forward_form(size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc, size_t dim,
+                                   size_t addresses, int* path, int* rows_per_tile);
+
 #ifdef __cplusplus
 }
 #endif

@@ -153,6 +153,8 @@ MEASURE_SIGNATURES = {
     "smx_measure_query_kernel_events": (_i, [_vp, _vp]),
     # kind, bsize, num, be, ne, bc, nc, dim, addresses, path, vec, waves, ahead
     "smx_measure_dense_backward_form": (_i, [_i] + [_sz] * 8 + [_vp] * 4),
+    # bsize, num, be, ne, bc, nc, dim, addresses, path, rows_per_tile
+    "smx_measure_dense_forward_form": (_i, [_sz] * 8 + [_vp] * 2),
 }
 
 

@@ -503,9 +503,8 @@ __global__ __launch_bounds__(kPqBwdWaves * kWave) void dense_rev_backward_kernel
 }
 
 template <int K>
-static int forward_rev(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L) {
-  int rows_per_tile = (int)L.num;
-  while (rows_per_tile > 8 && L.bsize * ((L.num + rows_per_tile - 1) / rows_per_tile) < 8192) rows_per_tile = (rows_per_tile + 1) / 2;
+static int forward_rev(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L,
+                       int rows_per_tile) {
   const int tiles = (int)((L.num + rows_per_tile - 1) / rows_per_tile);
   const size_t lds = (size_t)kind_mul(K) * L.dim * sizeof(float);
   hipLaunchKernelGGL((dense_rev_forward_kernel<K>), dim3((unsigned)(L.bsize * tiles)), dim3(256), lds, st, ent, q1, q2, dst,
@@ -530,12 +529,9 @@ static int backward_rev(hipStream_t st, const float* gout, const float* ent, con
 }
 
 template <int K, bool SHARED = false>
-static int forward_pq(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L) {
-  // enough workgroups to fill the chip, at least eight rows each when there are that many
-  int rows_per_tile = (int)L.num;
-  while (rows_per_tile > 8 && L.bsize * ((L.num + rows_per_tile - 1) / rows_per_tile) < 8192) rows_per_tile = (rows_per_tile + 1) / 2;
+static int forward_pq(hipStream_t st, const float* ent, const float* q1, const float* q2, float* dst, const Layout& L,
+                      int rows_per_tile) {
   const int tiles = (int)((L.num + rows_per_tile - 1) / rows_per_tile);
-  if (L.bsize * (size_t)tiles > 0x7fffffffull) return -1;
   const size_t lds = (size_t)kind_nq(K) * L.dim * sizeof(float);
   hipLaunchKernelGGL((dense_pq_forward_kernel<K, SHARED>), dim3((unsigned)(L.bsize * tiles)), dim3(256), lds, st, ent, q1, q2, dst,
                      (int)L.num, (int)L.dim, tiles, rows_per_tile);
@@ -635,30 +631,30 @@ int dense_forward(int kind, void* stream, const T* ent, const T* q1, const T* q2
   if (!ent || !q1 || !dst || (kind_nq(kind) == 2 && !q2)) return fail(SMX_ERR_ARG, "null tensor pointer");
   hipStream_t st = as_stream(stream);
   if constexpr (std::is_same<T, float>::value) {
-    const bool rows = rows_of_16_bytes(L, low_bits(ent, q1, q2, dst));
-    if (rows && per_query_layout(L)) {
+    const ForwardForm form = dense_forward_form(L, low_bits(ent, q1, q2, dst));
+    if (form.path == kPathPerQuery) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return forward_pq<KK>(st, ent, q1, q2, dst, L);
+    return forward_pq<KK>(st, ent, q1, q2, dst, L, form.rows_per_tile);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
     }
-    if (rows && shared_layout(L)) {
+    if (form.path == kPathShared) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return forward_pq<KK, true>(st, ent, q1, q2, dst, L);
+    return forward_pq<KK, true>(st, ent, q1, q2, dst, L, form.rows_per_tile);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
     }
-    if (rows && reverse_layout(L)) {
+    if (form.path == kPathReverse) {
       switch (kind) {
 #define X(KK) \
   case KK:    \
-    return forward_rev<KK>(st, ent, q1, q2, dst, L);
+    return forward_rev<KK>(st, ent, q1, q2, dst, L, form.rows_per_tile);
         SMX_FOR_EACH_KIND(X)
 #undef X
       }
@@ -757,6 +753,16 @@ int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t b
   *vec = form.vec;
   *waves = form.waves;
   *ahead = form.ahead;
+  return SMX_OK;
+}
+int smx_measure_dense_forward_form(size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc, size_t dim,
+                                   size_t addresses, int* path, int* rows_per_tile) {
+  using namespace smx;
+  const Layout L{bsize, num, be, ne, bc, nc, dim};
+  if (int rc = check_layout(L)) return rc;
+  const ForwardForm form = dense_forward_form(L, addresses);
+  *path = form.path;
+  *rows_per_tile = form.rows_per_tile;
   return SMX_OK;
 }
 

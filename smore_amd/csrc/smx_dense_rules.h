@@ -1,5 +1,5 @@
-// Which kernel a call of the dense operators' backward gets: rules on sizes and alignment alone, so that they can be asked
-// where there is no device (smx_measure_dense_backward_form).
+// Which kernel a call of the dense operators gets: rules on sizes and alignment alone, so that they can be asked where there
+// is no device (smx_measure_dense_backward_form, smx_measure_dense_forward_form).
 #pragma once
 #include <cstddef>
 
@@ -94,6 +94,24 @@ inline BackwardForm dense_backward_form(const Layout& L, int kind, size_t low) {
   }
   if (reverse_layout(L) && steppable(L.num) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
   return {kPathGeneral, 0, 0, 0};
+}
+
+// Per-query, shared and reverse forward: rows per workgroup, enough workgroups to fill the chip, at least eight rows each when
+// there are that many.  A tile's end, and a row number stepped by eight beyond it, are ints in those kernels.
+struct ForwardForm {
+  int path, rows_per_tile;
+};
+
+inline ForwardForm dense_forward_form(const Layout& L, size_t low) {
+  const ForwardForm general = {kPathGeneral, 0};
+  if (!rows_of_16_bytes(L, low)) return general;
+  const int path = per_query_layout(L) ? kPathPerQuery : shared_layout(L) ? kPathShared : reverse_layout(L) ? kPathReverse : kPathGeneral;
+  if (path == kPathGeneral) return general;
+  size_t rows = L.num;
+  auto tiles = [&] { return (L.num + rows - 1) / rows; };
+  while (rows > 8 && L.bsize * tiles() < 8192) rows = (rows + 1) / 2;
+  if (!steppable(L.num + rows) || !launchable(L.bsize * tiles(), 4)) return general;
+  return {path, (int)rows};
 }
 
 }  // namespace smx

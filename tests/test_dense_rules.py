@@ -1,4 +1,4 @@
-"""Which kernels the backward of the dense operators takes, asked on the host (smx_measure_dense_backward_form)."""
+"""Which kernels the dense operators take, asked on the host (smx_measure_dense_backward_form, smx_measure_dense_forward_form)."""
 import ctypes
 
 import pytest
@@ -59,3 +59,32 @@ def test_columns_by_row_length_and_alignment():
     assert form("box_out", 64, 40, 400, ne=1, nc=40)[0] == REVERSE
     assert form("box_out", 64, 40, 401, ne=1, nc=40)[0] == GENERAL
     assert form("box_out", 64, 40, 400, ne=40, nc=40)[0] == GENERAL
+
+
+def forward_form(bsize, num, dim, be=None, ne=None, nc=1, low=0):
+    path, rows = ctypes.c_int(), ctypes.c_int()
+    lib = _lib.load()
+    rc = lib.smx_measure_dense_forward_form(bsize, num, be or bsize, ne or num, bsize, nc, dim, low, ctypes.byref(path),
+                                            ctypes.byref(rows))
+    assert rc == 0, lib.smx_last_error()
+    return path.value, rows.value
+
+
+def test_forward_row_numbers_and_launches_stay_in_range():
+    """A tile's end and a row number stepped beyond it fit an int, and a launch has fewer than 2^32 threads; the general kernel,
+    whose grid is bounded and whose numbers are 64 bits wide, takes the rest."""
+    top = (1 << 31) - 1
+    for bsize in (1, 2, 3):
+        for num in (1, 9, 100_000, top // bsize - 300_000, top // bsize - 100_000, top // bsize - 8, top // bsize):
+            for layout, extra in ((PER_QUERY, {}), (SHARED, dict(be=1)), (REVERSE, dict(ne=1, nc=num))):
+                path, rows = forward_form(bsize, num, 4, **extra)
+                tiles = -(-num // rows) if rows else 0
+                if path == GENERAL:
+                    assert num > top - 300_000
+                else:
+                    assert path == layout or num == 1 or bsize == 1 and layout == SHARED
+                    assert tiles * rows + 8 <= top and bsize * tiles * 256 < 1 << 32
+    assert forward_form(1, top - 8, 4)[0] == forward_form(1, top - 100_000, 4)[0] == GENERAL
+    for bsize in ((1 << 24) - 1, 1 << 24):      # a workgroup of 256 threads per query
+        assert forward_form(bsize, 1, 4)[0] == (PER_QUERY if bsize < 1 << 24 else GENERAL)
+    assert forward_form(64, 40, 400, low=8)[0] == forward_form(64, 40, 401)[0] == GENERAL
