@@ -32,6 +32,10 @@ int smx_measure_backward_fused(int parts, int model, void* stream, const smx_pla
  * The events are used once; NULL, NULL clears a pair that was set and not used. */
 int smx_measure_query_kernel_events(void* before, void* after);
 
+/* No counterpart in the reference.  How smx_score_forward divides B x K pairs given by ids: the pairs of a workgroup
+ * (16: 16 or fewer, by the row's length) and whether it scores each distinct id among them once.  Host only. */
+int smx_measure_forward_tile(int model, size_t B, size_t K, int* tile, int* distinct);
+
 /* No counterpart in the reference.  smx_plan_build with the two knobs a test needs to see a plan give up while
  * every kernel still ends normally:
  *   spin_limit    polls a workgroup of the sort makes before it stops waiting for another one (the library

@@ -151,6 +151,8 @@ MEASURE_SIGNATURES = {
     # the arguments of smx_plan_build, then spin_limit, force_abort
     "smx_measure_plan_build": (_i, SIGNATURES["smx_plan_build"][1] + [_c.c_uint, _i]),
     "smx_measure_query_kernel_events": (_i, [_vp, _vp]),
+    # model, B, K, tile, distinct
+    "smx_measure_forward_tile": (_i, [_i, _sz, _sz, _vp, _vp]),
     # kind, bsize, num, be, ne, bc, nc, dim, addresses, path, vec, waves, ahead
     "smx_measure_dense_backward_form": (_i, [_i] + [_sz] * 8 + [_vp] * 4),
     # bsize, num, be, ne, bc, nc, dim, addresses, path, rows_per_tile

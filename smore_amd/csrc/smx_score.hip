@@ -698,6 +698,13 @@ int smx_measure_query_kernel_events(void* before, void* after) {
   return SMX_OK;
 }
 
+int smx_measure_forward_tile(int model, size_t B, size_t K, int* tile, int* distinct) {
+  if (model < 0 || model >= smx::mNumModels) return smx::fail(SMX_ERR_KIND, "unknown score model %d", model);
+  *tile = smx::forward_tile(B, K, 16);
+  *distinct = *tile >= smx::distinct_from(model);
+  return SMX_OK;
+}
+
 int smx_measure_backward_fused(int parts, int model, void* stream, const smx_plan_view* plan, float* table, size_t n_rows,
                                const int64_t* idx, const float* q1, const float* q2, const float* score,
                                const float* gscore, float* gq1, float* gq2, size_t B, size_t K, size_t dim,

@@ -783,23 +783,32 @@ constexpr int rows_in_flight(int nit, int mul) {
   return r < 1 ? 1 : r;
 }
 
+// Pairs of a forward workgroup: 64 per wavefront, fewer where the grid would not fill the chip.
+inline int forward_tile(size_t B, size_t K, int least) {
+  int tile_k = 256;
+  while (tile_k > least && (B * ((K + tile_k - 1) / tile_k) < 8192 || (size_t)tile_k / 2 >= K)) tile_k /= 2;
+  return tile_k;
+}
+
+// Tile length from which each distinct entity of a tile is scored once.  Not the short tiles of small batches: few of their ids
+// repeat, and the tables, the barriers and the LDS they take -- 49 KiB for sign codes of 400 floats, three workgroups per CU -- cost
+// more than the repeats.  Uniform / skewed ids, us with and without: box 512 x 128 x 400 46 / 43 -> 23 / 22, 400 x 400 x 400
+// 61 / 57 -> 39 / 30, L1 54 / 46 -> 36 / 27 at 1024 x 128 x 400, L2 512 x 128 x 200 12.8 / 11.5 -> 11.6 / 10.3.  Tiles of 64,
+// 1024 x 512 x 400: box 116 / 87 -> 113 / 68, but BetaE, whose pairs are arithmetic, 341 / 300 -> 337 / 336 at 200.  Tiles of 128,
+// 2000 x 1000 x 200: L2 162 / 77 -> 164 / 93.
+// Below it every pair is scored where it stands, and repeats of one id may then differ in their last bits, as those of two tiles may.
+constexpr int distinct_from(int model) { return model == mBetaKL ? 64 : 128; }
+
 template <int M, int VEC, int NIT, bool REG>
 int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
   constexpr int RIF = rows_in_flight(NIT, model_mul(M));
   const size_t B = (size_t)A.B, K = (size_t)A.K;
-  int tile_k = 256;  // 64 negatives per wavefront; smaller tiles when the grid would not fill the chip
-  while (tile_k > 4 * RIF && (B * ((K + tile_k - 1) / tile_k) < 8192 || (size_t)tile_k / 2 >= K)) tile_k /= 2;
+  const int tile_k = forward_tile(B, K, 4 * RIF);
   const int tiles = (int)((K + tile_k - 1) / tile_k);
   const size_t lds = ((size_t)model_nq(M) * A.ncol * VEC + 4 * kSlabDwords) * sizeof(float);
-  // ids given (not the dense layout, whose rows are all different): score each distinct entity of a
-  // tile once
-  // (not for a list of ids shared by the batch: a sampler's K negatives hardly ever repeat)
-  // (and not for the short tiles of small batches: few of their ids repeat, and the tables, the barriers and the LDS they
-  // take -- 49 KiB for sign codes of 400 floats, three workgroups per CU -- cost more than the repeats.  Uniform / skewed ids,
-  // us with and without: box 512 x 128 x 400 46 / 43 -> 23 / 22, 400 x 400 x 400 61 / 57 -> 39 / 30, L1 54 / 46 -> 36 / 27 at
-  // 1024 x 128 x 400, L2 512 x 128 x 200 12.8 / 11.5 -> 11.6 / 10.3.  Tiles of 64, 1024 x 512 x 400: box 116 / 87 -> 113 / 68, but
-  // BetaE, whose pairs are arithmetic, 341 / 300 -> 337 / 336 at 200.  Tiles of 128, 2000 x 1000 x 200: L2 162 / 77 -> 164 / 93.)
-  const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= (M == mBetaKL ? 64 : 128);
+  // (not the dense layout, whose rows are all different, nor a list of ids shared by the batch: a sampler's K negatives hardly
+  // ever repeat)
+  const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= distinct_from(M);
   if constexpr (model_coded(M) && !REG) {
     if (A.codes) {
       if (dedup)

@@ -1,6 +1,8 @@
 """Gather-fused path (score forward, query backward, segment plan, entity backward + sparse Adam)
 through the C ABI against the CPU oracle.  Integer results are compared bit for bit, floating
 point ones to the 1e-5 bar of tests/util.py."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -996,10 +998,9 @@ def test_several_index_streams_at_a_size_that_forks():
 
 
 @pytest.mark.parametrize("model,dim", [("box", 200), ("box", 400), ("l1", 30), ("l2", 64), ("rotate", 48), ("beta_kl", 20)])
-def test_forward_scores_each_distinct_entity_of_a_tile_once(model, dim):
-    """The forward de-duplicates ids inside a workgroup's tile of negatives: every pair must still get
-    the bits it would get alone.  Queries whose negatives are all one entity, all distinct, drawn from three
-    entities, and a last batch of 6 pairs (K = 70); scores against the dense layout (rows given pair by pair, no
+def test_forward_of_repeated_ids_in_short_tiles(model, dim):
+    """A batch so small that every pair is scored where it stands, with repeated ids: queries whose negatives are all one
+    entity, all distinct, drawn from three entities, and a last batch of 6 pairs (K = 70); scores against the dense layout (rows given pair by pair, no
     ids, no de-duplication) bit for bit and against the oracle; sign codes (box, l1) through the backward that
     reads them against the backward that recomputes from the rows, bit for bit."""
     from smore_amd import fused
@@ -1040,6 +1041,79 @@ def test_forward_scores_each_distinct_entity_of_a_tile_once(model, dim):
         assert_close(got[True][1].cpu().numpy(), got[False][1].cpu().numpy(), 1e-6, "gq1 from the forward's codes")
     else:
         assert codes is None
+
+
+def forward_tile(model, b, k):
+    """(pairs of a forward workgroup, whether it scores each distinct id among them once)"""
+    from smore_amd import _lib, fused
+    tile, distinct = ctypes.c_int(), ctypes.c_int()
+    _lib.call("smx_measure_forward_tile", fused.MODELS[model], b, k, ctypes.byref(tile), ctypes.byref(distinct))
+    return tile.value, bool(distinct.value)
+
+
+@pytest.mark.parametrize("model,dim,b,k,tile", [
+    ("box", 400, 2731, 300, 128), ("box", 30, 8192, 100, 128), ("box", 64, 8192, 130, 256), ("l1", 400, 8192, 128, 128),
+    ("l1", 30, 2731, 300, 128), ("l2", 64, 2731, 300, 128), ("rotate", 48, 2731, 300, 128), ("beta_kl", 20, 2731, 150, 64),
+    ("beta_kl_clamped", 20, 2731, 150, 64), ("beta_kl", 20, 2731, 300, 128), ("complex", 24, 2731, 300, 128),
+    ("complex_norm", 24, 2731, 300, 128), ("distmult", 24, 2731, 300, 128), ("distmult_norm", 24, 2731, 300, 128)])
+def test_forward_scores_each_distinct_entity_of_a_tile_once(model, dim, b, k, tile):
+    """The forward de-duplicates ids inside a workgroup's tile of negatives, in tiles as short as it does so and longer, with
+    and without a ragged last one.  Queries whose negatives are all one entity, all distinct, drawn from three entities, and all
+    equal but for the last tile; skewed ids in the others.  Repeats in a tile have the same bits; scores and sign codes (box,
+    l1) of three groups of queries against the same queries in a batch so small that every pair is scored where it stands, and
+    against the oracle; query gradients from the codes against those recomputed from the rows."""
+    from smore_amd import fused
+    assert forward_tile(model.split("_norm")[0].split("_clamped")[0], b, k) == (tile, True)
+    rng = np.random.default_rng(seed("dedup", model, dim, b, k))
+    gamma, norm, clamped = GAMMA[model.split("_clamped")[0]], model.endswith("_norm"), model.endswith("_clamped")
+    model = model.split("_norm")[0].split("_clamped")[0]
+    n = 500
+    table, q1, q2, idx, gs = make_problem(model, n, b, k, dim, rng, zipf=1.1)
+    if clamped:
+        table = (rng.standard_normal((n, 2 * dim)) * 1.5).astype(np.float32).astype(np.float64)
+    idx[0, :] = 7
+    idx[1, :] = np.arange(k)
+    idx[2, :] = rng.choice([3, 4, 88], size=k)
+    idx[3, :] = 11
+    idx[3, (k - 1) // tile * tile:] = np.arange(k - (k - 1) // tile * tile) + 20
+    idx[b - 1] = idx[2]
+    params = fused.score_params(gamma, 0.02, regularizer=(1.0, 0.05, 1e9) if clamped else None, norm=norm)
+    t_table, t_q1, t_q2 = dev(table), dev(q1), dev(q2)
+    t_idx = torch.tensor(idx, device="cuda")
+    codes = fused.new_codes(model, t_table, t_idx, t_q1)
+    assert (codes is not None) == (model in ("box", "l1"))
+    score = fused.score_forward(model, t_table, t_idx, t_q1, t_q2, params)
+    if codes is not None:
+        assert torch.equal(fused.score_forward(model, t_table, t_idx, t_q1, t_q2, params, codes=codes), score)
+        per_pair = codes.view(b, k, -1)
+    for q in (0, 2, 3, b - 1):
+        for k0 in range(0, k, tile):
+            ids = t_idx[q, k0:k0 + tile]
+            for e in ids.unique():
+                at = (ids == e).nonzero()[:, 0] + k0
+                assert bool((score[q, at] == score[q, at[0]]).all()), "repeats must have their representative's score"
+                assert codes is None or torch.equal(per_pair[q, at], per_pair[q, at[:1]].expand(len(at), -1))
+    for b0 in (0, b // 2, b - 16):
+        s = slice(b0, b0 + 16)
+        few_q2 = None if t_q2 is None else t_q2[s].contiguous()
+        assert not forward_tile(model, 16, k)[1]
+        few_codes = None if codes is None else fused.new_codes(model, t_table, t_idx[s], t_q1[s])
+        few = fused.score_forward(model, t_table, t_idx[s].contiguous(), t_q1[s].contiguous(), few_q2, params, codes=few_codes)
+        if codes is not None:
+            assert torch.equal(score[s], few), "every pair must get the bits it would get alone"
+            assert torch.equal(per_pair[s], few_codes.view(16, k, -1))
+        rows = orc.gather(orc.regularizer(table) if clamped else table, idx[s]).reshape(16, k, -1)
+        want = orc.score_forward(model, rows, q1[s][:, None], None if q2 is None else q2[s][:, None], gamma, 0.02, norm=norm)
+        signed = model in ("beta_kl", "complex", "distmult")
+        for got in (score[s], few):
+            assert_close(got.cpu().numpy(), want, REL_F32, f"{model} score with repeated ids", rms_floor=signed)
+    if codes is not None:
+        t_gs = dev(gs)
+        from_codes = fused.score_backward_query(model, t_table, t_idx, t_q1, t_q2, score, t_gs, params, codes=codes)
+        recomputed = fused.score_backward_query(model, t_table, t_idx, t_q1, t_q2, score, t_gs, params)
+        for got, ref in zip(from_codes, recomputed):
+            if ref is not None:
+                assert_close(got.cpu().numpy(), ref.cpu().numpy(), 1e-6, f"{model} query gradient from the forward's codes")
 
 
 @pytest.mark.parametrize("model,dim,n", [("box", 16, 3000), ("l2", 8, 200), ("box", 200, 100_000), ("rotate", 24, 700)])
