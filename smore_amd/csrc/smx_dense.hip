@@ -13,13 +13,14 @@
 //           in ascending job order, so every sum has a fixed order and no
 //           atomics are needed.
 //
-// Per-query kernels (fp32, 16-byte aligned rows, entity [B,N,dim*mul] against query [B,1,dim]: the
-// layout of the models' negatives [B,K] and positives [B,1], kg_reasoning.py:342-355): the query lives
-// in LDS / registers, every entity row is read once with 16-byte loads, and the backward writes the
-// row gradient and accumulates the query gradient in the same pass.  Shared negatives [1,N,.] and the
-// reverse layout (entity [B,1,.] against query [B,N,.]) have kernels of the same build.
-#include <type_traits>
-
+// Per-query kernels (fp32, entity [B,N,dim*mul] against query [B,1,dim]: the layout of the models'
+// negatives [B,K] and positives [B,1], kg_reasoning.py:342-355): the query lives in LDS / registers,
+// every entity row is read once, and the backward writes the row gradient and accumulates the query
+// gradient in the same pass.  Shared negatives [1,N,.] and the reverse layout (entity [B,1,.] against
+// query [B,N,.]) have kernels of the same build.  Rows of up to 1,024 floats in 16-byte columns; the
+// backward of the first two layouts also takes rows of up to 512 floats in 8- or 4-byte columns.
+// Everything else, and sizes that the kernels' ints or a launch cannot hold, is left to the general
+// kernels (smx_dense_rules.h).
 #include <type_traits>
 
 #include "../../include/smx_measure.h"
@@ -742,8 +743,7 @@ int smx_dist_backward_f64(int kind, void* stream, const double* gout, const doub
   return smx::dense_backward<double>(kind, stream, gout, ent, q1, q2, gent, gq1, gq2, bsize, num, be, ne, bc, nc, dim);
 }
 int smx_measure_dense_backward_form(int kind, size_t bsize, size_t num, size_t be, size_t ne, size_t bc, size_t nc, size_t dim,
-                                    size_t addresses, int* path, int* vec, int* waves,
-                                    int* ahead) {
+                                    size_t addresses, int* path, int* vec, int* waves, int* ahead) {
   using namespace smx;
   if (kind < 0 || kind >= kNumKinds) return fail(SMX_ERR_KIND, "unknown dist kind %d", kind);
   const Layout L{bsize, num, be, ne, bc, nc, dim};

@@ -89,7 +89,8 @@ inline BackwardForm dense_backward_form(const Layout& L, int kind, size_t low) {
   }
   if (shared_layout(L)) {
     const int vec = column_floats(L, low);
-    if (vec == 0 || !steppable(L.num) || !steppable(L.bsize) || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves)) return {kPathGeneral, 0, 0, 0};
+    if (vec == 0 || !steppable(L.num) || !steppable(L.bsize) || !launchable(L.bsize, kPqBwdWaves) || !launchable(L.num, kPqBwdWaves))
+      return {kPathGeneral, 0, 0, 0};
     return {kPathShared, vec, kPqBwdWaves, !(kind_heavy(kind) && vec == 4 && L.dim > 512)};
   }
   if (reverse_layout(L) && steppable(L.num) && rows_of_16_bytes(L, low)) return {kPathReverse, 4, kPqBwdWaves, 0};
