@@ -158,6 +158,10 @@ class EmbeddingOptimizer(ABC):
         sp_embed.register_state_dict_pre_hook(lambda module, prefix, keep_vars: self.poll_pending_id_check())
         self.prepare_state()
 
+    def __getstate__(self):
+        """A copy (copy.deepcopy of a model follows its table to its optimizer) records an event of its own."""
+        return {**self.__dict__, "_flag_copied": None}
+
     # -- set-up protocol of the trainer (embed_optimizer.py:71-75, 102-110; called as
     #    get_optim_class(args).prepare_optimizers(args, sparse_embeds) before the workers start)
     @classmethod

@@ -1,5 +1,6 @@
 """The sparse-embedding driver protocol (zero_grad -> lookups/scores -> backward -> apply_grad) on the
 HIP path, against the CPU oracle's float64 pipeline."""
+import copy
 import types
 
 import numpy as np
@@ -564,3 +565,28 @@ def test_an_undefined_gradient_of_the_scores_is_one_of_zeros():
         opt.check_ids()
         assert not torch.equal(emb.embedding[: b * k], before[: b * k]) and torch.equal(emb.embedding[b * k:], w0[b * k:])
     assert q.grad is not None and not bool(q.grad.any())
+
+
+def test_a_table_can_be_copied_between_steps():
+    """A deep copy of a table (an average of the weights, say) brings its optimizer along, and both go on by themselves."""
+    n, d, b, k, lr = 60, 16, 3, 5, 1e-2
+    emb, opt = _setup(n, d, 6)
+    ids = torch.arange(b * k, device="cuda").view(b, k)
+    q = torch.ones((b, d), device="cuda")
+
+    def step(opt):
+        opt.zero_grad()
+        opt.score_negatives("l1", ids, q.clone().requires_grad_(), None, gamma=12.0).sum().backward()
+        opt.apply_grad(lr)
+        opt.check_ids()
+        opt.zero_grad()
+
+    step(opt)
+    other = copy.deepcopy(emb)
+    theirs = other.fwd_delegate.__self__
+    assert theirs is not opt and theirs.sparse_embed is other and torch.equal(other.embedding, emb.embedding)
+    before = emb.embedding.detach().clone()
+    step(theirs)
+    assert torch.equal(emb.embedding, before) and not torch.equal(other.embedding, before)
+    step(opt)
+    assert torch.equal(other.embedding, emb.embedding) and torch.equal(other.state_sum_sq, emb.state_sum_sq)

@@ -2,11 +2,13 @@
 lazy and reach the fused scorer as ONE request with the right model / margin / coefficient / prologue, and which
 fall back to the looked-up rows.  The optimizer is replaced by a recorder whose scorer evaluates textbook torch
 expressions, so every result is also checked by value."""
+import copy
 import types
 
 import pytest
 import torch
 
+from smore_amd.embedding.embed_optimizer import AdamEmbedOptimizer
 from smore_amd.embedding.lazy_rows import LazyLogit, LazyRows
 from smore_amd.torchext import ext_ops
 
@@ -672,3 +674,14 @@ def test_comparisons_and_the_rarer_operators_give_what_the_tensor_gives():
     copy = LazyRows(opt, ids, None)
     copy[0] = 0.0                                                       # writes into the looked-up rows
     assert float(copy.materialize()[0].abs().sum()) == 0.0
+
+
+def test_an_optimizer_between_steps_can_be_copied():
+    """The event that every step records anew is not part of its state; the one that a step left for the next is."""
+    opt = AdamEmbedOptimizer.__new__(AdamEmbedOptimizer)
+    opt.step, opt._flag_event, opt._flag_copied = 3, None, torch.cuda.Event()
+    other = copy.deepcopy(opt)
+    assert other.step == 3 and other._flag_event is None and other._flag_copied is None and opt._flag_copied is not None
+    opt._flag_event = opt._flag_copied
+    with pytest.raises(TypeError):
+        copy.deepcopy(opt)
