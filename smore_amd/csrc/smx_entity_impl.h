@@ -62,6 +62,7 @@ struct EntityArgs : RowSink {
   float* head;    // [tiles, row_len]
   int* fix_list;   // [tiles] numbers of the tiles the fix-up pass has a segment to finish for (appended by the tile pass)
   int* fix_count;  // how many; cleared by the segment pass, which runs first
+  int one_launch;  // short and long segments share a launch: fix_list[t] says whether there is one for tile t, fix_count is not used
   int skip_single;  // segments of one pair were already finished by the query-backward kernel
   // sign codes written by the query-backward kernel, [n_pairs][NIT*64] bytes, or null (CODED kernels)
   const unsigned char* codes;
@@ -88,6 +89,12 @@ struct EntityArgs : RowSink {
   int rows_first;
   int share_rows;  // fix-up kernel: its LDS has room for one more row per wavefront, they share a segment's gradient rows
 };
+
+__device__ __forceinline__ void note_tile(const EntityArgs& A, int lane, int t, bool to_finish) {
+  if (lane != 0) return;
+  if (A.one_launch) A.fix_list[t] = to_finish;
+  else if (to_finish) A.fix_list[atomicAdd(A.fix_count, 1)] = t;
+}
 
 template <int SRC>
 __device__ __forceinline__ float second_coef(float c0, const ScoreParams& p) {
@@ -456,8 +463,7 @@ __device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int sg = A.seg_of_pos[p0];
     const int b0 = A.seg_start[sg], b1 = A.seg_start[sg + 1];
-    if (A.fix_list && lane == 0 && p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid)
-      A.fix_list[atomicAdd(A.fix_count, 1)] = t;
+    note_tile(A, lane, t, p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid);
   }
 
   // most tiles hold short segments only: find that out with one parallel look and leave
@@ -515,8 +521,8 @@ __device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   }
 }
 
-// One launch each, or (one_launch_tiles) one for both, the tiles first.  Nothing is
-// appended to the fix-up's list then (A.fix_list == null): that pass asks every tile itself.
+// One launch each, or (one_launch_tiles) one for both, the tiles first.  Nobody could clear the count of the fix-up's list then: the
+// tile pass leaves a word for every tile instead.
 template <int SRC, int VEC, int NIT, bool REG>
 __global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
@@ -544,19 +550,16 @@ __global__ __launch_bounds__(NW * 64) void entity_fixup_kernel(EntityArgs A) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = A.ncol * VEC;
   const size_t row_len = (size_t)half * MUL;
-  const int n_fix = A.fix_list ? *A.fix_count : (A.n_pairs + A.tile - 1) / A.tile;
-  const int n_valid = A.fix_list ? 0 : *A.n_uniq;
-  if (n_valid < 0) return;  // the plan's build gave up (then no tile is on the list)
+  const int n_fix = A.one_launch ? (A.n_pairs + A.tile - 1) / A.tile : *A.fix_count;
+  if (A.one_launch && *A.n_uniq < 0) return;  // the plan's build gave up (then no tile is on the list, and no word written)
   const bool mixed = SRC != kSrcRows && A.rows_first < A.n_pairs;
   for (int item = blockIdx.x; item < n_fix; item += gridDim.x) {  // uniform over the workgroup
-  const int t = A.fix_list ? A.fix_list[item] : item;
+  const int entry = A.fix_list[item];
+  if (A.one_launch && entry == 0) continue;
+  const int t = A.one_launch ? item : entry;
   const int p0 = t * A.tile;
   const int seg = A.seg_of_pos[p0];
   const int s0 = A.seg_start[seg];
-  if (!A.fix_list) {  // what the tile pass asks before it puts a tile on the list
-    const int end = A.seg_start[seg + 1];
-    if (p0 == 0 || s0 >= p0 || end > min(A.n_pairs, p0 + A.tile) || end - s0 <= A.short_max || seg >= n_valid) continue;
-  }
   const int ts = s0 / A.tile;
   const int n_parts = t - ts + 1;
   const int per_wave = (n_parts + NW - 1) / NW;
@@ -954,8 +957,7 @@ __device__ __forceinline__ void tile_pass_coded(const EntityArgs& A, unsigned ch
   };
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int s = at(sg, 0), s0 = at(b0, 0), s1 = at(b1, 0);
-    if (A.fix_list && lane == 0 && p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid)
-      A.fix_list[atomicAdd(A.fix_count, 1)] = t;
+    note_tile(A, lane, t, p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid);
   }
   bool any_long = false;
 #pragma unroll
@@ -1041,21 +1043,20 @@ __global__ __launch_bounds__(256, 4) void entity_small_coded_kernel(EntityArgs A
 }
 
 // Tiles of a plan up to which short and long segments go through one launch.  That saves a launch of 4 to 5 us, and with skewed
-// ids the two passes share the chip (28 us of 104 at 32,768 box pairs of 400 floats).  But the kernel has the registers
-// of the greater of the two, and the tiles' workgroups, which hardly find a long segment where ids are uniform, stand before the
-// segments': where two or fewer workgroups fit a CU, or fewer than of the segment pass alone, uniform ids lose from some size on.
-// The whole backward, uniform ids, two launches -> one, us:
-//   gradient rows 400 floats, 256 tiles 50 -> 47, 1600 floats 227 -> 248;  L2 200, 256 tiles 43 -> 40, 400 65 -> 63, 800 106 -> 114
-//   box 400, 32 tiles 31 -> 30, 128 61 -> 62, 512 90 -> 94;  from sign codes 200, 32 tiles 21 -> 20, 128 33 -> 36, 400 52 -> 51
-//   rotate 200, 32 tiles 29 -> 28, 256 62 -> 64;  400, 128 tiles 104 -> 102, 512 152 -> 157;  800, 8 tiles 43 -> 50
-template <int SRC, int VEC, int NIT>
-constexpr unsigned one_launch_tiles(bool coded) {
-  if (coded) return VEC == 4 && NIT == 2 ? 512 : 32;
-  if (VEC == 1) return 512;
-  if (SRC == kSrcRows) return NIT <= 4 ? 512 : 0;
-  if (NIT > 2) return 0;
-  if (src_mul(SRC) == 2) return NIT == 1 ? 32 : 128;
-  return SRC == mBox && NIT == 2 ? 64 : 512;
+// ids the two passes share the chip.  But the kernel has the registers of the greater of the two, and the tiles' workgroups, which
+// hardly find a long segment where ids are uniform, come on top of the segments': where fewer workgroups then fit a CU, uniform
+// ids lose a little of what skewed ones gain.  The whole backward, two launches -> one, us, uniform ids of 15 k / Zipf ids:
+//   gradient rows 400, 32 tiles 22 -> 19 / 71 -> 55, 512 tiles 81 -> 77 / 154 -> 102
+//   from sign codes, box 200, 128 tiles 30 -> 32 / 83 -> 66, 512 tiles 42 -> 42 / 121 -> 83;  400, 512 tiles 60 -> 59 / 160 -> 98
+//   L2 200, 32 tiles 20 -> 18 / 77 -> 62, 512 tiles 51 -> 49 / 130 -> 92;  800, 512 tiles 145 -> 154 / 236 -> 169
+//   rotate 200, 32 tiles 28 -> 27 / 79 -> 63, 512 tiles 79 -> 85 / 155 -> 106;  800, 32 tiles 88 -> 95 / 217 -> 167
+//   BetaE 200, 512 tiles 131 -> 138 / 234 -> 172;  600, 512 tiles 541 -> 566 / 761 -> 707
+// Beyond 512 tiles it is less: rotate 400, 1,024 tiles 363 -> 369 (ids of 1 M) / 496 -> 446, BetaE 574 -> 590 / 790 -> 776.  Rows of
+// more than 1,024 floats per half would spill up to 1,767 registers, gradient rows of that length lose up to half with uniform ids
+// (1,600 floats, 8 tiles 12 -> 18).
+template <int NIT>
+constexpr unsigned one_launch_tiles() {
+  return NIT <= 4 ? 512 : 0;
 }
 
 // Workgroups of 256 threads of `kernel` (with that much dynamic LDS) the current device keeps resident; asked
@@ -1083,7 +1084,7 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   // short segments: a fixed grid of wavefronts strides over the segment list (its length lives on the device)
   // (as many workgroups as the chip holds at once: a second wave of workgroups would run half empty)
   const unsigned want_blocks = (unsigned)(((A.n_pairs + A.chunk - 1) / A.chunk + 3) / 4);
-  constexpr unsigned kOneLaunch = one_launch_tiles<SRC, VEC, NIT>(false), kOneLaunchCoded = one_launch_tiles<SRC, VEC, NIT>(true);
+  constexpr unsigned kOneLaunch = one_launch_tiles<NIT>();
   const unsigned tile_blocks = (tiles + 3) / 4;
   EntityArgs F = A;
   bool coded = false;
@@ -1092,8 +1093,8 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   if (coded) {
     if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) {
       const size_t slabs = (size_t)4 * 64 * NIT * 64;  // one code record per lane and wavefront
-      if (tiles <= kOneLaunchCoded) {
-        F.fix_list = nullptr;
+      if (tiles <= kOneLaunch) {
+        F.one_launch = 1;
         const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_coded_kernel<SRC, VEC, NIT>, (int)slabs));
         hipLaunchKernelGGL((entity_small_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks + seg_blocks), dim3(256), slabs, st, F,
                            (int)tile_blocks);
@@ -1106,7 +1107,7 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   }
   if constexpr (kOneLaunch > 0) {
     if (!coded && tiles <= kOneLaunch) {
-      F.fix_list = nullptr;
+      F.one_launch = 1;
       const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_kernel<SRC, VEC, NIT, REG>, 0));
       hipLaunchKernelGGL((entity_small_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks + seg_blocks), dim3(256), 0, st, F,
                          (int)tile_blocks);

@@ -1381,15 +1381,16 @@ def _entity_pass_in_both_forms(n_pairs, dim):
 
 @pytest.mark.parametrize("n_pairs", [1, 255, 257, 131_072, 131_073])
 def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n_pairs):
-    """Up to 512 tiles of 256 pairs short and long segments of short rows go through one launch, and the fix-up finds its
-    tiles by itself: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
+    """Up to 512 tiles of 256 pairs short and long segments of short rows go through one launch, and the tile pass
+    leaves a word per tile for the fix-up: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
     gradient rows and, from sign codes and without, of box pairs, against float64."""
     _entity_pass_in_both_forms(n_pairs, 12)
 
 
 @pytest.mark.parametrize("n_pairs,dim", [(8192, 12), (8193, 12), (16_384, 260), (16_385, 260), (131_072, 50), (131_073, 50),
-                                         (8193, 30), (256, 516), (257, 1100)])
+                                         (8193, 30), (256, 516), (257, 1100), (131_072, 260), (131_073, 260), (131_072, 516),
+                                         (131_073, 516)])
 def test_entity_pass_around_the_sizes_of_other_row_lengths(n_pairs, dim):
-    """Where sign codes (32 tiles), box rows of two column groups (64) and rows of 4-byte columns (512) get launches of their
-    own for short and long segments, and rows so long that they always do."""
+    """The same with rows of two and four column groups, of 4-byte columns, from sign codes, at fewer tiles, and with rows so
+    long that short and long segments always get launches of their own."""
     _entity_pass_in_both_forms(n_pairs, dim)
