@@ -34,22 +34,20 @@ def _counts(n_hard):
     return torch.from_numpy(a.astype(np.int32))
 
 
-def _pinned(count, dtype, dev):
-    """Host memory a copy to the device need not be waited for from (it is given out again once that copy has passed).
-    Under graph capture pageable memory: such a call is refused, a replay would copy whatever then lies there."""
-    return torch.empty(count, dtype=dtype, pin_memory=dev.type == "cuda" and not torch.cuda.is_current_stream_capturing())
-
-
-def _to_device(host, dev):
-    return host.to(dev, non_blocking=dev.type == "cuda" and host.is_pinned())
+def _staging(count, dtype, dev):
+    """Host memory, and whether a copy from it to the device need not be waited for (pinned: it is given out again once that
+    copy has passed).  Under graph capture pageable memory: such a call is refused, a replay would copy whatever then lies
+    there."""
+    pinned = dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+    return torch.empty(count, dtype=dtype, pin_memory=pinned), pinned
 
 
 def _counts_on(counts, dev):
     if counts.device.type != "cpu":
         return counts.to(dev)
-    host = _pinned(counts.numel(), torch.int32, dev)
+    host, pinned = _staging(counts.numel(), torch.int32, dev)
     host.copy_(counts)
-    return _to_device(host, dev)
+    return host.to(dev, non_blocking=pinned)
 
 
 def _one_array(lists):
@@ -75,7 +73,7 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
     sizes = [(len(e), len(h)) for e, h in zip(easy_answers, hard_answers)]
     a = max(1, max(ne + nh for ne, nh in sizes))
     # ids [B, A] and the counts behind them travel to the device as one array, which nothing waits for
-    host = _pinned(b * a + (b + 1) // 2, torch.int64, table.device)
+    host, pinned = _staging(b * a + (b + 1) // 2, torch.int64, table.device)
     packed = host.numpy()
     packed[:] = 0
     ids, counts = packed[: b * a].reshape(b, a), packed[b * a:].view(np.int32)
@@ -97,7 +95,7 @@ def filtered_ranks(model, table, q1, q2, params, easy_answers, hard_answers, bra
     if (ordered[:, 1:] == ordered[:, :-1]).any():
         raise _lib.SmxError("an entity is listed twice among the answers of one query")
     dev = table.device
-    packed = _to_device(host, dev)
+    packed = host.to(dev, non_blocking=pinned)
     ids, counts = packed[: b * a].view(b, a), packed[b * a:]
     q1c = q1.reshape(b * branches, -1).contiguous()
     q2c = None if q2 is None else q2.reshape(b * branches, -1).contiguous()
