@@ -62,7 +62,6 @@ struct EntityArgs : RowSink {
   float* head;    // [tiles, row_len]
   int* fix_list;   // [tiles] numbers of the tiles the fix-up pass has a segment to finish for (appended by the tile pass)
   int* fix_count;  // how many; cleared by the segment pass, which runs first
-  int one_launch;  // short and long segments share a launch: fix_list[t] says whether there is one for tile t, fix_count is not used
   int skip_single;  // segments of one pair were already finished by the query-backward kernel
   // sign codes written by the query-backward kernel, [n_pairs][NIT*64] bytes, or null (CODED kernels)
   const unsigned char* codes;
@@ -89,12 +88,6 @@ struct EntityArgs : RowSink {
   int rows_first;
   int share_rows;  // fix-up kernel: its LDS has room for one more row per wavefront, they share a segment's gradient rows
 };
-
-__device__ __forceinline__ void note_tile(const EntityArgs& A, int lane, int t, bool to_finish) {
-  if (lane != 0) return;
-  if (A.one_launch) A.fix_list[t] = to_finish;
-  else if (to_finish) A.fix_list[atomicAdd(A.fix_count, 1)] = t;
-}
 
 template <int SRC>
 __device__ __forceinline__ float second_coef(float c0, const ScoreParams& p) {
@@ -463,7 +456,8 @@ __device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int sg = A.seg_of_pos[p0];
     const int b0 = A.seg_start[sg], b1 = A.seg_start[sg + 1];
-    note_tile(A, lane, t, p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid);
+    if (A.fix_list && lane == 0 && p0 > 0 && b0 < p0 && b1 <= p1 && b1 - b0 > A.short_max && sg < n_valid)
+      A.fix_list[atomicAdd(A.fix_count, 1)] = t;
   }
 
   // most tiles hold short segments only: find that out with one parallel look and leave
@@ -521,8 +515,9 @@ __device__ __forceinline__ void tile_pass(const EntityArgs& A, int block) {
   }
 }
 
-// One launch each, or (one_launch_tiles) one for both, the tiles first.  Nobody could clear the count of the fix-up's list then: the
-// tile pass leaves a word for every tile instead.
+// One launch each, or (one_launch_tiles) one for both, the tiles first.  Nothing is appended to the fix-up's list then
+// (A.fix_list == null): that pass asks every tile itself.  (A word per tile from the tile pass instead: 0.3 of 76 us with uniform
+// ids, up to 1.2 % slower with skewed ones.)
 template <int SRC, int VEC, int NIT, bool REG>
 __global__ __launch_bounds__(256) void entity_segment_kernel(EntityArgs A) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *A.fix_count = 0;  // the tile pass, launched after this one, appends to the list
@@ -550,16 +545,19 @@ __global__ __launch_bounds__(NW * 64) void entity_fixup_kernel(EntityArgs A) {
   const int wave = uniform(threadIdx.x >> 6);
   const int half = A.ncol * VEC;
   const size_t row_len = (size_t)half * MUL;
-  const int n_fix = A.one_launch ? (A.n_pairs + A.tile - 1) / A.tile : *A.fix_count;
-  if (A.one_launch && *A.n_uniq < 0) return;  // the plan's build gave up (then no tile is on the list, and no word written)
+  const int n_fix = A.fix_list ? *A.fix_count : (A.n_pairs + A.tile - 1) / A.tile;
+  const int n_valid = A.fix_list ? 0 : *A.n_uniq;
+  if (n_valid < 0) return;  // the plan's build gave up (then no tile is on the list)
   const bool mixed = SRC != kSrcRows && A.rows_first < A.n_pairs;
   for (int item = blockIdx.x; item < n_fix; item += gridDim.x) {  // uniform over the workgroup
-  const int entry = A.fix_list[item];
-  if (A.one_launch && entry == 0) continue;
-  const int t = A.one_launch ? item : entry;
+  const int t = A.fix_list ? A.fix_list[item] : item;
   const int p0 = t * A.tile;
   const int seg = A.seg_of_pos[p0];
   const int s0 = A.seg_start[seg];
+  if (!A.fix_list) {  // what the tile pass asks before it puts a tile on the list
+    const int end = A.seg_start[seg + 1];
+    if (p0 == 0 || s0 >= p0 || end > min(A.n_pairs, p0 + A.tile) || end - s0 <= A.short_max || seg >= n_valid) continue;
+  }
   const int ts = s0 / A.tile;
   const int n_parts = t - ts + 1;
   const int per_wave = (n_parts + NW - 1) / NW;
@@ -957,7 +955,8 @@ __device__ __forceinline__ void tile_pass_coded(const EntityArgs& A, unsigned ch
   };
   {  // does a long segment that came in from the left end inside this tile?  The fix-up pass finishes it.
     const int s = at(sg, 0), s0 = at(b0, 0), s1 = at(b1, 0);
-    note_tile(A, lane, t, p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid);
+    if (A.fix_list && lane == 0 && p0 > 0 && s0 < p0 && s1 <= p1 && s1 - s0 > A.short_max && s < n_valid)
+      A.fix_list[atomicAdd(A.fix_count, 1)] = t;
   }
   bool any_long = false;
 #pragma unroll
@@ -1094,7 +1093,7 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
     if constexpr (SRC != kSrcRows && model_coded(SRC) && !REG && NIT <= 2) {
       const size_t slabs = (size_t)4 * 64 * NIT * 64;  // one code record per lane and wavefront
       if (tiles <= kOneLaunch) {
-        F.one_launch = 1;
+        F.fix_list = nullptr;
         const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_coded_kernel<SRC, VEC, NIT>, (int)slabs));
         hipLaunchKernelGGL((entity_small_coded_kernel<SRC, VEC, NIT>), dim3(tile_blocks + seg_blocks), dim3(256), slabs, st, F,
                            (int)tile_blocks);
@@ -1107,7 +1106,7 @@ int launch_entity_reg(hipStream_t st, const EntityArgs& A) {
   }
   if constexpr (kOneLaunch > 0) {
     if (!coded && tiles <= kOneLaunch) {
-      F.one_launch = 1;
+      F.fix_list = nullptr;
       const unsigned seg_blocks = min(want_blocks, resident_blocks(entity_small_kernel<SRC, VEC, NIT, REG>, 0));
       hipLaunchKernelGGL((entity_small_kernel<SRC, VEC, NIT, REG>), dim3(tile_blocks + seg_blocks), dim3(256), 0, st, F,
                          (int)tile_blocks);

@@ -1381,8 +1381,8 @@ def _entity_pass_in_both_forms(n_pairs, dim):
 
 @pytest.mark.parametrize("n_pairs", [1, 255, 257, 131_072, 131_073])
 def test_entity_pass_around_the_size_from_which_its_tiles_get_their_own_launch(n_pairs):
-    """Up to 512 tiles of 256 pairs short and long segments of short rows go through one launch, and the tile pass
-    leaves a word per tile for the fix-up: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
+    """Up to 512 tiles of 256 pairs short and long segments of short rows go through one launch, and the fix-up finds its
+    tiles by itself: segments that span many tiles, end on a tile's last pair, begin on its first, lie inside one; sums of
     gradient rows and, from sign codes and without, of box pairs, against float64."""
     _entity_pass_in_both_forms(n_pairs, 12)
 
