@@ -166,6 +166,10 @@ __device__ __forceinline__ float stirling_of(const Shifted& s) {
 
 __device__ __forceinline__ bool fast_ok(float lo, float hi) { return lo >= kFastLo && hi <= kFastHi; }
 
+// (The general routines hand their results back in registers.  By reference they come back through scratch memory, and the
+// wait for those loads, where the branches meet, is one for every load in flight.)
+typedef float SlowTerms __attribute__((ext_vector_type(4)));
+
 // Entity-side quantities of KL(Beta(a,b) || .): lb = lgamma(a+b) - lgamma(a) - lgamma(b) and the
 // three digammas.  One call shares the shifted arguments, logarithms and reciprocals.
 static __device__ __noinline__ void beta_terms_slow(float a, float b, float& lb, float& pa, float& pb, float& ps) {
@@ -188,6 +192,94 @@ __device__ __forceinline__ void beta_terms(float a, float b, float& lb, float& p
   }
 }
 
+// ---- the same with the logarithms' sum taken apart -------------------------------------------------
+// With w = (x + 3) / 3, y = x + 3 and Stirling's series written out, everything of KL(Beta(a,b) || Beta(qa,qb)) that grows
+// with a logarithm has a coefficient of the query alone, because (y - 1/2) ln y of lgamma meets (x - q) ln y of (x - q) psi(x)
+// and y - x is 3:
+//   KL = k_q + (qs+2.5) ln ws - (qa+2.5) ln wa - (qb+2.5) ln wb + ln(C D(a) D(b) / D(s)) + S(s) - S(a) - S(b)
+//        - (a-qa) R(a) - (b-qb) R(b) + (s-qs) R(s)
+//   R(x) = ln y - psi(x) = 1/(2y) + V(y) + D'(x)/D(x),  D(x) = x (x + 1) (x + 2),  S, V: what Stirling's series of lgamma and
+//   psi leave after the terms written here,  C = e^3 / (3^2.5 sqrt(2 pi)): the constants that are left over,
+// and the logarithms are of numbers around 1.  V and S are polynomials of two steps in 1/y^2 fitted for y >= 3 (largest
+// error 3.9e-9 and 3.2e-9; the first terms left out of the series at y = x + 6: 2.5e-9 and 2.1e-9), so three steps of
+// recurrence do where six are taken above.  BetaE's kernels are bound by the number of their instructions (four cycles each:
+// a wavefront that has issued a transcendental one no longer shares its cycles with another), and this is 69 a feature
+// instead of 105 in the forward.  One feature's divergence has less than half the error (normal rows around 1: 0.66e-6 instead
+// of 1.7e-6).  512 x 512 pairs of 2 x 400 floats: forward 405 -> 358 us, query gradient 330 -> 299 (437 and 384 with a branch
+// per feature and the query's values in registers).  Good in the interval of fast_ok.
+constexpr float kLn2 = 0.693147180559945f;
+constexpr float kBetaConst = 5.14032259e-1f;   // C
+// A constant in a VGPR: an instruction takes one literal, and a scalar register halves the rate of those that have the full one.
+__device__ __forceinline__ float vector_const(float c) {
+  float v;
+  asm("v_mov_b32 %0, %1" : "=v"(v) : "i"(__builtin_bit_cast(int, c)));
+  return v;
+}
+struct BetaArg {
+  float w, r;      // (x + 3) / 3 and its reciprocal
+  float z;         // r^2
+  float d, rd;     // D(x) and its reciprocal; with POLE: (x + 1) (x + 2) and its reciprocal
+  float rx;        // POLE: 1/x
+  float rest;      // R(x)
+};
+// POLE: 1/x on its own, D'/D = 1/x + (2x + 3) / ((x + 1) (x + 2)); one special function more, and half the error of psi
+// below 5, where the pole is most of it.
+template <bool POLE>
+__device__ __forceinline__ BetaArg beta_arg(float x) {
+#pragma clang fp contract(off)
+  BetaArg s;
+  s.w = __builtin_fmaf(x, vector_const(3.33333343e-1f), 1.f);
+  s.r = f_rcp(s.w);
+  s.z = s.r * s.r;
+  const float tail = __builtin_fmaf(s.z, __builtin_fmaf(s.z, 4.478603748e-6f, vector_const(-1.023662279e-4f)), 9.259178391e-3f);
+  const float u = s.r * __builtin_fmaf(s.r, tail, 1.66666667e-1f);
+  if constexpr (POLE) {
+    s.d = __builtin_fmaf(x, x + 3.f, 2.f);
+    s.rd = f_rcp(s.d);
+    s.rx = f_rcp(x);
+    s.rest = __builtin_fmaf(__builtin_fmaf(x, 2.f, vector_const(3.f)), s.rd, u) + s.rx;
+  } else {
+    const float t = __builtin_fmaf(x, x, x + x);
+    s.d = t * (x + 1.f);
+    s.rd = f_rcp(s.d);
+    s.rx = 0.f;
+    s.rest = __builtin_fmaf(__builtin_fmaf(t, vector_const(3.f), 2.f), s.rd, u);
+  }
+  return s;
+}
+__device__ __forceinline__ float beta_stirling(const BetaArg& s) {   // S(x) / r
+#pragma clang fp contract(off)
+  return __builtin_fmaf(s.z, __builtin_fmaf(s.z, 2.867135899e-6f, vector_const(-1.026935902e-4f)), 2.777775529e-2f);
+}
+// lgamma(a+b) - lgamma(a) - lgamma(b) with ka = (qa+2.5) ln 2, kb likewise, ks = (qa+qb+2.5) ln 2 in the place of the row's own,
+// added to `from`
+__device__ __forceinline__ float beta_logs(float from, const BetaArg& a, const BetaArg& b, const BetaArg& s, float ka, float kb,
+                                           float ks) {
+#pragma clang fp contract(off)
+  float v = __builtin_fmaf(__builtin_amdgcn_logf((a.d * kBetaConst) * s.rd * b.d), kLn2, from);
+  v = __builtin_fmaf(ks, __builtin_amdgcn_logf(s.w), v);
+  v = __builtin_fmaf(-ka, __builtin_amdgcn_logf(a.w), v);
+  v = __builtin_fmaf(-kb, __builtin_amdgcn_logf(b.w), v);
+  v = __builtin_fmaf(s.r, beta_stirling(s), v);
+  v = __builtin_fmaf(-a.r, beta_stirling(a), v);
+  return __builtin_fmaf(-b.r, beta_stirling(b), v);
+}
+constexpr float kBetaShift = 2.5f * kLn2;
+__device__ __forceinline__ float beta_k(float q) { return __builtin_fmaf(q, kLn2, kBetaShift); }
+// psi'(x) out of the same parts (POLE): 1/x^2 + (2d + 1)/d^2 with d = (x + 1) (x + 2), and psi'(y) = 1/y + 1/(2y^2) plus a
+// polynomial fitted as V is (largest error 5.8e-9).  No special function more.
+__device__ __forceinline__ float beta_trigamma(const BetaArg& s) {
+#pragma clang fp contract(off)
+  const float tail = __builtin_fmaf(s.z, __builtin_fmaf(s.z, 8.307060779e-6f, vector_const(-1.356947031e-4f)), 6.172571429e-3f);
+  const float asym = __builtin_fmaf(s.r * s.z, tail, __builtin_fmaf(s.z, 5.55555556e-2f, s.r * 3.33333343e-1f));
+  return __builtin_fmaf(s.rx, s.rx, __builtin_fmaf(__builtin_fmaf(s.d, 2.f, 1.f), s.rd * s.rd, asym));
+}
+// psi(s) - psi(x)
+__device__ __forceinline__ float beta_psi_diff(const BetaArg& x, const BetaArg& s) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(__builtin_amdgcn_logf(s.w * x.r), kLn2, x.rest - s.rest);
+}
+
 static __device__ __noinline__ void digamma3_slow(float a, float b, float& pa, float& pb, float& ps) {
   pa = digamma(a);
   pb = digamma(b);
@@ -204,6 +296,12 @@ __device__ __forceinline__ void digamma3(float a, float b, float& pa, float& pb,
   }
 }
 
+static __device__ __noinline__ SlowTerms digamma3_any(float a, float b) {
+  float pa, pb, ps;
+  digamma3(a, b, pa, pb, ps);
+  return SlowTerms{pa, pb, ps, 0.f};
+}
+
 static __device__ __noinline__ void trigamma3_slow(float a, float b, float& ta, float& tb, float& ts) {
   ta = trigamma(a);
   tb = trigamma(b);
@@ -218,6 +316,12 @@ __device__ __forceinline__ void trigamma3(float a, float b, float& ta, float& tb
   } else {
     trigamma3_slow(a, b, ta, tb, ts);
   }
+}
+
+static __device__ __noinline__ SlowTerms trigamma3_any(float a, float b) {
+  float ta, tb, ts;
+  trigamma3(a, b, ta, tb, ts);
+  return SlowTerms{ta, tb, ts, 0.f};
 }
 
 }  // namespace smx

@@ -327,26 +327,51 @@ template <> struct ModelOps<mRotate> {
 struct QBeta {
   float a, b;  // alpha, beta of the query
   float k;     // forward: lgG(qa)+lgG(qb)-lgG(sq); query backward: psi(qa)-psi(sq)
-  float l;     // query backward: psi(qb)-psi(sq)
+  float l;     // forward: (qa + 2.5) ln 2, see beta_arg; query backward: psi(qb)-psi(sq)
+  float m;     // forward: (qb + 2.5) ln 2
 };
+
+// One pair's terms by the routines that take any argument; not inlined: rows that need it are rare.
+static __device__ __noinline__ float beta_pair_any(float ea, float eb, float qa, float qb, float k) {
+  float lb, pa, pb, ps;
+  beta_terms(ea, eb, lb, pa, pb, ps);
+  return (k + lb) + (ea - qa) * pa + (eb - qb) * pb + ((qa + qb) - (ea + eb)) * ps;
+}
 
 template <> struct ModelOps<mBetaKL> {
   using Q = QBeta;
-  static __device__ __forceinline__ Q prep(float q1, float q2) { return {q1, q2, 0.f, 0.f}; }
+  static __device__ __forceinline__ Q prep(float q1, float q2) { return {q1, q2, 0.f, 0.f, 0.f}; }
   static __device__ __forceinline__ Q prep_fwd(float q1, float q2) {
+    const float ka = beta_k(q1), kb = beta_k(q2), sum = q1 + q2;
     float lb, pa, pb, ps;
-    beta_terms(q1, q2, lb, pa, pb, ps);
-    return {q1, q2, -lb, 0.f};
+    if (fast_ok(fminf(q1, q2), sum)) lb = beta_logs(0.f, beta_arg<false>(q1), beta_arg<false>(q2), beta_arg<false>(sum), ka, kb, beta_k(sum));
+    else beta_terms(q1, q2, lb, pa, pb, ps);
+    return {q1, q2, -lb, ka, kb};
   }
   static __device__ __forceinline__ Q prep_bwd_q(float q1, float q2) {
     float pa, pb, ps;
     digamma3(q1, q2, pa, pb, ps);
-    return {q1, q2, pa - ps, pb - ps};
+    return {q1, q2, pa - ps, pb - ps, 0.f};
   }
   static __device__ __forceinline__ void fwd(float ea, float eb, const Q& q, float& a0, float&) {
-    float lb, pa, pb, ps;
-    beta_terms(ea, eb, lb, pa, pb, ps);
-    a0 += (q.k + lb) + (ea - q.a) * pa + (eb - q.b) * pb + ((q.a + q.b) - (ea + eb)) * ps;
+    a0 += beta_pair_any(ea, eb, q.a, q.b, q.k);
+  }
+  // The same for a row of which every feature lies in the interval of fast_ok.
+  static __device__ __forceinline__ void fwd_fast(float ea, float eb, const Q& q, float& a0) {
+#pragma clang fp contract(off)
+    const float sum = ea + eb;
+    const BetaArg a = beta_arg<false>(ea), b = beta_arg<false>(eb), s = beta_arg<false>(sum);
+    float v = beta_logs(q.k, a, b, s, q.l, q.m, (q.l + q.m) - kBetaShift);
+    const float da = ea - q.a, db = eb - q.b;
+    v = __builtin_fmaf(-da, a.rest, v);
+    v = __builtin_fmaf(-db, b.rest, v);
+    a0 += __builtin_fmaf(da + db, s.rest, v);
+  }
+  static __device__ __forceinline__ void bwd_q_fast(float c0, float e1, float e2, const Q& q, float& g1, float& g2) {
+#pragma clang fp contract(off)
+    const BetaArg a = beta_arg<true>(e1), b = beta_arg<true>(e2), s = beta_arg<true>(e1 + e2);
+    g1 = __builtin_fmaf(c0, q.k + beta_psi_diff(a, s), g1);
+    g2 = __builtin_fmaf(c0, q.l + beta_psi_diff(b, s), g2);
   }
   static __device__ __forceinline__ float fold(float a0, float, const ScoreParams&) { return a0; }
   static __device__ __forceinline__ float score(float folded, const ScoreParams& p) { return p.gamma - folded; }
@@ -360,19 +385,156 @@ template <> struct ModelOps<mBetaKL> {
     s2 += c0 * (e2 - q.b);
   }
   static __device__ __forceinline__ void finish_e(float e1, float e2, float& g1, float& g2) {
+#pragma clang fp contract(off)
+    const float sum = e1 + e2;
     float ta, tb, ts;
-    trigamma3(e1, e2, ta, tb, ts);
+    if (fast_ok(fminf(e1, e2), sum)) {
+      ta = beta_trigamma(beta_arg<true>(e1));
+      tb = beta_trigamma(beta_arg<true>(e2));
+      ts = beta_trigamma(beta_arg<true>(sum));
+    } else {
+      const SlowTerms t = trigamma3_any(e1, e2);
+      ta = t.x;
+      tb = t.y;
+      ts = t.z;
+    }
     const float common = ts * (g1 + g2);
-    g1 = ta * g1 - common;
-    g2 = tb * g2 - common;
+    g1 = __builtin_fmaf(ta, g1, -common);
+    g2 = __builtin_fmaf(tb, g2, -common);
   }
   static __device__ __forceinline__ void bwd_q(float c0, float, float e1, float e2, const Q& q, float& g1, float& g2) {
-    float pa, pb, ps;
-    digamma3(e1, e2, pa, pb, ps);
-    g1 += c0 * (q.k - pa + ps);
-    g2 += c0 * (q.l - pb + ps);
+    const SlowTerms t = digamma3_any(e1, e2);
+    g1 += c0 * (q.k - t.x + t.z);
+    g2 += c0 * (q.l - t.y + t.z);
   }
 };
+
+// BetaE's entity prologue in the kernels built for it: one v_med3 (a NaN gives the lower bound, as fminf(fmaxf()) does).
+struct BetaClamp {
+  float add, lo, hi;
+  bool low_ok;   // the lower bound already is in the interval of fast_ok
+  __device__ __forceinline__ BetaClamp(const ScoreParams& p) : add(p.reg_add), lo(fminf(p.reg_lo, p.reg_hi)), hi(p.reg_hi) {
+    low_ok = lo >= kFastLo;
+  }
+  __device__ __forceinline__ float operator()(float e) const { return __builtin_amdgcn_fmed3f(e + add, lo, hi); }
+};
+
+// The features of one row, clamped, and whether all of them, in all lanes, lie in the interval of fast_ok: one decision per
+// row instead of two compares, an exec mask and a branch per feature.  Their sum bounds each, as none is negative.
+template <int VEC, int NIT> struct BetaRow {
+  float a[NIT][VEC], b[NIT][VEC];
+  template <bool REG, class GetA, class GetB>
+  __device__ __forceinline__ bool load(const BetaClamp& clamp, GetA&& ga, GetB&& gb) {
+    float sum = 0.f;
+#pragma unroll
+    for (int it = 0; it < NIT; ++it)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        a[it][v] = REG ? clamp(ga(it, v)) : ga(it, v);
+        b[it][v] = REG ? clamp(gb(it, v)) : gb(it, v);
+        sum += a[it][v] + b[it][v];
+      }
+    bool ok = sum <= kFastHi;   // (not a NaN)
+    if (!(REG && clamp.low_ok)) {
+      float low = __builtin_inff();
+#pragma unroll
+      for (int it = 0; it < NIT; ++it)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) low = fminf(low, fminf(a[it][v], b[it][v]));
+      ok = ok && low >= kFastLo;
+    }
+    return __ballot(!ok) == 0ull;
+  }
+};
+
+// A lane's part of a row's divergence, and the row's part of the query gradient, from the row's values as they are stored.
+// get_q(it, q) fetches the query's values of a column group: the kernels that stream rows keep them in LDS, evaluated once per
+// workgroup, which leaves their registers to four wavefronts a SIMD (measured below with beta_arg).
+template <int VEC, int NIT, bool REG, class GetA, class GetB, class GetQ>
+__device__ __forceinline__ float beta_row_sum(const BetaClamp& clamp, GetA&& ga, GetB&& gb, GetQ&& get_q, int ncol, int lane) {
+  BetaRow<VEC, NIT> row;
+  const bool fast = row.template load<REG>(clamp, ga, gb);
+  float mine = 0.f;
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    QBeta q[VEC];
+    get_q(it, q);
+    float a0 = 0.f, a1 = 0.f;
+    if (fast) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::fwd_fast(row.a[it][v], row.b[it][v], q[v], a0);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::fwd(row.a[it][v], row.b[it][v], q[v], a0, a1);
+    }
+    mine += lane + 64 * it < ncol ? a0 : 0.f;
+  }
+  return mine;
+}
+template <int VEC, int NIT, bool REG, class GetA, class GetB, class GetQ>
+__device__ __forceinline__ void beta_row_query_grad(const BetaClamp& clamp, GetA&& ga, GetB&& gb, float c0, GetQ&& get_q,
+                                                    float (&g1)[NIT][VEC], float (&g2)[NIT][VEC]) {
+  BetaRow<VEC, NIT> row;
+  const bool fast = row.template load<REG>(clamp, ga, gb);
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    QBeta q[VEC];
+    get_q(it, q);
+    if (fast) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::bwd_q_fast(c0, row.a[it][v], row.b[it][v], q[v], g1[it][v], g2[it][v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::bwd_q(c0, 0.f, row.a[it][v], row.b[it][v], q[v], g1[it][v], g2[it][v]);
+    }
+  }
+}
+
+// ... and, for the row of a one-pair segment, its gradient with respect to the stored values as well (g = c0 (e - q) through
+// the trigammas and the clamp's mask): psi and psi' share every special function.
+template <int VEC, int NIT, bool REG, class GetA, class GetB, class GetQ>
+__device__ __forceinline__ void beta_row_both_grads(const BetaClamp& clamp, const ScoreParams& p, GetA&& ga, GetB&& gb, float c0,
+                                                    GetQ&& get_q, float (&g1)[NIT][VEC], float (&g2)[NIT][VEC],
+                                                    float (&ge1)[NIT][VEC], float (&ge2)[NIT][VEC]) {
+#pragma clang fp contract(off)
+  using O = ModelOps<mBetaKL>;
+  BetaRow<VEC, NIT> row;
+  const bool fast = row.template load<REG>(clamp, ga, gb);
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    QBeta q[VEC];
+    get_q(it, q);
+    if (fast) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const float ea = row.a[it][v], eb = row.b[it][v];
+        const BetaArg a = beta_arg<true>(ea), b = beta_arg<true>(eb), s = beta_arg<true>(ea + eb);
+        g1[it][v] = __builtin_fmaf(c0, q[v].k + beta_psi_diff(a, s), g1[it][v]);
+        g2[it][v] = __builtin_fmaf(c0, q[v].l + beta_psi_diff(b, s), g2[it][v]);
+        const float s1 = c0 * (ea - q[v].a), s2 = c0 * (eb - q[v].b), common = beta_trigamma(s) * (s1 + s2);
+        ge1[it][v] = __builtin_fmaf(beta_trigamma(a), s1, -common);
+        ge2[it][v] = __builtin_fmaf(beta_trigamma(b), s2, -common);
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const float ea = row.a[it][v], eb = row.b[it][v];
+        O::bwd_q(c0, 0.f, ea, eb, q[v], g1[it][v], g2[it][v]);
+        const SlowTerms t = trigamma3_any(ea, eb);
+        const float s1 = c0 * (ea - q[v].a), s2 = c0 * (eb - q[v].b), common = t.z * (s1 + s2);
+        ge1[it][v] = __builtin_fmaf(t.x, s1, -common);
+        ge2[it][v] = __builtin_fmaf(t.y, s2, -common);
+      }
+    }
+    if (REG) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        ge1[it][v] = reg_mask(ga(it, v), ge1[it][v], p);
+        ge2[it][v] = reg_mask(gb(it, v), ge2[it][v], p);
+      }
+    }
+  }
+}
 
 // ComplEx and DistMult score by similarity, not distance (dist_kernel.h:187-204, 324-349): the logit grows
 // with the inner product, so the upstream coefficient keeps its sign.

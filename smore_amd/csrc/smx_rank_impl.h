@@ -76,6 +76,14 @@ __device__ __forceinline__ float row_score(const float (&e1)[NIT][VEC], const fl
                                            const ScoreParams& p) {
   constexpr int MUL = model_mul(M);
   float mine = 0.f;
+  if constexpr (M == mBetaKL) {
+    mine = beta_row_sum<VEC, NIT, REG>(BetaClamp(p), [&](int it, int v) { return e1[it][v]; },
+                                       [&](int it, int v) { return e2[it][v]; },
+                                       [&](int it, QBeta (&to)[VEC]) {
+#pragma unroll
+                                         for (int v = 0; v < VEC; ++v) to[v] = q[it][v];
+                                       }, ncol, lane);
+  } else
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     float a0 = 0.f, a1 = 0.f;
@@ -196,12 +204,26 @@ __device__ __forceinline__ ScalarRow scalar_row(const float* p) {
 // psi cancel, digits that its fp32 sums would round away.  They are summed, and the three parts added, in 64 bits: once
 // per row, once per query, three additions per pair.  log_beta: with what the rounding of ea + eb changes in lgamma(ea + eb)
 // (the pair's sum is over ea and eb themselves, not over that rounded value).
-__device__ __forceinline__ double log_beta(float a, float b, float& pa, float& pb, float& ps) {
+// da, db: psi(a) - psi(a + b), psi(b) - psi(a + b).  The forms are those of the scoring kernels (beta_arg); the logarithms of
+// ratios, which are psi's as well, meet the row's own a + 2.5 and b + 2.5 in 64 bits.
+__device__ __forceinline__ double log_beta(float a, float b, float& da, float& db) {
 #pragma clang fp contract(off)
-  float lb;
-  beta_terms(a, b, lb, pa, pb, ps);
   const float sum = a + b, from_b = sum - a;
   const float rest = (a - (sum - from_b)) + (b - from_b);   // a + b = sum + rest
+  if (fast_ok(fminf(a, b), sum)) {
+    const BetaArg xa = beta_arg<false>(a), xb = beta_arg<false>(b), xs = beta_arg<false>(sum);
+    const float ga = __builtin_amdgcn_logf(xs.w * xa.r), gb = __builtin_amdgcn_logf(xs.w * xb.r);
+    const float gs = __builtin_amdgcn_logf(xs.w), gd = __builtin_amdgcn_logf((xa.d * kBetaConst) * xs.rd * xb.d);
+    da = -__builtin_fmaf(ga, kLn2, xa.rest - xs.rest);
+    db = -__builtin_fmaf(gb, kLn2, xb.rest - xs.rest);
+    const float tail = __builtin_fmaf(-xb.r, beta_stirling(xb), __builtin_fmaf(-xa.r, beta_stirling(xa), xs.r * beta_stirling(xs)));
+    const double logs = ((double)a + 2.5) * (double)ga + ((double)b + 2.5) * (double)gb + ((double)gd - 2.5 * (double)gs);
+    return __builtin_fma(logs, 0.69314718055994531, (double)(tail + rest * (1.f - xs.rest)));
+  }
+  float lb, pa, pb, ps;
+  beta_terms(a, b, lb, pa, pb, ps);
+  da = pa - ps;
+  db = pb - ps;
   return (double)lb + (double)(rest * ps);
 }
 // The sum with its error.  Past fp32 the error is a difference of infinities: the total alone then is what a plain sum
@@ -304,13 +326,9 @@ template <int M, bool NORM> struct ScanOps {
   static __device__ __forceinline__ double expand(float x1, float x2, const ScoreParams& p, float (&e)[kGroup]) {
 #pragma clang fp contract(off)
     if constexpr (M == mBetaKL) {
-      float pa, pb, ps;
       e[0] = reg_apply(x1, p);
       e[1] = reg_apply(x2, p);
-      const double lb = log_beta(e[0], e[1], pa, pb, ps);
-      e[2] = pa - ps;
-      e[3] = pb - ps;
-      return lb;
+      return log_beta(e[0], e[1], e[2], e[3]);
     } else {
       e[0] = x1;
       if constexpr (kGroup == 2) e[1] = x2;
@@ -335,8 +353,8 @@ __device__ __forceinline__ double query_const(const RankArgs& A, int bq, int dim
   if constexpr (M != mBetaKL) return 0.0;
   double mine = 0.0;
   for (int d = lane; d < dim; d += 64) {
-    float pa, pb, ps;
-    mine -= log_beta(A.q1[(size_t)bq * dim + d], A.q2[(size_t)bq * dim + d], pa, pb, ps);
+    float da, db;
+    mine -= log_beta(A.q1[(size_t)bq * dim + d], A.q2[(size_t)bq * dim + d], da, db);
   }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) mine += __shfl_xor(mine, d);   // (either order of a pair: the same sum in every lane)

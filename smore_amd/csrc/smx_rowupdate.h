@@ -219,7 +219,8 @@ struct NoExtraRows {
 // ADAM_STATIC: the caller knows at compile time that Adam is on (its m0 / v0 are loaded); otherwise the
 // run-time flag A.adam_on decides.  extra(g1, g2): adds what reaches the row from outside the score model
 // (gradient rows of the step's plain lookups) once the model's own gradient is complete, clamp mask included.
-template <int SRC, int VEC, int NIT, bool REG, bool ADAM_STATIC = false, class Extra = NoExtraRows>
+// DONE: g1 / g2 already are the row's gradient.
+template <int SRC, int VEC, int NIT, bool REG, bool ADAM_STATIC = false, bool DONE = false, class Extra = NoExtraRows>
 __device__ __forceinline__ void finish_row(const RowSink& A, int lane, unsigned row_id, int seg,
                                            float (&g1)[NIT][VEC], float (&g2)[NIT][VEC],
                                            const RowRegs<src_mul(SRC), VEC, NIT>& w,
@@ -228,7 +229,7 @@ __device__ __forceinline__ void finish_row(const RowSink& A, int lane, unsigned 
   constexpr int MUL = src_mul(SRC);
   const int half = A.ncol * VEC;
   const size_t row_len = (size_t)half * MUL;
-  if constexpr (SRC != kSrcRows) {
+  if constexpr (SRC != kSrcRows && !DONE) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it)
 #pragma unroll
@@ -242,7 +243,7 @@ __device__ __forceinline__ void finish_row(const RowSink& A, int lane, unsigned 
       if constexpr (MUL == 2) norm_project<VEC, NIT>(g2, A.ncol, lane, [&](int it, int x) { return w.h[MUL - 1][it].v[x]; });
     }
   }
-  if (REG) {
+  if (REG && !DONE) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it)
 #pragma unroll

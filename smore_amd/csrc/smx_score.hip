@@ -623,9 +623,10 @@ static int backward_fused(int parts, int model, void* stream, const smx_plan_vie
   // Without an optimizer the one-pair rows cost the query-gradient kernel one store each (nothing to
   // fetch), so they are always finished there.
   const bool q_beyond_l2 = queries_beyond_l2(model, B, dim);
-  const bool singles_here = !adam || q_beyond_l2;
-  A.pair_seg = singles_here ? plan->pair_seg : nullptr;
   fill_sink(&A, table, m, v, merged, adam);
+  A.stream_rows = beta_rows_in_stream(model, A.sink, vec, nit);
+  const bool singles_here = !adam || q_beyond_l2 || A.stream_rows;
+  A.pair_seg = singles_here ? plan->pair_seg : nullptr;
   // Sign codes (models that have them): when the entity pass would fetch query rows from beyond the L2,
   // the query-gradient kernel leaves each pair's derivative decisions in the workspace behind the
   // entity pass's own scratch, and the entity pass reads those instead of the query rows.  Used when

@@ -48,7 +48,18 @@ struct ScoreArgs {
   unsigned char* codes;  // [B*K][NIT*64] sign codes written by this kernel (forward or query backward), or null
   const unsigned char* codes_in;  // query backward: codes the forward left; the entity rows are then not read
   RowSink sink;
+  int stream_rows;       // one-pair segments are finished in the stream of the rows (beta_rows_in_stream)
 };
+
+// BetaE with Adam in place: the query-gradient kernel finishes the rows that occur once.  It is bound by the special functions
+// (VALU 95 % busy, the rows at 2.8 TB/s) and the entity pass by the rows' w, m and v, one after the other; here the first hides
+// behind the second, a row is read once for both, and psi' costs no special function beyond those of psi.  512 x 512 pairs,
+// 2 x 400 floats, 1 M entities, 201 k of 230 k rows occur once: query gradient 299 + entity pass 1001 us -> 849 + 186; 300 x 512
+// 1.04 ms a step against 1.31 before (its 300 workgroups take two turns of the 256 CUs), 128 x 1024 0.98 / 1.14, D = 200
+// 0.73 / 0.98.  Merged rows, v per row and other optimizers take the entity pass as before.
+inline bool beta_rows_in_stream(int model, const RowSink& sink, int vec, int nit) {
+  return model == mBetaKL && vec == 4 && nit <= 2 && sink.adam_on == kOptAdam && !sink.squeeze && !sink.merged;
+}
 
 template <int VEC> struct Pack {
   float v[VEC];
@@ -94,6 +105,58 @@ __device__ __forceinline__ void stage_query(float* lds, const float* __restrict_
     if (model_nq(M) == 2) lds[dim + d] = q2[b * dim + d];
   }
   __syncthreads();
+}
+
+// BetaE's per-query values in LDS, one stretch of dim floats per field, evaluated once per workgroup.  FWD: a, b, k, l, m of
+// QBeta; query backward: k, l and, where rows are finished in the stream (ROWS), a, b.
+__host__ __device__ constexpr int query_fields(int model, bool fwd, bool rows = false) {
+  return model != mBetaKL ? model_nq(model) : (fwd ? 5 : (rows ? 4 : 2));
+}
+template <bool FWD, bool ROWS = false>
+__device__ __forceinline__ void stage_beta_query(float* lds, const float* __restrict__ q1, const float* __restrict__ q2,
+                                                 size_t b, int dim) {
+  for (int d = threadIdx.x; d < dim; d += blockDim.x) {
+    const float x = q1[b * dim + d], y = q2[b * dim + d];
+    const QBeta q = FWD ? prep_forward<mBetaKL>(x, y) : prep_backward_query<mBetaKL>(x, y);
+    if constexpr (FWD) {
+      lds[d] = q.a;
+      lds[dim + d] = q.b;
+      lds[2 * dim + d] = q.k;
+      lds[3 * dim + d] = q.l;
+      lds[4 * dim + d] = q.m;
+    } else {
+      lds[d] = q.k;
+      lds[dim + d] = q.l;
+      if constexpr (ROWS) {
+        lds[2 * dim + d] = q.a;
+        lds[3 * dim + d] = q.b;
+      }
+    }
+  }
+  __syncthreads();
+}
+template <int VEC>
+__device__ __forceinline__ void lds_pack(const float* lds, int col, float (&x)[VEC]) {
+  if constexpr (VEC == 4) {
+    typedef float vec4 __attribute__((ext_vector_type(4)));
+    const vec4 t = reinterpret_cast<const vec4*>(lds)[col];
+    x[0] = t.x;
+    x[1] = t.y;
+    x[2] = t.z;
+    x[3] = t.w;
+  } else {
+    x[0] = lds[col];
+  }
+}
+template <int VEC, bool FWD, bool ROWS = false>
+__device__ __forceinline__ void beta_query(const float* lds, int dim, int col, QBeta (&q)[VEC]) {
+  float f[5][VEC];
+#pragma unroll
+  for (int i = 0; i < query_fields(mBetaKL, FWD, ROWS); ++i) lds_pack<VEC>(lds + i * dim, col, f[i]);
+#pragma unroll
+  for (int v = 0; v < VEC; ++v)
+    q[v] = FWD ? QBeta{f[0][v], f[1][v], f[2][v], f[3][v], f[4][v]}
+               : QBeta{ROWS ? f[2][v] : 0.f, ROWS ? f[3][v] : 0.f, f[0][v], f[1][v], 0.f};
 }
 
 // ---- streaming the rows of up to 64 pairs through a wavefront -----------------------------------
@@ -245,6 +308,13 @@ __device__ __forceinline__ void flush_codes(const unsigned char* stage, unsigned
   }
 }
 
+// Wavefronts per SIMD the compiler has to leave registers for: four where BetaE is bound by its arithmetic (with three, 2 x 400
+// floats: forward 415 instead of 405 us, query gradient 354 instead of 330; seven floats a lane do not fit the query gradient's
+// 128 registers: spills, 381 us instead of 299).
+constexpr int arithmetic_waves(int model, int floats_per_lane, bool fwd) {
+  return model == mBetaKL && floats_per_lane <= 8 && (fwd || floats_per_lane != 7) ? 4 : 1;
+}
+
 // DEDUP: a workgroup scores each DISTINCT entity among the (up to 256) pairs of its tile once.  With skewed ids a
 // query's negatives repeat the hot entities many times (Zipf 1.1: ~175 distinct among 256 consecutive negatives,
 // ~51 among 64), every repeat costs the same instructions as the first occurrence although its row comes from
@@ -260,7 +330,7 @@ constexpr unsigned kDedupEmpty = 0xffffffffu;  // (no id: the table has at most 
 constexpr size_t kDedupLds = kDedupSlots * 12 + 256 * 8 + 256 * 4 + 16;
 
 template <int M, int VEC, int NIT, int RIF, bool REG, bool CODED = false, bool DEDUP = false>
-__global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int tiles, int tile_k) {
+__global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void score_forward_kernel(ScoreArgs A, int tiles, int tile_k) {
   const float* __restrict__ table = A.table;
   const long long* __restrict__ idx = A.idx;
   const float* __restrict__ q1 = A.q1;
@@ -289,9 +359,10 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
     pb = load_pair_batch(idx, (A.ids_shared ? (size_t)0 : (size_t)(b / A.U) * K) + kw0, cnt, lane, row_len, n_rows, bad);
 
   // LDS: query | per-wavefront pair slabs | code stage (per wavefront; one for the tile with DEDUP) | DEDUP tables
-  unsigned* slab = reinterpret_cast<unsigned*>(lds + model_nq(M) * dim) + wave * kSlabDwords;
+  constexpr int QF = query_fields(M, true);
+  unsigned* slab = reinterpret_cast<unsigned*>(lds + QF * dim) + wave * kSlabDwords;
   constexpr int kStaged = DEDUP ? 256 : kStagePairs;  // pairs whose code bytes a stage holds (DEDUP: tile_k, at most that)
-  unsigned char* stage_base = reinterpret_cast<unsigned char*>(lds + model_nq(M) * dim + 4 * kSlabDwords);
+  unsigned char* stage_base = reinterpret_cast<unsigned char*>(lds + QF * dim + 4 * kSlabDwords);
   unsigned char* stage = DEDUP ? stage_base : stage_base + wave * (kStaged * NIT * 64);
   unsigned char* after_stage = stage_base + (CODED ? (size_t)(DEDUP ? tile_k : 4 * kStaged) * NIT * 64 : 0);
   unsigned* slot_id = reinterpret_cast<unsigned*>(after_stage);                   // [kDedupSlots]
@@ -307,9 +378,14 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
     }
   }
 
-  stage_query<M>(lds, q1, q2, b, dim);  // (ends with a barrier: the tables are cleared)
-  typename ModelOps<M>::Q q[NIT][VEC];
-  load_query_regs<M, VEC, NIT, true>(lds, dim, ncol, lane, q);
+  // (either ends with a barrier: the tables are cleared)
+  [[maybe_unused]] typename ModelOps<M>::Q q[NIT][VEC];
+  if constexpr (M == mBetaKL) {
+    stage_beta_query<true>(lds, q1, q2, b, dim);
+  } else {
+    stage_query<M>(lds, q1, q2, b, dim);
+    load_query_regs<M, VEC, NIT, true>(lds, dim, ncol, lane, q);
+  }
   if constexpr (!DEDUP) {
     if (cnt <= 0) return;
   }
@@ -366,6 +442,7 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
     stage_pairs(slab, lane, table, pb, 0.f, 0.f);
   }
 
+  [[maybe_unused]] const BetaClamp clamp(p);
   float neg_thr[NIT][VEC];
   if constexpr (CODED) {
 #pragma unroll
@@ -417,6 +494,12 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
     }
     // The logit is linear in the accumulators: fold them per lane, reduce once.
     float mine = 0.f;
+    if constexpr (M == mBetaKL) {
+      asm volatile("" ::: "memory");   // the query's values are read again for every row, see beta_row_sum
+      mine = beta_row_sum<VEC, NIT, REG>(
+          clamp, [&](int it, int v) { return e1[it].v[v]; }, [&](int it, int v) { return e2[it].v[v]; },
+          [&](int it, QBeta (&to)[VEC]) { beta_query<VEC, true>(lds, dim, min(lane + 64 * it, ncol - 1), to); }, ncol, lane);
+    } else
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       float a0 = 0.f, a1 = 0.f;
@@ -473,7 +556,8 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
 // row, so it finishes the row here (merged-gradient row and/or Adam on w, m, v) instead of leaving it
 // to the entity pass, which would have to fetch the query rows and the entity row again.
 // SINGLES: 0 = leave every segment to the entity pass, 1 = finish one-pair segments here as merged-gradient
-// rows, 2 = ... with Adam on w, m, v (and the merged row if asked for).
+// rows, 2 = ... with an optimizer on w, m, v (and the merged row if asked for), 3 = ... with Adam, in the stream of the rows
+// (BetaE, rows of up to 512 floats a half).
 // CODES (models with sign codes): 1 = also writes every pair's derivative decisions, one byte per lane
 // and column group, for the entity pass to use in place of the query rows; 2 = the forward pass left
 // the codes: the query gradient is summed from them and the entity rows are not read at all (except
@@ -483,7 +567,7 @@ __global__ __launch_bounds__(256) void score_forward_kernel(ScoreArgs A, int til
 // this is the half of the work that smx_score_backward_entity hands to this kernel when the query
 // gradients were taken earlier (autograd's backward) and the update comes later (apply_grad).
 template <int M, int VEC, int NIT, int RIF, int NW, bool REG, int SINGLES, int CODES = 0, bool GQ = true>
-__global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs A) {
+__global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * NIT, false) : 1) void score_backward_query_kernel(ScoreArgs A) {
   static_assert(GQ || (SINGLES == 2 && CODES == 0), "the one-pair-only form exists with an optimizer");
   const float* __restrict__ table = A.table;
   const long long* __restrict__ idx = A.idx;
@@ -498,6 +582,7 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
   const ScoreParams p = A.p;
   constexpr int MUL = model_mul(M);
   constexpr int NQ = model_nq(M);
+  constexpr int QF = query_fields(M, false, SINGLES == 3);
   extern __shared__ float lds[];
   // Queries are taken last to first: the forward walks them first to last, and what it touched last -- the sign
   // codes it wrote, the rows it read -- is what the memory-side cache still holds when this kernel starts
@@ -509,10 +594,15 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
   const int dim = ncol * VEC;
   const size_t row_len = (size_t)dim * MUL;
 
-  stage_query<M>(lds, q1, q2, b, dim);
-  typename ModelOps<M>::Q q[NIT][VEC];
-  load_query_regs<M, VEC, NIT, false>(lds, dim, ncol, lane, q);
+  [[maybe_unused]] typename ModelOps<M>::Q q[NIT][VEC];
+  if constexpr (M == mBetaKL) {
+    stage_beta_query<false, SINGLES == 3>(lds, q1, q2, b, dim);
+  } else {
+    stage_query<M>(lds, q1, q2, b, dim);
+    load_query_regs<M, VEC, NIT, false>(lds, dim, ncol, lane, q);
+  }
 
+  [[maybe_unused]] const BetaClamp clamp(p);
   float g1[NIT][VEC], g2[NIT][VEC];
   [[maybe_unused]] float neg_thr[NIT][VEC];  // sign-coded models, when this kernel makes the comparisons itself
 #pragma unroll
@@ -523,10 +613,19 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
       if constexpr (model_coded(M)) neg_thr[it][v] = ModelOps<M>::neg_threshold(q[it][v]);
     }
   // LDS: query | per-wavefront partial sums | per-wavefront pair slabs
-  unsigned* slab = reinterpret_cast<unsigned*>(lds + (NW + 1) * NQ * dim) + wave * kSlabDwords;
+  unsigned* slab = reinterpret_cast<unsigned*>(lds + (NW * NQ + QF) * dim) + wave * kSlabDwords;
   unsigned char* stage =
-      reinterpret_cast<unsigned char*>(lds + (NW + 1) * NQ * dim + NW * kSlabDwords) + wave * (kStagePairs * NIT * 64);
+      reinterpret_cast<unsigned char*>(lds + (NW * NQ + QF) * dim + NW * kSlabDwords) + wave * (kStagePairs * NIT * 64);
 
+  // the query's feature for the rows finished here
+  auto query_at = [&](int it, int v) {
+    if constexpr (M == mBetaKL) {
+      const int d = min(lane + 64 * it, ncol - 1) * VEC + v;
+      return QBeta{q1[(size_t)b * dim + d], q2[(size_t)b * dim + d], 0.f, 0.f, 0.f};   // (LDS holds k and l)
+    } else {
+      return q[it][v];
+    }
+  };
   // this wavefront's share of the query's negatives: a contiguous range, walked in batches of 64
   const int per_wave = (K + NW - 1) / NW;
   const int kw0 = wave * per_wave;
@@ -553,6 +652,17 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
     }
     float my_c0, my_c1;
     ModelOps<M>::coef(gscore[mine], score[mine], p, my_c0, my_c1);
+    if constexpr (SINGLES == 3) {
+      // the rows to finish to the front, in pair order, then the others: each kind streams without a branch on the other
+      const int first_other = __popcll(singles);
+      const int to = lane >= cnt ? lane
+                                 : ((singles >> lane) & 1ull ? (int)lanes_below_in(singles)
+                                                             : first_other + lane - (int)lanes_below_in(singles));
+      auto moved = [&](unsigned x) { return (unsigned)__builtin_amdgcn_ds_permute(to * 4, (int)x); };
+      pb = PairBatch{moved(pb.off_lo), moved(pb.off_hi), moved(pb.row)};
+      my_c0 = __uint_as_float(moved(__float_as_uint(my_c0)));
+      my_c1 = __uint_as_float(moved(__float_as_uint(my_c1)));
+    }
     // Without optimizer state to fetch, such a pair's row is finished the moment it streams by: its entity
     // row and query are in registers, the merged-gradient row is one more store.
     constexpr bool kInStream = SINGLES == 1 && CODES != 2;
@@ -628,11 +738,52 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
         slab_fence();
       }
     }
+    if constexpr (SINGLES == 3) {
+      // Rows that occur once, Adam: the row with its moments, one ahead of the one in work; every turn has the same number
+      // of loads and stores, so that no wait is for more than what it needs (after a branch that may have issued some, the
+      // wait is for all of them).
+      const int n_rows_here = __popcll(singles);
+      RowState<MUL, VEC, NIT> sa, sb;
+      auto request = [&](RowState<MUL, VEC, NIT>& s, int j) {
+        const unsigned long long off = batch_off(pb, min(j, n_rows_here - 1));
+        load_row<MUL, VEC, NIT>(s.e, table + off, dim, ncol, lane);
+        load_row<MUL, VEC, NIT, true>(s.m, A.sink.m + off, dim, ncol, lane);
+        load_row<MUL, VEC, NIT, true>(s.v, A.sink.v + off, dim, ncol, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      RowSink sink = A.sink;
+      sink.merged = nullptr;
+      sink.adam_on = kOptAdam;
+      sink.squeeze = 0;
+      auto finish = [&](const RowState<MUL, VEC, NIT>& s, int j) {
+        const float c0 = slab_coef(slab, j).x;
+        float ge1[NIT][VEC], ge2[NIT][VEC];
+        asm volatile("" ::: "memory");
+        beta_row_both_grads<VEC, NIT, REG>(
+            clamp, p, [&](int it, int v) { return s.e.h[0][it].v[v]; }, [&](int it, int v) { return s.e.h[MUL - 1][it].v[v]; }, c0,
+            [&](int it, QBeta (&to)[VEC]) { beta_query<VEC, false, true>(lds, dim, min(lane + 64 * it, ncol - 1), to); }, g1, g2,
+            ge1, ge2);
+        finish_row<M, VEC, NIT, REG, true, true>(sink, lane, (unsigned)__builtin_amdgcn_readlane((int)pb.row, j), 0, ge1, ge2, s.e,
+                                                 s.m, s.v);
+      };
+      if (n_rows_here > 0) {
+        request(sa, 0);
+        for (int j = 0; j < n_rows_here; j += 2) {
+          request(sb, j + 1);
+          finish(sa, j);
+          if (j + 1 >= n_rows_here) break;
+          request(sa, j + 2);
+          finish(sb, j + 1);
+        }
+      }
+      n_stream = cnt - n_rows_here;
+    }
     // lanes past the row end hold a copy of the last column: what they accumulate is never stored
+    const unsigned* const stream_from = SINGLES == 3 ? slab + 4 * (cnt - n_stream) : slab;
     if (n_stream > 0)
-    stream_batch<MUL, VEC, NIT, RIF>(slab, n_stream, dim, ncol, lane,
+    stream_batch<MUL, VEC, NIT, RIF>(stream_from, n_stream, dim, ncol, lane,
                                      [&](int j, const Pack<VEC>(&e1)[NIT], const Pack<VEC>(&e2)[NIT]) {
-      float2 c = slab_coef(slab, j);
+      float2 c = slab_coef(stream_from, j);
       [[maybe_unused]] const float c_raw = c.x;
       if constexpr (M == mL2)
         c.x = l2_pair_coef<VEC, NIT>(c.x, ncol, lane, [&](int it, int v) { return e1[it].v[v]; },
@@ -652,6 +803,11 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
           mine_b[64 * it] = (unsigned char)code;
         }
         flush_codes<NIT>(stage, A.codes, first, j, cnt, lane);
+      } else if constexpr (M == mBetaKL) {
+        asm volatile("" ::: "memory");   // (as in the forward)
+        beta_row_query_grad<VEC, NIT, REG>(
+            clamp, [&](int it, int v) { return e1[it].v[v]; }, [&](int it, int v) { return e2[it].v[v]; }, c.x,
+            [&](int it, QBeta (&to)[VEC]) { beta_query<VEC, false>(lds, dim, min(lane + 64 * it, ncol - 1), to); }, g1, g2);
       } else {
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
@@ -683,7 +839,7 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
               ge1[it][v] = ge2[it][v] = 0.f;
               const float x1 = REG ? reg_apply(e1[it].v[v], p) : e1[it].v[v];
               const float x2 = MUL == 2 ? (REG ? reg_apply(e2[it].v[v], p) : e2[it].v[v]) : 0.f;
-              ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, q[it][v], ge1[it][v], ge2[it][v]);
+              ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, query_at(it, v), ge1[it][v], ge2[it][v]);
             }
           const int seg = __builtin_amdgcn_readlane(my_ps, j) & 0x7fffffff;
           const unsigned row = (unsigned)__builtin_amdgcn_readlane((int)pb.row, j);
@@ -693,7 +849,7 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
     });
     }
 
-    if constexpr (SINGLES != 0 && !kInStream && !kFromCodes) {
+    if constexpr (SINGLES != 0 && SINGLES != 3 && !kInStream && !kFromCodes) {
       // S rows at a time per wavefront (their w, m, v loads are all requested before the first is
       // used): the row sets of the streaming loop are dead here, so this costs no extra registers, and
       // it divides the memory latency each one-pair row would otherwise expose by S.
@@ -736,7 +892,7 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
                 const float x1 = REG ? reg_apply(e[s].h[0][it].v[v], p) : e[s].h[0][it].v[v];
                 const float x2 =
                     MUL == 2 ? (REG ? reg_apply(e[s].h[MUL - 1][it].v[v], p) : e[s].h[MUL - 1][it].v[v]) : 0.f;
-                ModelOps<M>::bwd_e(c0, c1, x1, x2, q[it][v], ge1[it][v], ge2[it][v]);
+                ModelOps<M>::bwd_e(c0, c1, x1, x2, query_at(it, v), ge1[it][v], ge2[it][v]);
               }
             finish_row<M, VEC, NIT, REG, SINGLES == 2>(A.sink, lane, row, seg, ge1, ge2, e[s], m0[s], v0[s]);
           }
@@ -749,10 +905,11 @@ __global__ __launch_bounds__(NW * 64) void score_backward_query_kernel(ScoreArgs
 #pragma unroll
   for (int it = 0; it < NIT; ++it)
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) finish_query_grad<M>(q[it][v], g1[it][v], g2[it][v], p);
+    for (int v = 0; v < VEC; ++v)
+      if constexpr (M != mBetaKL) finish_query_grad<M>(q[it][v], g1[it][v], g2[it][v], p);
 
   // wavefront partials -> LDS -> fixed-order sum over wavefronts
-  float* part = lds + NQ * dim;  // [NW][NQ][dim]
+  float* part = lds + QF * dim;  // [NW][NQ][dim]
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = lane + 64 * it;
@@ -805,7 +962,7 @@ int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
   const size_t B = (size_t)A.B, K = (size_t)A.K;
   const int tile_k = forward_tile(B, K, 4 * RIF);
   const int tiles = (int)((K + tile_k - 1) / tile_k);
-  const size_t lds = ((size_t)model_nq(M) * A.ncol * VEC + 4 * kSlabDwords) * sizeof(float);
+  const size_t lds = ((size_t)query_fields(M, true) * A.ncol * VEC + 4 * kSlabDwords) * sizeof(float);
   // (not the dense layout, whose rows are all different, nor a list of ids shared by the batch: a sampler's K negatives hardly
   // ever repeat)
   const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= distinct_from(M);
@@ -867,6 +1024,14 @@ int launch_backward_query_reg(hipStream_t st, const ScoreArgs& A) {
       return check_launch("score backward (query, coded)");
     }
   }
+  if constexpr (M == mBetaKL && VEC == 4 && NIT <= 2 && NW == 8) {
+    if (A.pair_seg && A.stream_rows) {
+      const size_t fields = query_fields(M, false, true) - model_nq(M);
+      hipLaunchKernelGGL((score_backward_query_kernel<M, VEC, NIT, RIF, NW, REG, 3>), dim3((unsigned)A.B), dim3(NW * 64),
+                         lds + fields * A.ncol * VEC * sizeof(float), st, A);
+      return check_launch("score backward (query, rows in the stream)");
+    }
+  }
   if (A.pair_seg && A.sink.adam_on)
     hipLaunchKernelGGL((score_backward_query_kernel<M, VEC, NIT, RIF, NW, REG, 2>), dim3((unsigned)A.B),
                        dim3(NW * 64), lds, st, A);
@@ -906,9 +1071,38 @@ int launch_score(hipStream_t st, const ScoreArgs& A, bool forward) {
   return launch_backward_query_reg<M, VEC, NIT, 2, false>(st, A);
 }
 
+// BetaE's kernels pay for every feature a lane holds, also past the row's end: 512 for a row of 400 in columns of four floats,
+// 448 in single ones.  Those rows, and the short ones (128 floats: two a lane instead of four), are taken a float per lane and
+// step; the loads are still whole 256-byte stretches.  Forward, 512 x 512 pairs of 2 x 400 floats: 358 -> 311 us.  Not where
+// rows are finished as well: that is bound by memory.
+inline int beta_singles(int dim, int nit4) {
+  const int n = (dim + 63) / 64;
+  return n <= 7 && n < 4 * nit4 && n != 4 ? n : 0;
+}
+int beta_singles_dispatch(hipStream_t st, const ScoreArgs& A, int nit, bool forward);   // smx_score_inst_betakl_singles.hip
+template <int NIT>
+int launch_beta_singles(hipStream_t st, const ScoreArgs& A, bool forward) {
+  if (forward) return A.p.reg_on ? launch_forward_reg<mBetaKL, 1, NIT, true>(st, A) : launch_forward_reg<mBetaKL, 1, NIT, false>(st, A);
+  // (rows of up to 448 floats: eight wavefronts' partial sums fit)
+  const size_t lds = ((size_t)9 * 2 * A.ncol + 8 * kSlabDwords) * sizeof(float);
+  if (A.p.reg_on)
+    hipLaunchKernelGGL((score_backward_query_kernel<mBetaKL, 1, NIT, 1, 8, true, 0>), dim3((unsigned)A.B), dim3(512), lds, st, A);
+  else
+    hipLaunchKernelGGL((score_backward_query_kernel<mBetaKL, 1, NIT, 1, 8, false, 0>), dim3((unsigned)A.B), dim3(512), lds, st, A);
+  return check_launch("score backward (query)");
+}
+
 // Instantiated once per model in its own translation unit (smx_score_inst_*.hip).
 template <int M>
 int score_dispatch(hipStream_t st, const ScoreArgs& A, int vec, int nit, bool forward) {
+  if constexpr (M == mBetaKL) {
+    const int n = vec == 4 && (forward || (A.gq1 && !A.pair_seg)) ? beta_singles(A.ncol * 4, nit) : 0;
+    if (n) {
+      ScoreArgs S = A;
+      S.ncol = A.ncol * 4;
+      return beta_singles_dispatch(st, S, n, forward);
+    }
+  }
   if (vec == 4) {
     switch (nit) {
       case 1: return launch_score<M, 4, 1>(st, A, forward);
