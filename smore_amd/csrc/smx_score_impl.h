@@ -49,6 +49,7 @@ struct ScoreArgs {
   const unsigned char* codes_in;  // query backward: codes the forward left; the entity rows are then not read
   RowSink sink;
   int stream_rows;       // one-pair segments are finished in the stream of the rows (beta_rows_in_stream)
+  int rows_once;         // forward: no row is worth keeping in a cache (read_once)
 };
 
 // BetaE with Adam in place: the query-gradient kernel finishes the rows that occur once.  It is bound by the special functions
@@ -220,12 +221,14 @@ __device__ __forceinline__ GlobalRow slab_row(const unsigned* slab, int j) {
   const uint2 a = *reinterpret_cast<const uint2*>(slab + 4 * j);
   return reinterpret_cast<GlobalRow>(((unsigned long long)a.y << 32) | a.x);
 }
-template <int VEC>
+// ONCE: past the caches (read_once)
+template <int VEC, bool ONCE = false>
 __device__ __forceinline__ Pack<VEC> load_pack(GlobalRow base, int col) {
   Pack<VEC> r;
   if constexpr (VEC == 4) {
     typedef float vec4 __attribute__((ext_vector_type(4)));
-    const vec4 t = reinterpret_cast<const __attribute__((address_space(1))) vec4*>(base)[col];
+    const __attribute__((address_space(1))) vec4* p = reinterpret_cast<const __attribute__((address_space(1))) vec4*>(base) + col;
+    const vec4 t = ONCE ? __builtin_nontemporal_load(p) : *p;
     r.v[0] = t.x;
     r.v[1] = t.y;
     r.v[2] = t.z;
@@ -245,7 +248,7 @@ template <int MUL, int VEC, int NIT, int RIF> struct RowSet {
 };
 
 // Requests rows g0 .. g0+RIF-1 of the batch; g0 is a multiple of RIF, so the entries exist.
-template <int MUL, int VEC, int NIT, int RIF>
+template <int MUL, int VEC, int NIT, int RIF, bool ONCE = false>
 __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, const unsigned* slab, int g0, int dim,
                                              int ncol, int lane) {
   GlobalRow pe[RIF];
@@ -256,8 +259,8 @@ __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, con
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int c = min(lane + 64 * it, ncol - 1);
-      rs.e1[r][it] = load_pack<VEC>(pe[r], c);
-      if (MUL == 2) rs.e2[r][it] = load_pack<VEC>(pe[r] + dim, c);
+      rs.e1[r][it] = load_pack<VEC, ONCE>(pe[r], c);
+      if (MUL == 2) rs.e2[r][it] = load_pack<VEC, ONCE>(pe[r] + dim, c);
     }
     // Rows are used in the order r = 0, 1, ..: their loads must be issued in that order everywhere (the
     // scheduler is otherwise free to reverse them in the loop prologue), or the wait for row 0 at the top
@@ -266,20 +269,23 @@ __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, con
   }
 }
 
+// Forward kernels that have the form for rows read once: the models whose rows the memory bounds, in 16-byte columns.
+template <int M, int VEC, bool DEDUP> constexpr bool kReadOnce = DEDUP && VEC == 4 && M != mBetaKL;
+
 // Streams the cnt (<= 64) rows of a staged batch through `consume(j, e1, e2)`, j ascending.
-template <int MUL, int VEC, int NIT, int RIF, class Consume>
+template <int MUL, int VEC, int NIT, int RIF, bool ONCE = false, class Consume>
 __device__ __forceinline__ void stream_batch(const unsigned* slab, int cnt, int dim, int ncol, int lane,
                                              Consume&& consume) {
   static_assert(64 % RIF == 0, "a group of rows must not straddle the end of the slab");
   RowSet<MUL, VEC, NIT, RIF> a, b;
   const int last = ((cnt - 1) / RIF) * RIF;  // first row of the last group
-  request_rows<MUL, VEC, NIT, RIF>(a, slab, 0, dim, ncol, lane);
+  request_rows<MUL, VEC, NIT, RIF, ONCE>(a, slab, 0, dim, ncol, lane);
   for (int j0 = 0; j0 < cnt; j0 += 2 * RIF) {
-    request_rows<MUL, VEC, NIT, RIF>(b, slab, min(j0 + RIF, last), dim, ncol, lane);
+    request_rows<MUL, VEC, NIT, RIF, ONCE>(b, slab, min(j0 + RIF, last), dim, ncol, lane);
 #pragma unroll
     for (int r = 0; r < RIF; ++r)
       if (j0 + r < cnt) consume(j0 + r, a.e1[r], a.e2[r]);
-    request_rows<MUL, VEC, NIT, RIF>(a, slab, min(j0 + 2 * RIF, last), dim, ncol, lane);
+    request_rows<MUL, VEC, NIT, RIF, ONCE>(a, slab, min(j0 + 2 * RIF, last), dim, ncol, lane);
 #pragma unroll
     for (int r = 0; r < RIF; ++r)
       if (j0 + RIF + r < cnt) consume(j0 + RIF + r, b.e1[r], b.e2[r]);
@@ -392,6 +398,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
   int n_stream = cnt;        // rows this wavefront streams
   int first_rep = 0;         // DEDUP: position on the tile's list of the first of them
   int my_pos = lane;         // DEDUP: position on the list of the row my pair's score comes from
+  bool once = false;         // DEDUP: the tile's ids are all different and its rows come through once (read_once)
   if constexpr (DEDUP) {
     // The representative of an id is its first pair of the tile, and the list holds the representatives in pair
     // order: which wavefront scores which row is then the same in every run (a row's bits may depend on where it
@@ -429,6 +436,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
     }
     __syncthreads();
     if (lane < cnt) my_pos = slot_pos[s];
+    once = A.rows_once && n_reps == min(tile_k, K - tile * tile_k);
     const int share = (n_reps + 3) / 4;  // <= 64
     first_rep = wave * share;
     n_stream = max(0, min(share, n_reps - first_rep));
@@ -451,9 +459,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
       for (int v = 0; v < VEC; ++v) neg_thr[it][v] = ModelOps<M>::neg_threshold(q[it][v]);
   }
   float* out = score + (size_t)b * K + kw0;
-  if (n_stream > 0)
-  stream_batch<MUL, VEC, NIT, RIF>(slab, n_stream, dim, ncol, lane,
-                                   [&](int j, const Pack<VEC>(&e1)[NIT], const Pack<VEC>(&e2)[NIT]) {
+  auto take = [&](int j, const Pack<VEC>(&e1)[NIT], const Pack<VEC>(&e2)[NIT]) __attribute__((always_inline)) {
     // lanes past the row end hold a copy of the last column: they compute along and are dropped here.
     if constexpr (model_norm(M, REG)) {
       // unit-length halves: the two inner products and the two squared lengths are summed separately
@@ -526,7 +532,13 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
       if (lane == 63) out[j] = ModelOps<M>::score(folded, p);
       if constexpr (CODED) flush_codes<NIT>(stage, A.codes, (size_t)b * K + kw0, j, cnt, lane);
     }
-  });
+  };
+  if (n_stream > 0) {
+    if (kReadOnce<M, VEC, DEDUP> && once)
+      stream_batch<MUL, VEC, NIT, RIF, kReadOnce<M, VEC, DEDUP>>(slab, n_stream, dim, ncol, lane, take);
+    else
+      stream_batch<MUL, VEC, NIT, RIF>(slab, n_stream, dim, ncol, lane, take);
+  }
   if constexpr (DEDUP) {
     // every pair takes what its representative produced: the score from the tile's list ...
     __syncthreads();
@@ -956,8 +968,30 @@ inline int forward_tile(size_t B, size_t K, int least) {
 // Below it every pair is scored where it stands, and repeats of one id may then differ in their last bits, as those of two tiles may.
 constexpr int distinct_from(int model) { return model == mBetaKL ? 64 : 128; }
 
+// Rows that no cache will hold until they are asked for again are loaded past the caches (non-temporal), in the tiles whose ids
+// are all different: then the last-level cache (256 MB) keeps what is asked for again -- the sign codes and the logits, or the
+// lines that the query gradient starts with -- and the loads themselves are quicker (random rows of 800 bytes 6.0 TB/s against
+// 5.65).  Forward of 1024 x 1024 pairs, RotatE, rows of 4 KB of a table of 10 GB: 736 -> 674 us.  The lines, from whole steps
+// (forward, query gradient, entity pass), plain / past the caches in us:
+// a table from 1.5 GiB on (below, a share of the rows is still in the cache): box, rows of 800 bytes of 0.8 GB 498 / 507, of 1.7 GB
+// 546 / 536, of 8 GB 1054 / 1029; 1600 bytes of 2.4 GB 792 / 775; L1, 800 bytes of 0.8 GB 479 / 485, of 1.7 GB 532 / 521;
+// without codes the query gradient reads the rows again: a table from 4 GiB on (RotatE 4 KB of 1.6 GB 2156 / 2157, of 3.3 GB
+// 2378 / 2340, 1 KB of 1.7 GB 1308 / 1320, of 5 GB 1414 / 1400; L2 1600 bytes of 1.7 GB 1019 / 1033, of 13 GB 2179 / 2133) and a
+// pass of 1.5 GiB (L2 800 bytes x 1 M pairs 669 / 676, 1200 bytes 939 / 934; ComplEx 1600 bytes 1101 / 1095);
+// halves from 512 bytes on, or the lines that a row shares with its neighbours are most of it (RotatE, 2 x 400 bytes of 4 GB
+// 674 / 683, 2 x 512 bytes 739 / 736).  Not in the kernels that follow: the query gradient of RotatE 1468 / 1498.
+inline bool read_once(const ScoreArgs& A, int mul) {
+  constexpr size_t kGiB = (size_t)1 << 30;
+  const size_t half = (size_t)A.ncol * 4 * sizeof(float), row = mul * half;
+  if (half < 512) return false;
+  if (A.codes) return A.n_rows * row >= 3 * kGiB / 2;
+  return A.n_rows * row >= 4 * kGiB && (size_t)A.B * A.K * row >= 3 * kGiB / 2;
+}
+
 template <int M, int VEC, int NIT, bool REG>
-int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
+int launch_forward_reg(hipStream_t st, const ScoreArgs& args) {
+  ScoreArgs A = args;
+  A.rows_once = kReadOnce<M, VEC, true> && read_once(A, model_mul(M));
   constexpr int RIF = rows_in_flight(NIT, model_mul(M));
   const size_t B = (size_t)A.B, K = (size_t)A.K;
   const int tile_k = forward_tile(B, K, 4 * RIF);
