@@ -39,6 +39,8 @@ struct ScoreArgs {
   // Union queries (kg_reasoning.py:326, box.py:163): q1 / q2 hold U branch rows per query, [B*U, dim]; a kernel's
   // "query" is then one branch row, number bq = b * U + u, which scores the ids of query b.
   int U;                 // branches per query (1: none of this)
+  bool stream_rows;      // one-pair segments are finished in the stream of the rows (beta_rows_in_stream)
+  bool rows_once;        // forward: no row is worth keeping in a cache (read_once)
   const unsigned char* winner;  // query backward, [B, K]: the branch that gave the pair's logit; a branch row sums its own pairs only
   unsigned long long n_rows;
   ScoreParams p;
@@ -48,8 +50,6 @@ struct ScoreArgs {
   unsigned char* codes;  // [B*K][NIT*64] sign codes written by this kernel (forward or query backward), or null
   const unsigned char* codes_in;  // query backward: codes the forward left; the entity rows are then not read
   RowSink sink;
-  int stream_rows;       // one-pair segments are finished in the stream of the rows (beta_rows_in_stream)
-  int rows_once;         // forward: no row is worth keeping in a cache (read_once)
 };
 
 // BetaE with Adam in place: the query-gradient kernel finishes the rows that occur once.  It is bound by the special functions
@@ -791,11 +791,14 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
       n_stream = cnt - n_rows_here;
     }
     // lanes past the row end hold a copy of the last column: what they accumulate is never stored
-    const unsigned* const stream_from = SINGLES == 3 ? slab + 4 * (cnt - n_stream) : slab;
+    auto stream_from = [&]() -> const unsigned* {
+      if constexpr (SINGLES == 3) return slab + 4 * (cnt - n_stream);
+      return slab;
+    };
     if (n_stream > 0)
-    stream_batch<MUL, VEC, NIT, RIF>(stream_from, n_stream, dim, ncol, lane,
+    stream_batch<MUL, VEC, NIT, RIF>(stream_from(), n_stream, dim, ncol, lane,
                                      [&](int j, const Pack<VEC>(&e1)[NIT], const Pack<VEC>(&e2)[NIT]) {
-      float2 c = slab_coef(stream_from, j);
+      float2 c = slab_coef(stream_from(), j);
       [[maybe_unused]] const float c_raw = c.x;
       if constexpr (M == mL2)
         c.x = l2_pair_coef<VEC, NIT>(c.x, ncol, lane, [&](int it, int v) { return e1[it].v[v]; },
