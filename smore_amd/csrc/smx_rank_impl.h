@@ -831,7 +831,8 @@ __global__ __launch_bounds__(kScanThreads) void rank_scan_kernel(RankArgs A) {
 // 64 candidates, 5 us instead of 8.)
 // Scores: a wavefront takes `per_wave` consecutive candidates of one query, the next row on its way while one is summed.
 constexpr int kCandFused = 64;
-template <int M, int VEC, int NIT, bool REG, bool UNION, bool FUSED>
+// ONCE: rows past the caches (candidates_read_once)
+template <int M, int VEC, int NIT, bool REG, bool UNION, bool FUSED, bool ONCE = false>
 __global__ __launch_bounds__(FUSED ? 1024 : 256) void cand_score_kernel(RankArgs A, int tiles, int per_wave) {
   constexpr int MUL = model_mul(M);
   const int b = blockIdx.x / tiles;
@@ -859,7 +860,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void cand_score_kernel(RankArgs
     auto request = [&](int i) {
       const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)off, i);
       const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(off >> 32), i);
-      load_entity<VEC, NIT, MUL>(A.table + (((unsigned long long)hi << 32) | lo), dim, A.ncol, lane, next1, next2);
+      load_entity<VEC, NIT, MUL, ONCE>(A.table + (((unsigned long long)hi << 32) | lo), dim, A.ncol, lane, next1, next2);
     };
     request(0);
     for (int i = 0; i < n; ++i) {
@@ -1027,8 +1028,19 @@ static __global__ __launch_bounds__(256) void rank_prepare_kernel(RankArgs A, in
   }
 }
 
+// Rows of long lists out of a table that the last-level cache (256 MB) does not hold are loaded past it: no list comes back to
+// them, and random rows come at 6.0 TB/s instead of 5.65.  256 lists of 1,500: RotatE 2 x 400 floats, 3.2 GB, 258 -> 243 us, box
+// 400 floats, 1.6 GB, 158 -> 152; 256 x 700 x 260 62 -> 58.  The halves' features from 1 GiB on (RotatE
+// 2 x 500 floats of 0.7 GB a half 293 / 295, box 128 floats of 0.15 GB 54 / 59, L1 300 floats of 1.1 GB 42.5 / 42.1), lists from 96 MiB on (64 x 400 of 400 floats 38.6 / 39.2), halves from 512 bytes on (440 bytes
+// 115 / 114: as good); not BetaE, which is bound by its arithmetic.
+inline bool candidates_read_once(const RankArgs& A, int mul) {
+  const size_t half = (size_t)A.ncol * 4 * sizeof(float), row = mul * half;
+  return half >= 512 && A.n_rows * half >= ((size_t)1 << 30) && (size_t)A.B * A.C * row >= ((size_t)96 << 20);
+}
+
 template <int M, int VEC, int NIT, bool REG>
 int launch_candidates(hipStream_t st, const RankArgs& A) {
+  constexpr bool kOnce = VEC == 4 && M != mBetaKL;
   int per_wave = 16;   // candidates of a wavefront: fewer when the grid would not fill the chip
   while (per_wave > 1 && (size_t)A.B * ((A.C + 4 * per_wave - 1) / (4 * per_wave)) < 2048) per_wave /= 2;
   const int tiles = (A.C + 4 * per_wave - 1) / (4 * per_wave);
@@ -1038,6 +1050,8 @@ int launch_candidates(hipStream_t st, const RankArgs& A) {
   }
   if (A.U > 1)
     hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, true, false>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
+  else if (kOnce && candidates_read_once(A, model_mul(M)))
+    hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, false, false, kOnce>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
   else
     hipLaunchKernelGGL((cand_score_kernel<M, VEC, NIT, REG, false, false>), dim3((unsigned)A.B * tiles), dim3(256), 0, st, A, tiles, per_wave);
   if (int rc = check_launch("candidate scores")) return rc;

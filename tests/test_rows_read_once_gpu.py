@@ -42,3 +42,29 @@ def test_same_bits_as_a_small_table(model, dim, n, b, k):
                                  24.0, *([0.02] if model == "box" else []))
         # the terms of a row: at most some 2 each
         assert_close(got[i].cpu().numpy(), want[0], REL_F32, "score", sum_abs=24.0 + 2.0 * dim)
+
+
+# 1.27 GiB a half, lists of 128 MiB; the last wavefront of a list takes nine candidates of its sixteen
+@pytest.mark.parametrize("model,dim,n", [("box", 260, 1_320_000), ("l1", 132, 2_600_000), ("rotate", 132, 2_600_000), ("complex", 260, 1_320_000)])
+def test_candidates_as_from_a_small_table(model, dim, n):
+    from smore_amd import fused
+    from smore_amd.evaluation import candidate_ranks
+    rng = np.random.default_rng(seed("candidates read once", model, dim))
+    width = dim * (2 if model in ("rotate", "complex") else 1)
+    b, c = -(-(1 << 27) // (width * 4 * 1001)), 1001
+    pool = np.unique(np.concatenate([[0, n - 1], rng.integers(0, n, 5000)]))
+    pick = rng.integers(0, pool.size, (b, c))
+    pick[0, :2] = (0, pool.size - 1)
+    small = torch.tensor(rng.standard_normal((pool.size, width)) * 0.5, dtype=torch.float32, device="cuda")
+    rows = torch.tensor(pool, device="cuda")
+    large = torch.empty(n, width, dtype=torch.float32, device="cuda")
+    large[rows] = small
+    local = torch.tensor(pick, device="cuda")
+    ids = rows[local]
+    local[:, -30:], ids[:, -30:] = -1, -1                 # padding reads entity 0, the same row in both
+    q1 = torch.tensor(rng.standard_normal((b, dim)) * 0.5, dtype=torch.float32, device="cuda")
+    q2 = None if model == "l1" else torch.tensor(rng.random((b, dim)), dtype=torch.float32, device="cuda")
+    params = fused.score_params(24.0, 0.02)
+    n_hard = rng.integers(1, 11, b).tolist()
+    for got, ref in zip(candidate_ranks(model, large, q1, q2, params, ids, n_hard), candidate_ranks(model, small, q1, q2, params, local, n_hard)):
+        assert torch.equal(got, ref)
