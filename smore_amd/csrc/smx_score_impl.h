@@ -40,7 +40,6 @@ struct ScoreArgs {
   // "query" is then one branch row, number bq = b * U + u, which scores the ids of query b.
   int U;                 // branches per query (1: none of this)
   bool stream_rows;      // one-pair segments are finished in the stream of the rows (beta_rows_in_stream)
-  bool rows_once;        // forward: no row is worth keeping in a cache (read_once)
   const unsigned char* winner;  // query backward, [B, K]: the branch that gave the pair's logit; a branch row sums its own pairs only
   unsigned long long n_rows;
   ScoreParams p;
@@ -269,9 +268,6 @@ __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, con
   }
 }
 
-// Forward kernels that have the form for rows read once: the models whose rows the memory bounds, in 16-byte columns.
-template <int M, int VEC, bool DEDUP> constexpr bool kReadOnce = DEDUP && VEC == 4 && M != mBetaKL;
-
 // Streams the cnt (<= 64) rows of a staged batch through `consume(j, e1, e2)`, j ascending.
 template <int MUL, int VEC, int NIT, int RIF, bool ONCE = false, class Consume>
 __device__ __forceinline__ void stream_batch(const unsigned* slab, int cnt, int dim, int ncol, int lane,
@@ -335,7 +331,9 @@ constexpr unsigned kDedupEmpty = 0xffffffffu;  // (no id: the table has at most 
 // scores of the list, representatives per wavefront
 constexpr size_t kDedupLds = kDedupSlots * 12 + 256 * 8 + 256 * 4 + 16;
 
-template <int M, int VEC, int NIT, int RIF, bool REG, bool CODED = false, bool DEDUP = false>
+// ONCE (with DEDUP): tiles of different ids load their rows past the caches (read_once).  A kernel of its own, as the second
+// loop costs the first 8 to 28 registers.
+template <int M, int VEC, int NIT, int RIF, bool REG, bool CODED = false, bool DEDUP = false, bool ONCE = false>
 __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void score_forward_kernel(ScoreArgs A, int tiles, int tile_k) {
   const float* __restrict__ table = A.table;
   const long long* __restrict__ idx = A.idx;
@@ -398,7 +396,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
   int n_stream = cnt;        // rows this wavefront streams
   int first_rep = 0;         // DEDUP: position on the tile's list of the first of them
   int my_pos = lane;         // DEDUP: position on the list of the row my pair's score comes from
-  bool once = false;         // DEDUP: the tile's ids are all different and its rows come through once (read_once)
+  [[maybe_unused]] bool once = false;   // ONCE: the tile's ids are all different
   if constexpr (DEDUP) {
     // The representative of an id is its first pair of the tile, and the list holds the representatives in pair
     // order: which wavefront scores which row is then the same in every run (a row's bits may depend on where it
@@ -436,7 +434,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
     }
     __syncthreads();
     if (lane < cnt) my_pos = slot_pos[s];
-    once = A.rows_once && n_reps == min(tile_k, K - tile * tile_k);
+    if constexpr (ONCE) once = n_reps == min(tile_k, K - tile * tile_k);
     const int share = (n_reps + 3) / 4;  // <= 64
     first_rep = wave * share;
     n_stream = max(0, min(share, n_reps - first_rep));
@@ -534,8 +532,8 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
     }
   };
   if (n_stream > 0) {
-    if (kReadOnce<M, VEC, DEDUP> && once)
-      stream_batch<MUL, VEC, NIT, RIF, kReadOnce<M, VEC, DEDUP>>(slab, n_stream, dim, ncol, lane, take);
+    if (ONCE && once)
+      stream_batch<MUL, VEC, NIT, RIF, ONCE>(slab, n_stream, dim, ncol, lane, take);
     else
       stream_batch<MUL, VEC, NIT, RIF>(slab, n_stream, dim, ncol, lane, take);
   }
@@ -992,9 +990,9 @@ inline bool read_once(const ScoreArgs& A, int mul) {
 }
 
 template <int M, int VEC, int NIT, bool REG>
-int launch_forward_reg(hipStream_t st, const ScoreArgs& args) {
-  ScoreArgs A = args;
-  A.rows_once = kReadOnce<M, VEC, true> && read_once(A, model_mul(M));
+int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
+  constexpr bool kOnce = VEC == 4 && NIT <= 2 && M != mBetaKL;   // (BetaE is bound by its arithmetic, longer rows lose a wavefront)
+  const bool once = kOnce && read_once(A, model_mul(M));
   constexpr int RIF = rows_in_flight(NIT, model_mul(M));
   const size_t B = (size_t)A.B, K = (size_t)A.K;
   const int tile_k = forward_tile(B, K, 4 * RIF);
@@ -1005,7 +1003,10 @@ int launch_forward_reg(hipStream_t st, const ScoreArgs& args) {
   const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= distinct_from(M);
   if constexpr (model_coded(M) && !REG) {
     if (A.codes) {
-      if (dedup)
+      if (dedup && once)
+        hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, true, true, kOnce>), dim3((unsigned)(B * tiles)),
+                           dim3(256), lds + (size_t)tile_k * NIT * 64 + kDedupLds, st, A, tiles, tile_k);
+      else if (dedup)
         hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, true, true>), dim3((unsigned)(B * tiles)),
                            dim3(256), lds + (size_t)tile_k * NIT * 64 + kDedupLds, st, A, tiles, tile_k);
       else
@@ -1014,7 +1015,10 @@ int launch_forward_reg(hipStream_t st, const ScoreArgs& args) {
       return check_launch("score forward (coded)");
     }
   }
-  if (dedup)
+  if (dedup && once)
+    hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, false, true, kOnce>), dim3((unsigned)(B * tiles)),
+                       dim3(256), lds + kDedupLds, st, A, tiles, tile_k);
+  else if (dedup)
     hipLaunchKernelGGL((score_forward_kernel<M, VEC, NIT, RIF, REG, false, true>), dim3((unsigned)(B * tiles)),
                        dim3(256), lds + kDedupLds, st, A, tiles, tile_k);
   else
