@@ -36,6 +36,12 @@ int smx_measure_query_kernel_events(void* before, void* after);
  * (16: 16 or fewer, by the row's length) and whether it scores each distinct id among them once.  Host only. */
 int smx_measure_forward_tile(int model, size_t B, size_t K, int* tile, int* distinct);
 
+/* No counterpart in the reference.  How a wavefront of the row-finishing query-gradient kernel walks a batch of cnt
+ * (1 .. 64) pairs, of which those in the mask `singles` are finished on their own: place[64], the slab entry of each
+ * lane's pair; taken[64], the entries whose rows are streamed, in order (-1 behind the last); lowest, highest, the range
+ * of the entries asked for by the stream, in groups of rif (1, 2 or 4).  Host only, the kernel's own arithmetic. */
+int smx_measure_slab_walk(int cnt, unsigned long long singles, int rif, int* place, int* taken, int* lowest, int* highest);
+
 /* No counterpart in the reference.  smx_plan_build with the two knobs a test needs to see a plan give up while
  * every kernel still ends normally:
  *   spin_limit    polls a workgroup of the sort makes before it stops waiting for another one (the library

@@ -153,6 +153,8 @@ MEASURE_SIGNATURES = {
     "smx_measure_query_kernel_events": (_i, [_vp, _vp]),
     # model, B, K, tile, distinct
     "smx_measure_forward_tile": (_i, [_i, _sz, _sz, _vp, _vp]),
+    # cnt, singles, rif, place, taken, lowest, highest
+    "smx_measure_slab_walk": (_i, [_i, _c.c_ulonglong, _i] + [_vp] * 4),
     # kind, bsize, num, be, ne, bc, nc, dim, addresses, path, vec, waves, ahead
     "smx_measure_dense_backward_form": (_i, [_i] + [_sz] * 8 + [_vp] * 4),
     # bsize, num, be, ne, bc, nc, dim, addresses, path, rows_per_tile

@@ -706,6 +706,33 @@ int smx_measure_forward_tile(int model, size_t B, size_t K, int* tile, int* dist
   return SMX_OK;
 }
 
+int smx_measure_slab_walk(int cnt, unsigned long long singles, int rif, int* place, int* taken, int* lowest, int* highest) {
+  if (cnt < 1 || cnt > smx::kSlabEntries || (rif != 1 && rif != 2 && rif != 4)) return smx::fail(SMX_ERR_ARG, "no such batch");
+  if (cnt < smx::kSlabEntries) singles &= (1ull << cnt) - 1;
+  const int n_singles = __builtin_popcountll(singles);
+  for (int lane = 0; lane < smx::kSlabEntries; ++lane) {
+    const bool single = (singles >> lane) & 1ull;
+    place[lane] = smx::slab_place(lane, cnt, n_singles, single, __builtin_popcountll(singles & ((1ull << lane) - 1)));
+    taken[lane] = -1;
+  }
+  *lowest = smx::kSlabEntries;
+  *highest = -1;
+  const int n = cnt - n_singles;
+  if (n == 0) return SMX_OK;
+  auto request = [&](int group) {
+    *lowest = std::min(*lowest, group);
+    *highest = std::max(*highest, group + rif - 1);
+  };
+  const int last = smx::last_group(n, rif);
+  request(0);
+  for (int j0 = 0; j0 < n; j0 += 2 * rif) {   // (as stream_batch)
+    request(std::min(j0 + rif, last));
+    request(std::min(j0 + 2 * rif, last));
+    for (int j = j0; j < std::min(j0 + 2 * rif, n); ++j) taken[j] = j;
+  }
+  return SMX_OK;
+}
+
 int smx_measure_backward_fused(int parts, int model, void* stream, const smx_plan_view* plan, float* table, size_t n_rows,
                                const int64_t* idx, const float* q1, const float* q2, const float* score,
                                const float* gscore, float* gq1, float* gq2, size_t B, size_t K, size_t dim,

@@ -20,6 +20,7 @@
 #include "smx_common.h"
 #include "smx_models.h"
 #include "smx_rowupdate.h"
+#include "smx_slab.h"
 #include "smx_wave.h"
 
 namespace smx {
@@ -193,7 +194,7 @@ __device__ __forceinline__ unsigned long long batch_off(const PairBatch& pb, int
   return ((unsigned long long)hi << 32) | lo;
 }
 
-constexpr int kSlabDwords = 64 * 4;  // per wavefront: 64 entries of {address lo, address hi, c0, c1}
+constexpr int kSlabDwords = kSlabEntries * 4;  // per wavefront: 64 entries of {address lo, address hi, c0, c1}
 
 // Orders a wavefront's own LDS writes before its later LDS reads (other lanes' entries).
 __device__ __forceinline__ void slab_fence() {
@@ -246,7 +247,7 @@ template <int MUL, int VEC, int NIT, int RIF> struct RowSet {
   Pack<VEC> e2[RIF][NIT];
 };
 
-// Requests rows g0 .. g0+RIF-1 of the batch; g0 is a multiple of RIF, so the entries exist.
+// Requests rows g0 .. g0+RIF-1 of the batch, g0 a multiple of RIF: the entries exist (last_group).
 template <int MUL, int VEC, int NIT, int RIF, bool ONCE = false>
 __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, const unsigned* slab, int g0, int dim,
                                              int ncol, int lane) {
@@ -268,13 +269,14 @@ __device__ __forceinline__ void request_rows(RowSet<MUL, VEC, NIT, RIF>& rs, con
   }
 }
 
-// Streams the cnt (<= 64) rows of a staged batch through `consume(j, e1, e2)`, j ascending.
+// Streams the first cnt (1 .. 64) rows of a staged batch through `consume(j, e1, e2)`, j ascending.  `slab` is the start of the
+// wavefront's own: every group has to lie in it (last_group).
 template <int MUL, int VEC, int NIT, int RIF, bool ONCE = false, class Consume>
 __device__ __forceinline__ void stream_batch(const unsigned* slab, int cnt, int dim, int ncol, int lane,
                                              Consume&& consume) {
-  static_assert(64 % RIF == 0, "a group of rows must not straddle the end of the slab");
+  static_assert(kSlabEntries % RIF == 0, "a group of rows must not straddle the end of the slab");
   RowSet<MUL, VEC, NIT, RIF> a, b;
-  const int last = ((cnt - 1) / RIF) * RIF;  // first row of the last group
+  const int last = last_group(cnt, RIF);
   request_rows<MUL, VEC, NIT, RIF, ONCE>(a, slab, 0, dim, ncol, lane);
   for (int j0 = 0; j0 < cnt; j0 += 2 * RIF) {
     request_rows<MUL, VEC, NIT, RIF, ONCE>(b, slab, min(j0 + RIF, last), dim, ncol, lane);
@@ -663,11 +665,8 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
     float my_c0, my_c1;
     ModelOps<M>::coef(gscore[mine], score[mine], p, my_c0, my_c1);
     if constexpr (SINGLES == 3) {
-      // the rows to finish to the front, in pair order, then the others: each kind streams without a branch on the other
-      const int first_other = __popcll(singles);
-      const int to = lane >= cnt ? lane
-                                 : ((singles >> lane) & 1ull ? (int)lanes_below_in(singles)
-                                                             : first_other + lane - (int)lanes_below_in(singles));
+      // the rows to finish behind the others, each kind in pair order: each streams without a branch on the other
+      const int to = slab_place(lane, cnt, __popcll(singles), (singles >> lane) & 1ull, (int)lanes_below_in(singles));
       auto moved = [&](unsigned x) { return (unsigned)__builtin_amdgcn_ds_permute(to * 4, (int)x); };
       pb = PairBatch{moved(pb.off_lo), moved(pb.off_hi), moved(pb.row)};
       my_c0 = __uint_as_float(moved(__float_as_uint(my_c0)));
@@ -752,10 +751,10 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
       // Rows that occur once, Adam: the row with its moments, one ahead of the one in work; every turn has the same number
       // of loads and stores, so that no wait is for more than what it needs (after a branch that may have issued some, the
       // wait is for all of them).
-      const int n_rows_here = __popcll(singles);
+      n_stream = cnt - __popcll(singles);   // the rows to finish are n_stream .. cnt - 1
       RowState<MUL, VEC, NIT> sa, sb;
       auto request = [&](RowState<MUL, VEC, NIT>& s, int j) {
-        const unsigned long long off = batch_off(pb, min(j, n_rows_here - 1));
+        const unsigned long long off = batch_off(pb, min(j, cnt - 1));
         load_row<MUL, VEC, NIT>(s.e, table + off, dim, ncol, lane);
         load_row<MUL, VEC, NIT, true>(s.m, A.sink.m + off, dim, ncol, lane);
         load_row<MUL, VEC, NIT, true>(s.v, A.sink.v + off, dim, ncol, lane);
@@ -776,27 +775,22 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
         finish_row<M, VEC, NIT, REG, true, true>(sink, lane, (unsigned)__builtin_amdgcn_readlane((int)pb.row, j), 0, ge1, ge2, s.e,
                                                  s.m, s.v);
       };
-      if (n_rows_here > 0) {
-        request(sa, 0);
-        for (int j = 0; j < n_rows_here; j += 2) {
+      if (n_stream < cnt) {
+        request(sa, n_stream);
+        for (int j = n_stream; j < cnt; j += 2) {
           request(sb, j + 1);
           finish(sa, j);
-          if (j + 1 >= n_rows_here) break;
+          if (j + 1 >= cnt) break;
           request(sa, j + 2);
           finish(sb, j + 1);
         }
       }
-      n_stream = cnt - n_rows_here;
     }
     // lanes past the row end hold a copy of the last column: what they accumulate is never stored
-    auto stream_from = [&]() -> const unsigned* {
-      if constexpr (SINGLES == 3) return slab + 4 * (cnt - n_stream);
-      return slab;
-    };
     if (n_stream > 0)
-    stream_batch<MUL, VEC, NIT, RIF>(stream_from(), n_stream, dim, ncol, lane,
+    stream_batch<MUL, VEC, NIT, RIF>(slab, n_stream, dim, ncol, lane,
                                      [&](int j, const Pack<VEC>(&e1)[NIT], const Pack<VEC>(&e2)[NIT]) {
-      float2 c = slab_coef(stream_from(), j);
+      float2 c = slab_coef(slab, j);
       [[maybe_unused]] const float c_raw = c.x;
       if constexpr (M == mL2)
         c.x = l2_pair_coef<VEC, NIT>(c.x, ncol, lane, [&](int it, int v) { return e1[it].v[v]; },
