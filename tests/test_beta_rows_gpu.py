@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dim", [4, 64, 68, 128, 132, 192, 196, 256, 260, 320, 324, 384, 388, 448, 452, 512])
 @pytest.mark.parametrize("clamped", [True, False])
 def test_row_lengths(dim, clamped):
+    from smore_amd import fused
     rng = np.random.default_rng(seed("beta rows", dim, clamped))
     n, b, k = 300, 5, 67                  # 335 pairs: a third of the touched rows occur once; 67: a remainder per wavefront
     f32 = lambda x: x.astype(np.float32).astype(np.float64)
@@ -26,40 +27,6 @@ def test_row_lengths(dim, clamped):
     idx = rng.integers(0, n, (b, k))
     idx[0, :3] = (7, 8, 9)
     gs = f32(rng.standard_normal((b, k)))
-    # entity 9: lgamma and (x - q) psi(x) of 1,201 are 7,313 and 8,500, and four terms of that size cancel: an ulp of each
-    one_step(raw, qa, qb, idx, gs, clamped, score_terms=4 * 8500.0 * (idx == 9))
-
-
-# Pairs that are a segment of their own, per wavefront of eight and per batch of 64: none, all, all but one, odd and even counts.
-# K = 512: full batches; 520: 64 + 1; 1,024: two full batches; 300: 38 each, the last one 34.  Features on both sides of 256: two
-# rows requested at a time and one.
-@pytest.mark.parametrize("k", [300, 512, 520, 1024])
-@pytest.mark.parametrize("dim", [64, 128, 256, 260, 400])
-def test_rows_in_the_stream_in_every_batch(dim, k):
-    rng = np.random.default_rng(seed("beta rows in the stream", dim, k))
-    b, per_wave = 4, -(-k // 8)
-    hot = 24                               # ids that occur again and again
-    idx, fresh = np.empty((b, k), dtype=np.int64), hot
-    counts = iter(rng.permutation([0, 1, 2, 31, 32, 33, 62, 63, 64] * 16))
-    for q in range(b):
-        idx[q] = np.arange(k) % hot
-        for first in range(0, k, per_wave):
-            for at in range(first, min(first + per_wave, k), 64):
-                cnt = min(64, first + per_wave - at, k - at)
-                n = min(int(next(counts)), cnt)
-                idx[q, at + np.sort(rng.permutation(cnt)[:n])] = fresh + np.arange(n)
-                fresh += n
-    f32 = lambda x: x.astype(np.float32).astype(np.float64)
-    place = rng.permutation(fresh + 50)
-    raw = f32(rng.standard_normal((fresh + 50, 2 * dim)) * 0.5)
-    qa, qb = (f32(np.clip(1 + 0.5 * rng.standard_normal((b, dim)), 0.05, 1e9)) for _ in range(2))
-    one_step(raw, qa, qb, place[idx], f32(rng.standard_normal((b, k))), True)
-
-
-def one_step(raw, qa, qb, idx, gs, clamped, score_terms=None):
-    """Scores, query gradients and the one-call backward with Adam, against the oracle."""
-    from smore_amd import fused
-    n, dim, (b, k) = raw.shape[0], qa.shape[1], idx.shape
     reg = orc.regularizer(raw) if clamped else raw
     rows = orc.gather(reg, idx).reshape(b, k, -1)
     want = orc.score_forward("beta_kl", rows, qa[:, None], qb[:, None], 60.0)
@@ -74,7 +41,8 @@ def one_step(raw, qa, qb, idx, gs, clamped, score_terms=None):
     table, q1, q2, g, ids = dev(raw), dev(qa), dev(qb), dev(gs), torch.tensor(idx, device="cuda")
     params = fused.score_params(60.0, 0.0, regularizer=(1.0, 0.05, 1e9) if clamped else None)
     score = fused.score_forward("beta_kl", table, ids, q1, q2, params)
-    assert_close(score.cpu().numpy(), want, REL_F32, "score", sum_abs=score_terms)
+    # entity 9: lgamma and (x - q) psi(x) of 1,201 are 7,313 and 8,500, and four terms of that size cancel: an ulp of each
+    assert_close(score.cpu().numpy(), want, REL_F32, "score", sum_abs=4 * 8500.0 * (idx == 9))
     gq = fused.score_backward_query("beta_kl", table, ids, q1, q2, score, g, params)
     plan = fused.build_plan(ids, n)
     assert (plan.pair_seg < 0).any() and (plan.pair_seg >= 0).any()
@@ -90,4 +58,4 @@ def one_step(raw, qa, qb, idx, gs, clamped, score_terms=None):
     w = raw.copy()
     orc.adam_rows(w, np.zeros_like(raw), np.zeros_like(raw), uniq, m.cpu().numpy()[uniq].astype(np.float64) / np.float32(0.1), 1e-3, 1)
     # a first step moves a weight by at most the learning rate, known to a few ulps from the moments the device holds
-    assert np.all(np.abs(table.cpu().numpy()[uniq] - w[uniq]) <= 1e-3 * 1e-4 + 2.0 ** -22 * np.abs(w[uniq]))
+    assert np.abs(table.cpu().numpy()[uniq] - w[uniq]).max() <= 1e-3 * 1e-4 + 2.0 ** -23 * np.abs(w[uniq]).max()
