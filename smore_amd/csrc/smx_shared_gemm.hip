@@ -71,14 +71,18 @@ __global__ __launch_bounds__(256) void beta_row_terms_kernel(const float* __rest
   }
 }
 
-// Qk [B]: one wavefront per query
+// Qk [B]: one wavefront per query, in the form of the rows' constants: what the two are off by in the same way cancels
 __global__ __launch_bounds__(256) void beta_query_terms_kernel(const float* __restrict__ q1, const float* __restrict__ q2,
                                                                int B, int dim, float* __restrict__ Qk) {
   const int lane = threadIdx.x & 63;
   const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (b >= B) return;
   float mine = 0.f;
-  for (int d = lane; d < dim; d += 64) mine += ModelOps<mBetaKL>::prep_fwd(q1[(size_t)b * dim + d], q2[(size_t)b * dim + d]).k;
+  for (int d = lane; d < dim; d += 64) {
+    float lb, pa, pb, ps;
+    beta_terms(q1[(size_t)b * dim + d], q2[(size_t)b * dim + d], lb, pa, pb, ps);
+    mine -= lb;
+  }
   const float total = wave_sum_last_f32(mine);
   if (lane == 63) Qk[b] = total;
 }
