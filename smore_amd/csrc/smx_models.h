@@ -326,16 +326,29 @@ template <> struct ModelOps<mRotate> {
 // once when the segment is finished.
 struct QBeta {
   float a, b;  // alpha, beta of the query
-  float k;     // forward: lgG(qa)+lgG(qb)-lgG(sq); query backward: psi(qa)-psi(sq)
+  float k;     // forward: lgG(qa)+lgG(qb)-lgG(sq)+ln C, see beta_logs; query backward: psi(qa)-psi(sq)
   float l;     // forward: (qa + 2.5) ln 2, see beta_arg; query backward: psi(qb)-psi(sq)
   float m;     // forward: (qb + 2.5) ln 2
 };
 
-// One pair's terms by the routines that take any argument; not inlined: rows that need it are rare.
+// One feature of a row in the interval of fast_ok (see beta_arg).
+static __device__ __forceinline__ float beta_pair_fast(float ea, float eb, const QBeta& q) {
+#pragma clang fp contract(off)
+  const BetaArg a = beta_arg<false>(ea), b = beta_arg<false>(eb), s = beta_arg<false>(ea + eb);
+  float v = q.k + beta_logs(a, b, s, q.l, q.m);
+  const float da = ea - q.a, db = eb - q.b;
+  v = __builtin_fmaf(-da, a.rest, v);
+  v = __builtin_fmaf(-db, b.rest, v);
+  return __builtin_fmaf(da + db, s.rest, v);
+}
+// ... of any row, the same bits where the feature is in the interval: which form a feature takes is the feature's own affair, as
+// it is the query's in prep_fwd.  Not inlined: rows that need it are rare.  (The query's coefficients are formed again: as two
+// arguments more they cost the rows of seven floats a lane 17 spilled registers, 584 us instead of 280 for 2 x 400 floats.)
 static __device__ __noinline__ float beta_pair_any(float ea, float eb, float qa, float qb, float k) {
+  if (fast_ok(fminf(ea, eb), ea + eb)) return beta_pair_fast(ea, eb, {qa, qb, k, beta_k(qa), beta_k(qb)});
   float lb, pa, pb, ps;
-  beta_terms(ea, eb, lb, pa, pb, ps);
-  return (k + lb) + (ea - qa) * pa + (eb - qb) * pb + ((qa + qb) - (ea + eb)) * ps;
+  beta_terms_slow(ea, eb, lb, pa, pb, ps);
+  return (k + (lb - kLnBetaConst)) + (ea - qa) * pa + (eb - qb) * pb + ((qa + qb) - (ea + eb)) * ps;
 }
 
 template <> struct ModelOps<mBetaKL> {
@@ -344,28 +357,17 @@ template <> struct ModelOps<mBetaKL> {
   static __device__ __forceinline__ Q prep_fwd(float q1, float q2) {
     const float ka = beta_k(q1), kb = beta_k(q2), sum = q1 + q2;
     float lb, pa, pb, ps;
-    if (fast_ok(fminf(q1, q2), sum)) lb = beta_logs(0.f, beta_arg<false>(q1), beta_arg<false>(q2), beta_arg<false>(sum), ka, kb, beta_k(sum));
-    else beta_terms(q1, q2, lb, pa, pb, ps);
+    if (fast_ok(fminf(q1, q2), sum)) lb = beta_logs(beta_arg<false>(q1), beta_arg<false>(q2), beta_arg<false>(sum), ka, kb);
+    else {
+      beta_terms_slow(q1, q2, lb, pa, pb, ps);
+      lb -= kLnBetaConst;
+    }
     return {q1, q2, -lb, ka, kb};
   }
   static __device__ __forceinline__ Q prep_bwd_q(float q1, float q2) {
     float pa, pb, ps;
     digamma3(q1, q2, pa, pb, ps);
     return {q1, q2, pa - ps, pb - ps, 0.f};
-  }
-  static __device__ __forceinline__ void fwd(float ea, float eb, const Q& q, float& a0, float&) {
-    a0 += beta_pair_any(ea, eb, q.a, q.b, q.k);
-  }
-  // The same for a row of which every feature lies in the interval of fast_ok.
-  static __device__ __forceinline__ void fwd_fast(float ea, float eb, const Q& q, float& a0) {
-#pragma clang fp contract(off)
-    const float sum = ea + eb;
-    const BetaArg a = beta_arg<false>(ea), b = beta_arg<false>(eb), s = beta_arg<false>(sum);
-    float v = beta_logs(q.k, a, b, s, q.l, q.m, (q.l + q.m) - kBetaShift);
-    const float da = ea - q.a, db = eb - q.b;
-    v = __builtin_fmaf(-da, a.rest, v);
-    v = __builtin_fmaf(-db, b.rest, v);
-    a0 += __builtin_fmaf(da + db, s.rest, v);
   }
   static __device__ __forceinline__ void bwd_q_fast(float c0, float e1, float e2, const Q& q, float& g1, float& g2) {
 #pragma clang fp contract(off)
@@ -459,13 +461,19 @@ __device__ __forceinline__ float beta_row_sum(const BetaClamp& clamp, GetA&& ga,
   for (int it = 0; it < NIT; ++it) {
     QBeta q[VEC];
     get_q(it, q);
-    float a0 = 0.f, a1 = 0.f;
+    float a0;
     if (fast) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::fwd_fast(row.a[it][v], row.b[it][v], q[v], a0);
+      for (int v = 0; v < VEC; ++v) {
+        const float x = beta_pair_fast(row.a[it][v], row.b[it][v], q[v]);
+        a0 = v == 0 ? x : a0 + x;
+      }
     } else {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) ModelOps<mBetaKL>::fwd(row.a[it][v], row.b[it][v], q[v], a0, a1);
+      for (int v = 0; v < VEC; ++v) {
+        const float x = beta_pair_any(row.a[it][v], row.b[it][v], q[v].a, q[v].b, q[v].k);
+        a0 = v == 0 ? x : a0 + x;
+      }
     }
     mine += lane + 64 * it < ncol ? a0 : 0.f;
   }

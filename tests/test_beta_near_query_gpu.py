@@ -4,6 +4,7 @@ feature."""
 import numpy as np
 import pytest
 import torch
+from scipy.special import gammaln, psi
 
 from tests.util import seed
 
@@ -12,6 +13,15 @@ pytestmark = pytest.mark.gpu
 
 def _dev(x):
     return torch.tensor(x, dtype=torch.float32, device="cuda")
+
+
+def _rms(x):
+    return float(np.sqrt(np.mean(np.square(x))))
+
+
+def _kl(ea, eb, qa, qb):
+    log_beta = lambda a, b: gammaln(a) + gammaln(b) - gammaln(a + b)
+    return log_beta(qa, qb) - log_beta(ea, eb) + (ea - qa) * psi(ea) + (eb - qb) * psi(eb) + (qa + qb - ea - eb) * psi(ea + eb)
 
 
 def _draw(rng, low, high, shape):
@@ -32,3 +42,57 @@ def test_shared_list_constants_of_row_and_query_are_of_one_form():
     table = _dev(np.concatenate([qa, qb], 1))
     score = fused.score_forward_shared("beta_kl", table, torch.arange(n, device="cuda"), _dev(qa), _dev(qb), fused.score_params(0.0))
     assert abs(score.diagonal().double().mean().item()) <= 1.0e-4
+
+
+def _mixed(rng, shape):
+    """Features in the interval of the fast forms, below it, beyond it and at its ends, the sum of a pair included."""
+    x = _draw(rng, 0.05, 60.0, shape)
+    x[..., ::7] = _draw(rng, 0.001, 0.019, x[..., ::7].shape)
+    x[..., 3::11] = _draw(rng, 1001.0, 5000.0, x[..., 3::11].shape)
+    x[0, 0], x[1, 1], x[2, 2], x[3, 3] = np.float32(0.02), 1000.0, 999.5, np.float32(0.0199)
+    return x
+
+
+# every number of floats per lane, in columns of one and of four, and rows that are not
+WIDTHS = [4, 33, 64, 200, 256, 260, 400, 452, 512, 516, 1000]
+
+
+@pytest.mark.parametrize("inside", [True, False])
+@pytest.mark.parametrize("dim", WIDTHS)
+def test_a_row_is_at_no_distance_from_itself(dim, inside):
+    from smore_amd import fused
+    from smore_amd.evaluation import candidate_ranks
+    rng = np.random.default_rng(seed("itself", dim, inside))
+    n, k = 40, 140
+    qa, qb = (_draw(rng, 0.05, 60.0, (n, dim)) if inside else _mixed(rng, (n, dim)) for _ in range(2))
+    table, q1, q2 = _dev(np.concatenate([qa, qb], 1)), _dev(qa), _dev(qb)
+    idx = torch.tensor(rng.integers(0, n, (n, k)), device="cuda")
+    own = torch.tensor(rng.integers(0, k, n), device="cuda")
+    at = torch.arange(n, device="cuda")
+    idx[at, own] = at
+    params = fused.score_params(60.0)
+    score = fused.score_forward("beta_kl", table, idx, q1, q2, params)
+    logit = candidate_ranks("beta_kl", table, q1, q2, params, idx, [1] * n)[0]
+    assert (score[at, own] == 60.0).all() and (logit[at, own] == 60.0).all()
+    assert torch.isfinite(score).all()
+
+
+# widths with one and two columns of four a lane, in single columns, unaligned
+@pytest.mark.parametrize("low,high", [(None, None), (0.05, 5.0), (1.0, 5.0), (1.0, 20.0), (20.0, 60.0), (60.0, 480.0)])
+@pytest.mark.parametrize("near", [0.01, 0.1])
+@pytest.mark.parametrize("dim", [36, 250, 400, 512])
+def test_scores_near_the_query_round_no_worse_than_the_general_forms(dim, near, low, high):
+    """The operators sum a row's features in another order: a tenth for that and for the spread of two samples of 2,048."""
+    from smore_amd import fused
+    from smore_amd.torchext import ext_ops
+    rng = np.random.default_rng(seed("near", dim, near, low))
+    b, k = 256, 8
+    qa, qb = (_draw(rng, low, high, (b, dim)) for _ in range(2))
+    ea, eb = ((np.repeat(q, k, 0) * rng.uniform(1 - near, 1 + near, (b * k, dim))).astype(np.float32).astype(np.float64) for q in (qa, qb))
+    want = _kl(ea, eb, np.repeat(qa, k, 0), np.repeat(qb, k, 0)).sum(1).reshape(b, k)
+    rows, q1, q2 = _dev(np.concatenate([ea, eb], 1)), _dev(qa), _dev(qb)
+    idx = torch.arange(b * k, device="cuda").reshape(b, k)
+    got = -fused.score_forward("beta_kl", rows, idx, q1, q2, fused.score_params(0.0)).cpu().numpy().astype(np.float64)
+    with torch.no_grad():
+        general = ext_ops.beta_kl(rows.view(b, k, -1), ext_ops.BetaDist(q1[:, None], q2[:, None])).cpu().numpy().astype(np.float64)
+    assert _rms(got - want) <= 1.1 * _rms(general - want)
