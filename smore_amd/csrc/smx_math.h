@@ -299,11 +299,19 @@ __device__ __forceinline__ void digamma3(float a, float b, float& pa, float& pb,
   }
 }
 
-static __device__ __noinline__ SlowTerms digamma3_any(float a, float b) {
+// psi(a) - psi(a + b) and psi(b) - psi(a + b), x and y.  In the interval of fast_ok the form of beta_psi_diff, for rows and queries
+// alike: a row that equals its query does not pull at it.
+__device__ __forceinline__ SlowTerms beta_psi_diffs(float a, float b) {
+  const float sum = a + b;
+  if (fast_ok(fminf(a, b), sum)) {
+    const BetaArg s = beta_arg<true>(sum);
+    return SlowTerms{-beta_psi_diff(beta_arg<true>(a), s), -beta_psi_diff(beta_arg<true>(b), s), 0.f, 0.f};
+  }
   float pa, pb, ps;
-  digamma3(a, b, pa, pb, ps);
-  return SlowTerms{pa, pb, ps, 0.f};
+  digamma3_slow(a, b, pa, pb, ps);
+  return SlowTerms{pa - ps, pb - ps, 0.f, 0.f};
 }
+static __device__ __noinline__ SlowTerms beta_psi_diffs_any(float a, float b) { return beta_psi_diffs(a, b); }
 
 static __device__ __noinline__ void trigamma3_slow(float a, float b, float& ta, float& tb, float& ts) {
   ta = trigamma(a);

@@ -365,9 +365,8 @@ template <> struct ModelOps<mBetaKL> {
     return {q1, q2, -lb, ka, kb};
   }
   static __device__ __forceinline__ Q prep_bwd_q(float q1, float q2) {
-    float pa, pb, ps;
-    digamma3(q1, q2, pa, pb, ps);
-    return {q1, q2, pa - ps, pb - ps, 0.f};
+    const SlowTerms t = beta_psi_diffs(q1, q2);
+    return {q1, q2, t.x, t.y, 0.f};
   }
   static __device__ __forceinline__ void bwd_q_fast(float c0, float e1, float e2, const Q& q, float& g1, float& g2) {
 #pragma clang fp contract(off)
@@ -405,9 +404,9 @@ template <> struct ModelOps<mBetaKL> {
     g2 = __builtin_fmaf(tb, g2, -common);
   }
   static __device__ __forceinline__ void bwd_q(float c0, float, float e1, float e2, const Q& q, float& g1, float& g2) {
-    const SlowTerms t = digamma3_any(e1, e2);
-    g1 += c0 * (q.k - t.x + t.z);
-    g2 += c0 * (q.l - t.y + t.z);
+    const SlowTerms t = beta_psi_diffs_any(e1, e2);
+    g1 = __builtin_fmaf(c0, q.k - t.x, g1);
+    g2 = __builtin_fmaf(c0, q.l - t.y, g2);
   }
 };
 

@@ -329,8 +329,9 @@ __global__ __launch_bounds__(8 * kTileN) void shared_gemm_kernel(GemmArgs A) {
       if (m < M && n < N) {
         float v = sum[r];
         if constexpr (BETA) {
-          const QBeta q = ModelOps<mBetaKL>::prep_bwd_q(A.q1[(size_t)m * dim + d], A.q2[(size_t)m * dim + d]);
-          v = -(v + (n < dim ? q.k : q.l) * g);
+          float pa, pb, ps;   // (the rows' digammas are of this form)
+          digamma3(A.q1[(size_t)m * dim + d], A.q2[(size_t)m * dim + d], pa, pb, ps);
+          v = -(v + ((n < dim ? pa : pb) - ps) * g);
         }
         (n < dim ? A.out1 : A.out2)[(size_t)m * dim + d] = v;
       }

@@ -96,3 +96,46 @@ def test_scores_near_the_query_round_no_worse_than_the_general_forms(dim, near, 
     with torch.no_grad():
         general = ext_ops.beta_kl(rows.view(b, k, -1), ext_ops.BetaDist(q1[:, None], q2[:, None])).cpu().numpy().astype(np.float64)
     assert _rms(got - want) <= 1.1 * _rms(general - want)
+
+
+@pytest.mark.parametrize("inside", [True, False])
+@pytest.mark.parametrize("dim", WIDTHS)
+def test_a_row_does_not_pull_at_a_query_that_equals_it(dim, inside):
+    """One pair a query: the query gradient is that pair's, and the row's own is 0 in every form of the backward."""
+    from smore_amd import fused
+    rng = np.random.default_rng(seed("pull", dim, inside))
+    n = 40
+    qa, qb = (_draw(rng, 0.05, 60.0, (n, dim)) if inside else _mixed(rng, (n, dim)) for _ in range(2))
+    table, q1, q2 = _dev(np.concatenate([qa, qb], 1)), _dev(qa), _dev(qb)
+    idx = torch.arange(n, device="cuda").reshape(n, 1)
+    gs, params = _dev(rng.standard_normal((n, 1))), fused.score_params(60.0)
+    score = fused.score_forward("beta_kl", table, idx, q1, q2, params)
+    for g in fused.score_backward_query("beta_kl", table, idx, q1, q2, score, gs, params):
+        assert not g.any()
+    plan = fused.build_plan(idx, n)
+    m, v, before = torch.zeros_like(table), torch.zeros_like(table), table.clone()
+    for g in fused.score_backward_fused("beta_kl", plan, table, idx, q1, q2, score, gs, params, m=m, v=v, adam=fused.adam_params(1e-3, 1)):
+        assert not g.any()
+    assert not m.any() and not v.any() and torch.equal(table, before)
+
+
+@pytest.mark.parametrize("outside", [0.004, 1500.0])
+@pytest.mark.parametrize("dim", WIDTHS)
+def test_a_feature_outside_the_interval_changes_no_other(dim, outside):
+    """The form is chosen by the feature, whatever path its row takes."""
+    from smore_amd import fused
+    rng = np.random.default_rng(seed("outside", dim, outside))
+    n = 40
+    qa, qb = (_draw(rng, 0.05, 60.0, (n, dim)) for _ in range(2))
+    rows = np.concatenate([_draw(rng, None, None, (n, dim)), _draw(rng, 1.0, 60.0, (n, dim))], 1)
+    idx = torch.arange(n, device="cuda").reshape(n, 1)
+    q1, q2, gs, params = _dev(qa), _dev(qb), _dev(rng.standard_normal((n, 1))), fused.score_params(60.0)
+    score = torch.zeros_like(gs)
+    at = rng.integers(0, dim, n)
+    moved = rows.copy()
+    moved[np.arange(n), at] = outside
+    plain, other = (fused.score_backward_query("beta_kl", _dev(t), idx, q1, q2, score, gs, params) for t in (rows, moved))
+    same = torch.ones(n, dim, dtype=torch.bool, device="cuda")
+    same[torch.arange(n), torch.tensor(at)] = False
+    for a, b in zip(plain, other):
+        assert torch.equal(a[same], b[same]) and not torch.equal(a, b)
