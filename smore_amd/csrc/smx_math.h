@@ -270,12 +270,15 @@ __device__ __forceinline__ float beta_logs(const BetaArg& a, const BetaArg& b, c
   return __builtin_fmaf(-b.r, beta_stirling(b), v);
 }
 // psi'(x) out of the same parts (POLE): 1/x^2 + (2d + 1)/d^2 with d = (x + 1) (x + 2), and psi'(y) = 1/y + 1/(2y^2) plus a
-// polynomial fitted as V is (largest error 5.8e-9).  No special function more.
+// polynomial fitted as V is (largest error 5.8e-9).  No special function more.  The sum goes from the small terms to 1/y, nearly all
+// of it for large x, and 1/x^2, nearly all of it for small x: one rounding each.  (With 1/y first, the gradients of rows at 20 to 60
+// had a tenth more error than with the six-step form.)
 __device__ __forceinline__ float beta_trigamma(const BetaArg& s) {
 #pragma clang fp contract(off)
   const float tail = __builtin_fmaf(s.z, __builtin_fmaf(s.z, 8.307060779e-6f, vector_const(-1.356947031e-4f)), 6.172571429e-3f);
-  const float asym = __builtin_fmaf(s.r * s.z, tail, __builtin_fmaf(s.z, 5.55555556e-2f, s.r * 3.33333343e-1f));
-  return __builtin_fmaf(s.rx, s.rx, __builtin_fmaf(__builtin_fmaf(s.d, 2.f, 1.f), s.rd * s.rd, asym));
+  float v = __builtin_fmaf(s.r * s.z, tail, s.z * 5.55555556e-2f);
+  v = __builtin_fmaf(__builtin_fmaf(s.d, 2.f, 1.f), s.rd * s.rd, v);
+  return __builtin_fmaf(s.rx, s.rx, __builtin_fmaf(s.r, 3.33333343e-1f, v));
 }
 // psi(s) - psi(x)
 __device__ __forceinline__ float beta_psi_diff(const BetaArg& x, const BetaArg& s) {
