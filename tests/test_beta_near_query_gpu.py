@@ -162,3 +162,21 @@ def test_gradients_of_rows_round_no_worse_than_the_general_forms(low, high):
     want = 0.25 * (polygamma(1, ea) - polygamma(1, ea + eb))
     error = lambda g: _rms((g.detach().cpu().numpy().astype(np.float64).reshape(n, -1)[:, :dim] / want - 1))
     assert error(merged) <= error(rows.grad)
+
+
+def test_ranking_knows_the_digamma_to_an_ulp():
+    """Features of 1/31 to 1/17, where psi(x) - psi(x + 1) = -1/x is 17 to 31 and an ulp 2^-19: 1/x and the sum are off by 0.58 and 0.29
+    of one, the difference by 0.29 more, the logit's own roundings by 0.2 each.  The logit is that difference times about
+    -40, plus parts in 64 bits."""
+    from smore_amd import fused
+    from tests.test_rank_numerics_gpu import _all_ids, _keys
+    rng = np.random.default_rng(seed("digamma"))
+    n, dim = 2000, 4
+    ea, eb = np.full((n, dim), 1.0), np.full((n, dim), 1.0)
+    ea[:, 0] = _draw(rng, 1 / 31, 1 / 17, n)
+    qa, qb = np.ones((1, dim)), np.ones((1, dim))
+    qa[0, 0] = 40.0
+    want = -_kl(ea, eb, qa, qb).sum(1)
+    got = _keys("beta_kl", _dev(np.concatenate([ea, eb], 1)), _dev(qa), _dev(qb), fused.score_params(0.0), _all_ids(1, n))[0]
+    error = (got.cpu().numpy().astype(np.float64)[0] - want) / (ea[:, 0] - 40.0)
+    assert _rms(error) <= 2.0 ** -19
