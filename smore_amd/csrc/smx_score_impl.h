@@ -108,12 +108,14 @@ __device__ __forceinline__ void stage_query(float* lds, const float* __restrict_
   __syncthreads();
 }
 
-// BetaE's per-query values in LDS, one stretch of dim floats per field, evaluated once per workgroup.  FWD: a, b, k, l, m of
-// QBeta; query backward: k, l and, where rows are finished in the stream (ROWS), a, b.
-__host__ __device__ constexpr int query_fields(int model, bool fwd, bool rows = false) {
-  return model != mBetaKL ? model_nq(model) : (fwd ? 5 : (rows ? 4 : 2));
+// BetaE's per-query values in LDS, one stretch of dim floats per field, evaluated once per workgroup.  FWD: a, b, k of QBeta, and
+// l, m where a lane reads columns of four; a lane that takes single floats forms them again, two multiply-adds in the place of two
+// reads with their addresses and a wait (2 x 400 floats, 512 x 512 pairs: 291 -> 286 us).  Query backward: k, l and, where rows are
+// finished in the stream (ROWS), a, b.
+__host__ __device__ constexpr int query_fields(int model, int vec, bool fwd, bool rows = false) {
+  return model != mBetaKL ? model_nq(model) : (fwd ? (vec == 1 ? 3 : 5) : (rows ? 4 : 2));
 }
-template <bool FWD, bool ROWS = false>
+template <int VEC, bool FWD, bool ROWS = false>
 __device__ __forceinline__ void stage_beta_query(float* lds, const float* __restrict__ q1, const float* __restrict__ q2,
                                                  size_t b, int dim) {
   for (int d = threadIdx.x; d < dim; d += blockDim.x) {
@@ -123,8 +125,10 @@ __device__ __forceinline__ void stage_beta_query(float* lds, const float* __rest
       lds[d] = q.a;
       lds[dim + d] = q.b;
       lds[2 * dim + d] = q.k;
-      lds[3 * dim + d] = q.l;
-      lds[4 * dim + d] = q.m;
+      if constexpr (VEC != 1) {
+        lds[3 * dim + d] = q.l;
+        lds[4 * dim + d] = q.m;
+      }
     } else {
       lds[d] = q.k;
       lds[dim + d] = q.l;
@@ -153,7 +157,11 @@ template <int VEC, bool FWD, bool ROWS = false>
 __device__ __forceinline__ void beta_query(const float* lds, int dim, int col, QBeta (&q)[VEC]) {
   float f[5][VEC];
 #pragma unroll
-  for (int i = 0; i < query_fields(mBetaKL, FWD, ROWS); ++i) lds_pack<VEC>(lds + i * dim, col, f[i]);
+  for (int i = 0; i < query_fields(mBetaKL, VEC, FWD, ROWS); ++i) lds_pack<VEC>(lds + i * dim, col, f[i]);
+  if constexpr (FWD && VEC == 1) {
+    f[3][0] = beta_k(f[0][0]);
+    f[4][0] = beta_k(f[1][0]);
+  }
 #pragma unroll
   for (int v = 0; v < VEC; ++v)
     q[v] = FWD ? QBeta{f[0][v], f[1][v], f[2][v], f[3][v], f[4][v]}
@@ -365,7 +373,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
     pb = load_pair_batch(idx, (A.ids_shared ? (size_t)0 : (size_t)(b / A.U) * K) + kw0, cnt, lane, row_len, n_rows, bad);
 
   // LDS: query | per-wavefront pair slabs | code stage (per wavefront; one for the tile with DEDUP) | DEDUP tables
-  constexpr int QF = query_fields(M, true);
+  constexpr int QF = query_fields(M, VEC, true);
   unsigned* slab = reinterpret_cast<unsigned*>(lds + QF * dim) + wave * kSlabDwords;
   constexpr int kStaged = DEDUP ? 256 : kStagePairs;  // pairs whose code bytes a stage holds (DEDUP: tile_k, at most that)
   unsigned char* stage_base = reinterpret_cast<unsigned char*>(lds + QF * dim + 4 * kSlabDwords);
@@ -387,7 +395,7 @@ __global__ __launch_bounds__(256, arithmetic_waves(M, VEC * NIT, true)) void sco
   // (either ends with a barrier: the tables are cleared)
   [[maybe_unused]] typename ModelOps<M>::Q q[NIT][VEC];
   if constexpr (M == mBetaKL) {
-    stage_beta_query<true>(lds, q1, q2, b, dim);
+    stage_beta_query<VEC, true>(lds, q1, q2, b, dim);
   } else {
     stage_query<M>(lds, q1, q2, b, dim);
     load_query_regs<M, VEC, NIT, true>(lds, dim, ncol, lane, q);
@@ -594,7 +602,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
   const ScoreParams p = A.p;
   constexpr int MUL = model_mul(M);
   constexpr int NQ = model_nq(M);
-  constexpr int QF = query_fields(M, false, SINGLES == 3);
+  constexpr int QF = query_fields(M, VEC, false, SINGLES == 3);
   extern __shared__ float lds[];
   // Queries are taken last to first: the forward walks them first to last, and what it touched last -- the sign
   // codes it wrote, the rows it read -- is what the memory-side cache still holds when this kernel starts
@@ -608,7 +616,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
 
   [[maybe_unused]] typename ModelOps<M>::Q q[NIT][VEC];
   if constexpr (M == mBetaKL) {
-    stage_beta_query<false, SINGLES == 3>(lds, q1, q2, b, dim);
+    stage_beta_query<VEC, false, SINGLES == 3>(lds, q1, q2, b, dim);
   } else {
     stage_query<M>(lds, q1, q2, b, dim);
     load_query_regs<M, VEC, NIT, false>(lds, dim, ncol, lane, q);
@@ -991,7 +999,7 @@ int launch_forward_reg(hipStream_t st, const ScoreArgs& A) {
   const size_t B = (size_t)A.B, K = (size_t)A.K;
   const int tile_k = forward_tile(B, K, 4 * RIF);
   const int tiles = (int)((K + tile_k - 1) / tile_k);
-  const size_t lds = ((size_t)query_fields(M, true) * A.ncol * VEC + 4 * kSlabDwords) * sizeof(float);
+  const size_t lds = ((size_t)query_fields(M, VEC, true) * A.ncol * VEC + 4 * kSlabDwords) * sizeof(float);
   // (not the dense layout, whose rows are all different, nor a list of ids shared by the batch: a sampler's K negatives hardly
   // ever repeat)
   const bool dedup = A.idx != nullptr && !A.ids_shared && tile_k >= distinct_from(M);
@@ -1061,7 +1069,7 @@ int launch_backward_query_reg(hipStream_t st, const ScoreArgs& A) {
   }
   if constexpr (M == mBetaKL && VEC == 4 && NIT <= 2 && NW == 8) {
     if (A.pair_seg && A.stream_rows) {
-      const size_t fields = query_fields(M, false, true) - model_nq(M);
+      const size_t fields = query_fields(M, VEC, false, true) - model_nq(M);
       hipLaunchKernelGGL((score_backward_query_kernel<M, VEC, NIT, RIF, NW, REG, 3>), dim3((unsigned)A.B), dim3(NW * 64),
                          lds + fields * A.ncol * VEC * sizeof(float), st, A);
       return check_launch("score backward (query, rows in the stream)");
