@@ -111,7 +111,7 @@ __device__ __forceinline__ void stage_query(float* lds, const float* __restrict_
 // BetaE's per-query values in LDS, one stretch of dim floats per field, evaluated once per workgroup.  FWD: a, b, k of QBeta, and
 // l, m where a lane reads columns of four; a lane that takes single floats forms them again, two multiply-adds in the place of two
 // reads with their addresses and a wait (2 x 400 floats, 512 x 512 pairs: 291 -> 286 us).  Query backward: k, l and, where rows are
-// finished in the stream (ROWS), a, b.
+// finished (ROWS), a, b.
 __host__ __device__ constexpr int query_fields(int model, int vec, bool fwd, bool rows = false) {
   return model != mBetaKL ? model_nq(model) : (fwd ? (vec == 1 ? 3 : 5) : (rows ? 4 : 2));
 }
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
 
   [[maybe_unused]] typename ModelOps<M>::Q q[NIT][VEC];
   if constexpr (M == mBetaKL) {
-    stage_beta_query<VEC, false, SINGLES == 3>(lds, q1, q2, b, dim);
+    stage_beta_query<VEC, false, SINGLES != 0>(lds, q1, q2, b, dim);
   } else {
     stage_query<M>(lds, q1, q2, b, dim);
     load_query_regs<M, VEC, NIT, false>(lds, dim, ncol, lane, q);
@@ -637,13 +637,20 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
   unsigned char* stage =
       reinterpret_cast<unsigned char*>(lds + (NW * NQ + QF) * dim + NW * kSlabDwords) + wave * (kStagePairs * NIT * 64);
 
-  // the query's feature for the rows finished here
-  auto query_at = [&](int it, int v) {
+  // the query's features of a column group for the rows finished here; BetaE's stand behind k and l (SINGLES 1 and 2: where the
+  // partial sums go once every wavefront is done with them).  Fetched from memory for each row instead: 4096 x 128 pairs of 2 x 400
+  // floats 1457 us against 1450 with merged rows, 2341 against 2330 with Adam and v per row.
+  auto query_at = [&](int it, typename ModelOps<M>::Q(&to)[VEC]) {
     if constexpr (M == mBetaKL) {
-      const int d = min(lane + 64 * it, ncol - 1) * VEC + v;
-      return QBeta{q1[(size_t)b * dim + d], q2[(size_t)b * dim + d], 0.f, 0.f, 0.f};   // (LDS holds k and l)
+      float fa[VEC], fb[VEC];
+      const int col = min(lane + 64 * it, ncol - 1);
+      lds_pack<VEC>(lds + 2 * dim, col, fa);
+      lds_pack<VEC>(lds + 3 * dim, col, fb);
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) to[v] = QBeta{fa[v], fb[v], 0.f, 0.f, 0.f};
     } else {
-      return q[it][v];
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) to[v] = q[it][v];
     }
   };
   // this wavefront's share of the query's negatives: a contiguous range, walked in batches of 64
@@ -846,7 +853,9 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
           RowRegs<MUL, VEC, NIT> w, none;
           float ge1[NIT][VEC], ge2[NIT][VEC];
 #pragma unroll
-          for (int it = 0; it < NIT; ++it)
+          for (int it = 0; it < NIT; ++it) {
+            typename ModelOps<M>::Q qa[VEC];
+            query_at(it, qa);
 #pragma unroll
             for (int v = 0; v < VEC; ++v) {
               w.h[0][it].v[v] = e1[it].v[v];
@@ -854,8 +863,9 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
               ge1[it][v] = ge2[it][v] = 0.f;
               const float x1 = REG ? reg_apply(e1[it].v[v], p) : e1[it].v[v];
               const float x2 = MUL == 2 ? (REG ? reg_apply(e2[it].v[v], p) : e2[it].v[v]) : 0.f;
-              ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, query_at(it, v), ge1[it][v], ge2[it][v]);
+              ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, qa[v], ge1[it][v], ge2[it][v]);
             }
+          }
           const int seg = __builtin_amdgcn_readlane(my_ps, j) & 0x7fffffff;
           const unsigned row = (unsigned)__builtin_amdgcn_readlane((int)pb.row, j);
           finish_row<M, VEC, NIT, REG, false>(A.sink, lane, row, seg, ge1, ge2, w, none, none);
@@ -900,15 +910,18 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
             const unsigned row = (unsigned)__builtin_amdgcn_readlane((int)pb.row, j);
             float ge1[NIT][VEC], ge2[NIT][VEC];
 #pragma unroll
-            for (int it = 0; it < NIT; ++it)
+            for (int it = 0; it < NIT; ++it) {
+              typename ModelOps<M>::Q qa[VEC];
+              query_at(it, qa);
 #pragma unroll
               for (int v = 0; v < VEC; ++v) {
                 ge1[it][v] = ge2[it][v] = 0.f;
                 const float x1 = REG ? reg_apply(e[s].h[0][it].v[v], p) : e[s].h[0][it].v[v];
                 const float x2 =
                     MUL == 2 ? (REG ? reg_apply(e[s].h[MUL - 1][it].v[v], p) : e[s].h[MUL - 1][it].v[v]) : 0.f;
-                ModelOps<M>::bwd_e(c0, c1, x1, x2, query_at(it, v), ge1[it][v], ge2[it][v]);
+                ModelOps<M>::bwd_e(c0, c1, x1, x2, qa[v], ge1[it][v], ge2[it][v]);
               }
+            }
             finish_row<M, VEC, NIT, REG, SINGLES == 2>(A.sink, lane, row, seg, ge1, ge2, e[s], m0[s], v0[s]);
           }
         }
@@ -925,6 +938,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
 
   // wavefront partials -> LDS -> fixed-order sum over wavefronts
   float* part = lds + QF * dim;  // [NW][NQ][dim]
+  if constexpr (M == mBetaKL && (SINGLES == 1 || SINGLES == 2)) __syncthreads();   // (query_at)
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = lane + 64 * it;

@@ -69,3 +69,40 @@ def one_step(raw, qa, qb, idx, gs):
     orc.adam_rows(w, np.zeros_like(raw), np.zeros_like(raw), uniq, m.cpu().numpy()[uniq].astype(np.float64) / np.float32(0.1), 1e-3, 1)
     # a first step moves a weight by at most the learning rate, known to a few ulps from the moments the device holds
     assert np.all(np.abs(table.cpu().numpy()[uniq] - w[uniq]) <= 1e-3 * 1e-4 + 2.0 ** -22 * np.abs(w[uniq]))
+
+
+# queries of more than 4 MiB: rows of one pair are finished by the query-gradient kernel whatever the optimizer
+@pytest.mark.parametrize("kind", ["merged", "squeeze", "adam and merged"])
+@pytest.mark.parametrize("dim,b", [(64, 8300), (260, 2100), (516, 1100), (33, 16000)])
+def test_rows_finished_outside_the_stream(dim, b, kind):
+    """The one call against its two halves: query gradients, and the entity pass's rows."""
+    from smore_amd import fused
+    rng = np.random.default_rng(seed("outside the stream", dim, kind))
+    k = 70
+    n = b * k // 2
+    table = torch.tensor(rng.standard_normal((n, 2 * dim)) * 0.5, dtype=torch.float32, device="cuda")
+    q1, q2 = (torch.tensor(np.clip(1 + 0.5 * rng.standard_normal((b, dim)), 0.05, None), dtype=torch.float32, device="cuda") for _ in range(2))
+    ids = torch.tensor(rng.integers(0, n, (b, k)), device="cuda")
+    g = torch.tensor(rng.standard_normal((b, k)), dtype=torch.float32, device="cuda")
+    params = fused.score_params(60.0, 0.0, regularizer=(1.0, 0.05, 1e9))
+    score = fused.score_forward("beta_kl", table, ids, q1, q2, params)
+    plan = fused.build_plan(ids, n)
+    want_q = fused.score_backward_query("beta_kl", table, ids, q1, q2, score, g, params)
+    want = torch.empty(plan.uniq.numel(), 2 * dim, device="cuda")
+    fused.score_backward_entity("beta_kl", plan, table, q1, q2, score, g, params, merged=want)
+    merged = None if kind == "squeeze" else torch.empty_like(want)
+    state = {}
+    if kind != "merged":
+        squeeze = kind == "squeeze"
+        state = dict(m=torch.zeros_like(table), v=torch.zeros(n, 1, device="cuda") if squeeze else torch.zeros_like(table),
+                     adam=fused.adam_params(1e-3, 1, squeeze=squeeze))
+    got_q = fused.score_backward_fused("beta_kl", plan, table, ids, q1, q2, score, g, params, merged=merged, **state)
+    uniq = plan.uniq[:int(plan.n_uniq)]
+    want = want[:uniq.numel()]
+    for a, w in zip(got_q, want_q):
+        # the wavefronts' sums may be of other lengths: an ulp of the terms' magnitudes
+        assert_close(a.cpu().numpy(), w.cpu().numpy(), REL_F32, "query gradient", sum_abs=g.abs().sum(1, keepdim=True).cpu().numpy() * np.ones(dim))
+    if merged is not None:
+        assert_close(merged[:uniq.numel()].cpu().numpy(), want.cpu().numpy(), REL_F32, "merged rows")
+    if state:
+        assert_close(state["m"][uniq].cpu().numpy(), 0.1 * want.cpu().numpy(), REL_F32, "first moments")
