@@ -1134,7 +1134,7 @@ int launch_score(hipStream_t st, const ScoreArgs& A, bool forward) {
 // rows are finished as well: that is bound by memory.
 inline int beta_singles(int dim, int nit4) {
   const int n = (dim + 63) / 64;
-  return n <= 7 && n < 4 * nit4 && n != 4 ? n : 0;
+  return n <= 7 && n < 4 * nit4 ? n : 0;   // (never four: rows of 193 to 256 floats fill their columns of four)
 }
 int beta_singles_dispatch(hipStream_t st, const ScoreArgs& A, int nit, bool forward);   // smx_score_inst_betakl_singles.hip
 template <int NIT>
