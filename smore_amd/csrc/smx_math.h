@@ -222,6 +222,7 @@ struct BetaArg {
   float d, rd;     // D(x) and its reciprocal; with POLE: (x + 1) (x + 2) and its reciprocal
   float rx;        // POLE: 1/x
   float rest;      // R(x)
+  float quot, u;   // not POLE: D'(x)/D(x) and the rest of R(x) without it
 };
 // POLE: 1/x on its own, D'/D = 1/x + (2x + 3) / ((x + 1) (x + 2)); one special function more, and half the error of psi
 // below 5, where the pole is most of it.
@@ -239,13 +240,17 @@ __device__ __forceinline__ BetaArg beta_arg(float x) {
     s.rd = f_rcp(s.d);
     s.rx = f_rcp(x);
     s.rest = __builtin_fmaf(__builtin_fmaf(x, 2.f, vector_const(3.f)), s.rd, u) + s.rx;
+    s.quot = 0.f;
   } else {
     const float t = __builtin_fmaf(x, x, x + x);
     s.d = t * (x + 1.f);
     s.rd = f_rcp(s.d);
     s.rx = 0.f;
-    s.rest = __builtin_fmaf(__builtin_fmaf(t, vector_const(3.f), 2.f), s.rd, u);
+    const float num = __builtin_fmaf(t, vector_const(3.f), 2.f);
+    s.rest = __builtin_fmaf(num, s.rd, u);
+    s.quot = num * s.rd;
   }
+  s.u = u;
   return s;
 }
 __device__ __forceinline__ float beta_stirling(const BetaArg& s) {   // S(x) / r
