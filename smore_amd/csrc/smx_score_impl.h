@@ -637,22 +637,18 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
   unsigned char* stage =
       reinterpret_cast<unsigned char*>(lds + (NW * NQ + QF) * dim + NW * kSlabDwords) + wave * (kStagePairs * NIT * 64);
 
-  // the query's features of a column group for the rows finished here; BetaE's stand behind k and l (SINGLES 1 and 2: where the
+  // BetaE: the query's features of a column group for the rows finished here.  They stand behind k and l (SINGLES 1 and 2: where the
   // partial sums go once every wavefront is done with them).  Fetched from memory for each row instead: 4096 x 128 pairs of 2 x 400
   // floats 1457 us against 1450 with merged rows, 2341 against 2330 with Adam and v per row.
-  auto query_at = [&](int it, typename ModelOps<M>::Q(&to)[VEC]) {
-    if constexpr (M == mBetaKL) {
-      float fa[VEC], fb[VEC];
-      const int col = min(lane + 64 * it, ncol - 1);
-      lds_pack<VEC>(lds + 2 * dim, col, fa);
-      lds_pack<VEC>(lds + 3 * dim, col, fb);
+  [[maybe_unused]] auto query_features = [&](int it, QBeta (&to)[VEC]) {
+    float fa[VEC], fb[VEC];
+    const int col = min(lane + 64 * it, ncol - 1);
+    lds_pack<VEC>(lds + 2 * dim, col, fa);
+    lds_pack<VEC>(lds + 3 * dim, col, fb);
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) to[v] = QBeta{fa[v], fb[v], 0.f, 0.f, 0.f};
-    } else {
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) to[v] = q[it][v];
-    }
+    for (int v = 0; v < VEC; ++v) to[v] = QBeta{fa[v], fb[v], 0.f, 0.f, 0.f};
   };
+  [[maybe_unused]] QBeta qf[VEC];
   // this wavefront's share of the query's negatives: a contiguous range, walked in batches of 64
   const int per_wave = (K + NW - 1) / NW;
   const int kw0 = wave * per_wave;
@@ -854,8 +850,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
           float ge1[NIT][VEC], ge2[NIT][VEC];
 #pragma unroll
           for (int it = 0; it < NIT; ++it) {
-            typename ModelOps<M>::Q qa[VEC];
-            query_at(it, qa);
+            if constexpr (M == mBetaKL) query_features(it, qf);
 #pragma unroll
             for (int v = 0; v < VEC; ++v) {
               w.h[0][it].v[v] = e1[it].v[v];
@@ -863,7 +858,8 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
               ge1[it][v] = ge2[it][v] = 0.f;
               const float x1 = REG ? reg_apply(e1[it].v[v], p) : e1[it].v[v];
               const float x2 = MUL == 2 ? (REG ? reg_apply(e2[it].v[v], p) : e2[it].v[v]) : 0.f;
-              ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, qa[v], ge1[it][v], ge2[it][v]);
+              if constexpr (M == mBetaKL) ModelOps<M>::bwd_e(c.x, c.y, x1, x2, qf[v], ge1[it][v], ge2[it][v]);
+              else ModelOps<M>::bwd_e(model_norm(M, REG) ? c_raw : c.x, c.y, x1, x2, q[it][v], ge1[it][v], ge2[it][v]);
             }
           }
           const int seg = __builtin_amdgcn_readlane(my_ps, j) & 0x7fffffff;
@@ -911,15 +907,15 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
             float ge1[NIT][VEC], ge2[NIT][VEC];
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
-              typename ModelOps<M>::Q qa[VEC];
-              query_at(it, qa);
+              if constexpr (M == mBetaKL) query_features(it, qf);
 #pragma unroll
               for (int v = 0; v < VEC; ++v) {
                 ge1[it][v] = ge2[it][v] = 0.f;
                 const float x1 = REG ? reg_apply(e[s].h[0][it].v[v], p) : e[s].h[0][it].v[v];
                 const float x2 =
                     MUL == 2 ? (REG ? reg_apply(e[s].h[MUL - 1][it].v[v], p) : e[s].h[MUL - 1][it].v[v]) : 0.f;
-                ModelOps<M>::bwd_e(c0, c1, x1, x2, qa[v], ge1[it][v], ge2[it][v]);
+                if constexpr (M == mBetaKL) ModelOps<M>::bwd_e(c0, c1, x1, x2, qf[v], ge1[it][v], ge2[it][v]);
+                else ModelOps<M>::bwd_e(c0, c1, x1, x2, q[it][v], ge1[it][v], ge2[it][v]);
               }
             }
             finish_row<M, VEC, NIT, REG, SINGLES == 2>(A.sink, lane, row, seg, ge1, ge2, e[s], m0[s], v0[s]);
@@ -938,7 +934,7 @@ __global__ __launch_bounds__(NW * 64, SINGLES == 0 ? arithmetic_waves(M, VEC * N
 
   // wavefront partials -> LDS -> fixed-order sum over wavefronts
   float* part = lds + QF * dim;  // [NW][NQ][dim]
-  if constexpr (M == mBetaKL && (SINGLES == 1 || SINGLES == 2)) __syncthreads();   // (query_at)
+  if constexpr (M == mBetaKL && (SINGLES == 1 || SINGLES == 2)) __syncthreads();   // (query_features)
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = lane + 64 * it;
