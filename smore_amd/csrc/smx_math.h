@@ -203,10 +203,10 @@ __device__ __forceinline__ void beta_terms(float a, float b, float& lb, float& p
 // and the logarithms are of numbers around 1.  V and S are polynomials of two steps in 1/y^2 fitted for y >= 3 (largest
 // error 3.9e-9 and 3.2e-9; the first terms left out of the series at y = x + 6: 2.5e-9 and 2.1e-9), so three steps of
 // recurrence do where six are taken above.  BetaE's kernels are bound by the number of their instructions (four cycles each:
-// a wavefront that has issued a transcendental one no longer shares its cycles with another), and this is 69 a feature
-// instead of 105 in the forward.  One feature's divergence has less than half the error (normal rows around 1: 0.66e-6 instead
-// of 1.7e-6).  512 x 512 pairs of 2 x 400 floats: forward 405 -> 358 us, query gradient 330 -> 299 (437 and 384 with a branch
-// per feature and the query's values in registers).  Good in the interval of fast_ok.
+// a wavefront that has issued a transcendental one no longer shares its cycles with another), and this is 71 a feature
+// instead of 105 in the forward.  One feature's divergence has less than a third of the error (normal rows around 1: 0.5e-6
+// instead of 1.7e-6 rms).  512 x 512 pairs of 2 x 400 floats, the forms alone: forward 405 -> 358 us, query gradient 330 -> 299 (437
+// and 384 with a branch per feature and the query's values in registers).  Good in the interval of fast_ok.
 constexpr float kLn2 = 0.693147180559945f;
 constexpr float kBetaConst = 5.14032259e-1f;   // C
 constexpr float kLnBetaConst = -6.65469255e-1f;   // ln C
@@ -337,9 +337,13 @@ __device__ __forceinline__ void trigamma3(float a, float b, float& ta, float& tb
   }
 }
 
-static __device__ __noinline__ SlowTerms trigamma3_any(float a, float b) {
+// psi' of a, b and their sum: in the interval of fast_ok the form of the entity pass, whatever path the row takes.
+static __device__ __noinline__ SlowTerms beta_trigammas_any(float a, float b) {
+  const float sum = a + b;
+  if (fast_ok(fminf(a, b), sum))
+    return SlowTerms{beta_trigamma(beta_arg<true>(a)), beta_trigamma(beta_arg<true>(b)), beta_trigamma(beta_arg<true>(sum)), 0.f};
   float ta, tb, ts;
-  trigamma3(a, b, ta, tb, ts);
+  trigamma3_slow(a, b, ta, tb, ts);
   return SlowTerms{ta, tb, ts, 0.f};
 }
 

@@ -399,7 +399,7 @@ template <> struct ModelOps<mBetaKL> {
       tb = beta_trigamma(beta_arg<true>(e2));
       ts = beta_trigamma(beta_arg<true>(sum));
     } else {
-      const SlowTerms t = trigamma3_any(e1, e2);
+      const SlowTerms t = beta_trigammas_any(e1, e2);
       ta = t.x;
       tb = t.y;
       ts = t.z;
@@ -534,7 +534,7 @@ __device__ __forceinline__ void beta_row_both_grads(const BetaClamp& clamp, cons
       for (int v = 0; v < VEC; ++v) {
         const float ea = row.a[it][v], eb = row.b[it][v];
         O::bwd_q(c0, 0.f, ea, eb, q[v], g1[it][v], g2[it][v]);
-        const SlowTerms t = trigamma3_any(ea, eb);
+        const SlowTerms t = beta_trigammas_any(ea, eb);
         const float s1 = c0 * (ea - q[v].a), s2 = c0 * (eb - q[v].b), common = t.z * (s1 + s2);
         ge1[it][v] = __builtin_fmaf(t.x, s1, -common);
         ge2[it][v] = __builtin_fmaf(t.y, s2, -common);

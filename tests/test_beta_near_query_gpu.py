@@ -180,3 +180,30 @@ def test_ranking_knows_the_digamma_to_an_ulp():
     got = _keys("beta_kl", _dev(np.concatenate([ea, eb], 1)), _dev(qa), _dev(qb), fused.score_params(0.0), _all_ids(1, n))[0]
     error = (got.cpu().numpy().astype(np.float64)[0] - want) / (ea[:, 0] - 40.0)
     assert _rms(error) <= 2.0 ** -19
+
+
+@pytest.mark.parametrize("outside", [0.004, 1500.0])
+@pytest.mark.parametrize("dim", WIDTHS)
+def test_a_feature_outside_the_interval_changes_no_other_gradient_of_its_row(dim, outside):
+    """One pair a query and Adam: rows finished in the stream up to 512 floats a half, by the entity pass beyond."""
+    from smore_amd import fused
+    rng = np.random.default_rng(seed("outside, rows", dim, outside))
+    n = 40
+    qa, qb = (_draw(rng, 0.05, 60.0, (n, dim)) for _ in range(2))
+    rows = np.concatenate([_draw(rng, None, None, (n, dim)), _draw(rng, 1.0, 60.0, (n, dim))], 1)
+    idx = torch.arange(n, device="cuda").reshape(n, 1)
+    q1, q2, gs, params = _dev(qa), _dev(qb), _dev(rng.standard_normal((n, 1))), fused.score_params(60.0)
+    score, plan = torch.zeros_like(gs), fused.build_plan(idx, n)
+    at = rng.integers(0, dim, n)
+    moved = rows.copy()
+    moved[np.arange(n), at] = outside
+    moments = []
+    for t in (rows, moved):
+        table = _dev(t)
+        m, v = torch.zeros_like(table), torch.zeros_like(table)
+        fused.score_backward_fused("beta_kl", plan, table, idx, q1, q2, score, gs, params, m=m, v=v, adam=fused.adam_params(1e-3, 1))
+        moments.append(m)
+    same = torch.ones(n, 2 * dim, dtype=torch.bool, device="cuda")
+    for half in (0, dim):
+        same[torch.arange(n), torch.tensor(at + half)] = False
+    assert torch.equal(moments[0][same], moments[1][same]) and not torch.equal(moments[0], moments[1])
