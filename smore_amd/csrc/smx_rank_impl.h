@@ -206,7 +206,7 @@ __device__ __forceinline__ ScalarRow scalar_row(const float* p) {
 // (the pair's sum is over ea and eb themselves, not over that rounded value).
 // da, db: psi(a) - psi(a + b), psi(b) - psi(a + b).  The forms are those of the scoring kernels (beta_arg), with the poles of psi(a) and
 // psi(b) on their own: at 1/31 to 1/17 these are off by 0.85 of an ulp rms, without by 1.16, in the six-step form by 1.07.  (4 queries
-// among 400,000 rows of 2 x 400 floats: 705, 680 and 707 us.)  The logarithms of ratios, which are psi's as well, meet the row's own
+// among 400,000 rows of 2 x 400 floats: 717, 697 and 730 us.)  The logarithms of ratios, which are psi's as well, meet the row's own
 // a + 2.5 and b + 2.5 in 64 bits.
 __device__ __forceinline__ double log_beta(float a, float b, float& da, float& db) {
 #pragma clang fp contract(off)
